@@ -88,37 +88,39 @@ struct Mma<double> {
 // ------------------------------------------------------------------------------------------
 // One tap, forward, tap-major (mode 2 with wvol == 1 and ld == F): Ap[c][f] = w[f][c], a plain
 // transposition of an F x C matrix -- what a matrix product's left operand needs.  32 x 32
-// tiles through LDS: read along c, written along f, both coalesced.
+// tiles through LDS: read along c, written along f, both coalesced; zeros up to `depth` rows of
+// `ld` values.
 template <typename T>
-__global__ void __launch_bounds__(256) pack_transpose_kernel(const T *__restrict__ w, T *__restrict__ ap, int F, int C) {
+__global__ void __launch_bounds__(256) pack_transpose_kernel(const T *__restrict__ w, T *__restrict__ ap, int F, int C, int ld,
+                                                             int depth) {
   __shared__ T tile[32][33];
   const int c0 = blockIdx.x * 32, f0 = blockIdx.y * 32;
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int f = f0 + ty + 8 * j, c = c0 + tx;
-    if (f < F && c < C) tile[ty + 8 * j][tx] = w[(long long)f * C + c];
+    tile[ty + 8 * j][tx] = f < F && c < C ? w[(long long)f * C + c] : T(0);
   }
   __syncthreads();
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int c = c0 + ty + 8 * j, f = f0 + tx;
-    if (f < F && c < C) ap[(long long)c * F + f] = tile[tx][ty + 8 * j];
+    if (f < ld && c < depth) ap[(long long)c * ld + f] = tile[tx][ty + 8 * j];
   }
 }
 
-// Stride phases as rows (see GemmParams::phase_count): Ap[(e * F + f)][c * phases + phase] = w[f][c][tap of offset e in
-// that phase], zero where the phase has no tap at that offset; taps[e * phases + phase] names the tap (-1: none).
+// Stride phases as rows (see GemmParams::phase_count): Ap[(e * depth + f)][c * phases + phase] = w[f][c][tap of offset e in
+// that phase], zero for f >= F and where the phase has no tap at that offset; taps[e * phases + phase] names the tap (-1: none).
 template <typename T>
 __global__ void __launch_bounds__(256) pack_phase_rows_kernel(const T *__restrict__ w, T *__restrict__ ap, const int *__restrict__ taps,
-                                                              int entries, int phases, int F, int C, int wvol, int ld) {
-  const long long total = (long long)entries * F * ld;
+                                                              int entries, int phases, int F, int depth, int C, int wvol, int ld) {
+  const long long total = (long long)entries * depth * ld;
   for (long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += (long long)gridDim.x * blockDim.x) {
     const int m = (int)(idx % ld);
     const long long row = idx / ld;
-    const int f = (int)(row % F), e = (int)(row / F);
+    const int f = (int)(row % depth), e = (int)(row / depth);
     T v = T(0);
-    if (m < phases * C) {
+    if (m < phases * C && f < F) {
       const int tap = taps[e * phases + m % phases];
       if (tap >= 0) v = w[((long long)f * C + m / phases) * wvol + tap];
     }
@@ -128,9 +130,9 @@ __global__ void __launch_bounds__(256) pack_phase_rows_kernel(const T *__restric
 
 template <typename T>
 __global__ void __launch_bounds__(256) pack_filters_kernel(const T *__restrict__ w, T *__restrict__ ap, int F, int C,
-                                                           int wvol, int mode, int ld) {
+                                                           int wvol, int mode, int ld, int depth) {
   const int M = (mode == 2 || mode == 6) ? F : mode == 3 ? C : mode == 4 ? 3 * C : 3 * F;
-  const int total = (F * C * wvol / M) * ld;
+  const int total = (mode == 4 || mode == 5 ? wvol / 3 : wvol) * depth * ld;
   for (int idx = blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += gridDim.x * blockDim.x) {
     // idx enumerates the packed layout so that stores are coalesced
     const int m = idx % ld;
@@ -141,9 +143,9 @@ __global__ void __launch_bounds__(256) pack_filters_kernel(const T *__restrict__
       const int n = mode == 4 ? C : F;
       const int one = (m / 48) * 16 + m % 16, tap = (m % 48) / 16;
       T v = T(0);
-      if (one < n) {
-        const int f = mode == 4 ? row % F : one, c = mode == 4 ? one : row % C;
-        const int t = (row / (mode == 4 ? F : C)) * 3 + (mode == 4 ? tap : 2 - tap);
+      const int f = mode == 4 ? row % depth : one, c = mode == 4 ? one : row % depth;
+      if (one < n && f < F && c < C) {
+        const int t = (row / depth) * 3 + (mode == 4 ? tap : 2 - tap);
         v = w[((long long)f * C + c) * wvol + t];
       }
       ap[idx] = v;
@@ -156,26 +158,27 @@ __global__ void __launch_bounds__(256) pack_filters_kernel(const T *__restrict__
     int f, c, t;
     if (mode == 2) {
       f = m;
-      c = row % C;
-      t = row / C;
+      c = row % depth;
+      t = row / depth;
     } else if (mode == 6) {
       f = m;
       t = row % wvol;
       c = row / wvol;
     } else if (mode == 3) {
       c = m;
-      f = row % F;
-      t = row / F;
+      f = row % depth;
+      t = row / depth;
     } else if (mode == 4) {
       c = m / 3;
-      f = row % F;
-      t = (row / F) * 3 + m % 3;
+      f = row % depth;
+      t = (row / depth) * 3 + m % 3;
     } else {
       f = m / 3;
-      c = row % C;
-      t = (row / C) * 3 + 2 - m % 3;
+      c = row % depth;
+      t = (row / depth) * 3 + 2 - m % 3;
     }
-    ap[idx] = w[((long long)f * C + c) * wvol + t];
+    // (rows beyond the channels or filters there are: zeros)
+    ap[idx] = f < F && c < C ? w[((long long)f * C + c) * wvol + t] : T(0);
   }
 }
 
@@ -574,15 +577,38 @@ bool fits_buffer_loads(const Geometry &g) {
   const long long elem = g.dtype == MG_F64 ? 8 : 4;
   const long long limit = 1ll << 31;
   return (long long)g.N * g.C * g.xvol * elem < limit && (long long)g.N * g.F * g.gvol * elem < limit &&
-         (long long)(g.F + 3) * (g.C + 3) * g.wvol * elem < limit;  // packed filter rows are padded to 4 values
+         (long long)(g.F + 15) * (g.C + 15) * g.wvol * elem < limit;  // packed filters: whole K tiles of rows, 4 values to a row
 }
 
 // K tile of the gather-GEMMs (positions x filters-or-channels x BK).
 int gemm_bk(int dtype) { return dtype == MG_F64 ? 8 : 16; }
+
+double conv_flops(const Geometry &g) {
+  return 2.0 * (double)g.N * (double)g.F * (double)g.gvol * (double)g.C * (double)g.wvol;
+}
+
+// Channels that the tap-major kernels contract per tap (filters, for the data gradient) for a count
+// of `channels`: the count itself where it fills whole K tiles, else rounded up to whole tiles of 16
+// whose last one has fewer live rows; 0 where the table of rows is the better form: a small problem,
+// or more than a third of dead rows (a product has one tap, and its table rows no structure to use:
+// any count).  MYGRAD_HIP_PAD=0 leaves every awkward count to the table of rows.
+int whole_channels(const Geometry &g, int channels) {
+  if (channels % 16 == 0) return channels;
+  static const bool on = [] {
+    const char *flag = getenv("MYGRAD_HIP_PAD");
+    return !(flag && flag[0] == '0');
+  }();
+  const int up = (channels + 15) / 16 * 16;
+  if (on && conv_flops(g) >= 2.0e8 && (3 * up <= 4 * channels || g.wvol == 1)) return up;
+  return channels % gemm_bk(g.dtype) == 0 ? channels : 0;
+}
 // K tile of a tap-major plan that contracts `channels` channels per tap.  Double precision: 16
 // where the channels allow it -- a K tile of 8 is 64 MFMAs per wave between two barriers, and
 // the barriers then cost a tenth of the time (config 4: forward 122 -> 115 us, dx 130 -> 119 us).
 int tap_bk(int dtype, int channels) { return dtype == MG_F64 && channels % 16 != 0 ? 8 : 16; }
+
+// KTile::dead of a K tile of `bk` rows with `left` channels from its first row on.
+unsigned dead_rows(int bk, int left) { return left >= bk ? 0u : (unsigned)(((1ull << bk) - 1) & ~((1ull << left) - 1)); }
 
 struct Plan {
   void *blob = nullptr;  // one device allocation holding every table below
@@ -607,6 +633,8 @@ struct Plan {
   ShareFix *share_fix = nullptr;
   int share_grid = 0, share_slots = 0, share_fixes = 0;
   bool tap_major = false;  // which kernel family the tables are for
+  bool ragged = false;     // tap-major: some K tile has dead rows (KTile::dead)
+  int depth = 0;           // tap-major: rows of the packed filters per tap (whole_channels)
   bool single_dense_phase = false;  // positions enumerate the destination tensor in order
   bool table_rows = false;          // tap-major kernel whose K tiles are rows of the gather table (channel count no multiple of the K tile)
   int table_count = 0;              // data gradient on table rows: rows of the (padded) table = rows of the packed filters
@@ -687,14 +715,26 @@ int check_desc(const mg_conv_desc *d, Geometry *g) {
   return MG_OK;
 }
 
-// Largest row tile whose round-up waste stays small.
-int pick_bm(int M) {
-  const int cands[4] = {128, 64, 32, 16};
-  for (int c : cands) {
-    const int padded = (int)ceil_div(M, c) * c;
-    if (padded - M <= M / 8) return c;
+// Row tile: the one whose rounded-up rows cost least, at the relative cost of a row in a tile of that
+// height (`thirds`: the heights that are multiples of 48 are built).  The costs are the rates of the
+// tiles on row counts that they divide, 64 channels, 3x3 at 56x56 and 9 taps along 9409 positions:
+// single precision 125 / 122 / 124 / 119 / 115 / 92 TFLOP/s for 128 / 96 / 64 / 48 / 32 / 16 rows,
+// double 54 / 54 / 51 / 48 / 52 / 40.  (45 rows: 86 -> 113 TFLOP/s with 48 instead of three times 16,
+// 83 rows: 81 -> 106 with 96 instead of six times 16, 160 rows: 107 -> 117 with 32 instead of 64.)
+int pick_bm(int M, bool thirds, bool f64) {
+  struct Rows {
+    int bm;
+    double cost, cost64;
+  };
+  static const Rows cands[] = {{128, 1.00, 1.00}, {96, 1.02, 1.01}, {64, 1.00, 1.06}, {48, 1.04, 1.11}, {32, 1.08, 1.05}, {16, 1.36, 1.34}};
+  int best = 16;
+  double least = 0;
+  for (const Rows &c : cands) {
+    if (c.bm % 48 == 0 && !thirds) continue;
+    const double cost = (double)(ceil_div(M, c.bm) * c.bm) * (f64 ? c.cost64 : c.cost);
+    if (least == 0 || cost < least) best = c.bm, least = cost;
   }
-  return 16;
+  return best;
 }
 
 template <typename K>
@@ -711,8 +751,10 @@ int resident_blocks(K kernel, int threads) {
 #define MG_GEMM_SHAPES(T, X) \
   X(T, 128, 128, 64, 64)     \
   X(T, 128, 64, 64, 32)      \
+  X(T, 96, 128, 48, 64)      \
   X(T, 64, 256, 64, 64)      \
   X(T, 64, 128, 32, 64)      \
+  X(T, 48, 256, 48, 64)      \
   X(T, 32, 256, 32, 64)      \
   X(T, 32, 128, 16, 64)      \
   X(T, 16, 256, 16, 64)
@@ -788,12 +830,12 @@ TileChoice choose_tile(int M, const std::vector<long long> &phase_npos, int min_
     double penalty;  // relative cost of a flop in this tile shape
     bool tap_only;
   };
-  static const Cfg plain[] = {{128, 128, 1.00, false}, {128, 64, 1.05, true}, {64, 256, 1.00, false}, {64, 128, 1.08, true},
-                              {32, 256, 1.00, false},  {32, 128, 1.10, true}, {16, 256, 1.00, false}};
+  static const Cfg plain[] = {{128, 128, 1.00, false}, {128, 64, 1.05, true}, {96, 128, 1.00, true},   {64, 256, 1.00, false},
+                              {64, 128, 1.08, true},   {48, 256, 1.00, true},  {32, 256, 1.00, false},  {32, 128, 1.10, true}, {16, 256, 1.00, false}};
   static const Cfg fused2[] = {{128, 64, 1.05, true}, {64, 128, 1.08, true}, {32, 256, 1.00, true}, {16, 256, 1.00, true}};
   static const Cfg fused4[] = {{64, 64, 1.10, true}, {32, 128, 1.10, true}, {16, 256, 1.00, true}};
   const Cfg *cfgs = nph == 4 ? fused4 : nph == 2 ? fused2 : plain;
-  const int ncfgs = nph == 4 ? 3 : nph == 2 ? 4 : 7;
+  const int ncfgs = nph == 4 ? 3 : nph == 2 ? 4 : 9;
   // MYGRAD_HIP_TILE="rows,positions[,blocks per unit]" (diagnostics and the tests of every tile shape;
   // read whenever a plan is built, and part of the plan's key): only that tile shape, where it exists
   struct Forced {
@@ -813,7 +855,7 @@ TileChoice choose_tile(int M, const std::vector<long long> &phase_npos, int min_
   for (int ci = 0; ci < ncfgs; ++ci)
     forced_fits |= cfgs[ci].bm == forced.bm && cfgs[ci].bn == forced.bn && (!cfgs[ci].tap_only || tap_major) &&
                    !(tap_major && elem == 8 && cfgs[ci].bn * cfgs[ci].bm >= 128 * 128);  // (no such double-precision tile)
-  const int bm = forced_fits ? forced.bm : nph == 4 ? std::min(pick_bm(M), 64) : pick_bm(M);
+  const int bm = forced_fits ? forced.bm : nph == 4 ? std::min(pick_bm(M, false, false), 64) : pick_bm(M, tap_major && nph == 1, elem == 8);
   const int cus = runtime().props.multiProcessorCount;
   TileChoice best{};
   double best_cost = 0;
@@ -1300,7 +1342,7 @@ void thin_tables(Plan &pl, Tables &t, const std::vector<ThinUse> &uses, int nph,
 
 int build_fwd_plan(const Geometry &g, Plan &pl) {
   Tables t;
-  if ((g.F <= 4 || (g.F <= 1024 && g.C % gemm_bk(g.dtype) != 0)) && thin_applies(g, g.F, (long long)g.N * g.gvol, (long long)g.C * g.wvol, 1)) {
+  if ((g.F <= 4 || (g.F <= 1024 && whole_channels(g, g.C) == 0)) && thin_applies(g, g.F, (long long)g.N * g.gvol, (long long)g.C * g.wvol, 1)) {
     // up to four filters, or a first layer (channels that fill no K tile; passes of 64 filters), in
     // single precision: one output position per lane
     const int qs[3] = {g.X[1] * g.X[2], g.X[2], 1};
@@ -1323,7 +1365,9 @@ int build_fwd_plan(const Geometry &g, Plan &pl) {
     pl.bm = 4, pl.bn = 256;
     return upload_plan(pl, t);
   }
-  pl.tap_major = g.C % gemm_bk(g.dtype) == 0 && fits_buffer_loads(g);
+  pl.depth = whole_channels(g, g.C);
+  pl.ragged = pl.depth > g.C;
+  pl.tap_major = pl.depth != 0 && fits_buffer_loads(g);
   // Channels that do not fill K tiles (a first layer's one or three): the same kernel, its K
   // tiles 16 rows of the gather table each -- unless the problem is tiny (few launches matter
   // more) or MYGRAD_HIP_TABLE_ROWS=0 asks for the plain table-driven kernel.
@@ -1333,12 +1377,12 @@ int build_fwd_plan(const Geometry &g, Plan &pl) {
   }();
   pl.table_rows = rows_on && !pl.tap_major && fits_buffer_loads(g) && !tiny_table(g, g.F, (long long)g.C * g.wvol);
   if (pl.table_rows) pl.tap_major = true;
-  const int bk = pl.table_rows ? 16 : pl.tap_major ? tap_bk(g.dtype, g.C) : gemm_bk(g.dtype);
+  const int bk = pl.table_rows ? 16 : pl.tap_major ? tap_bk(g.dtype, pl.depth) : gemm_bk(g.dtype);
   pl.bk = bk;
   pl.single_dense_phase = true;
   {
     const long long ktiles = pl.table_rows ? ceil_div((long long)g.C * g.wvol, bk)
-                             : pl.tap_major ? g.wvol * (g.C / bk) : ceil_div((long long)g.C * g.wvol, bk);
+                             : pl.tap_major ? g.wvol * (pl.depth / bk) : ceil_div((long long)g.C * g.wvol, bk);
     const TileChoice tc = choose_tile(g.F, {(long long)g.N * g.gvol}, (int)ktiles, pl.tap_major, g.dtype == MG_F64 ? 8 : 4, 1, bk);
     pl.bm = tc.bm, pl.bn = tc.bn, pl.m_tiles = tc.m_tiles, pl.full_tiles = tc.full_tiles, pl.tail_split = tc.tail_split, pl.blocks_per_cu = tc.blocks_per_cu;
     deepen_if_tiny(g, pl);
@@ -1371,17 +1415,18 @@ int build_fwd_plan(const Geometry &g, Plan &pl) {
     pl.pos_blocks = (int)ceil_div(ph.npos, pl.bn);
     return upload_plan(pl, t);
   }
-  if (pl.tap_major && fold_applies(g, g.F, g.C)) {
+  if (pl.tap_major && fold_applies(g, g.F, pl.depth)) {
     // rows (filter, tap of the last axis); K tiles over the taps of the other axes
     const int qs[3] = {g.X[1] * g.X[2], g.X[2], 1};
     for (int c0 = 0; c0 < g.C; c0 += bk)
       for (int t0 = 0; t0 < g.W[0]; ++t0)
         for (int t1 = 0; t1 < g.W[1]; ++t1) {
           KTile e{};
+          e.dead = dead_rows(bk, g.C - c0);
           e.d0 = t0 * g.D[0] - g.P[0];
           e.d1 = t1 * g.D[1] - g.P[1];
           e.d2 = 0;
-          e.a_row0 = (t0 * g.W[1] + t1) * g.C + c0;
+          e.a_row0 = (t0 * g.W[1] + t1) * pl.depth + c0;
           e.coff = (int)(c0 * g.xvol) + e.d0 * qs[0] + e.d1 * qs[1];
           t.ktiles.push_back(e);
         }
@@ -1404,10 +1449,11 @@ int build_fwd_plan(const Geometry &g, Plan &pl) {
           for (int t2 = 0; t2 < g.W[2]; ++t2) {
             const int tflat = (t0 * g.W[1] + t1) * g.W[2] + t2;
             KTile e{};
+            e.dead = dead_rows(bk, g.C - c0);
             e.d0 = t0 * g.D[0] - g.P[0];
             e.d1 = t1 * g.D[1] - g.P[1];
             e.d2 = t2 * g.D[2] - g.P[2];
-            e.a_row0 = tflat * g.C + c0;
+            e.a_row0 = tflat * pl.depth + c0;
             e.coff = (int)(c0 * g.xvol) + e.d0 * qs[0] + e.d1 * qs[1] + e.d2 * qs[2];
             t.ktiles.push_back(e);
           }
@@ -1437,12 +1483,14 @@ int build_dgrad_plan(const Geometry &g, Plan &pl) {
   // with its deep K tiles needs neither packed filters nor a pass over partial sums.  (Measured,
   // whole steps: 3 channels 38.5 -> 28 us; with 16 channels the tap-major kernels are 4 us
   // ahead, and with 32 or 64 the table-driven kernel's few, long-running blocks cost 2 - 5 x.)
-  pl.tap_major = g.F % gemm_bk(g.dtype) == 0 && fits_buffer_loads(g) && !(tiny_table(g, g.C, (long long)g.F * g.wvol) && g.C <= 8);
+  pl.depth = whole_channels(g, g.F);
+  pl.ragged = pl.depth > g.F;
+  pl.tap_major = pl.depth != 0 && fits_buffer_loads(g) && !(tiny_table(g, g.C, (long long)g.F * g.wvol) && g.C <= 8);
   // filter counts that fill no K tile (10, 20, ...): the tap-major kernel on rows of the gather
   // table, as in the forward pass (MYGRAD_HIP_TABLE_ROWS=0: the plain table-driven kernel)
-  pl.table_rows = table_rows_on() && g.F % gemm_bk(g.dtype) != 0 && fits_buffer_loads(g) && !tiny_table(g, g.C, (long long)g.F * g.wvol);
+  pl.table_rows = table_rows_on() && pl.depth == 0 && fits_buffer_loads(g) && !tiny_table(g, g.C, (long long)g.F * g.wvol);
   if (pl.table_rows) pl.tap_major = true;
-  const int bk = pl.table_rows ? 16 : pl.tap_major ? tap_bk(g.dtype, g.F) : gemm_bk(g.dtype);
+  const int bk = pl.table_rows ? 16 : pl.tap_major ? tap_bk(g.dtype, pl.depth) : gemm_bk(g.dtype);
   pl.bk = bk;
   pl.single_dense_phase = g.S[0] == 1 && g.S[1] == 1 && g.S[2] == 1;
   const int gs[3] = {g.G[1] * g.G[2], g.G[2], 1};
@@ -1529,17 +1577,18 @@ int build_dgrad_plan(const Geometry &g, Plan &pl) {
   // matrix pipes -- and the epilogue adds the three rows of a channel, shifted along the last
   // axis, into dx.  A wave's 64 positions must be whole rows: rows of up to 64 positions, padded
   // to a power of two.
-  if (fold_applies(g, g.C, g.F) && pl.tap_major && !pl.table_rows && nphase == 1 && found.size() == 1) {
+  if (fold_applies(g, g.C, pl.depth) && pl.tap_major && !pl.table_rows && nphase == 1 && found.size() == 1) {
     const PhaseTaps &pt = found[0];
     Phase ph = pt.ph;
     for (int f0 = 0; f0 < g.F; f0 += bk)
       for (size_t a = 0; a < pt.taps[0].size(); ++a)
         for (size_t b = 0; b < pt.taps[1].size(); ++b) {
           KTile e{};
+          e.dead = dead_rows(bk, g.F - f0);
           e.d0 = pt.offs[0][a];
           e.d1 = pt.offs[1][b];
           e.d2 = 0;
-          e.a_row0 = (pt.taps[0][a] * g.W[1] + pt.taps[1][b]) * g.F + f0;
+          e.a_row0 = (pt.taps[0][a] * g.W[1] + pt.taps[1][b]) * pl.depth + f0;
           e.coff = (int)(f0 * g.gvol) + e.d0 * gs[0] + e.d1 * gs[1];
           t.ktiles.push_back(e);
         }
@@ -1592,8 +1641,9 @@ int build_dgrad_plan(const Geometry &g, Plan &pl) {
     for (int f0 = 0; f0 < g.F; f0 += bk)  // filter block outermost: its offsets share a neighbourhood of grad
       for (int e = 0; e < entries; ++e) {
         KTile kt{};
+        kt.dead = dead_rows(bk, g.F - f0);
         kt.d0 = offsets[e][0], kt.d1 = offsets[e][1], kt.d2 = offsets[e][2];
-        kt.a_row0 = e * g.F + f0;
+        kt.a_row0 = e * pl.depth + f0;
         kt.coff = (int)(f0 * g.gvol) + kt.d0 * gs[0] + kt.d1 * gs[1] + kt.d2 * gs[2];
         t.ktiles.push_back(kt);
       }
@@ -1649,7 +1699,7 @@ int build_dgrad_plan(const Geometry &g, Plan &pl) {
     pl.nph = (int)nphase;
     // Four phases share a tile's time: a K tile of 16 would be 16 MFMAs per wave between two
     // barriers.  With 32 filters per K tile the barriers cost half as much.
-    const int fbk = nphase == 4 && g.F % 32 == 0 && deep_fused_on() ? 32 : bk;
+    const int fbk = nphase == 4 && pl.depth % 32 == 0 && deep_fused_on() ? 32 : bk;
     pl.bk = fbk;
     Phase coarse{};
     long long total_ktiles = 0;
@@ -1674,10 +1724,11 @@ int build_dgrad_plan(const Geometry &g, Plan &pl) {
             for (size_t c = 0; c < pt.taps[2].size(); ++c) {
               const int tflat = (pt.taps[0][a] * g.W[1] + pt.taps[1][b]) * g.W[2] + pt.taps[2][c];
               KTile e{};
+              e.dead = dead_rows(fbk, g.F - f0);
               e.d0 = pt.offs[0][a];
               e.d1 = pt.offs[1][b];
               e.d2 = pt.offs[2][c];
-              e.a_row0 = tflat * g.F + f0;
+              e.a_row0 = tflat * pl.depth + f0;
               e.coff = (int)(f0 * g.gvol) + e.d0 * gs[0] + e.d1 * gs[1] + e.d2 * gs[2];
               t.ktiles.push_back(e);
             }
@@ -1714,7 +1765,7 @@ int build_dgrad_plan(const Geometry &g, Plan &pl) {
     for (const PhaseTaps &pt : found) {
       npos.push_back(pt.ph.npos);
       const long long ntaps = (long long)pt.taps[0].size() * pt.taps[1].size() * pt.taps[2].size();
-      min_ktiles = std::min(min_ktiles, pl.tap_major && !pl.table_rows ? ntaps * (g.F / bk) : ceil_div(ntaps * g.F, bk));
+      min_ktiles = std::min(min_ktiles, pl.tap_major && !pl.table_rows ? ntaps * (pl.depth / bk) : ceil_div(ntaps * g.F, bk));
     }
     long long all_ktiles = 0, all_pos = 0;
     for (const PhaseTaps &pt : found) {
@@ -1769,10 +1820,11 @@ int build_dgrad_plan(const Geometry &g, Plan &pl) {
             for (size_t c = 0; c < pt.taps[2].size(); ++c) {
               const int tflat = (pt.taps[0][a] * g.W[1] + pt.taps[1][b]) * g.W[2] + pt.taps[2][c];
               KTile e{};
+              e.dead = dead_rows(bk, g.F - f0);
               e.d0 = pt.offs[0][a];
               e.d1 = pt.offs[1][b];
               e.d2 = pt.offs[2][c];
-              e.a_row0 = tflat * g.F + f0;
+              e.a_row0 = tflat * pl.depth + f0;
               e.coff = (int)(f0 * g.gvol) + e.d0 * gs[0] + e.d1 * gs[1] + e.d2 * gs[2];
               t.ktiles.push_back(e);
             }
@@ -1806,11 +1858,33 @@ int build_dgrad_plan(const Geometry &g, Plan &pl) {
 #define MG_WGRAD_SHAPES(T, X)                                                          \
   X(T, 128, 128, (sizeof(T) == 8 ? 16 : 32), 64, 64)                                   \
   X(T, 64, 64, (sizeof(T) == 8 ? 32 : 64), 32, 32)                                     \
+  X(T, 48, 64, (sizeof(T) == 8 ? 32 : 64), 48, 16)                                     \
   X(T, 32, 128, (sizeof(T) == 8 ? 16 : 32), 32, 32)                                    \
   X(T, 32, 64, (sizeof(T) == 8 ? 32 : 64), 32, 16)                                     \
   X(T, 16, 64, (sizeof(T) == 8 ? 32 : 64), 16, 16)
 
 // Blocks of the filter-gradient kernel that fit on one compute unit at a time.
+// Row tile of the filter gradient for F filters, at most `limit` rows: the one whose rounded-up rows
+// cost least at the relative cost of a row (the last tile is moved back to end with the last filter, so
+// a tile has no more rows than there are filters).  The costs are the tiles' rates on filter counts
+// that they divide: single precision 122 / 125 / 117 / 109 / 80 TFLOP/s with 128 / 64 / 48 / 32 / 16 rows, double
+// 50 / 50 / 45 / 45 / 36 (83 filters: 71 TFLOP/s on 16 rows, 94 on 32; 80 filters: 78 and 91).
+int wgrad_rows(int F, int limit) {
+  struct Rows {
+    int bm;
+    double cost;
+  };
+  static const Rows cands[] = {{128, 1.00}, {64, 1.00}, {48, 1.06}, {32, 1.12}, {16, 1.50}};
+  int best = 0;
+  double least = 0;
+  for (const Rows &c : cands) {
+    if (F < c.bm || c.bm > limit) continue;
+    const double cost = (double)(ceil_div(F, c.bm) * c.bm) * c.cost;
+    if (least == 0 || cost < least) best = c.bm, least = cost;
+  }
+  return best;
+}
+
 // Tile shapes that only the table-row mode of the tap-major filter-gradient kernel has.
 #define MG_WGRAD_TABLE_SHAPES(T, X)                \
   X(T, 64, 80, (sizeof(T) == 8 ? 32 : 64), 16, 80) \
@@ -1825,7 +1899,7 @@ int wgrad_blocks_per_cu(int bm, int bn, bool tap_major) {
 #define MG_OCC(TT, BM, BN, BK, WM, WN)                                                     \
   if (bm == BM && bn == BN) {                                                              \
     if (tap_major) return resident_blocks(tap_wgrad_kernel<TT, BM, BN, BK, WM, WN, true>, 512);  \
-    if constexpr (BN == 64) return resident_blocks(wgrad_kernel<TT, BM, BN, BK, WM, WN>, 256); \
+    if constexpr (BN == 64 && BM != 48) return resident_blocks(wgrad_kernel<TT, BM, BN, BK, WM, WN>, 256); \
   }
   MG_WGRAD_SHAPES(T, MG_OCC)
 #undef MG_OCC
@@ -1895,7 +1969,12 @@ int build_pos_table(const Geometry &g, Plan &pl) {
 int build_wgrad_plan(const Geometry &g, Plan &pl) {
   Tables t;
   const bool f64 = g.dtype == MG_F64;
-  const long long ct = (long long)g.C * g.wvol;
+  // tap-major columns: whole groups of 16 channels per tap (the last group moved back, see WGroup),
+  // which takes 16 channels to move in
+  const bool ragged_c = g.C % 16 != 0 && g.C >= 16 && whole_channels(g, g.C) % 16 == 0 && whole_channels(g, g.C) != 0;
+  const bool whole_c = g.C % 16 == 0 || ragged_c;
+  pl.depth = ragged_c ? whole_channels(g, g.C) : g.C;
+  long long ct = (long long)pl.depth * g.wvol;
   const long long kpos = (long long)g.N * g.gvol;
   const int cus = runtime().props.multiProcessorCount;
   // Split K so that all blocks are resident at once (one round: no half-empty second
@@ -1925,7 +2004,8 @@ int build_wgrad_plan(const Geometry &g, Plan &pl) {
     }
     return std::max<long long>(1, std::min(slots / tiles, max_splits));
   };
-  // Tap-major candidates in the order of preference: the first shape wins that divides F, wastes
+  // Tap-major candidates in the order of preference: the first shape wins that has the row tile for F
+  // filters (wgrad_rows), wastes
   // little on padding the columns to whole tiles and still fills most block slots of the device
   // with tiles x K splits.  128 x 128 re-reads grad and x least.  With 64 filters the tile is square
   // with the K tile 64 deep (half the barriers, one column group per gathering thread): tiles of
@@ -1935,7 +2015,7 @@ int build_wgrad_plan(const Geometry &g, Plan &pl) {
   struct Cand {
     int bm, bn, bk;
   };
-  const Cand cands[] = {{128, 128, f64 ? 16 : 32}, {64, 64, f64 ? 32 : 64}, {32, 128, f64 ? 16 : 32},
+  const Cand cands[] = {{128, 128, f64 ? 16 : 32}, {64, 64, f64 ? 32 : 64}, {48, 64, f64 ? 32 : 64}, {32, 128, f64 ? 16 : 32},
                         {32, 64, f64 ? 32 : 64},   {16, 64, f64 ? 32 : 64}};
   long long best_splits = 1;
   pl.bm = 0;
@@ -1945,22 +2025,26 @@ int build_wgrad_plan(const Geometry &g, Plan &pl) {
   if (const char *v = getenv("MYGRAD_HIP_WGRAD_TILE")) sscanf(v, "%d,%d", &forced_bm, &forced_bn);
   bool forced = false;
   for (const Cand &c : cands)
-    forced |= c.bm == forced_bm && c.bn == forced_bn && g.F % c.bm == 0 && !(c.bm == 32 && c.bn == 128 && !f64);
-  if (g.C % 16 == 0 && fits_buffer_loads(g)) {
+    forced |= c.bm == forced_bm && c.bn == forced_bn && g.F >= c.bm && !(c.bm == 32 && c.bn == 128 && !f64);
+  if (whole_c && fits_buffer_loads(g)) {
+    int limit = 128;
     for (const Cand &c : cands) {
       if (forced && (c.bm != forced_bm || c.bn != forced_bn)) continue;
-      if (g.F % c.bm != 0) continue;
+      if (!forced && wgrad_rows(g.F, limit) != c.bm) continue;
       // 32x64 double-precision tiles are bound by LDS reads (the 4x4x4 MFMA takes an operand
       // per 512 flops); the wider tile halves them per flop and is worth more padding.
       // In single precision 32x128 measured slower than 32x64.
       if (c.bm == 32 && c.bn == 128 && !f64) continue;
-      const long long col_tiles = ceil_div(ct, c.bn), row_tiles = g.F / c.bm;
+      const long long col_tiles = ceil_div(ct, c.bn), row_tiles = ceil_div(g.F, c.bm);
       const long long splits = splits_for(c.bm, c.bn, c.bk, true);
       if (c.bn > 64 && !forced) {
         const int per_cu = f64 ? wgrad_blocks_per_cu<double>(c.bm, c.bn, true) : wgrad_blocks_per_cu<float>(c.bm, c.bn, true);
         const double waste = (double)(col_tiles * c.bn - ct) / (double)ct;
         const double filled = (double)(col_tiles * row_tiles * splits) / ((double)per_cu * cus);
-        if (waste > (c.bm == 32 ? 0.15 : 0.12) || filled < 0.75) continue;
+        if (waste > (c.bm == 32 ? 0.15 : 0.12) || filled < 0.75) {
+          limit = std::min(limit, c.bm == 128 ? 64 : limit);
+          continue;
+        }
       }
       best_splits = splits;
       pl.bm = c.bm, pl.bn = c.bn, pl.bk = c.bk;
@@ -1969,6 +2053,8 @@ int build_wgrad_plan(const Geometry &g, Plan &pl) {
   }
   pl.tap_major = pl.bm != 0;
   if (!pl.tap_major) {
+    pl.depth = g.C;
+    ct = (long long)g.C * g.wvol;
     // Channels that fill no group of 16 columns: the tap-major kernel with one table row per
     // column (64-column tiles, filters in whole row tiles), unless the problem is tiny or
     // MYGRAD_HIP_TABLE_ROWS=0 asks for the plain table-driven kernel.
@@ -2015,7 +2101,7 @@ int build_wgrad_plan(const Geometry &g, Plan &pl) {
       WGroup e{};
       const long long col = gi * 16;  // group gi = (channel block, tap), taps innermost
       if (col < ct) {
-        const int tflat = (int)(gi % g.wvol), c0 = (int)(gi / g.wvol) * 16;
+        const int tflat = (int)(gi % g.wvol), c0 = std::min((int)(gi / g.wvol) * 16, g.C - 16);
         const int t2 = tflat % g.W[2], t1 = (tflat / g.W[2]) % g.W[1], t0 = tflat / (g.W[2] * g.W[1]);
         e.d0 = t0 * g.D[0] - g.P[0];
         e.d1 = t1 * g.D[1] - g.P[1];
@@ -2074,8 +2160,10 @@ int get_plan(ConvOp op, const mg_conv_desc *d, const Geometry &g, Plan **out) {
   return MG_OK;
 }
 
-template <typename T, int BM, int BN, int BK, int WM, int WN, int NPH = 1, bool FOLD = false, bool ROWS = false>
+template <typename T, int BM, int BN, int BK, int WM, int WN, int NPH = 1, bool FOLD = false, bool ROWS = false, bool DEAD = false>
 void launch_gemm(GemmParams &gp, const Plan &pl, hipStream_t s) {
+  if constexpr (!DEAD && !ROWS && tap_gemm_dead_apart(BM, BN, NPH, (int)sizeof(T)))
+    if (pl.ragged) return launch_gemm<T, BM, BN, BK, WM, WN, NPH, FOLD, ROWS, true>(gp, pl, s);
   if (pl.tap_major) {
     const long long tiles = (long long)pl.pos_blocks * pl.m_tiles;
     const long long tail_tiles = tiles - pl.full_tiles;
@@ -2084,7 +2172,7 @@ void launch_gemm(GemmParams &gp, const Plan &pl, hipStream_t s) {
     if (pl.share_grid > 0) {
       // whole tiles b, b + grid, ... and then one even share of the remaining tiles' K tiles per block
       gp.items = pl.full_tiles;
-      hipLaunchKernelGGL((tap_gemm_kernel<T, BM, BN, BK, WM, WN, NPH, FOLD, ROWS>), dim3((unsigned)pl.share_grid), dim3(512), 0, s, gp);
+      hipLaunchKernelGGL((tap_gemm_kernel<T, BM, BN, BK, WM, WN, NPH, FOLD, ROWS, DEAD>), dim3((unsigned)pl.share_grid), dim3(512), 0, s, gp);
       if (pl.share_fixes > 0)
         hipLaunchKernelGGL((tail_fixup_kernel<T, BM, BN, NPH>), dim3((unsigned)ceil_div(BM * BN, 256), (unsigned)pl.share_fixes),
                            dim3(256), 0, s, gp);
@@ -2099,11 +2187,11 @@ void launch_gemm(GemmParams &gp, const Plan &pl, hipStream_t s) {
     }();
     const int c = pl.m_tiles;
     gp.xcd_chunk = chunks_on && tap_gemm_streams(BM, (int)sizeof(T)) && grid == slots && (c == 2 || c == 4 || c == 8) && grid % (8 * c) == 0 ? c : 1;
-    hipLaunchKernelGGL((tap_gemm_kernel<T, BM, BN, BK, WM, WN, NPH, FOLD, ROWS>), dim3((unsigned)grid), dim3(512), 0, s, gp);
+    hipLaunchKernelGGL((tap_gemm_kernel<T, BM, BN, BK, WM, WN, NPH, FOLD, ROWS, DEAD>), dim3((unsigned)grid), dim3(512), 0, s, gp);
     if (tail_tiles > 0)
       hipLaunchKernelGGL((tail_fixup_kernel<T, BM, BN, NPH>), dim3((unsigned)ceil_div(BM * BN, 256), (unsigned)tail_tiles),
                          dim3(256), 0, s, gp);
-  } else if constexpr (NPH == 1 && !FOLD && !ROWS) {
+  } else if constexpr (NPH == 1 && !FOLD && !ROWS && !DEAD && BM % 48 != 0) {
     const dim3 grid((unsigned)pl.pos_blocks, (unsigned)pl.m_tiles);
     hipLaunchKernelGGL((gather_gemm_kernel<T, BM, BN, BK, WM, WN>), grid, dim3(256), 0, s, gp);
   }
@@ -2254,12 +2342,12 @@ int folded_ld(int n) {
 }
 
 template <typename T>
-int pack_filters(const Geometry &g, const void *w, int mode, void **packed, size_t extra = 0, void **behind = nullptr) {
+int pack_filters(const Geometry &g, const void *w, int mode, int depth, void **packed, size_t extra = 0, void **behind = nullptr) {
   const int M = (mode == 2 || mode == 6) ? g.F : mode == 3 ? g.C : mode == 4 ? 3 * g.C : 3 * g.F;
   const int ld = mode == 4 || mode == 5 ? folded_ld<T>(M / 3) : packed_ld(M, true);
-  const size_t count = (size_t)g.F * g.C * g.wvol / M * ld;
+  const size_t count = (size_t)(mode == 4 || mode == 5 ? g.wvol / 3 : g.wvol) * depth * ld;
   const size_t packed_bytes = (count * sizeof(T) + 255) & ~size_t(255);
-  if (mode == 3 && g.wvol == 1 && ld == g.C && reinterpret_cast<uintptr_t>(w) % 16 == 0) {
+  if (mode == 3 && g.wvol == 1 && ld == g.C && depth == g.F && reinterpret_cast<uintptr_t>(w) % 16 == 0) {
     // one tap, input gradient: the packed layout [f][c] is w's own, nothing to do
     void *scratch = nullptr;
     if (int rc = workspace(extra, &scratch)) return rc;
@@ -2269,18 +2357,18 @@ int pack_filters(const Geometry &g, const void *w, int mode, void **packed, size
   }
   if (int rc = workspace(packed_bytes + extra, packed)) return rc;
   if (behind) *behind = static_cast<char *>(*packed) + packed_bytes;
-  if (mode == 2 && g.wvol == 1 && ld == g.F) {
+  if (mode == 2 && g.wvol == 1) {
     // one tap, forward: a transposition of the F x C matrix
     ScopedTiming timed(TAG_PACK_FILTERS);
-    hipLaunchKernelGGL(pack_transpose_kernel<T>, dim3((unsigned)ceil_div(g.C, 32), (unsigned)ceil_div(g.F, 32)), dim3(256), 0,
-                       runtime().stream, static_cast<const T *>(w), static_cast<T *>(*packed), (int)g.F, (int)g.C);
+    hipLaunchKernelGGL(pack_transpose_kernel<T>, dim3((unsigned)ceil_div(depth, 32), (unsigned)ceil_div(ld, 32)), dim3(256), 0,
+                       runtime().stream, static_cast<const T *>(w), static_cast<T *>(*packed), (int)g.F, (int)g.C, ld, depth);
     MG_HIP(hipGetLastError());
     return MG_OK;
   }
   const unsigned blocks = (unsigned)std::min<long long>(ceil_div((long long)count, 256), 4096);
   ScopedTiming timed(TAG_PACK_FILTERS);
   hipLaunchKernelGGL(pack_filters_kernel<T>, dim3(blocks), dim3(256), 0, runtime().stream, static_cast<const T *>(w),
-                     static_cast<T *>(*packed), g.F, g.C, (int)g.wvol, mode, ld);
+                     static_cast<T *>(*packed), g.F, g.C, (int)g.wvol, mode, ld, depth);
   MG_HIP(hipGetLastError());
   return MG_OK;
 }
@@ -2355,7 +2443,7 @@ int conv_fwd_impl(const Geometry &g, const Plan &pl, const void *x, const void *
   void *partial = nullptr;
   if (!pl.tap_major) {
     packed = const_cast<void *>(w);  // read in place: row k = (c, taps) of filter m lies at w[m * C*taps + k]
-  } else if (int rc = pack_filters<T>(g, w, pl.table_rows ? 6 : pl.fold_row ? 5 : 2, &packed, tail_bytes(pl, sizeof(T)), &partial)) {
+  } else if (int rc = pack_filters<T>(g, w, pl.table_rows ? 6 : pl.fold_row ? 5 : 2, pl.table_rows ? g.C : pl.depth, &packed, tail_bytes(pl, sizeof(T)), &partial)) {
     return rc;
   }
   GemmParams gp{};
@@ -2379,7 +2467,7 @@ int conv_fwd_impl(const Geometry &g, const Plan &pl, const void *x, const void *
   gp.src_nstride = (long long)g.C * g.xvol;
   gp.dst_nstride = (long long)g.F * g.gvol;
   gp.a_ld = pl.fold_row ? folded_ld<T>(g.F) : packed_ld(g.F, pl.tap_major);
-  gp.a_bytes = (unsigned)((size_t)g.C * (pl.fold_row ? g.wvol / 3 : g.wvol) * gp.a_ld * sizeof(T));
+  gp.a_bytes = (unsigned)((size_t)(pl.tap_major && !pl.table_rows ? pl.depth : g.C) * (pl.fold_row ? g.wvol / 3 : g.wvol) * gp.a_ld * sizeof(T));
   gp.src_bytes = pl.tap_major ? (unsigned)((size_t)g.N * g.C * g.xvol * sizeof(T)) : 0;
   return run_gemm<T>(gp, pl, TAG_CONV_FWD, runtime().stream);
 }
@@ -2424,15 +2512,15 @@ int conv_dgrad_impl(const Geometry &g, const Plan &pl, const void *grad, const v
     }
   } else if (pl.phase_rows) {
     const int ld = packed_ld(pl.phase_count * g.C, true);
-    const size_t packed_bytes = ((size_t)pl.table_count * g.F * ld * sizeof(T) + 255) & ~size_t(255);
+    const size_t packed_bytes = ((size_t)pl.table_count * pl.depth * ld * sizeof(T) + 255) & ~size_t(255);
     if (int rc = workspace(packed_bytes + tail_bytes(pl, sizeof(T)), &packed)) return rc;
     partial = static_cast<char *>(packed) + packed_bytes;
     ScopedTiming timed(TAG_PACK_FILTERS);
-    const unsigned blocks = (unsigned)std::min<long long>(ceil_div((long long)pl.table_count * g.F * ld, 256), 4096);
+    const unsigned blocks = (unsigned)std::min<long long>(ceil_div((long long)pl.table_count * pl.depth * ld, 256), 4096);
     hipLaunchKernelGGL(pack_phase_rows_kernel<T>, dim3(blocks), dim3(256), 0, runtime().stream, static_cast<const T *>(w),
-                       static_cast<T *>(packed), pl.arow, pl.table_count, pl.phase_count, (int)g.F, (int)g.C, (int)g.wvol, ld);
+                       static_cast<T *>(packed), pl.arow, pl.table_count, pl.phase_count, (int)g.F, pl.depth, (int)g.C, (int)g.wvol, ld);
     MG_HIP(hipGetLastError());
-  } else if (int rc = pack_filters<T>(g, w, pl.fold_row ? 4 : 3, &packed, tail_bytes(pl, sizeof(T)), &partial)) {
+  } else if (int rc = pack_filters<T>(g, w, pl.fold_row ? 4 : 3, pl.depth, &packed, tail_bytes(pl, sizeof(T)), &partial)) {
     return rc;
   }
   GemmParams gp{};
@@ -2457,10 +2545,10 @@ int conv_dgrad_impl(const Geometry &g, const Plan &pl, const void *grad, const v
   gp.dst_nstride = (long long)g.C * g.xvol;
   gp.a_ld = pl.fold_row ? folded_ld<T>(g.C) : packed_ld(g.C, pl.tap_major);
   gp.a_bytes = pl.table_rows ? (unsigned)((size_t)pl.table_count * gp.a_ld * sizeof(T))
-                             : (unsigned)((size_t)g.F * (pl.fold_row ? g.wvol / 3 : g.wvol) * gp.a_ld * sizeof(T));
+                             : (unsigned)((size_t)(pl.tap_major ? pl.depth : g.F) * (pl.fold_row ? g.wvol / 3 : g.wvol) * gp.a_ld * sizeof(T));
   if (pl.phase_rows) {
     gp.a_ld = packed_ld(pl.phase_count * g.C, true);
-    gp.a_bytes = (unsigned)((size_t)pl.table_count * g.F * gp.a_ld * sizeof(T));
+    gp.a_bytes = (unsigned)((size_t)pl.table_count * pl.depth * gp.a_ld * sizeof(T));
   }
   gp.src_bytes = pl.tap_major ? (unsigned)((size_t)g.N * g.F * g.gvol * sizeof(T)) : 0;
   return run_gemm<T>(gp, pl, TAG_CONV_DGRAD, runtime().stream);
@@ -2489,7 +2577,7 @@ void launch_wgrad(WgradParams &wp, bool tap_major, bool table_rows, hipStream_t 
   wp.col_tiles = (int)ceil_div(wp.CT, BN);
   wp.row_tiles = (int)ceil_div(wp.F, BM);
   if (table_rows) {
-    if constexpr (BN == 64) launch_table_wgrad<T, BM, BN, BK, WM, WN>(wp, s);
+    if constexpr (BN == 64 && BM != 48) launch_table_wgrad<T, BM, BN, BK, WM, WN>(wp, s);
   } else if (tap_major) {
     // one-dimensional grid, runs of (split, tile) pairs per XCD (see the kernel)
     const long long blocks = (long long)wp.splits * wp.col_tiles * wp.row_tiles;
@@ -2497,7 +2585,7 @@ void launch_wgrad(WgradParams &wp, bool tap_major, bool table_rows, hipStream_t 
       hipLaunchKernelGGL((tap_wgrad_kernel<T, BM, BN, BK, WM, WN, true>), dim3((unsigned)blocks), dim3(512), 0, s, wp);
     else
       hipLaunchKernelGGL((tap_wgrad_kernel<T, BM, BN, BK, WM, WN, false>), dim3((unsigned)blocks), dim3(512), 0, s, wp);
-  } else if constexpr (BN == 64) {
+  } else if constexpr (BN == 64 && BM != 48) {
     const dim3 grid((unsigned)wp.col_tiles, (unsigned)wp.row_tiles, (unsigned)wp.splits);
     hipLaunchKernelGGL((wgrad_kernel<T, BM, BN, BK, WM, WN>), grid, dim3(256), 0, s, wp);
   }
@@ -2506,11 +2594,11 @@ void launch_wgrad(WgradParams &wp, bool tap_major, bool table_rows, hipStream_t 
 template <typename T>
 int conv_wgrad_impl(const Geometry &g, const Plan &pl, const void *grad, const void *x, void *dw) {
   hipStream_t s = runtime().stream;
-  const int ct = (int)(g.C * g.wvol);
   // The tap-major kernel writes its columns in (tap, channel) order, so its result goes
   // through the reduction kernel, which also restores (channel, tap) -- unless there is a
   // single tap (a matrix product), where the two orders are the same, and a single split.
   const bool staged = pl.splits > 1 || (pl.tap_major && !pl.table_rows && g.wvol > 1);
+  const int ct = (int)((staged ? pl.depth : g.C) * g.wvol);
   void *target = dw;
   if (staged)
     if (int rc = workspace((size_t)pl.splits * g.F * ct * sizeof(T), &target)) return rc;
@@ -2544,6 +2632,8 @@ int conv_wgrad_impl(const Geometry &g, const Plan &pl, const void *grad, const v
   wp.by_g2 = make_fastdiv((unsigned)g.G[2]);
   wp.pos_tab = pl.pos_tab;
   wp.wvol = (int)g.wvol;
+  wp.shift_from = staged || pl.depth == g.C ? 1 << 30 : pl.depth - 16;
+  wp.col_shift = pl.depth - g.C;
   {
     ScopedTiming timed(TAG_CONV_WGRAD);
     bool launched = false;
@@ -2573,10 +2663,10 @@ int conv_wgrad_impl(const Geometry &g, const Plan &pl, const void *grad, const v
       // four runs of splits per element when one thread per element would leave units idle
       if (ceil_div(count, 256) < runtime().props.multiProcessorCount && pl.splits >= 16)
         hipLaunchKernelGGL((tap_reduce_kernel<T, 4>), dim3((unsigned)ceil_div(count, 64)), dim3(256), 0, s,
-                           static_cast<const T *>(target), static_cast<T *>(dw), g.F, g.C, (int)g.wvol, pl.splits);
+                           static_cast<const T *>(target), static_cast<T *>(dw), g.F, g.C, (int)g.wvol, pl.splits, ct);
       else
         hipLaunchKernelGGL((tap_reduce_kernel<T, 1>), dim3((unsigned)ceil_div(count, 256)), dim3(256), 0, s,
-                           static_cast<const T *>(target), static_cast<T *>(dw), g.F, g.C, (int)g.wvol, pl.splits);
+                           static_cast<const T *>(target), static_cast<T *>(dw), g.F, g.C, (int)g.wvol, pl.splits, ct);
     } else {
       if (ceil_div(count, 256) < runtime().props.multiProcessorCount / 8 && pl.splits >= 64)
         hipLaunchKernelGGL((splitk_reduce_kernel<T, 16>), dim3((unsigned)ceil_div(count, 16)), dim3(256), 0, s,
@@ -2605,88 +2695,6 @@ void release_conv_plans() {
 
 using namespace mg;
 
-// The fast (tap-major) kernels need the reduction -- K for the product and for da, M for dx --
-// and da's row count M to be multiples of 16.  A large product whose extents are not is run on
-// zero-padded copies of its operands (two bandwidth-bound passes over the operands against a
-// matrix product that runs more than twice as fast); small ones take the table-driven kernels.
-namespace {
-constexpr int64_t kMatmulUnit = 16;
-inline int64_t padded(int64_t n) { return (n + kMatmulUnit - 1) / kMatmulUnit * kMatmulUnit; }
-// MYGRAD_HIP_PAD=0 leaves every operand as it is (the table-driven kernels then take the
-// awkward extents): for comparisons
-inline bool padding_allowed() {
-  static const bool on = [] {
-    const char *flag = getenv("MYGRAD_HIP_PAD");
-    return !(flag && flag[0] == '0');
-  }();
-  return on;
-}
-inline bool worth_padding(int64_t batch, int64_t M, int64_t K, int64_t N) {
-  return padding_allowed() && 2.0 * (double)batch * (double)M * (double)K * (double)N >= 2.0e8;
-}
-
-// dst:(batch, drows, dcols) takes src:(batch, srows, scols) where both have an element, zero elsewhere
-template <typename T>
-__global__ void __launch_bounds__(256) pad2d_kernel(const T *__restrict__ src, T *__restrict__ dst, long long total, int srows,
-                                                    int scols, int drows, int dcols) {
-  const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= total) return;
-  const long long plane = (long long)drows * dcols;
-  const long long b = idx / plane;
-  const int rem = (int)(idx - b * plane);
-  const int r = rem / dcols, c = rem - r * dcols;
-  dst[idx] = (r < srows && c < scols) ? src[(b * srows + r) * scols + c] : T(0);
-}
-
-// src:(batch, srows, scols) re-laid as (batch, drows, dcols) into dst
-int relay_into(int dtype, const void *src, int64_t batch, int64_t srows, int64_t scols, int64_t drows, int64_t dcols, void *dst) {
-  void *where = dst;
-  void **block = &where;
-  const long long total = batch * drows * dcols;
-  if (srows >= (1ll << 31) || scols >= (1ll << 31) || drows * dcols >= (1ll << 31) || ceil_div(total, 256) >= (1ll << 31))
-    return fail(MG_ERR_UNSUPPORTED, "matrix product: an extent of 2^31 or more");
-  std::lock_guard<std::recursive_mutex> guard(api_mutex());
-  const dim3 grid((unsigned)ceil_div(total, 256)), blk(256);
-  ScopedTiming timed(TAG_COPY);
-  if (dtype == MG_F32)
-    hipLaunchKernelGGL(pad2d_kernel<float>, grid, blk, 0, runtime().stream, (const float *)src, (float *)*block, total, (int)srows,
-                       (int)scols, (int)drows, (int)dcols);
-  else
-    hipLaunchKernelGGL(pad2d_kernel<double>, grid, blk, 0, runtime().stream, (const double *)src, (double *)*block, total, (int)srows,
-                       (int)scols, (int)drows, (int)dcols);
-  MG_HIP(hipGetLastError());
-  return MG_OK;
-}
-
-// a pooled block holding src:(batch, srows, scols) re-laid as (batch, drows, dcols)
-int relaid(int dtype, const void *src, int64_t batch, int64_t srows, int64_t scols, int64_t drows, int64_t dcols, void **block) {
-  if (int rc = mg_malloc(block, (size_t)(batch * drows * dcols) * (dtype == MG_F32 ? 4 : 8))) return rc;
-  return relay_into(dtype, src, batch, srows, scols, drows, dcols, *block);
-}
-
-// Channel (or filter) count to zero-pad `channels` to so that the tap-major kernels apply, or 0
-// to leave it: already a multiple of 16, too small a problem to repay two extra passes over
-// the operands, or more than a third of padding.
-inline double conv_flops(const Geometry &g) {
-  return 2.0 * (double)g.N * (double)g.F * (double)g.gvol * (double)g.C * (double)g.wvol;
-}
-inline int64_t channels_to_pad_to(int64_t channels, double flops) {
-  if (channels % kMatmulUnit == 0 || flops < 2.0e8 || !padding_allowed()) return 0;
-  const int64_t up = padded(channels);
-  return 3 * up <= 4 * channels ? up : 0;
-}
-
-// frees pooled blocks when the call that used them returns (the pool keeps them in stream order)
-struct Blocks {
-  void *held[4] = {nullptr, nullptr, nullptr, nullptr};
-  ~Blocks() {
-    for (void *p : held)
-      if (p) (void)mg_free(p);
-  }
-};
-}  // namespace
-
-
 extern "C" {
 
 int mg_conv_fwd(const mg_conv_desc *desc, const void *x, const void *w, void *out) {
@@ -2695,15 +2703,6 @@ int mg_conv_fwd(const mg_conv_desc *desc, const void *x, const void *w, void *ou
   Geometry g;
   if (int rc = check_desc(desc, &g)) return rc;
   if (!x || !w || !out) return fail(MG_ERR_BAD_ARG, "null tensor pointer in mg_conv_fwd");
-  if (const int64_t Cp = channels_to_pad_to(g.C, conv_flops(g))) {
-    // zero channels added to x and to the filters: the same sums, on the tap-major kernels
-    Blocks tmp;
-    if (int rc = relaid(g.dtype, x, g.N, g.C, g.xvol, Cp, g.xvol, &tmp.held[0])) return rc;
-    if (int rc = relaid(g.dtype, w, g.F, g.C, g.wvol, Cp, g.wvol, &tmp.held[1])) return rc;
-    mg_conv_desc wider = *desc;
-    wider.C = Cp;
-    return mg_conv_fwd(&wider, tmp.held[0], tmp.held[1], out);
-  }
   Plan *pl = nullptr;
   if (int rc = get_plan(OP_FWD, desc, g, &pl)) return rc;
   return g.dtype == MG_F32 ? conv_fwd_impl<float>(g, *pl, x, w, out) : conv_fwd_impl<double>(g, *pl, x, w, out);
@@ -2715,15 +2714,6 @@ int mg_conv_dgrad(const mg_conv_desc *desc, const void *grad, const void *w, voi
   Geometry g;
   if (int rc = check_desc(desc, &g)) return rc;
   if (!grad || !w || !dx) return fail(MG_ERR_BAD_ARG, "null tensor pointer in mg_conv_dgrad");
-  if (const int64_t Fp = channels_to_pad_to(g.F, conv_flops(g))) {
-    // zero filters added to grad and to the filter bank
-    Blocks tmp;
-    if (int rc = relaid(g.dtype, grad, g.N, g.F, g.gvol, Fp, g.gvol, &tmp.held[0])) return rc;
-    if (int rc = relaid(g.dtype, w, 1, g.F, (int64_t)g.C * g.wvol, Fp, (int64_t)g.C * g.wvol, &tmp.held[1])) return rc;
-    mg_conv_desc wider = *desc;
-    wider.F = Fp;
-    return mg_conv_dgrad(&wider, tmp.held[0], tmp.held[1], dx);
-  }
   Plan *pl = nullptr;
   if (int rc = get_plan(OP_DGRAD, desc, g, &pl)) return rc;
   return g.dtype == MG_F32 ? conv_dgrad_impl<float>(g, *pl, grad, w, dx)
@@ -2736,29 +2726,6 @@ int mg_conv_wgrad(const mg_conv_desc *desc, const void *grad, const void *x, voi
   Geometry g;
   if (int rc = check_desc(desc, &g)) return rc;
   if (!grad || !x || !dw) return fail(MG_ERR_BAD_ARG, "null tensor pointer in mg_conv_wgrad");
-  {
-    const int64_t Cp = channels_to_pad_to(g.C, conv_flops(g)), Fp = channels_to_pad_to(g.F, conv_flops(g));
-    if (Cp || Fp) {
-      // zero channels / filters added to x / grad; the rows and columns of dw that exist are kept
-      const int64_t C2 = Cp ? Cp : g.C, F2 = Fp ? Fp : g.F;
-      Blocks tmp;
-      const void *x2 = x, *g2 = grad;
-      if (Cp) {
-        if (int rc = relaid(g.dtype, x, g.N, g.C, g.xvol, Cp, g.xvol, &tmp.held[0])) return rc;
-        x2 = tmp.held[0];
-      }
-      if (Fp) {
-        if (int rc = relaid(g.dtype, grad, g.N, g.F, g.gvol, Fp, g.gvol, &tmp.held[1])) return rc;
-        g2 = tmp.held[1];
-      }
-      if (int rc = mg_malloc(&tmp.held[2], (size_t)(F2 * C2 * g.wvol) * (g.dtype == MG_F32 ? 4 : 8))) return rc;
-      mg_conv_desc wider = *desc;
-      wider.C = C2;
-      wider.F = F2;
-      if (int rc = mg_conv_wgrad(&wider, g2, x2, tmp.held[2])) return rc;
-      return relay_into(g.dtype, tmp.held[2], g.F, C2, g.wvol, g.C, g.wvol, dw);
-    }
-  }
   Plan *pl = nullptr;
   if (int rc = get_plan(OP_WGRAD, desc, g, &pl)) return rc;
   return g.dtype == MG_F32 ? conv_wgrad_impl<float>(g, *pl, grad, x, dw)
@@ -2790,57 +2757,18 @@ int matmul_desc(const char *who, int dtype, int64_t batch, int64_t M, int64_t K,
 int mg_matmul(int dtype, int64_t batch, int64_t M, int64_t K, int64_t N, const void *a, const void *x, void *out) {
   mg_conv_desc d;
   if (int rc = matmul_desc("mg_matmul", dtype, batch, M, K, N, &d)) return rc;
-  if (K % kMatmulUnit != 0 && (dtype == MG_F32 || dtype == MG_F64) && a && x && out && worth_padding(batch, M, K, N)) {
-    const int64_t Kp = padded(K);
-    Blocks tmp;
-    if (int rc = relaid(dtype, a, 1, M, K, M, Kp, &tmp.held[0])) return rc;          // zero columns
-    if (int rc = relaid(dtype, x, batch, K, N, Kp, N, &tmp.held[1])) return rc;      // zero rows
-    if (int rc = matmul_desc("mg_matmul", dtype, batch, M, Kp, N, &d)) return rc;
-    return mg_conv_fwd(&d, tmp.held[1], tmp.held[0], out);
-  }
   return mg_conv_fwd(&d, x, a, out);
 }
 
 int mg_matmul_da(int dtype, int64_t batch, int64_t M, int64_t K, int64_t N, const void *grad, const void *x, void *da) {
   mg_conv_desc d;
   if (int rc = matmul_desc("mg_matmul_da", dtype, batch, M, K, N, &d)) return rc;
-  // da's rows are the filter-gradient kernel's tile rows, which must divide M: a large M is padded
-  // to whole 128-row (64-row) tiles rather than left to the 16- or 32-row ones
-  const int64_t row_unit = M >= 1024 ? 128 : (M >= 256 ? 64 : kMatmulUnit);
-  const int64_t Mp = (M + row_unit - 1) / row_unit * row_unit;
-  if ((K % kMatmulUnit != 0 || Mp != M) && (dtype == MG_F32 || dtype == MG_F64) && grad && x && da &&
-      worth_padding(batch, M, K, N)) {
-    const int64_t Kp = padded(K);
-    Blocks tmp;
-    const void *g2 = grad, *x2 = x;
-    if (Mp != M) {
-      if (int rc = relaid(dtype, grad, batch, M, N, Mp, N, &tmp.held[0])) return rc;
-      g2 = tmp.held[0];
-    }
-    if (Kp != K) {
-      if (int rc = relaid(dtype, x, batch, K, N, Kp, N, &tmp.held[1])) return rc;
-      x2 = tmp.held[1];
-    }
-    if (int rc = mg_malloc(&tmp.held[2], (size_t)Mp * Kp * (dtype == MG_F32 ? 4 : 8))) return rc;
-    if (int rc = matmul_desc("mg_matmul_da", dtype, batch, Mp, Kp, N, &d)) return rc;
-    if (int rc = mg_conv_wgrad(&d, g2, x2, tmp.held[2])) return rc;
-    // the rows and columns that belong to da
-    return relay_into(dtype, tmp.held[2], 1, Mp, Kp, M, K, da);
-  }
   return mg_conv_wgrad(&d, grad, x, da);
 }
 
 int mg_matmul_dx(int dtype, int64_t batch, int64_t M, int64_t K, int64_t N, const void *grad, const void *a, void *dx) {
   mg_conv_desc d;
   if (int rc = matmul_desc("mg_matmul_dx", dtype, batch, M, K, N, &d)) return rc;
-  if (M % kMatmulUnit != 0 && (dtype == MG_F32 || dtype == MG_F64) && grad && a && dx && worth_padding(batch, M, K, N)) {
-    const int64_t Mp = padded(M);
-    Blocks tmp;
-    if (int rc = relaid(dtype, a, 1, M, K, Mp, K, &tmp.held[0])) return rc;          // zero rows
-    if (int rc = relaid(dtype, grad, batch, M, N, Mp, N, &tmp.held[1])) return rc;   // zero rows
-    if (int rc = matmul_desc("mg_matmul_dx", dtype, batch, Mp, K, N, &d)) return rc;
-    return mg_conv_dgrad(&d, tmp.held[1], tmp.held[0], dx);
-  }
   return mg_conv_dgrad(&d, grad, a, dx);
 }
 

@@ -42,18 +42,24 @@ struct TabEntry {
 // One K tile of the tap-major gather-GEMM: BK consecutive channels (forward) or
 // filters (data gradient) under one filter tap.  Rows a_row0.. of the packed
 // filter matrix multiply the gathered elements at `coff` + i * channel stride;
-// all of them share the tap's coordinate offsets d[k], hence one validity test.
+// all of them share the tap's coordinate offsets d[k], hence one validity test.  Channels that
+// are no multiple of BK leave the last tile of a tap fewer live rows: bit i of `dead` is set for a row i
+// beyond the last channel, which reads as zero (whatever lies behind the tensor's channels, Inf or
+// NaN included, is not touched) and meets zero filters.
 struct KTile {
   int a_row0;
   int coff;
   int d0, d1, d2;
-  int pad0_, pad1_, pad2_;
+  unsigned dead;
+  int pad1_, pad2_;
 };
 
 // Sixteen consecutive columns of the filter-gradient matrix as the tap-major kernel
 // lays it out: one tap, channels c0..c0+15 (c0 a multiple of 16); the groups of one
 // channel block follow each other, one per tap.  `coff` = c0 * channel stride + the
-// tap's element offset.
+// tap's element offset.  With a channel count C that is no multiple of 16 the last block is
+// the channels C-16..C-1 (C >= 16), so that nothing outside x is read; what it shares with the
+// block before it is computed twice and used once.
 struct WGroup {
   int coff;
   int d0, d1, d2;
@@ -211,7 +217,7 @@ struct WgradParams {
   const void *x;
   void *out;            // dw itself when splits == 1, else the partial-sum workspace
   const TabEntry *tab;  // one row per column (c, tap): the forward table
-  int F, CT;            // rows and columns of dw viewed as a matrix
+  int F, CT;            // rows of dw viewed as a matrix; columns of `out` (whole channel blocks per tap where it is the workspace)
   int G[3], Q[3], sj[3], qs[3];
   int gvol;
   long long x_nstride, g_nstride;
@@ -231,6 +237,9 @@ struct WgradParams {
   // position's sample adds to the byte offset of grad[0][f][position]: n * (F - 1) * gvol elements.
   const void *pos_tab;
   int wvol;  // taps of the window
+  // One tap and channels that are no multiple of 16 (out is in dw's own layout): columns from
+  // shift_from on are the last, shifted channel block; column col there is channel col - col_shift.
+  int shift_from, col_shift;
 };
 
 }  // namespace mg

@@ -10,8 +10,8 @@
 // of zeros in device memory, so no select follows the load either.  The filter
 // gradient orders its columns by channel block of 16, then tap, then channel.
 //
-// Needs the channel count (filter count for dgrad) to be a multiple of BK; other
-// shapes take the table-driven kernels.
+// Channel counts (filter counts for dgrad) that are no multiple of BK: the last K tile of a tap
+// has fewer live rows (KTile::dead), which costs what its dead rows cost in MFMAs.
 #pragma once
 
 #include <type_traits>
@@ -129,7 +129,13 @@ struct Quad {
 // ------------------------------------------------------------------------------------------
 // forward and data gradient
 // ------------------------------------------------------------------------------------------
-template <typename T, int BM, int BN, int BK, int WM, int WN, int NPH = 1, bool FOLD = false, bool ROWS = false>
+// Whether the kernel for channels that are no multiple of BK is an instance of its own (DEAD): in the
+// others the test of KTile::dead costs nothing measurable (64 x 256: 260 -> 251 us on 64 channels
+// at 56x56), but the 128 x 128 float tile loses 1.2 % with it (4096^3: 991 -> 1003 us) and the four
+// fused phases 1 %.
+constexpr bool tap_gemm_dead_apart(int bm, int bn, int nph, int elem) { return elem == 4 && (nph == 4 || (bm == 128 && bn == 128)); }
+
+template <typename T, int BM, int BN, int BK, int WM, int WN, int NPH = 1, bool FOLD = false, bool ROWS = false, bool DEAD = false>
 __global__ void __launch_bounds__(512) tap_gemm_kernel(const GemmParams p) {
   // ROWS: the BK rows of a K tile are any rows of the gather table (GemmParams::tab: element
   // offset and coordinate offsets of one (channel, tap) each), not BK channels under one tap;
@@ -317,8 +323,17 @@ __global__ void __launch_bounds__(512) tap_gemm_kernel(const GemmParams p) {
         const bool ok = pos_ok & ((unsigned)(qb0 + e[2]) < (unsigned)p.Q[0]) & ((unsigned)(qb1 + e[3]) < (unsigned)p.Q[1]) &
                         ((unsigned)(qb2 + e[4]) < (unsigned)p.Q[2]);
         const unsigned at = ok ? src_at + (unsigned)(e[1] * (int)sizeof(T)) : kOutside;
+        // (wave-uniform branch, the same loads on both sides: only the short last tile of a tap
+        // pays an instruction per row, which sends its dead rows outside)
+        if (!(DEAD || !tap_gemm_dead_apart(BM, BN, NPH, (int)sizeof(T))) || __builtin_expect(e[5] == 0, 1)) {
 #pragma unroll
-        for (int r = 0; r < BLOADS; ++r) rb[r] = buffer_load<T>(src_buf, at, (unsigned)r * b_step);
+          for (int r = 0; r < BLOADS; ++r) rb[r] = buffer_load<T>(src_buf, at, (unsigned)r * b_step);
+        } else {
+          const unsigned dead = (unsigned)e[5] >> brow0;
+#pragma unroll
+          for (int r = 0; r < BLOADS; ++r)
+            rb[r] = buffer_load<T>(src_buf, at | ((dead << (31 - r * BROWS)) & kOutside), (unsigned)r * b_step);
+        }
       }
       if (live) {
         ++requested;
@@ -1065,7 +1080,10 @@ __global__ void __launch_bounds__(512) tap_wgrad_kernel(const WgradParams p) {
   const int split = pair / tiles_per_split;
   const int tile = pair % tiles_per_split;
   const int n0 = (tile % p.col_tiles) * BN;  // first column
-  const int m0 = (tile / p.col_tiles) * BM;  // first filter (F % BM == 0)
+  // First filter.  Filters that fill no whole number of tiles: the last tile is moved back to end
+  // with the last filter, so that nothing beyond grad is read, and stores only its own rows (m_own on).
+  const int m_own = (tile / p.col_tiles) * BM;
+  const int m0 = p.F >= BM ? min(m_own, p.F - BM) : m_own;
   const int kbeg = split * p.kchunk;
   const int kend = min(kbeg + p.kchunk, p.kpos);
 
@@ -1295,6 +1313,12 @@ __global__ void __launch_bounds__(512) tap_wgrad_kernel(const WgradParams p) {
   // and cost a 4096^3 matrix product 4 %, so it is not set there).
   __builtin_amdgcn_s_setprio(3);
 
+  // column of `out` that column `col` of the tiles belongs in, negative if another column holds it
+  auto out_column = [&](int col) -> int {
+    if (TABLE || col < p.shift_from) return col;
+    return col - p.col_shift >= p.shift_from ? col - p.col_shift : -1;
+  };
+
   if constexpr (sizeof(T) == 8) {
     // 4x4x4 four-block MFMAs on 8-row x 8-column patches (see Quad); quarter-wave lk
     // contracts the K indices lk*KQ .. lk*KQ+KQ-1, four adjacent ones per LDS read
@@ -1342,12 +1366,12 @@ __global__ void __launch_bounds__(512) tap_wgrad_kernel(const WgradParams p) {
     T *__restrict__ out = static_cast<T *>(p.out) + (long long)split * p.F * p.CT;
 #pragma unroll
     for (int j = 0; j < GN; ++j) {
-      const int col = n0 + bcol8 + j * 8;
-      if (col >= p.CT) continue;
+      const int col = out_column(n0 + bcol8 + j * 8);
+      if (col < 0 || col >= p.CT) continue;
 #pragma unroll
       for (int i = 0; i < GM; ++i) {
         const int f = m0 + drow + i * 8;
-        if (f < p.F) out[(long long)f * p.CT + col] = acc[i][j];
+        if (f >= m_own && f < p.F) out[(long long)f * p.CT + col] = acc[i][j];
       }
     }
     return;
@@ -1407,21 +1431,22 @@ __global__ void __launch_bounds__(512) tap_wgrad_kernel(const WgradParams p) {
   T *__restrict__ out = static_cast<T *>(p.out) + (long long)split * p.F * p.CT;
 #pragma unroll
   for (int j = 0; j < TN; ++j) {
-    const int col = n0 + wn0 + j * 16 + l16;
-    if (col >= p.CT) continue;
+    const int col = out_column(n0 + wn0 + j * 16 + l16);
+    if (col < 0 || col >= p.CT) continue;
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int f = m0 + wm0 + i * 16 + Mma<T>::row_of(lane, q);
-        if (f < p.F) out[(long long)f * p.CT + col] = acc[i][j][q];
+        if (f >= m_own && f < p.F) out[(long long)f * p.CT + col] = acc[i][j][q];
       }
   }
 }
 
 // dw[f][c][t] = the sum over K splits of part[s][f][col], where the columns run over
 // channel blocks of 16, then taps, then the channel inside the block:
-// col = ((c/16) * wvol + t) * 16 + c%16.
+// col = ((c/16) * wvol + t) * 16 + c%16; `ct` columns in all.  With C no multiple of 16 the last
+// block holds channels C-16..C-1, of which those of the block before it are passed over.
 // The splits are cut into RUNS runs (1 or 4); wave q of the block adds run q in split
 // order for 256 / RUNS consecutive elements, and the run sums are added in run order:
 // always the same association for a given plan, so the result repeats exactly.  Four
@@ -1429,26 +1454,26 @@ __global__ void __launch_bounds__(512) tap_wgrad_kernel(const WgradParams p) {
 // the device with one thread per element.
 template <typename T, int RUNS>
 __global__ void __launch_bounds__(256) tap_reduce_kernel(const T *__restrict__ part, T *__restrict__ dw, int F, int C,
-                                                         int wvol, int splits) {
+                                                         int wvol, int splits, int ct) {
   constexpr int WIDTH = 256 / RUNS;
   __shared__ T runs[4][64];
-  const int count = F * C * wvol;
+  const int count = F * ct;
   const int q = threadIdx.x / WIDTH, lane = threadIdx.x % WIDTH;
   // Threads run through the partial sums' own layout, so a wave reads consecutive
   // addresses of every split (the few stores to dw are the scattered side).
-  const int src = blockIdx.x * WIDTH + lane;  // index into one split: f * C*wvol + column
+  const int src = blockIdx.x * WIDTH + lane;  // index into one split: f * ct + column
   const int per = (splits + RUNS - 1) / RUNS;
   const int first = min(q * per, splits), last = min(first + per, splits);
   T sum = T(0);
   int i = count;  // index into dw
   if (src < count) {
-    const int ct = C * wvol;
     const int f = src / ct;
     const int col = src - f * ct;
     const int group = col / 16;  // (channel block, tap)
     const int cb = group / wvol, t = group - cb * wvol;
-    i = f * ct + (cb * 16 + col % 16) * wvol + t;
-    if (first < last) sum = sum_in_order(part + (long long)first * count + src, count, last - first);
+    const int c = min(cb * 16, max(C - 16, 0)) + col % 16;
+    if (c >= cb * 16) i = (f * C + c) * wvol + t;
+    if (i < count && first < last) sum = sum_in_order(part + (long long)first * count + src, count, last - first);
   }
   if constexpr (RUNS == 1) {
     if (i < count) dw[i] = sum;

@@ -653,7 +653,7 @@ def test_data_gradient_with_the_stride_phases_as_rows(abi, dtype, x_shape, w_sha
 # Every tile shape of the forward / data-gradient kernels, forced in turn (the planner would take
 # one or two of them for any given problem): rows x positions, and for the data gradient under a
 # stride the shapes of its fused stride phases.
-ALL_TILES = ["128,128", "128,64", "64,256", "64,128", "32,256", "32,128", "16,256", "64,64"]
+ALL_TILES = ["128,128", "128,64", "64,256", "64,128", "32,256", "32,128", "16,256", "64,64", "96,128", "48,256"]
 TILE_PROBLEMS = [
     # (x, w, stride, padding, dilation): odd extents, so that row ends and sample ends fall inside tiles
     ((3, 32, 29, 27), (160, 32, 3, 3), (1, 1), (1, 1), (1, 1)),       # 160 rows: one and a quarter tiles of 128
@@ -714,7 +714,7 @@ def test_row_tiles_of_a_position_block_on_one_xcd(abi, monkeypatch, x_shape, w_s
     assert np.array_equal(bits(got), bits(abi.conv_fwd(x, w, 1, 1, 1)))
 
 
-WGRAD_TILES = ["128,128", "64,64", "32,128", "32,64", "16,64"]
+WGRAD_TILES = ["48,64", "128,128", "64,64", "32,128", "32,64", "16,64"]
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
@@ -966,6 +966,45 @@ def test_conv_awkward_channel_counts_on_padded_copies(abi, dtype, case):
     assert rel_err(abi.conv_fwd(x, w, s, p, d), want_out) <= tol
     assert rel_err(abi.conv_dgrad(g, x_shape, w, s, p, d), direct.conv_backward_x(g, x_shape, w, s, p, d)) <= tol
     assert rel_err(abi.conv_wgrad(g, x, w_shape, s, p, d), direct.conv_backward_w(g, x, w_shape, s, p, d)) <= tol
+
+
+# Counts that fill no K tile (channels forward, filters in the data gradient) or no row tile, read where they lie:
+# one row short of and one beyond a K tile, of each row tile and of a group of 16 columns; strides (fused
+# phases, phases as rows), folded taps, one tap (the filter gradient written without a pass over
+# partial sums), an odd number of positions.
+RAGGED_CASES = [
+    # x shape, w shape, stride, padding, dilation
+    ((2, 47, 41, 37), (83, 47, 3, 3), (1, 1), (1, 1), (1, 1)),
+    ((2, 33, 47, 43), (65, 33, 3, 3), (2, 2), (1, 1), (1, 1)),
+    ((3, 45, 30, 64), (31, 45, 3, 3), (1, 1), (1, 1), (1, 1)),
+    ((2, 4, 113, 113), (95, 4, 5, 5), (2, 2), (2, 2), (1, 1)),
+    ((2, 49, 1501), (129, 49, 9), (1,), (4,), (1,)),
+    ((1, 81, 9001), (161, 81, 1), (1,), (0,), (1,)),
+    ((4, 18, 6, 25, 25), (47, 18, 3, 3, 1), (1, 2, 2), (1, 0, 0), (1, 1, 1)),
+]
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("case", range(len(RAGGED_CASES)))
+def test_conv_counts_that_fill_no_tile_in_place(abi, dtype, case):
+    x_shape, w_shape, s, p, d = RAGGED_CASES[case]
+    rng = np.random.default_rng(1700 + case)
+    print("ragged", np.dtype(dtype).name, x_shape, w_shape, s, p, d, flush=True)
+    # small integers: every sum is exact in both precisions, so the results are compared as they are
+    x = rng.integers(-3, 4, x_shape).astype(dtype)
+    w = rng.integers(-2, 3, w_shape).astype(dtype)
+    want = direct.conv_forward(x, w, s, p, d).astype(dtype)
+    g = rng.integers(-2, 3, want.shape).astype(dtype)
+    assert np.array_equal(abi.conv_fwd(x, w, s, p, d), want)
+    assert np.array_equal(abi.conv_dgrad(g, x_shape, w, s, p, d), direct.conv_backward_x(g, x_shape, w, s, p, d).astype(dtype))
+    assert np.array_equal(abi.conv_wgrad(g, x, w_shape, s, p, d), direct.conv_backward_w(g, x, w_shape, s, p, d).astype(dtype))
+    # what lies behind a sample's channels (the next sample's first ones) stays out of its sums, NaN and all
+    if x_shape[0] > 1:
+        xn, gn = x.copy(), g.copy()
+        xn[1:], gn[1:] = np.nan, np.nan
+        assert np.array_equal(abi.conv_fwd(xn, w, s, p, d)[0], want[0])
+        dx = direct.conv_backward_x(g[:1], (1, *x_shape[1:]), w, s, p, d).astype(dtype)
+        assert np.array_equal(abi.conv_dgrad(gn, x_shape, w, s, p, d)[0], dx[0])
 
 
 KERNEL_VARIANT_CASES = [
