@@ -4,8 +4,8 @@
 // the result carry) is bound by launches, not arithmetic, when each pair gets a launch of the
 // convolution kernels; here a wavefront makes one 16x16 tile of one product on the matrix cores,
 // reading its operands where they lie (a transposed operand is a pair of swapped strides), so the
-// whole stack is one grid.  Pairs of 32 x 32 results or more go through a second kernel, where a
-// block of four wavefronts makes a 64 x 64 tile of one product from operands it has copied to
+// whole stack is one grid.  Results larger than 32 x 32 go through a second kernel, where a
+// block of four wavefronts makes a tile of one product from operands it has copied to
 // LDS once (16 bytes per lane, coalesced) instead of every wavefront fetching its own rows and
 // columns through L1.  Large pairs stay with the tiled convolution kernels.
 #include "internal.h"
@@ -43,6 +43,7 @@ struct Tile<double> {
 struct BatchedParams {
   int M, K, N;
   int row_tiles, col_tiles;
+  int pairs, dealt;                  // staged kernel: pairs, and whether they are dealt out to the XCDs in turn
   long long tiles;                   // batch * row_tiles * col_tiles
   long long a_pair, a_row, a_col;    // element strides of op(a): between pairs, along M, along K
   long long b_pair, b_row, b_col;    // of op(b): between pairs, along K, along N
@@ -128,153 +129,204 @@ __global__ void __launch_bounds__(256) batched_product_kernel(BatchedParams p, c
 }
 
 
-// ---- 64 x 64 tiles of one product per block, operands staged in LDS ---------------------------
-// A block copies the 64 x 64 pieces of op(a) and op(b) that its tile needs, K chunk by K chunk,
-// into LDS in the orientation they have in memory (a transposed operand is read differently, not
-// stored differently), zeros beyond the matrices' edges.  Wavefront w makes the 32 x 32 quarter
-// (w / 2, w % 2) of the tile: per step of four k, two fragments of each operand and four MFMAs.
-// Row lengths in LDS: an operand whose MFMA lanes (lane % 16) run down its memory rows gets
-// 64 + 4 floats per row (sixteen rows start in sixteen different groups of four banks), one
-// whose lanes run along a row gets 64 + 16 (the four k of a step start sixteen banks apart).
-template <typename T, bool ROWS_ARE_LANES>
-struct StagedLd {
-  static constexpr int value = sizeof(T) == 4 ? (ROWS_ARE_LANES ? 68 : 80) : (ROWS_ARE_LANES ? 66 : 72);
-};
-
-template <typename T, bool TA, bool TB, bool VA, bool VB>
+// ---- a tile of one product per block, operands staged in LDS -----------------------------------
+// A block copies the pieces of op(a) and op(b) that its BM x BN tile needs, K chunk by K chunk, into
+// LDS in the orientation they have in memory (a transposed operand is read differently, not stored
+// differently), zeros beyond the matrices' edges, 16 bytes per lane whatever the row length (a
+// global load of 16 bytes needs the alignment of an element only; the one piece of a row that the
+// matrix's edge cuts goes element by element).  Each of the four wavefronts makes a 32 x 32 part.
+//
+// What bounds it: the trips of a chunk from memory to LDS to registers, not the matrix pipes, so
+// the loads of the next chunk are issued before this one is multiplied, chunks are short (128 bytes
+// of k: six or seven blocks on a unit cover for one another; 256 bytes: 794 x (86,117,322) 117 us
+// instead of 103), and the LDS reads are wide.  Measured, single precision, forward / da / db: 96 x
+// (197,64,197) 14.1 / 13.8 / 13.7 us (34 TFLOP/s; 19.9 / 17.3 / 20.4 with element loads and
+// element LDS reads, which rows that are no whole pieces and every row took before), 794 x
+// (86,117,322) 103 / 91 / 104 us (147 / 130 / 139), 8 x 512^3 29 / 28 / 30 us.
+// The sum over k may run in any order that both operands share: in a block of 4 * VEC values of k
+// (VEC = 16 bytes) the lane groups (lane / 16 = q) take k = VEC * q + s at step s, so an operand
+// that lies along k gives a lane VEC steps per LDS read; of one that lies along its rows or columns
+// a lane takes two neighbours, the two MFMA fragments it feeds, per read.
+template <typename T, bool TA, bool TB, int BM, int BN>
 __global__ void __launch_bounds__(256) batched_staged_kernel(BatchedParams p, const T *__restrict__ a, const T *__restrict__ b,
                                                              T *__restrict__ out) {
   constexpr int VEC = 16 / sizeof(T);
   typedef T V __attribute__((ext_vector_type(VEC)));
-  constexpr int LDA = StagedLd<T, !TA>::value;  // not transposed: memory rows are m, the lanes' index
-  constexpr int LDB = StagedLd<T, TB>::value;   // transposed: memory rows are n, the lanes' index
-  __shared__ __attribute__((aligned(16))) T As[64 * LDA];
-  __shared__ __attribute__((aligned(16))) T Bs[64 * LDB];
+  typedef T VU __attribute__((ext_vector_type(VEC), aligned(sizeof(T))));
+  typedef T Pair __attribute__((ext_vector_type(2)));
+  typedef T PairU __attribute__((ext_vector_type(2), aligned(sizeof(T))));
+  static_assert((BM / 32) * (BN / 32) == 4, "four wavefronts of 32 x 32");
+  constexpr int KC = 128 / sizeof(T);  // depth of a chunk
+  // The stored pieces: rows x columns as in memory, rows 16-byte aligned in LDS.  Of pieces with k down
+  // their rows the lane groups read rows VEC apart: 8 floats of padding put two groups' 32 banks
+  // side by side.
+  constexpr int AR = TA ? KC : BM, AC = TA ? BM : KC, LDA = AC + (TA ? 32 / (int)sizeof(T) : VEC);
+  constexpr int BR = TB ? BN : KC, BC = TB ? KC : BN, LDB = BC + (TB ? VEC : 32 / (int)sizeof(T));
+  constexpr int NA = AR * AC / VEC / 256, NB = BR * BC / VEC / 256;
+  __shared__ __attribute__((aligned(16))) T As[AR * LDA];
+  __shared__ __attribute__((aligned(16))) T Bs[BR * LDB];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l16 = lane & 15, lk = lane >> 4;
+  // Blocks are handed to the 8 XCDs round-robin, each with its own L2, in which the tiles of a pair
+  // should meet: the pairs are dealt out to the XCDs in turn, so that all of them work on one
+  // stretch of memory, or, with few pairs, an XCD takes one run of consecutive tiles, so that none
+  // idles.  (Runs for 8192 pairs of 64^3: 76 -> 88 us, the XCDs' streams a power of two apart.)
+  const int xcd = blockIdx.x % 8, nth = blockIdx.x / 8;
   const int per_pair = p.row_tiles * p.col_tiles;
-  const long long pair = (long long)blockIdx.x / per_pair;
-  const int within = (int)((long long)blockIdx.x - pair * per_pair);
-  const int row0 = (within / p.col_tiles) * 64, col0 = (within % p.col_tiles) * 64;
-  const T *pa = a + pair * p.a_pair;
-  const T *pb = b + pair * p.b_pair;
+  int pair, within;
+  if (p.dealt) {
+    pair = nth / per_pair * 8 + xcd;
+    within = nth % per_pair;
+    if (pair >= p.pairs) return;  // (the whole block)
+  } else {
+    const int per_xcd = gridDim.x / 8, extra = gridDim.x % 8;
+    const int tile = xcd * per_xcd + min(xcd, extra) + nth;
+    pair = tile / per_pair;
+    within = tile - pair * per_pair;
+  }
+  const int row0 = (within / p.col_tiles) * BM, col0 = (within % p.col_tiles) * BN;
+  const T *pa = a + (long long)pair * p.a_pair;
+  const T *pb = b + (long long)pair * p.b_pair;
 
-  // The 64 x 64 piece of a stored matrix (`rows` x `cols`, row-major) that starts at (r0, c0)
-  // travels through registers (`fetch`, zeros outside the matrix) into LDS (`park`, row length
-  // `ld`); the loads of both operands are issued before either is parked, so that a chunk
-  // costs one trip to memory, not two.
-  constexpr int PIECES = 64 / VEC, PASS = 256 / PIECES, NV = 64 / PASS;
-  struct Regs {
-    V v[NV];   // 16-byte pieces: rows tid / PIECES + i * PASS, piece tid % PIECES
-    T e[16];   // single elements: rows tid / 64 + 4 * i, column tid % 64
-  };
-  auto fetch = [&](const T *src, int rows, int cols, int r0, int c0, Regs &reg, auto vec) {
-    if constexpr (decltype(vec)::value) {
-      const int piece = tid % PIECES, r = tid / PIECES;
+  // R x C elements of a stored matrix (`rows` x `cols`, row-major) from (r0, c0): through registers
+  // (zeros outside the matrix) into LDS; the loads of both operands are issued before either is
+  // parked, so that a chunk costs one trip to memory, not two
+  auto fetch = [&](auto rc, auto cc, const T *src, int rows, int cols, int r0, int c0, auto &reg) {
+    constexpr int R = decltype(rc)::value, C = decltype(cc)::value, PIECES = C / VEC, PASS = 256 / PIECES;
+    const int c = c0 + (tid % PIECES) * VEC;
+    const T *at = src + (long long)(r0 + tid / PIECES) * cols + c;
 #pragma unroll
-      for (int i = 0; i < NV; ++i) {
-        const int rr = r0 + r + i * PASS, cc = c0 + piece * VEC;
-        reg.v[i] = V{};
-        if (rr < rows && cc < cols) reg.v[i] = *reinterpret_cast<const V *>(src + (long long)rr * cols + cc);  // cols % VEC == 0
-      }
-    } else {
-      const int c = tid % 64, r = tid / 64;
+    for (int i = 0; i < R / PASS; ++i) {
+      reg[i] = V{};
+      if (r0 + tid / PIECES + i * PASS < rows) {
+        const T *piece = at + (long long)(i * PASS) * cols;
+        if (c + VEC <= cols) {
+          reg[i] = *reinterpret_cast<const VU *>(piece);
+        } else {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int rr = r0 + r + i * 4, cc = c0 + c;
-        reg.e[i] = (rr < rows && cc < cols) ? src[(long long)rr * cols + cc] : T(0);
+          for (int s = 0; s < VEC - 1; ++s)
+            if (c + s < cols) reg[i][s] = piece[s];
+        }
       }
     }
   };
-  auto park = [&](const Regs &reg, T *dst, int ld, auto vec) {
-    if constexpr (decltype(vec)::value) {
-      const int piece = tid % PIECES, r = tid / PIECES;
+  auto park = [&](auto rc, auto cc, T *dst, auto ld, const auto &reg) {
+    constexpr int R = decltype(rc)::value, C = decltype(cc)::value, PIECES = C / VEC, PASS = 256 / PIECES;
 #pragma unroll
-      for (int i = 0; i < NV; ++i) *reinterpret_cast<V *>(dst + (r + i * PASS) * ld + piece * VEC) = reg.v[i];
-    } else {
-      const int c = tid % 64, r = tid / 64;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) dst[(r + i * 4) * ld + c] = reg.e[i];
-    }
+    for (int i = 0; i < R / PASS; ++i)
+      *reinterpret_cast<V *>(dst + (tid / PIECES + i * PASS) * decltype(ld)::value + (tid % PIECES) * VEC) = reg[i];
   };
-  const std::integral_constant<bool, VA> vec_a{};
-  const std::integral_constant<bool, VB> vec_b{};
-  auto fetch_chunk = [&](int k0, Regs &ra, Regs &rb) {
-    if constexpr (TA)
-      fetch(pa, p.K, p.M, k0, row0, ra, vec_a);  // stored (K, M)
-    else
-      fetch(pa, p.M, p.K, row0, k0, ra, vec_a);  // stored (M, K)
-    if constexpr (TB)
-      fetch(pb, p.N, p.K, col0, k0, rb, vec_b);  // stored (N, K)
-    else
-      fetch(pb, p.K, p.N, k0, col0, rb, vec_b);  // stored (K, N)
+  const std::integral_constant<int, AR> ar{};
+  const std::integral_constant<int, AC> ac{};
+  const std::integral_constant<int, BR> br{};
+  const std::integral_constant<int, BC> bc{};
+  V ra[NA], rb[NB];
+  auto fetch_chunk = [&](int k0) {
+    fetch(ar, ac, pa, TA ? p.K : p.M, TA ? p.M : p.K, TA ? k0 : row0, TA ? row0 : k0, ra);
+    fetch(br, bc, pb, TB ? p.N : p.K, TB ? p.K : p.N, TB ? col0 : k0, TB ? k0 : col0, rb);
   };
 
-  const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
+  constexpr int WAVES_N = BN / 32;
+  const int wr = (wave / WAVES_N) * 32, wc = (wave % WAVES_N) * 32;
+  const bool live = row0 + wr < p.M && col0 + wc < p.N;  // (the same for a whole wavefront)
   typename Tile<T>::Acc acc[2][2];
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = typename Tile<T>::Acc{0, 0, 0, 0};
 
-  Regs ra, rb;
-  fetch_chunk(0, ra, rb);
-  for (int k0 = 0; k0 < p.K; k0 += 64) {
+  fetch_chunk(0);
+  for (int k0 = 0; k0 < p.K; k0 += KC) {
     if (k0 > 0) __syncthreads();  // everyone has finished with the previous chunk
-    park(ra, As, LDA, vec_a);
-    park(rb, Bs, LDB, vec_b);
+    park(ar, ac, As, std::integral_constant<int, LDA>{}, ra);
+    park(br, bc, Bs, std::integral_constant<int, LDB>{}, rb);
     __syncthreads();
-    if (k0 + 64 < p.K) fetch_chunk(k0 + 64, ra, rb);  // on its way while this chunk is multiplied
-    const int steps = (min(64, p.K - k0) + 3) / 4;
-    for (int ks = 0; ks < steps; ++ks) {
-      const int k = ks * 4 + lk;
-      T av[2], bv[2];
+    if (k0 + KC < p.K) fetch_chunk(k0 + KC);  // on its way while this chunk is multiplied
+    const int blocks = live ? (min(KC, p.K - k0) + 4 * VEC - 1) / (4 * VEC) : 0;
+    for (int kb = 0; kb < blocks; ++kb) {
+      const int k = kb * (4 * VEC) + lk * VEC;
+      T av[2][VEC], bv[2][VEC];
+      // rows of the tile: fragment i's are wr + 16 i + l16, or (op(a) along its rows) wr + 2 l16 + i
+      if constexpr (TA) {
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int m = wr + i * 16 + l16;
-        av[i] = TA ? As[k * LDA + m] : As[m * LDA + k];
+        for (int s = 0; s < VEC; ++s) {
+          const Pair two = *reinterpret_cast<const Pair *>(As + (k + s) * LDA + wr + 2 * l16);
+          av[0][s] = two[0], av[1][s] = two[1];
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const V v = *reinterpret_cast<const V *>(As + (wr + i * 16 + l16) * LDA + k);
+#pragma unroll
+          for (int s = 0; s < VEC; ++s) av[i][s] = v[s];
+        }
+      }
+      // columns: fragment j's are wc + 2 l16 + j
+      if constexpr (TB) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const V v = *reinterpret_cast<const V *>(Bs + (wc + 2 * l16 + j) * LDB + k);
+#pragma unroll
+          for (int s = 0; s < VEC; ++s) bv[j][s] = v[s];
+        }
+      } else {
+#pragma unroll
+        for (int s = 0; s < VEC; ++s) {
+          const Pair two = *reinterpret_cast<const Pair *>(Bs + (k + s) * LDB + wc + 2 * l16);
+          bv[0][s] = two[0], bv[1][s] = two[1];
+        }
       }
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int n = wc + j * 16 + l16;
-        bv[j] = TB ? Bs[n * LDB + k] : Bs[k * LDB + n];
-      }
+      for (int s = 0; s < VEC; ++s)
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = Tile<T>::run(av[i], bv[j], acc[i][j]);
+          for (int j = 0; j < 2; ++j) acc[i][j] = Tile<T>::run(av[i][s], bv[j][s], acc[i][j]);
     }
   }
 
-  T *po = out + pair * ((long long)p.M * p.N);
+  const int col = col0 + wc + 2 * l16;
+  if (!live || col >= p.N) return;
+  T *po = out + pair * ((long long)p.M * p.N) + col;
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int col = col0 + wc + j * 16 + l16;
-    if (col >= p.N) continue;
+  for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = row0 + wr + i * 16 + Tile<T>::row_of(lane, r);
-        if (row < p.M) po[(long long)row * p.N + col] = acc[i][j][r];
+    for (int r = 0; r < 4; ++r) {
+      const int m = Tile<T>::row_of(lane, r);
+      const int row = row0 + wr + (TA ? 2 * m + i : i * 16 + m);
+      if (row >= p.M) continue;
+      if (col + 1 < p.N) {
+        PairU two;
+        two[0] = acc[i][0][r], two[1] = acc[i][1][r];
+        *reinterpret_cast<PairU *>(po + (long long)row * p.N) = two;
+      } else {
+        po[(long long)row * p.N] = acc[i][0][r];
       }
-  }
+    }
+}
+
+// Rows of the tile: of 128 x 32, 64 x 64 and 32 x 128, all four wavefronts of 32 x 32, the one that covers
+// M x N with the least area (the squarer one where they come out the same: it loads less).
+inline int staged_rows(int64_t M, int64_t N) {
+  int best = 64;
+  int64_t least = ceil_div(M, 64) * ceil_div(N, 64);
+  for (int bm : {128, 32})
+    if (ceil_div(M, bm) * ceil_div(N, 4096 / bm) < least) best = bm, least = ceil_div(M, bm) * ceil_div(N, 4096 / bm);
+  return best;
 }
 
 template <typename T>
-void launch_staged(const BatchedParams &p, long long batch, bool ta, bool tb, bool va, bool vb, const void *a, const void *b,
-                   void *out, hipStream_t s) {
-  const dim3 grid((unsigned)(batch * p.row_tiles * p.col_tiles)), block(256);
-#define MG_STAGED(TA, TB, VA, VB)                                                                                      \
-  if (ta == TA && tb == TB && va == VA && vb == VB)                                                                    \
-    hipLaunchKernelGGL((batched_staged_kernel<T, TA, TB, VA, VB>), grid, block, 0, s, p, (const T *)a, (const T *)b, (T *)out);
-#define MG_STAGED_V(TA, TB) MG_STAGED(TA, TB, false, false) MG_STAGED(TA, TB, false, true) MG_STAGED(TA, TB, true, false) MG_STAGED(TA, TB, true, true)
-  MG_STAGED_V(false, false)
-  MG_STAGED_V(false, true)
-  MG_STAGED_V(true, false)
-  MG_STAGED_V(true, true)
-#undef MG_STAGED_V
+void launch_staged(const BatchedParams &p, int bm, unsigned blocks, bool ta, bool tb, const void *a, const void *b, void *out, hipStream_t s) {
+#define MG_STAGED(TA, TB, BM)                    \
+  if (ta == TA && tb == TB && bm == BM)          \
+    hipLaunchKernelGGL((batched_staged_kernel<T, TA, TB, BM, 4096 / BM>), dim3(blocks), dim3(256), 0, s, p, (const T *)a, (const T *)b, (T *)out);
+#define MG_STAGED_BM(TA, TB) MG_STAGED(TA, TB, 64) MG_STAGED(TA, TB, 128) MG_STAGED(TA, TB, 32)
+  MG_STAGED_BM(false, false)
+  MG_STAGED_BM(false, true)
+  MG_STAGED_BM(true, false)
+  MG_STAGED_BM(true, true)
+#undef MG_STAGED_BM
 #undef MG_STAGED
 }
 
@@ -307,25 +359,28 @@ int mg_matmul_batched(int dtype, int64_t batch, int64_t M, int64_t K, int64_t N,
   p.b_row = trans_b ? 1 : N, p.b_col = trans_b ? K : 1;  // b[p] is stored (N, K) when transposed
   hipStream_t s = runtime().stream;
   ScopedTiming timed(TAG_BATCHED_PRODUCT);
-  // Pairs of 32 x 32 results or more whose 64 x 64 tiles are at least half full: staged in LDS.
   // MYGRAD_HIP_BMM_STAGED=0 keeps every pair on the kernel that reads its operands in place.
   static const bool staged_on = [] {
     const char *flag = getenv("MYGRAD_HIP_BMM_STAGED");
     return !(flag && flag[0] == '0');
   }();
-  const long long t64 = ceil_div(M, 64) * ceil_div(N, 64);
-  if (staged_on && K > 0 && M >= 32 && N >= 32 && 2 * M * N >= t64 * 64 * 64 && batch * t64 < (1ll << 31)) {
-    const int vec = dtype == MG_F32 ? 4 : 2;
-    // 16-byte pieces along a stored matrix's rows: the row length is a whole number of pieces
-    // (so is the distance between pairs, then) and the stack itself is aligned
-    const bool va = (trans_a ? M : K) % vec == 0 && reinterpret_cast<uintptr_t>(a) % 16 == 0;
-    const bool vb = (trans_b ? K : N) % vec == 0 && reinterpret_cast<uintptr_t>(b) % 16 == 0;
-    p.row_tiles = (int)ceil_div(M, 64);
-    p.col_tiles = (int)ceil_div(N, 64);
+  const int bm = staged_rows(M, N);
+  p.dealt = batch >= 64;
+  const long long blocks = (p.dealt ? ceil_div(batch, 8) * 8 : batch) * ceil_div(M, bm) * ceil_div(N, 4096 / bm);
+  p.pairs = (int)batch;
+  // A result of one wavefront's 32 x 32 or of 16 rows or columns stays with the kernel above (300 x
+  // (20,100,20): 5.6 us there, 8.0 staged).  In double precision, whose 16x16x4 MFMA takes three
+  // times as long, 32 x 32 parts that are less than 0.6 full lose too (64 x (300,400,18): 48 / 57 us;
+  // 34 x (310,259,31): 31 / 21) unless 64 x 64 tiles are half full.
+  const long long parts = ceil_div(M, 32) * ceil_div(N, 32) * 1024, t64 = ceil_div(M, 64) * ceil_div(N, 64) * 4096;
+  const bool full = dtype == MG_F32 || 10 * M * N >= 6 * parts || (M >= 32 && N >= 32 && 2 * M * N >= t64);
+  if (staged_on && K > 0 && M > 16 && N > 16 && (M > 32 || N > 32) && full && blocks < (1ll << 31)) {
+    p.row_tiles = (int)ceil_div(M, bm);
+    p.col_tiles = (int)ceil_div(N, 4096 / bm);
     if (dtype == MG_F32)
-      launch_staged<float>(p, batch, trans_a != 0, trans_b != 0, va, vb, a, b, out, s);
+      launch_staged<float>(p, bm, (unsigned)blocks, trans_a != 0, trans_b != 0, a, b, out, s);
     else
-      launch_staged<double>(p, batch, trans_a != 0, trans_b != 0, va, vb, a, b, out, s);
+      launch_staged<double>(p, bm, (unsigned)blocks, trans_a != 0, trans_b != 0, a, b, out, s);
     MG_HIP(hipGetLastError());
     return MG_OK;
   }

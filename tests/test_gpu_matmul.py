@@ -84,7 +84,9 @@ BATCHED = [(1, 1, 1, 1), (3, 16, 16, 16), (5, 17, 3, 33), (2, 1, 70, 1), (300, 8
            (3, 100, 129, 50),
            # 32 x 32 results or more per pair: 64 x 64 tiles staged in LDS -- whole tiles, ragged edges in M, N
            # and K, several K chunks, row lengths that are and are not whole 16-byte pieces
-           (9, 64, 64, 64), (3, 130, 70, 96), (2, 32, 200, 32), (5, 47, 33, 61), (2, 128, 64, 192)]
+           (9, 64, 64, 64), (3, 130, 70, 96), (2, 32, 200, 32), (5, 47, 33, 61), (2, 128, 64, 192),
+           # tiles of 128 x 32 and 32 x 128, one past a wavefront's part, a K of one and of one past a chunk, nine blocks
+           (2, 127, 33, 32), (3, 31, 65, 129), (1, 33, 1, 33), (2, 17, 17, 97), (9, 65, 32, 33)]
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
