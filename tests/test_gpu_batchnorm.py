@@ -267,3 +267,22 @@ def test_conv_batchnorm_relu_pool_chain_stays_on_the_device():
     want_dx = ora.conv_backward_x(want_dy, x.shape, x.dtype, w.data, stride=1, padding=1)
     want_dw = ora.conv_backward_w(want_dy, x.data, w.shape, stride=1, padding=1)
     assert err(x.grad, want_dx) <= 1e-10 and err(w.grad, want_dw) <= 1e-10
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("shape", [(1, 2, 64), (3, 2, 65), (5, 3, 66), (2, 1, 67), (4, 5, 9, 15), (300, 2, 11, 11), (2, 3, 5003)])
+def test_rows_that_are_no_whole_16_byte_pieces(abi, shape, dtype):
+    """The last piece of a row shares elements with the one before it: each counts once in the sums,
+    and nothing of the neighbouring rows is touched.  Sums of small integers are exact, so are the
+    statistics' totals; the bar of the other tests holds for what is divided."""
+    dtype = np.dtype(dtype)
+    rng = np.random.default_rng(list(shape))
+    x, grad = rng.integers(-8, 9, shape).astype(dtype), rng.integers(-8, 9, shape).astype(dtype)
+    y, mean, var = abi.batchnorm_fwd(x, eps=1e-5)
+    want_y, want_mean, want_var = ora.batchnorm_forward(x.astype(np.float64), eps=1e-5)
+    assert err(mean, want_mean) <= STAT_TOL[dtype] and err(var, want_var) <= STAT_TOL[dtype] and err(y, want_y) <= TOL[dtype]
+    dx, dgamma, dbeta = abi.batchnorm_bwd(grad, x, mean, var, np.ones(shape[1], dtype), eps=1e-5, want=("x", "gamma", "beta"))
+    axes = (0, *range(2, len(shape)))
+    assert np.array_equal(dbeta, grad.sum(axes).astype(dtype))
+    one = np.ones(shape[1])
+    assert err(dx, ora.batchnorm_backward(grad.astype(np.float64), x.astype(np.float64), one, eps=1e-5)[0]) <= TOL[dtype]
