@@ -65,7 +65,7 @@ def _count(shape):
 
 def _free_device(ptr):
     try:
-        _hip.load_library().mg_free(ptr)
+        _hip._lib.mg_free(ptr)  # loaded: something allocated `ptr`
     except Exception:  # interpreter shutdown
         pass
 
@@ -93,6 +93,14 @@ class DeviceBuffer:
         arr = np.ascontiguousarray(arr)
         assert arr.nbytes <= self.nbytes
         _hip.check(_hip.lib().mg_memcpy_h2d(self.ptr, arr.ctypes.data, arr.nbytes))
+        stats["h2d_bytes"] += arr.nbytes
+
+    def stage(self, arr):
+        """:meth:`upload` for a buffer that only operations read (they are ordered after it): the
+        copy is not waited for."""
+        arr = np.ascontiguousarray(arr)
+        assert arr.nbytes <= self.nbytes
+        _hip.check(_hip.lib().mg_upload(self.ptr, arr.ctypes.data, arr.nbytes))
         stats["h2d_bytes"] += arr.nbytes
 
     def download_into(self, arr):
@@ -193,7 +201,7 @@ class DeviceArray:
 
     def __init__(self, buf, shape, dtype, base=None):
         self.buf = buf
-        self.shape = tuple(int(n) for n in shape)
+        self.shape = tuple(map(int, shape))
         self.dtype = np.dtype(dtype)
         self.base = base
         self._host = None
@@ -401,7 +409,7 @@ def hold_gradient(arr):
     if arr.dtype not in (np.float32, np.float64) or lookup(arr) is not None:
         return
     buf = DeviceBuffer(arr.nbytes)
-    buf.upload(arr)
+    buf.stage(arr)
     stats["uploads"] += 1
     attach_transient(arr, buf)
 
@@ -446,7 +454,7 @@ def to_device(arr, dtype=None):
             stats["mirror_hits"] += 1
             return buf
     buf = DeviceBuffer(arr.nbytes)
-    buf.upload(arr)
+    buf.stage(arr)
     stats["uploads"] += 1
     key = _key(arr)
     if key in _locked:

@@ -125,6 +125,7 @@ _SIGNATURES = {
     "mg_host_alloc": [ctypes.POINTER(_vp), ctypes.c_size_t],
     "mg_host_free": [_vp],
     "mg_memcpy_h2d": [_vp, _vp, ctypes.c_size_t],
+    "mg_upload": [_vp, _vp, ctypes.c_size_t],
     "mg_memcpy_d2h": [_vp, _vp, ctypes.c_size_t],
     "mg_memcpy_d2d": [_vp, _vp, ctypes.c_size_t],
     "mg_memset_zero": [_vp, ctypes.c_size_t],

@@ -162,6 +162,13 @@ __global__ void __launch_bounds__(256) copy16_kernel(const uint4 *__restrict__ s
   for (; i < n16; i += step) dst[i] = src[i];
 }
 
+// The same for a copy between device memory and pinned host memory, `n` bytes, both ends 16-byte aligned.
+__global__ void __launch_bounds__(256) copy_link_kernel(const char *__restrict__ src, char *__restrict__ dst, size_t n) {
+  const size_t i = size_t(blockIdx.x) * 256 + threadIdx.x;
+  if (i < n / 16) reinterpret_cast<uint4 *>(dst)[i] = reinterpret_cast<const uint4 *>(src)[i];
+  if (blockIdx.x == 0 && threadIdx.x < n % 16) dst[n / 16 * 16 + threadIdx.x] = src[n / 16 * 16 + threadIdx.x];
+}
+
 __global__ void fill_zero_bytes_kernel(uint8_t *p, size_t n) {
   size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i < n) p[i] = 0;
@@ -255,6 +262,37 @@ BlockPool &host_pool() {
   p.pinned = true;
   return p;
 }
+// Staging memory of mg_upload: four pinned segments, filled one after the other; the event recorded
+// when a segment is left says when the copies out of it are done.
+struct Staging {
+  static constexpr size_t kSegment = size_t(1) << 20;
+  static constexpr int kSegments = 4;
+  char *base = nullptr;
+  size_t offset = 0;
+  int segment = 0;
+  hipEvent_t left[kSegments] = {};
+  bool pending[kSegments] = {};
+};
+Staging &staging() {
+  static Staging s;
+  return s;
+}
+void staging_release() {
+  Staging &st = staging();
+  if (st.base) (void)hipHostFree(st.base);
+  for (hipEvent_t e : st.left)
+    if (e) (void)hipEventDestroy(e);
+  st = Staging{};
+}
+// Copies of at most this many bytes between device and pinned memory are a kernel of this library: a
+// launch and the link's latency, where the runtime's copy costs about twice that.  Larger ones leave
+// the link to the runtime's copy.
+constexpr size_t kLinkKernelBytes = size_t(64) << 10;
+
+void launch_copy_link(const void *src, void *dst, size_t nbytes) {
+  hipLaunchKernelGGL(copy_link_kernel, dim3((unsigned)((nbytes / 16 + 255) / 256 + (nbytes < 16 ? 1 : 0))), dim3(256), 0, runtime().stream,
+                     static_cast<const char *>(src), static_cast<char *>(dst), nbytes);
+}
 size_t pool_round(size_t n) {
   const size_t unit = n <= (size_t(1) << 20) ? 512 : (size_t(1) << 21);
   return (n + unit - 1) / unit * unit;
@@ -324,6 +362,7 @@ int mg_shutdown(void) {
   MG_HIP(hipStreamSynchronize(rt.stream));
   release_conv_plans();
   timing_release();
+  staging_release();
   if (rt.workspace) MG_HIP(hipFree(rt.workspace));
   rt.workspace = nullptr;
   rt.workspace_bytes = 0;
@@ -479,12 +518,55 @@ int mg_memcpy_h2d(void *dst_dev, const void *src_host, size_t nbytes) {
   return MG_OK;
 }
 
+int mg_upload(void *dst_dev, const void *src_host, size_t nbytes) {
+  MG_LOCK();
+  MG_REQUIRE_INIT();
+  if (nbytes == 0) return MG_OK;
+  if (!dst_dev || !src_host) return fail(MG_ERR_BAD_ARG, "null pointer in mg_upload");
+  // large arrays: the runtime's own staging overlaps its copies, which a single one here would not
+  if (nbytes > Staging::kSegment / 4) return mg_memcpy_h2d(dst_dev, src_host, nbytes);
+  Runtime &rt = runtime();
+  Staging &st = staging();
+  if (!st.base) {
+    if (hipHostMalloc(reinterpret_cast<void **>(&st.base), Staging::kSegment * Staging::kSegments, hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      st.base = nullptr;
+      return mg_memcpy_h2d(dst_dev, src_host, nbytes);
+    }
+    for (hipEvent_t &e : st.left) MG_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  }
+  if (st.offset + nbytes > Staging::kSegment) {
+    MG_HIP(hipEventRecord(st.left[st.segment], rt.stream));
+    st.pending[st.segment] = true;
+    st.segment = (st.segment + 1) % Staging::kSegments;
+    st.offset = 0;
+    if (st.pending[st.segment]) MG_HIP(hipEventSynchronize(st.left[st.segment]));
+    st.pending[st.segment] = false;
+  }
+  char *at = st.base + st.segment * Staging::kSegment + st.offset;
+  st.offset += (nbytes + 255) & ~size_t(255);
+  memcpy(at, src_host, nbytes);
+  if (nbytes <= kLinkKernelBytes && reinterpret_cast<uintptr_t>(dst_dev) % 16 == 0) {
+    launch_copy_link(at, dst_dev, nbytes);
+    MG_HIP(hipGetLastError());
+  } else {
+    MG_HIP(hipMemcpyAsync(dst_dev, at, nbytes, hipMemcpyHostToDevice, rt.stream));
+  }
+  return MG_OK;
+}
+
 int mg_memcpy_d2h(void *dst_host, const void *src_dev, size_t nbytes) {
   MG_LOCK();
   MG_REQUIRE_INIT();
   if (nbytes == 0) return MG_OK;
   if (!dst_host || !src_dev) return fail(MG_ERR_BAD_ARG, "null pointer in mg_memcpy_d2h");
   Runtime &rt = runtime();
+  if (nbytes <= kLinkKernelBytes && reinterpret_cast<uintptr_t>(src_dev) % 16 == 0 && host_pool().size_of.count(dst_host) != 0) {
+    launch_copy_link(src_dev, dst_host, nbytes);  // (the start of a pinned block of the pool)
+    MG_HIP(hipGetLastError());
+    MG_HIP(hipStreamSynchronize(rt.stream));
+    return MG_OK;
+  }
   MG_HIP(hipMemcpyAsync(dst_host, src_dev, nbytes, hipMemcpyDeviceToHost, rt.stream));
   MG_HIP(hipStreamSynchronize(rt.stream));
   return MG_OK;

@@ -10,6 +10,8 @@ broadcast operand is summed back on the device (carried in double, rounded once:
 NumPy's pairwise sum to rounding).
 Floating-point operands only; other argument patterns raise (there is no CPU fallback)."""
 
+from math import prod
+
 import numpy as np
 
 from ... import _device, _hip, _reduce
@@ -34,7 +36,7 @@ def _spread(arr, shape, dtype):
 def device_multiply(a, b, dtype, shape=None):
     """``a * b`` for two host arrays that broadcast to ``shape`` -> (host result, its device buffer)."""
     shape = a.shape if shape is None else tuple(shape)
-    size = int(np.prod(shape, dtype=np.int64))
+    size = prod(shape)
     if size == 0:
         return np.empty(shape, dtype=dtype), None
     ob = None
@@ -71,7 +73,7 @@ class Multiply(Operation):
         dtype = np.dtype(np.result_type(grad.dtype, other.dtype))
         if grad.shape != self._shape or dtype not in (np.float32, np.float64):
             raise NotImplementedError(f"multiply backward for gradient {grad.shape} {grad.dtype} (no CPU fallback)")
-        if var.size == int(np.prod(self._shape, dtype=np.int64)):  # nothing to add up (axes of length one at most)
+        if var.size == prod(self._shape):  # nothing to add up (axes of length one at most)
             out, ob = device_multiply(grad, _device.value_of(other), dtype, self._shape)
             if ob is None:
                 return np.zeros(var.shape, dtype=dtype)

@@ -13,6 +13,8 @@ else one launch of the tiled kernels per matrix pair); two stacks that broadcast
 (each is first spread to the common batch shape on the device, and the gradient of a stack
 that was spread is summed back over the axes it was spread along)."""
 
+from math import prod
+
 import numpy as np
 
 from ... import _device, _hip, _reduce
@@ -29,8 +31,25 @@ __all__ = ["MatMul"]
 SMALL_PAIR_FLOPS = 2 * 768**3
 
 
-def _prod(shape):
-    return int(np.prod(shape, dtype=np.int64))
+# Shape of the product of two operands taken without rows and columns (the batch shape, then zeros) per
+# pair of operand shapes that passed NumPy's checks: a layer multiplies the same shapes at every step
+_PROBE_SHAPES = {}
+
+
+def _probe_shape(x_shape, y_shape):
+    key = (x_shape, y_shape)
+    shape = _PROBE_SHAPES.get(key)
+    if shape is None:
+        # NumPy's own checks (scalars, core dimensions, batch broadcasting) on operands
+        # without rows and columns: the same errors, the batch shape of the result, no arithmetic
+        shape = np.matmul(
+            np.empty(x_shape if len(x_shape) < 2 else (*x_shape[:-2], 0, x_shape[-1]), dtype=np.int8),
+            np.empty(y_shape if len(y_shape) < 2 else (*y_shape[:-2], y_shape[-2], 0), dtype=np.int8),
+        ).shape
+        if len(_PROBE_SHAPES) >= 1024:
+            _PROBE_SHAPES.clear()
+        _PROBE_SHAPES[key] = shape
+    return shape
 
 
 class MatMul(Operation):
@@ -41,12 +60,7 @@ class MatMul(Operation):
     def __call__(self, a, b):
         self.variables = (a, b)
         x, y = _device.value_of(a), _device.value_of(b)
-        # NumPy's own checks (scalars, core dimensions, batch broadcasting) on operands
-        # without rows and columns: the same errors, the batch shape of the result, no arithmetic
-        probe = np.matmul(
-            np.empty(x.shape if x.ndim < 2 else (*x.shape[:-2], 0, x.shape[-1]), dtype=np.int8),
-            np.empty(y.shape if y.ndim < 2 else (*y.shape[:-2], y.shape[-2], 0), dtype=np.int8),
-        )
+        probe = _probe_shape(tuple(x.shape), tuple(y.shape))
         dtype = np.dtype(np.result_type(x.dtype, y.dtype))
         if dtype not in (np.float32, np.float64):
             raise TypeError(f"matmul runs on the GPU in float32 or float64, got {x.dtype} and {y.dtype} (there is no CPU fallback)")
@@ -59,10 +73,10 @@ class MatMul(Operation):
         self._spread = bool(stack_a and stack_b and stack_a != stack_b)
         self._own_stacks = (stack_a, stack_b)
         if self._spread:
-            stack_a = stack_b = tuple(probe.shape[: probe.ndim - 2])
+            stack_a = stack_b = probe[: len(probe) - 2]
         batch_shape = stack_a or stack_b
         out_shape = batch_shape + (() if x.ndim == 1 else (M,)) + (() if y.ndim == 1 else (N,))
-        assert len(out_shape) == probe.ndim
+        assert len(out_shape) == len(probe)
         self._dtype, self._dims = dtype, (M, K, N)
         self._stacks = (stack_a, stack_b)
         self._promoted = (x2_shape, y2_shape)
@@ -70,7 +84,7 @@ class MatMul(Operation):
             return np.zeros(out_shape, dtype=dtype)
 
         ab, bb = self._operand(x, 0), self._operand(y, 1)
-        ob = _device.DeviceBuffer(max(_prod(out_shape) * dtype.itemsize, 16))
+        ob = _device.DeviceBuffer(max(prod(out_shape) * dtype.itemsize, 16))
         self._launch("mg_matmul", ab, bb, ob, a_like=0, x_like=1, out_like=2)
         out = _device.download(ob, out_shape, dtype)
         _device.attach(out, ob)
@@ -95,14 +109,14 @@ class MatMul(Operation):
         code, item = _hip.dtype_code(self._dtype), self._dtype.itemsize
         fn = getattr(_hip.lib(), entry)
         if not stack_a:
-            _hip.check(fn(code, _prod(stack_b), M, K, N, first.ptr, second.ptr, result.ptr))
+            _hip.check(fn(code, prod(stack_b), M, K, N, first.ptr, second.ptr, result.ptr))
         elif not stack_b:
-            _hip.check(fn(code, 1, _prod(stack_a) * M, K, N, first.ptr, second.ptr, result.ptr))
+            _hip.check(fn(code, 1, prod(stack_a) * M, K, N, first.ptr, second.ptr, result.ptr))
         elif 2 * M * K * N <= SMALL_PAIR_FLOPS:
             # a stack of small pairs: one launch, the gradients by transposed reads
             # (entry: first, second -> result)   mg_matmul: a, b -> a @ b;
             # mg_matmul_da: grad, b -> grad @ b^T;   mg_matmul_dx: grad, a -> a^T @ grad
-            pairs = _prod(stack_a)
+            pairs = prod(stack_a)
             batched = _hip.lib().mg_matmul_batched
             if entry == "mg_matmul":
                 _hip.check(batched(code, pairs, M, K, N, 0, 0, first.ptr, second.ptr, result.ptr))
@@ -112,7 +126,7 @@ class MatMul(Operation):
                 _hip.check(batched(code, pairs, K, M, N, 1, 0, second.ptr, first.ptr, result.ptr))
         else:
             per = (M * K * item, K * N * item, M * N * item)
-            for i in range(_prod(stack_a)):
+            for i in range(prod(stack_a)):
                 _hip.check(
                     fn(code, 1, M, K, N, first.ptr + i * per[a_like], second.ptr + i * per[x_like], result.ptr + i * per[out_like])
                 )
@@ -125,14 +139,14 @@ class MatMul(Operation):
             return np.zeros(var.shape, dtype=dtype)
         M, K, N = self._dims
         stack_a, stack_b = self._stacks
-        batch = _prod(stack_a or stack_b)
+        batch = prod(stack_a or stack_b)
         if grad.size != batch * M * N:
             raise ValueError(f"matmul backward: gradient of shape {grad.shape} does not match the product")
         gb = _device.to_device(grad, dtype)
         own, full = self._own_stacks[index], self._stacks[index]
         widened = self._spread and own != full
         core = self._promoted[index][-2:]
-        count = _prod(full + core) if widened else var.size
+        count = prod(full + core) if widened else var.size
         ob = _device.DeviceBuffer(max(count * dtype.itemsize, 16))
         if index == 0:
             # d a = grad @ b^T, summed over a batch that `a` was shared by (ops.py:107-114)

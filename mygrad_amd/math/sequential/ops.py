@@ -37,7 +37,7 @@ class Sum(Operation):
         kept_shape = tuple(1 if i in axes else n for i, n in enumerate(x.shape))
         self._kept_shape = kept_shape
         out_shape = kept_shape if keepdims else tuple(n for i, n in enumerate(x.shape) if i not in axes)
-        if int(np.prod(out_shape, dtype=np.int64)) == 0:
+        if 0 in out_shape:
             return np.zeros(out_shape, dtype=x.dtype)
         if x.size == 0:  # something is left, nothing to add to it
             return np.zeros(out_shape, dtype=x.dtype)

@@ -3,6 +3,7 @@ signature, argument checks and errors (``mygrad/nnet/layers/conv.py``), whose
 forward pass, ``dx`` and ``dw`` run as implicit-GEMM kernels in
 ``libmygrad_hip.so``."""
 
+from math import prod
 from numbers import Integral
 
 import numpy as np
@@ -127,7 +128,7 @@ class ConvND(Operation):
         padding, stride, dilation, out_shape = checked
         self.padding, self.stride, self.dilation = padding, stride, dilation
 
-        if np.iscomplexobj(xd) or np.iscomplexobj(wd):
+        if xd.dtype.kind == "c" or wd.dtype.kind == "c":
             return self._complex_forward(xd, wd)
         dtype, result_dtype = _kernel_dtype(xd, wd)
         if result_dtype.kind in "iu" and xd.size and wd.size:
@@ -158,7 +159,7 @@ class ConvND(Operation):
         else:
             self._desc = _hip.shared_desc(_hip.conv_desc, dtype, tuple(xd.shape), tuple(wd.shape), grid, tuple(stride), tuple(padding),
                                           tuple(dilation))
-            ob = _device.DeviceBuffer(int(np.prod(out_full)) * dtype.itemsize)
+            ob = _device.DeviceBuffer(prod(out_full) * dtype.itemsize)
             _hip.check(_hip.lib().mg_conv_fwd(self._desc, xb.ptr, wb.ptr, ob.ptr))
         out, ob = _narrowed(ob, out_full, dtype, result_dtype)
         _device.attach(out, ob)

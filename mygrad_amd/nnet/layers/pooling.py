@@ -74,6 +74,10 @@ def plan_stages(lead, pooled, pool, stride, most=_hip.MG_MAX_ND):
     return stages
 
 
+# what the checks of MaxPoolND made of (shape, window, stride), for calls that passed them
+_CHECKED = {}
+
+
 class MaxPoolND(Operation):
     """Max-pooling over the trailing ``len(pool)`` axes of ``x``.
 
@@ -102,10 +106,10 @@ class MaxPoolND(Operation):
         """Argmax bytes of the forward pass (of its one stage, for up to three pooled axes)."""
         return self._stages[0].argmax if self._stages else None
 
-    def __call__(self, x, pool, stride):
-        self.variables = (x,)
-        xd = _device.value_of(x)
-
+    @staticmethod
+    def _check(xd, pool, stride):
+        """The reference's checks of a call (pooling.py:60-88); returns the window and stride as arrays, the
+        pooled extents, the grid and the leading pooled axes that pool nothing."""
         assert isinstance(pool, (tuple, list, np.ndarray)) and all(
             i >= 0 and isinstance(i, Integral) for i in pool
         )
@@ -119,9 +123,7 @@ class MaxPoolND(Operation):
         )
         assert len(stride) == len(pool) and all(s >= 1 and isinstance(s, Integral) for s in stride)
 
-        self.pool, self.stride = pool, stride
         m = len(pool)
-        lead_shape = xd.shape[: xd.ndim - m]
         pooled = np.array(xd.shape[xd.ndim - m :])
 
         out_shape = (pooled - pool) / stride + 1
@@ -140,6 +142,33 @@ class MaxPoolND(Operation):
         skip = 0
         while m - skip > 1 and pool[skip] == 1 and stride[skip] == 1:
             skip += 1
+        return pool, stride, tuple(int(n) for n in pooled), tuple(int(g) for g in out_shape), skip
+
+    def __call__(self, x, pool, stride):
+        self.variables = (x,)
+        xd = _device.value_of(x)
+
+        # A layer is called with the same shapes and windows at every step: what the checks made of
+        # them the first time (they passed) is kept and handed out again.
+        # (Plain ints only: 2.0 equals 2 as a key and is refused as a window.)
+        key = checked = None
+        if type(pool) is tuple and all([type(i) is int for i in pool]) and (
+            type(stride) is int or type(stride) is tuple and all([type(i) is int for i in stride])
+        ):
+            key = (tuple(xd.shape), pool, stride)
+            checked = _CHECKED.get(key)
+        if checked is None:
+            checked = self._check(xd, pool, stride)
+            if key is not None:
+                for arr in checked[:2]:
+                    arr.flags.writeable = False  # shared between the operations that hit this entry
+                if len(_CHECKED) >= 1024:
+                    _CHECKED.clear()
+                _CHECKED[key] = checked
+        self.pool, self.stride, pooled, grid, skip = checked
+        pool, stride = self.pool, self.stride
+        m = len(pool)
+        lead_shape = xd.shape[: xd.ndim - m]
         self._skip = skip
         result_dtype = xd.dtype
         if xd.dtype.kind in "iu":
@@ -159,7 +188,6 @@ class MaxPoolND(Operation):
         # pick the same maxima, and the result is narrowed again (exactly: it consists of inputs)
         if xd.dtype == np.float16:
             xd = xd.astype(np.float32)  # on the device for a value that lives there, else on the host
-        grid = tuple(int(g) for g in out_shape)
         self._grid = grid
         self._lead = prod(int(n) for n in lead_shape)
         out_full = (*lead_shape, *grid)

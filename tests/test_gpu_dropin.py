@@ -804,3 +804,23 @@ def test_complex_operands_under_no_autodiff_carry_a_complex_step():
     with mg.no_autodiff:
         z = np.asarray(conv_nd(x, wc, **kwargs).data)
     assert rel_err(z.imag, ora.conv_forward(x.astype(np.complex128), wc, **kwargs).imag) <= 1e-10
+
+
+def test_uploads_that_are_not_waited_for():
+    """More uploads than the staging memory holds, each source overwritten as soon as the call returns, at the sizes
+    where the way of the copy changes; and back through pinned and through ordinary memory."""
+    from mygrad_amd import _device
+
+    sizes = [1, 15, 16, 17, 4095, 65536, 65537, 262144, 262145, 700001] + [200003] * 60
+    kept = []
+    for i, n in enumerate(sizes):
+        source = np.full(n, i + 1, dtype=np.uint8)
+        source[-1] = 200 + i % 50
+        buf = _device.DeviceBuffer(n)
+        buf.stage(source)
+        source[:] = 0
+        kept.append(buf)
+    for i, (n, buf) in enumerate(zip(sizes, kept)):
+        for back in (_device.pinned_empty((n,), np.uint8), np.zeros(n, dtype=np.uint8)):
+            buf.download_into(back)
+            assert back[-1] == 200 + i % 50 and (back[:-1] == i + 1).all(), (i, n)

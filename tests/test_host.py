@@ -687,3 +687,29 @@ def test_shared_descriptors_are_built_once_per_distinct_layer():
     assert (c.N, c.C, c.F, list(c.pad)) == (2, 3, 4, [0, 1, 1])
     fresh = _hip.conv_desc(f64, (2, 3, 8, 8), (4, 3, 3, 3), (8, 8), (1, 1), (1, 1), (1, 1))
     assert fresh is not c  # the builders themselves always build
+
+
+def test_reused_checks_refuse_what_the_checks_refuse():
+    """A call whose shapes and settings equal (as numbers) those of a call that passed is still checked:
+    2.0 is no window, and shapes that do not multiply do not."""
+    from mygrad_amd.math.misc.ops import _probe_shape
+    from mygrad_amd.nnet.layers.pooling import _CHECKED, MaxPoolND
+
+    _CHECKED.clear()
+    x = mg.Tensor(np.zeros((2, 3, 8, 8), dtype=np.float32))
+    try:
+        max_pool(x, (2, 2), 2)  # (with no device the launch is refused; the checks have passed by then)
+    except mg.HipUnavailable:
+        pass
+    assert len(_CHECKED) == 1
+    for pool, stride in (((2.0, 2.0), 2), ((2, 2), 2.5), ((2, 2), (2, 2, 2)), ((0, 2), 2), ((2, 2), 0)):
+        with pytest.raises((AssertionError, TypeError)):
+            MaxPoolND()(x, pool, stride)
+    with pytest.raises(ValueError):
+        MaxPoolND()(x, (3, 3), 2)
+    assert len(_CHECKED) == 1
+    assert _probe_shape((5, 3, 4), (4, 2)) == (5, 0, 0) == _probe_shape((5, 3, 4), (4, 2))
+    for a, b in (((3, 4), (3, 4)), ((), (4, 2)), ((2, 3, 4), (3, 4, 5))):
+        for _ in range(2):
+            with pytest.raises(ValueError):
+                _probe_shape(a, b)
