@@ -531,7 +531,7 @@ __global__ void __launch_bounds__(256) sum_middle_finish_kernel(MiddleParams p, 
   out[e] = (T)total;
 }
 
-// many_channels: the caller cuts its launches to the grid's y extent of 65535 itself
+// many_channels: the caller cuts its launches to the grid's extent itself
 int make_params(const mg_bn_desc *d, BnParams *p, const char *who, bool many_channels = false) {
   if (!d) return fail(MG_ERR_BAD_ARG, "%s: descriptor is null", who);
   if (d->dtype != MG_F32 && d->dtype != MG_F64) return fail(MG_ERR_UNSUPPORTED, "%s: dtype %d (only float32=0 / float64=1)", who, d->dtype);
@@ -665,7 +665,14 @@ int axis_sum_impl(BnParams p, const void *x, const void *y, void *out) {
     else
       MG_BN_LAUNCH(axis_sum_kernel, walk, p, (const T *)x, (double *)partial);
   };
-  launch(grid_for(p));
+  if (p.walk == COLS) {
+    launch(grid_for(p));
+  } else {
+    // a launch has fewer than 2^32 threads along x, which is 2^24 - 1 blocks
+    const int channels = p.C, most = 1 << 23;
+    for (; p.c0 < channels; p.c0 += most) launch(dim3((unsigned)std::min(most, channels - p.c0), (unsigned)p.chunks));
+    p.c0 = 0;
+  }
   hipLaunchKernelGGL(axis_sum_finish_kernel<T>, dim3((unsigned)ceil_div(p.C, 4)), block, 0, s, p, (const double *)partial, (T *)out);
   MG_HIP(hipGetLastError());
   return MG_OK;

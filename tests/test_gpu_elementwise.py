@@ -158,6 +158,14 @@ def test_sum_over_full_size(abi):
         assert np.all(np.abs(got - want) <= SUM_TOL[np.dtype(np.float32)] * scale)
 
 
+def test_sum_over_more_rows_than_one_launch_has_blocks(abi):
+    """2^24 + 5 rows of 64 (a launch is limited to fewer than 2^32 threads along an axis), told apart by one element."""
+    rows = 2**24 + 5
+    x = np.zeros((1, rows, 64), dtype=np.float32)
+    x[0, :, 63] = np.arange(rows) % 1009
+    assert np.array_equal(abi.sum_over(x, 0), x[0, :, 63])
+
+
 def test_sum_over_closed_forms_and_bad_arguments(abi):
     from mygrad_amd import _device, _hip
 
