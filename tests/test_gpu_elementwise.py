@@ -57,6 +57,18 @@ def test_multiply_and_relu_bit_exact(abi, dtype, shape):
         assert np.array_equal(bits(abi.relu_bwd_mask(mask, g)), bits(ora.relu_backward(a, g)))
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n", [7, 8, 9, 511, 512, 513, 1024, 4 * 512 + 505, 2**23 + 519])
+def test_masked_relu_where_a_wavefront_has_all_or_none_of_its_elements(abi, dtype, n):
+    rng = np.random.default_rng(n)
+    a, g = (_specials(rng, (n,), dtype) for _ in range(2))
+    with np.errstate(all="ignore"):
+        out, mask = abi.relu_fwd_mask(a)
+        assert np.array_equal(bits(out), bits(ora.relu_forward(a)))
+        assert np.array_equal(mask, np.packbits(a > 0, bitorder="little"))
+        assert np.array_equal(bits(abi.relu_bwd_mask(mask, g)), bits(ora.relu_backward(a, g)))
+
+
 def test_relu_reference_docstring_vectors(abi, kats):
     for case in kats["relu"]:
         x = np.array(case["x"])
