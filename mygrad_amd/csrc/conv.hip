@@ -573,9 +573,12 @@ struct Geometry {
 
 // The tap-major kernels address their operands with 32-bit byte offsets and mark
 // padding with an offset of 2 GiB, so every tensor they read must be smaller.
+// MYGRAD_HIP_BUFFER_LIMIT=bytes lowers that limit, so that the tests reach what larger tensors run on with
+// small ones (read whenever a plan is built, and part of the plan's key).
 bool fits_buffer_loads(const Geometry &g) {
   const long long elem = g.dtype == MG_F64 ? 8 : 4;
-  const long long limit = 1ll << 31;
+  const char *lower = getenv("MYGRAD_HIP_BUFFER_LIMIT");
+  const long long limit = lower ? std::min(1ll << 31, atoll(lower)) : 1ll << 31;
   return (long long)g.N * g.C * g.xvol * elem < limit && (long long)g.N * g.F * g.gvol * elem < limit &&
          (long long)(g.F + 15) * (g.C + 15) * g.wvol * elem < limit;  // packed filters: whole K tiles of rows, 4 values to a row
 }
@@ -1366,8 +1369,8 @@ int build_fwd_plan(const Geometry &g, Plan &pl) {
     return upload_plan(pl, t);
   }
   pl.depth = whole_channels(g, g.C);
-  pl.ragged = pl.depth > g.C;
   pl.tap_major = pl.depth != 0 && fits_buffer_loads(g);
+  pl.ragged = pl.tap_major && pl.depth > g.C;
   // Channels that do not fill K tiles (a first layer's one or three): the same kernel, its K
   // tiles 16 rows of the gather table each -- unless the problem is tiny (few launches matter
   // more) or MYGRAD_HIP_TABLE_ROWS=0 asks for the plain table-driven kernel.
@@ -1484,8 +1487,8 @@ int build_dgrad_plan(const Geometry &g, Plan &pl) {
   // whole steps: 3 channels 38.5 -> 28 us; with 16 channels the tap-major kernels are 4 us
   // ahead, and with 32 or 64 the table-driven kernel's few, long-running blocks cost 2 - 5 x.)
   pl.depth = whole_channels(g, g.F);
-  pl.ragged = pl.depth > g.F;
   pl.tap_major = pl.depth != 0 && fits_buffer_loads(g) && !(tiny_table(g, g.C, (long long)g.F * g.wvol) && g.C <= 8);
+  pl.ragged = pl.tap_major && pl.depth > g.F;
   // filter counts that fill no K tile (10, 20, ...): the tap-major kernel on rows of the gather
   // table, as in the forward pass (MYGRAD_HIP_TABLE_ROWS=0: the plain table-driven kernel)
   pl.table_rows = table_rows_on() && pl.depth == 0 && fits_buffer_loads(g) && !tiny_table(g, g.C, (long long)g.F * g.wvol);
@@ -2128,6 +2131,7 @@ int get_plan(ConvOp op, const mg_conv_desc *d, const Geometry &g, Plan **out) {
   if (const char *tile = getenv("MYGRAD_HIP_TILE")) key.append(tile);
   if (const char *tile = getenv("MYGRAD_HIP_WGRAD_TILE")) key.append("w").append(tile);
   if (const char *row = getenv("MYGRAD_HIP_FUSE_MIN_ROW")) key.append("r").append(row);
+  if (const char *limit = getenv("MYGRAD_HIP_BUFFER_LIMIT")) key.append("b").append(limit);
   auto it = plans().find(key);
   if (it == plans().end()) {
     if (plans().size() >= 256) {
@@ -2160,8 +2164,9 @@ int get_plan(ConvOp op, const mg_conv_desc *d, const Geometry &g, Plan **out) {
   return MG_OK;
 }
 
+// Whether there is a kernel for the plan in this tile shape; launches it if so.
 template <typename T, int BM, int BN, int BK, int WM, int WN, int NPH = 1, bool FOLD = false, bool ROWS = false, bool DEAD = false>
-void launch_gemm(GemmParams &gp, const Plan &pl, hipStream_t s) {
+bool launch_gemm(GemmParams &gp, const Plan &pl, hipStream_t s) {
   if constexpr (!DEAD && !ROWS && tap_gemm_dead_apart(BM, BN, NPH, (int)sizeof(T)))
     if (pl.ragged) return launch_gemm<T, BM, BN, BK, WM, WN, NPH, FOLD, ROWS, true>(gp, pl, s);
   if (pl.tap_major) {
@@ -2176,7 +2181,7 @@ void launch_gemm(GemmParams &gp, const Plan &pl, hipStream_t s) {
       if (pl.share_fixes > 0)
         hipLaunchKernelGGL((tail_fixup_kernel<T, BM, BN, NPH>), dim3((unsigned)ceil_div(BM * BN, 256), (unsigned)pl.share_fixes),
                            dim3(256), 0, s, gp);
-      return;
+      return true;
     }
     gp.items = (int)(pl.full_tiles + tail_tiles * pl.tail_split);
     const long long grid = std::min<long long>(gp.items, slots);
@@ -2191,10 +2196,13 @@ void launch_gemm(GemmParams &gp, const Plan &pl, hipStream_t s) {
     if (tail_tiles > 0)
       hipLaunchKernelGGL((tail_fixup_kernel<T, BM, BN, NPH>), dim3((unsigned)ceil_div(BM * BN, 256), (unsigned)tail_tiles),
                          dim3(256), 0, s, gp);
+    return true;
   } else if constexpr (NPH == 1 && !FOLD && !ROWS && !DEAD && BM % 48 != 0) {
     const dim3 grid((unsigned)pl.pos_blocks, (unsigned)pl.m_tiles);
     hipLaunchKernelGGL((gather_gemm_kernel<T, BM, BN, BK, WM, WN>), grid, dim3(256), 0, s, gp);
+    return true;
   }
+  return false;
 }
 
 // Bytes of partial sums the shared tail tiles of this plan need.
@@ -2244,15 +2252,13 @@ int run_gemm(GemmParams &gp, const Plan &pl, int tag, hipStream_t s) {
   ScopedTiming timed(tag);
   bool launched = false;
   if (pl.deep_k) {
-    launch_gemm<T, 16, 64, 4 * BK, 16, 16>(gp, pl, s);
-    launched = true;
+    launched = launch_gemm<T, 16, 64, 4 * BK, 16, 16>(gp, pl, s);
   }
   if constexpr (sizeof(T) == 8) {
     if (pl.tap_major && pl.bk == 2 * BK && !pl.table_rows && !pl.fold_row) {
 #define MG_LAUNCH_DEEP(TT, BM, BN, WM, WN)                \
   if (!launched && pl.bm == BM && pl.bn == BN) {          \
-    launch_gemm<TT, BM, BN, 2 * BK, WM, WN>(gp, pl, s);   \
-    launched = true;                                      \
+    launched = launch_gemm<TT, BM, BN, 2 * BK, WM, WN>(gp, pl, s); \
   }
       MG_GEMM_SHAPES(T, MG_LAUNCH_DEEP)
 #undef MG_LAUNCH_DEEP
@@ -2261,8 +2267,7 @@ int run_gemm(GemmParams &gp, const Plan &pl, int tag, hipStream_t s) {
   if (pl.table_rows) {
 #define MG_LAUNCH_ROWS(TT, BM, BN, WM, WN)                              \
   if (!launched && pl.bm == BM && pl.bn == BN) {                        \
-    launch_gemm<TT, BM, BN, 16, WM, WN, 1, false, true>(gp, pl, s);     \
-    launched = true;                                                    \
+    launched = launch_gemm<TT, BM, BN, 16, WM, WN, 1, false, true>(gp, pl, s); \
   }
     MG_GEMM_SHAPES(T, MG_LAUNCH_ROWS)
 #undef MG_LAUNCH_ROWS
@@ -2278,30 +2283,26 @@ int run_gemm(GemmParams &gp, const Plan &pl, int tag, hipStream_t s) {
   if (pl.fold_row && !launched) {
     if (pl.bk == 2 * BK && sizeof(T) == 8) {
       if (pl.bm == 48)
-        launch_gemm<T, 48, 256, (sizeof(T) == 8 ? 2 * BK : BK), 48, 64, 1, true>(gp, pl, s);
+        launched = launch_gemm<T, 48, 256, (sizeof(T) == 8 ? 2 * BK : BK), 48, 64, 1, true>(gp, pl, s);
       else
-        launch_gemm<T, 96, 128, (sizeof(T) == 8 ? 2 * BK : BK), 48, 64, 1, true>(gp, pl, s);
+        launched = launch_gemm<T, 96, 128, (sizeof(T) == 8 ? 2 * BK : BK), 48, 64, 1, true>(gp, pl, s);
     } else if (pl.bm == 48) {
-      launch_gemm<T, 48, 256, BK, 48, 64, 1, true>(gp, pl, s);
+      launched = launch_gemm<T, 48, 256, BK, 48, 64, 1, true>(gp, pl, s);
     } else {
-      launch_gemm<T, 96, 128, BK, 48, 64, 1, true>(gp, pl, s);
+      launched = launch_gemm<T, 96, 128, BK, 48, 64, 1, true>(gp, pl, s);
     }
-    launched = true;
   }
 #define MG_LAUNCH(TT, BM, BN, WM, WN)                     \
   if (!launched && pl.bm == BM && pl.bn == BN) {          \
-    launch_gemm<TT, BM, BN, BK, WM, WN>(gp, pl, s);       \
-    launched = true;                                      \
+    launched = launch_gemm<TT, BM, BN, BK, WM, WN>(gp, pl, s); \
   }
 #define MG_LAUNCH2(TT, BM, BN, WM, WN)                    \
   if (!launched && pl.bm == BM && pl.bn == BN) {          \
-    launch_gemm<TT, BM, BN, BK, WM, WN, 2>(gp, pl, s);    \
-    launched = true;                                      \
+    launched = launch_gemm<TT, BM, BN, BK, WM, WN, 2>(gp, pl, s); \
   }
 #define MG_LAUNCH4(TT, BM, BN, WM, WN)                    \
   if (!launched && pl.bm == BM && pl.bn == BN) {          \
-    launch_gemm<TT, BM, BN, BK, WM, WN, 4>(gp, pl, s);    \
-    launched = true;                                      \
+    launched = launch_gemm<TT, BM, BN, BK, WM, WN, 4>(gp, pl, s); \
   }
   if constexpr (sizeof(T) == 4) {
     if (pl.nph == 2) {
@@ -2309,8 +2310,7 @@ int run_gemm(GemmParams &gp, const Plan &pl, int tag, hipStream_t s) {
     } else if (pl.nph == 4 && pl.bk == 2 * BK) {
 #define MG_LAUNCH4_DEEP(TT, BM, BN, WM, WN)                      \
   if (!launched && pl.bm == BM && pl.bn == BN) {                 \
-    launch_gemm<TT, BM, BN, 2 * BK, WM, WN, 4>(gp, pl, s);       \
-    launched = true;                                             \
+    launched = launch_gemm<TT, BM, BN, 2 * BK, WM, WN, 4>(gp, pl, s); \
   }
       MG_FUSED4_SHAPES(T, MG_LAUNCH4_DEEP)
 #undef MG_LAUNCH4_DEEP

@@ -1007,6 +1007,34 @@ def test_conv_counts_that_fill_no_tile_in_place(abi, dtype, case):
         assert np.array_equal(abi.conv_dgrad(gn, x_shape, w, s, p, d)[0], dx[0])
 
 
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("x_shape,w_shape,s", [
+    ((2, 45, 41, 37), (128, 45, 3, 3), 1),   # ragged channels, forward on 128-row tiles
+    ((2, 128, 41, 37), (45, 128, 3, 3), 1),  # ragged filters, data gradient on 128-row tiles
+    ((5, 128, 41, 37), (45, 128, 3, 3), 2),
+    ((3, 1001, 400), (512, 1001, 1), 1),     # a matrix product
+])
+def test_ragged_counts_in_tensors_too_large_for_buffer_loads(abi, monkeypatch, dtype, x_shape, w_shape, s):
+    """What tensors of 2 GiB and more run on, reached with small ones: every pass launches a kernel and
+    writes its result."""
+    from mygrad_amd import _hip
+
+    monkeypatch.setenv("MYGRAD_HIP_BUFFER_LIMIT", "4096")
+    rng = np.random.default_rng(list(x_shape))
+    nd = len(w_shape) - 2
+    conf = (s,) * nd, (w_shape[2] // 2,) * nd, (1,) * nd
+    print("large", np.dtype(dtype).name, x_shape, w_shape, s, flush=True)
+    x, w = rng.integers(-3, 4, x_shape).astype(dtype), rng.integers(-2, 3, w_shape).astype(dtype)
+    want = direct.conv_forward(x, w, *conf).astype(dtype)
+    g = rng.integers(-2, 3, want.shape).astype(dtype)
+    assert np.array_equal(abi.conv_fwd(x, w, *conf), want)
+    assert "table-driven" in _hip.last_plan()
+    assert np.array_equal(abi.conv_dgrad(g, x_shape, w, *conf), direct.conv_backward_x(g, x_shape, w, *conf).astype(dtype))
+    assert "table-driven" in _hip.last_plan()
+    assert np.array_equal(abi.conv_wgrad(g, x, w_shape, *conf), direct.conv_backward_w(g, x, w_shape, *conf).astype(dtype))
+    assert "table-driven" in _hip.last_plan()
+
+
 KERNEL_VARIANT_CASES = [
     # x shape, w shape, stride, padding, dilation
     ((8, 128, 28, 28), (128, 128, 3, 3), (1, 1), (1, 1), (1, 1)),   # 128-row tiles, wgrad 128x128
