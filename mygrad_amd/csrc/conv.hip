@@ -18,6 +18,7 @@
 
 #include <algorithm>
 #include <array>
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -718,26 +719,24 @@ int check_desc(const mg_conv_desc *d, Geometry *g) {
   return MG_OK;
 }
 
-// Row tile: the one whose rounded-up rows cost least, at the relative cost of a row in a tile of that
-// height (`thirds`: the heights that are multiples of 48 are built).  The costs are the rates of the
-// tiles on row counts that they divide, 64 channels, 3x3 at 56x56 and 9 taps along 9409 positions:
-// single precision 125 / 122 / 124 / 119 / 115 / 92 TFLOP/s for 128 / 96 / 64 / 48 / 32 / 16 rows,
-// double 54 / 54 / 51 / 48 / 52 / 40.  (45 rows: 86 -> 113 TFLOP/s with 48 instead of three times 16,
-// 83 rows: 81 -> 106 with 96 instead of six times 16, 160 rows: 107 -> 117 with 32 instead of 64.)
-int pick_bm(int M, bool thirds, bool f64) {
-  struct Rows {
-    int bm;
-    double cost, cost64;
-  };
-  static const Rows cands[] = {{128, 1.00, 1.00}, {96, 1.02, 1.01}, {64, 1.00, 1.06}, {48, 1.04, 1.11}, {32, 1.08, 1.05}, {16, 1.36, 1.34}};
-  int best = 16;
-  double least = 0;
-  for (const Rows &c : cands) {
-    if (c.bm % 48 == 0 && !thirds) continue;
-    const double cost = (double)(ceil_div(M, c.bm) * c.bm) * (f64 ? c.cost64 : c.cost);
-    if (least == 0 || cost < least) best = c.bm, least = cost;
-  }
-  return best;
+// The largest row tile whose round-up waste stays small.
+int rows_of_little_waste(int M) {
+  for (int c : {128, 64, 32, 16})
+    if (ceil_div(M, c) * c - M <= M / 8) return c;
+  return 16;
+}
+
+// Row tile of the table-driven kernel: that one, and 16 rows (with the K tile four times as deep, see
+// deepen_if_tiny) for a `tiny` problem whose 16 x 64 tiles number no more than three per unit: what
+// counts there is how many blocks share the chain of K tiles.  Measured on 122 such passes, 16 rows
+// against the best of the other heights: 5.6 us instead of 12 - 20 (2 - 700 blocks), 13 - 18 instead of
+// 9 - 11 beyond (1000 - 2700 blocks; from there on at least 32 rows).
+int table_driven_rows(int M, const std::vector<long long> &phase_npos, bool tiny) {
+  const int bm = rows_of_little_waste(M);
+  if (!tiny || M <= 16) return bm;
+  long long blocks = 0;
+  for (long long n : phase_npos) blocks += ceil_div(n, 64) * ceil_div(M, 16);
+  return blocks <= 3ll * runtime().props.multiProcessorCount ? 16 : std::max(bm, 32);
 }
 
 template <typename K>
@@ -777,7 +776,7 @@ int resident_blocks(K kernel, int threads) {
 
 // Blocks of the persistent tap-major gather-GEMM that a compute unit holds at once.
 template <typename T>
-int gemm_blocks_per_cu(int bm, int bn, int nph = 1, int bk = 0) {
+int ask_gemm_blocks_per_cu(int bm, int bn, int nph, int bk) {
   constexpr int BK = sizeof(T) == 8 ? 8 : 16;
 #define MG_OCC(TT, BM, BN, WM, WN)                                                                                       \
   if (bm == BM && bn == BN)                                                                                              \
@@ -806,6 +805,15 @@ int gemm_blocks_per_cu(int bm, int bn, int nph = 1, int bk = 0) {
   return 1;
 }
 
+// (the runtime's answer, asked for once per kernel: a plan compares up to nine)
+template <typename T>
+int gemm_blocks_per_cu(int bm, int bn, int nph = 1, int bk = 0) {
+  static std::map<std::array<int, 4>, int> known;
+  int &n = known[{bm, bn, nph, bk}];
+  if (n == 0) n = ask_gemm_blocks_per_cu<T>(bm, bn, nph, bk);
+  return n;
+}
+
 // Picks the tile of the gather-GEMM, how many persistent blocks run per compute unit
 // and how the last, partial round of tiles is shared out.  With r blocks per unit the
 // grid has r x CUs blocks; block b takes tiles b, b + grid, ...  A unit's MFMA pipes are
@@ -814,7 +822,7 @@ int gemm_blocks_per_cu(int bm, int bn, int nph = 1, int bk = 0) {
 // units busy; each of those is cut into `split` K slices so that every unit gets
 // about the same share of them (the busiest gets ceil(rem x split / CUs) slices).
 // Smaller tiles give more tiles (finer balance, less padding) at some cost in operand
-// reuse.  Kernels that do not stream run one block per tile (r = 1 in this arithmetic:
+// reuse; the shapes, each shared out in its best way, are compared by tile_time.  Kernels that do not stream run one block per tile (r = 1 in this arithmetic:
 // the hardware refills a unit as soon as a block leaves).
 // Fewest K tiles in a block's share of the leftover tiles (see build_shares).
 constexpr long long kMinRun = 8;
@@ -825,12 +833,67 @@ struct TileChoice {
   long long tiles;
 };
 
-TileChoice choose_tile(int M, const std::vector<long long> &phase_npos, int min_ktiles, bool tap_major, size_t elem, int nph = 1, int bk = 0,
-                       int avg_ktiles = -1) {
+// What a tap-major gather-GEMM is bound by, per tile shape: the chain of K tiles that one block works
+// off, at `step` microseconds for 16 rows of K (a trip to memory and the barriers, whatever the other
+// blocks do), or the matrix pipes of the unit with the most K tiles, at `rate` (single precision) or
+// `rate64` of their peak.  Fitted to 5843 timed pairs of a pass (905 convolutions and products of 1e4 to
+// 3e10 flops, forward and data gradient) and a tile shape forced on it.  Of the shapes of a pass the
+// one that costs least here is 1.2 % slower than the best on average (5.8 % at the 95th percentile; 3 %
+// and 18 % under choose_tile's limit on mean_chain); the shape whose rounded-up rows cost least is 18 %
+// slower (68 %), because how many blocks share a small pass counts for more than its padding.  (Double precision is bound by the pipes throughout.)
+struct TileRate {
+  int nph, bm, bn;
+  double step, rate, rate64;
+};
+constexpr TileRate kTileRates[] = {
+    {1, 16, 256, 0.50, 0.42, 0.42}, {1, 32, 128, 0.35, 0.59, 0.62},  {1, 32, 256, 0.55, 0.63, 0.64}, {1, 48, 256, 0.62, 0.70, 0.67},
+    {1, 64, 128, 0.47, 0.77, 0.70}, {1, 64, 256, 0.78, 0.83, 0.00},  {1, 96, 128, 0.56, 0.82, 0.80}, {1, 128, 64, 0.27, 0.81, 0.87},
+    {1, 128, 128, 0.63, 0.86, 0.0}, {2, 16, 256, 0.53, 0.50, 0.00},  {2, 32, 256, 0.47, 0.70, 0.00}, {2, 64, 128, 0.45, 0.82, 0.00},
+    {2, 128, 64, 0.23, 0.82, 0.00}, {4, 16, 256, 0.20, 0.38, 0.00},  {4, 32, 128, 0.20, 0.51, 0.00}, {4, 64, 64, 0.50, 0.78, 0.00}};
+
+// Microseconds of the launch described by `t` (without what every shape costs alike): `ktiles` K tiles of
+// `bk` rows per tile, `resident` blocks to a unit.
+double tile_time(const TileChoice &t, long long ktiles, int bk, size_t elem, int nph, int resident, bool table_rows) {
+  const double cus = runtime().props.multiProcessorCount;
+  const double left = (double)(t.tiles - t.full_tiles), kt = (double)ktiles, grid = resident * cus;
+  double chain, work, slices = 0;  // K tiles one after the other in a block; K tiles of the busiest unit; tiles of partial sums
+  if (t.tail_split == 0) {
+    const double runs = std::max(1.0, std::min(grid, std::floor(left * kt / (double)kMinRun))), run = std::ceil(left * kt / runs);
+    work = (double)t.full_tiles / cus * kt + run * std::ceil(runs / cus);
+    chain = std::ceil((double)t.full_tiles / grid) * kt + run;
+    slices = (runs - 1) + std::min(left, runs - 1);
+  } else {
+    const double share = std::ceil(kt / t.tail_split), items = left * t.tail_split;
+    work = std::ceil((double)t.full_tiles / cus) * kt + std::ceil(items / cus) * share;
+    chain = std::ceil((double)t.full_tiles / grid) * kt + std::ceil(items / grid) * share;
+    if (t.tail_split > 1) slices = items;
+  }
+  const TileRate *r = kTileRates;
+  while (r->nph != nph || r->bm != t.bm || r->bn != t.bn) ++r;
+  const double tile = (double)t.bm * t.bn;
+  double a = 0, b = work * 2.0 * tile * bk * cus / (elem == 8 ? 78.6e6 * r->rate64 : 157.3e6 * r->rate);
+  if (elem == 4) a = chain * r->step * bk / 16;
+  if (elem == 4 && table_rows) a *= 2.1, b *= 1.2;  // (its gathers look up a row of the table per element)
+  return std::sqrt(std::sqrt(a * a * a * a + b * b * b * b)) + slices * tile * (double)elem * nph * 2.0 / 4.0e6;
+}
+
+// K tiles that one accumulator sums up without a break, on average over the results.
+double mean_chain(const TileChoice &t, long long ktiles, int resident) {
+  const double kt = (double)ktiles, left = (double)(t.tiles - t.full_tiles);
+  double run = std::ceil(kt / std::max(t.tail_split, 1));
+  if (t.tail_split == 0) {
+    const double runs = std::max(1.0, std::min((double)resident * runtime().props.multiProcessorCount, std::floor(left * kt / (double)kMinRun)));
+    run = std::min(kt, std::ceil(left * kt / runs));
+  }
+  return ((double)t.full_tiles * kt + left * run) / (double)t.tiles;
+}
+
+TileChoice choose_tile(int M, const std::vector<long long> &phase_npos, int min_ktiles, bool tap_major, size_t elem, int nph, int bk, bool table_rows,
+                       bool tiny, int avg_ktiles = -1) {
   if (avg_ktiles < 0) avg_ktiles = min_ktiles;  // K tiles of an average tile (phases of a data gradient differ)
   struct Cfg {
     int bm, bn;
-    double penalty;  // relative cost of a flop in this tile shape
+    double penalty;  // relative cost of a flop, among shapes of one height
     bool tap_only;
   };
   static const Cfg plain[] = {{128, 128, 1.00, false}, {128, 64, 1.05, true}, {96, 128, 1.00, true},   {64, 256, 1.00, false},
@@ -858,13 +921,25 @@ TileChoice choose_tile(int M, const std::vector<long long> &phase_npos, int min_
   for (int ci = 0; ci < ncfgs; ++ci)
     forced_fits |= cfgs[ci].bm == forced.bm && cfgs[ci].bn == forced.bn && (!cfgs[ci].tap_only || tap_major) &&
                    !(tap_major && elem == 8 && cfgs[ci].bn * cfgs[ci].bm >= 128 * 128);  // (no such double-precision tile)
-  const int bm = forced_fits ? forced.bm : nph == 4 ? std::min(pick_bm(M, false, false), 64) : pick_bm(M, tap_major && nph == 1, elem == 8);
+  const int bm = forced_fits ? forced.bm : tap_major ? 0 : table_driven_rows(M, phase_npos, tiny);  // 0: whichever costs least
   const int cus = runtime().props.multiProcessorCount;
-  TileChoice best{};
-  double best_cost = 0;
+  struct Candidate {
+    TileChoice tile;
+    double time, chain;
+  };
+  std::vector<Candidate> candidates;
+  // A sum's rounding errors grow with the number of terms that one accumulator takes, and how often K is
+  // cut differs between the shapes of a small pass: none is taken whose chain is longer than that of
+  // the height of little waste, at the width that wastes least of the rounds.  (Without this limit single
+  // errors against 64 bits were 2.4 times as large, in single precision: (353,777) @ (777,2631) 2.4e-7
+  // on 128 rows, 5.0e-7 on 32.)
+  const int usual = std::min(rows_of_little_waste(M), nph == 4 ? 64 : 128);
+  double usual_cost = 0, longest = 0;
   for (int ci = 0; ci < ncfgs; ++ci) {
     const Cfg &c = cfgs[ci];
-    if (c.bm != bm || (c.tap_only && !tap_major) || (forced_fits && c.bn != forced.bn)) continue;
+    TileChoice best{};  // of this shape: how many blocks per unit, how the last round is shared out
+    double best_cost = 0;
+    if ((bm != 0 && c.bm != bm) || (c.tap_only && !tap_major) || (forced_fits && c.bn != forced.bn)) continue;
     // 64x64 fp64 wave tiles hold 128 accumulator registers: only one 8-wave block
     // fits on a compute unit, so the tap-major kernels use the half-size shapes
     if (tap_major && elem == 8 && c.bn * c.bm >= 128 * 128) continue;
@@ -918,7 +993,7 @@ TileChoice choose_tile(int M, const std::vector<long long> &phase_npos, int min_
           const double fix_seconds = slices * c.bm * c.bn * (double)elem * nph * 2.0 / 4.0e12 + 4e-6;
           units += fix_seconds / tile_seconds;
         }
-        const double cost = units * alone * c.bm * c.bn * c.penalty;
+        const double cost = units * alone;
         if (best.bm == 0 || cost < best_cost) {
           best = t;
           best_cost = cost;
@@ -942,7 +1017,7 @@ TileChoice choose_tile(int M, const std::vector<long long> &phase_npos, int min_
           if (t.tail_split > 1) t.full_tiles = (int)(t.tiles - rem);
         }
       }
-      const double cost = ((double)(t.tiles / grid) * r + tail) * alone * c.bm * c.bn * c.penalty;
+      const double cost = ((double)(t.tiles / grid) * r + tail) * alone;
       if (best.bm == 0 || cost < best_cost) {
         best = t;
         best_cost = cost;
@@ -970,15 +1045,23 @@ TileChoice choose_tile(int M, const std::vector<long long> &phase_npos, int min_
           if (u.tail_split > 1) u.full_tiles = (int)(q * cus);
           time += share;
         }
-        const double ucost = time * c.bm * c.bn * c.penalty;
-        if (q > 0 && ucost < best_cost) {
+        if (q > 0 && time < best_cost) {
           best = u;
-          best_cost = ucost;
+          best_cost = time;
         }
       }
     }
+    if (!tap_major) return best;
+    const int resident = stream ? best.blocks_per_cu : elem == 8 ? gemm_blocks_per_cu<double>(c.bm, c.bn, 1, bk) : gemm_blocks_per_cu<float>(c.bm, c.bn, nph, bk);
+    const long long ktiles = std::max(avg_ktiles, 1);
+    candidates.push_back({best, tile_time(best, ktiles, bk, elem, nph, resident, table_rows), mean_chain(best, ktiles, resident)});
+    const double cost = best_cost * c.bm * c.bn * c.penalty;
+    if (c.bm == usual && (longest == 0 || cost < usual_cost)) usual_cost = cost, longest = candidates.back().chain;
   }
-  return best;
+  const Candidate *chosen = nullptr;
+  for (const Candidate &c : candidates)
+    if ((longest == 0 || c.chain <= 1.05 * longest) && (!chosen || c.time < chosen->time)) chosen = &c;
+  return chosen ? chosen->tile : TileChoice{};
 }
 
 void set_divisors(Phase &ph) {
@@ -1386,7 +1469,7 @@ int build_fwd_plan(const Geometry &g, Plan &pl) {
   {
     const long long ktiles = pl.table_rows ? ceil_div((long long)g.C * g.wvol, bk)
                              : pl.tap_major ? g.wvol * (pl.depth / bk) : ceil_div((long long)g.C * g.wvol, bk);
-    const TileChoice tc = choose_tile(g.F, {(long long)g.N * g.gvol}, (int)ktiles, pl.tap_major, g.dtype == MG_F64 ? 8 : 4, 1, bk);
+    const TileChoice tc = choose_tile(g.F, {(long long)g.N * g.gvol}, (int)ktiles, pl.tap_major, g.dtype == MG_F64 ? 8 : 4, 1, bk, pl.table_rows, is_tiny(g));
     pl.bm = tc.bm, pl.bn = tc.bn, pl.m_tiles = tc.m_tiles, pl.full_tiles = tc.full_tiles, pl.tail_split = tc.tail_split, pl.blocks_per_cu = tc.blocks_per_cu;
     deepen_if_tiny(g, pl);
   }
@@ -1657,7 +1740,7 @@ int build_dgrad_plan(const Geometry &g, Plan &pl) {
     coarse.blk_begin = 0;
     coarse.npos = (int)((long long)g.N * coarse.J[0] * coarse.J[1] * coarse.J[2]);
     set_divisors(coarse);
-    const TileChoice tc = choose_tile((int)nphase * g.C, {(long long)coarse.npos}, coarse.k_count, true, g.dtype == MG_F64 ? 8 : 4, 1, bk);
+    const TileChoice tc = choose_tile((int)nphase * g.C, {(long long)coarse.npos}, coarse.k_count, true, g.dtype == MG_F64 ? 8 : 4, 1, bk, false, false);
     if (tc.bm != 0 && coarse.k_count > 0) {
       pl.bm = tc.bm, pl.bn = tc.bn, pl.m_tiles = tc.m_tiles, pl.full_tiles = tc.full_tiles, pl.tail_split = tc.tail_split, pl.blocks_per_cu = tc.blocks_per_cu;
       pl.phase_rows = g.C;
@@ -1742,7 +1825,7 @@ int build_dgrad_plan(const Geometry &g, Plan &pl) {
     coarse.blk_begin = 0;
     coarse.npos = (int)((long long)g.N * coarse.J[0] * coarse.J[1] * coarse.J[2]);
     set_divisors(coarse);
-    const TileChoice tc = choose_tile(g.C, {(long long)coarse.npos}, (int)total_ktiles, true, 4, pl.nph, fbk);
+    const TileChoice tc = choose_tile(g.C, {(long long)coarse.npos}, (int)total_ktiles, true, 4, pl.nph, fbk, false, false);
     if (tc.bm != 0 && total_ktiles > 0) {
       pl.bm = tc.bm, pl.bn = tc.bn, pl.m_tiles = tc.m_tiles, pl.full_tiles = tc.full_tiles, pl.tail_split = tc.tail_split, pl.blocks_per_cu = tc.blocks_per_cu;
       t.phases.push_back(coarse);
@@ -1773,11 +1856,11 @@ int build_dgrad_plan(const Geometry &g, Plan &pl) {
     long long all_ktiles = 0, all_pos = 0;
     for (const PhaseTaps &pt : found) {
       const long long ntaps = (long long)pt.taps[0].size() * pt.taps[1].size() * pt.taps[2].size();
-      all_ktiles += ceil_div(ntaps * g.F, bk) * pt.ph.npos;
+      all_ktiles += (pl.tap_major && !pl.table_rows ? ntaps * (pl.depth / bk) : ceil_div(ntaps * g.F, bk)) * pt.ph.npos;
       all_pos += pt.ph.npos;
     }
-    const TileChoice tc = choose_tile(g.C, npos, (int)std::max<long long>(min_ktiles, 0), pl.tap_major, g.dtype == MG_F64 ? 8 : 4, 1, bk,
-                                      (int)(all_ktiles / std::max<long long>(all_pos, 1)));
+    const TileChoice tc = choose_tile(g.C, npos, (int)std::max<long long>(min_ktiles, 0), pl.tap_major, g.dtype == MG_F64 ? 8 : 4, 1, bk, pl.table_rows,
+                                      is_tiny(g), (int)(all_ktiles / std::max<long long>(all_pos, 1)));
     pl.bm = tc.bm, pl.bn = tc.bn, pl.m_tiles = tc.m_tiles, pl.full_tiles = tc.full_tiles, pl.tail_split = tc.tail_split, pl.blocks_per_cu = tc.blocks_per_cu;
     deepen_if_tiny(g, pl);
   }

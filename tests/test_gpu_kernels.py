@@ -1035,6 +1035,53 @@ def test_ragged_counts_in_tensors_too_large_for_buffer_loads(abi, monkeypatch, d
     assert "table-driven" in _hip.last_plan()
 
 
+# A pass that does not fill the device is shared out by how many blocks its tiles make, not only by their
+# padding: (dtype, x, w, stride, padding, pass, what the plan must say, what it must not)
+SMALL_PASSES = [
+    (np.float32, (1, 7, 17, 28), (37, 7, 3, 3), 1, 0, "fwd", "tile 16x64x", None),      # 24 blocks, 2 on 64 rows
+    (np.float32, (4, 4, 14, 69), (84, 4, 5, 3), (1, 2), (0, 1), "fwd", "tile 16x64x", None),
+    (np.float32, (64, 8, 56, 56), (24, 8, 1, 1), 1, 0, "fwd", "table-driven", "tile 16x64x"),  # thousands of blocks either way
+    (np.float64, (25, 7, 19, 29), (102, 7, 1, 3), 2, 0, "fwd", "tile 16x64x", None),
+    (np.float64, (8, 259, 26, 31), (27, 259, 3, 3), (1, 2), (0, 2), "dx", "tap-major", "tile 96x128x"),
+    (np.float64, (1, 808, 3317), (93, 808, 1), 1, 0, "dx", "tap-major", "tile 96x128x"),
+    (np.float64, (1, 184, 375), (41, 184, 1), 1, 0, "fwd", "tap-major", "tile 48x256x"),
+    (np.float32, (1, 72, 23, 42), (55, 72, 3, 1), 1, (1, 0), "fwd", "tap-major", "tile 64x256x"),
+    (np.float32, (1, 216, 171), (96, 216, 1), 1, 0, "fwd", "tap-major", "tile 96x128x"),
+]
+
+
+@pytest.mark.parametrize("case", range(len(SMALL_PASSES)))
+def test_small_passes_are_spread_over_the_device(abi, case):
+    from mygrad_amd import _hip
+
+    dtype, x_shape, w_shape, s, p, which, has, has_not = SMALL_PASSES[case]
+    nd = len(x_shape) - 2
+    s, p = ((v,) * nd if isinstance(v, int) else v for v in (s, p))
+    rng = np.random.default_rng(case)
+    x, w = rng.integers(-3, 4, x_shape).astype(dtype), rng.integers(-2, 3, w_shape).astype(dtype)
+    want = direct.conv_forward(x, w, s, p, (1,) * nd).astype(dtype)
+    if which == "fwd":
+        got = abi.conv_fwd(x, w, s, p, 1)
+    else:
+        g = rng.integers(-2, 3, want.shape).astype(dtype)
+        want = direct.conv_backward_x(g, x_shape, w, s, p, (1,) * nd).astype(dtype)
+        got = abi.conv_dgrad(g, x_shape, w, s, p, 1)
+    plan = _hip.last_plan()
+    assert np.array_equal(got, want)
+    assert has in plan and (has_not is None or has_not not in plan), plan
+
+
+@pytest.mark.parametrize("m,k,n", [(353, 777, 2631), (622, 1357, 491), (463, 102, 2473)])
+def test_small_products_add_up_no_longer_chains(abi, m, k, n):
+    """Spreading K over blocks also shortens the sum that one accumulator takes: the bound is what these products
+    showed where their K was cut (2.4e-7, 2.2e-7, 1.6e-7), a third above it; uncut they show up to 5.0e-7."""
+    rng = np.random.default_rng(m)
+    a, b = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((k, n)).astype(np.float32)
+    want = a.astype(np.float64) @ b
+    got = abi.conv_fwd(b[None], a[:, :, None], 1, 0, 1)[0]
+    assert np.linalg.norm(got - want) <= 3.3e-7 * np.linalg.norm(want)
+
+
 KERNEL_VARIANT_CASES = [
     # x shape, w shape, stride, padding, dilation
     ((8, 128, 28, 28), (128, 128, 3, 3), (1, 1), (1, 1), (1, 1)),   # 128-row tiles, wgrad 128x128
