@@ -730,13 +730,14 @@ int rows_of_little_waste(int M) {
 // deepen_if_tiny) for a `tiny` problem whose 16 x 64 tiles number no more than three per unit: what
 // counts there is how many blocks share the chain of K tiles.  Measured on 122 such passes, 16 rows
 // against the best of the other heights: 5.6 us instead of 12 - 20 (2 - 700 blocks), 13 - 18 instead of
-// 9 - 11 beyond (1000 - 2700 blocks; from there on at least 32 rows).
-int table_driven_rows(int M, const std::vector<long long> &phase_npos, bool tiny) {
+// 9 - 11 beyond (1000 - 2700 blocks; from there on at least 32 rows, and in double precision, where taller
+// tiles hold a block per unit, no more: 32 x 256 10.5 us, 64 x 256 13.4, 128 x 128 12.8).
+int table_driven_rows(int M, const std::vector<long long> &phase_npos, bool tiny, bool f64) {
   const int bm = rows_of_little_waste(M);
   if (!tiny || M <= 16) return bm;
   long long blocks = 0;
   for (long long n : phase_npos) blocks += ceil_div(n, 64) * ceil_div(M, 16);
-  return blocks <= 3ll * runtime().props.multiProcessorCount ? 16 : std::max(bm, 32);
+  return blocks <= 3ll * runtime().props.multiProcessorCount ? 16 : f64 ? 32 : std::max(bm, 32);
 }
 
 template <typename K>
@@ -838,8 +839,8 @@ struct TileChoice {
 // blocks do), or the matrix pipes of the unit with the most K tiles, at `rate` (single precision) or
 // `rate64` of their peak.  Fitted to 5843 timed pairs of a pass (905 convolutions and products of 1e4 to
 // 3e10 flops, forward and data gradient) and a tile shape forced on it.  Of the shapes of a pass the
-// one that costs least here is 1.2 % slower than the best on average (5.8 % at the 95th percentile; 3 %
-// and 18 % under choose_tile's limit on mean_chain); the shape whose rounded-up rows cost least is 18 %
+// one that costs least here is 1.2 % slower than the best on average (5.8 % at the 95th percentile; 2.3 %
+// and 13 % under choose_tile's limit on mean_chain); the shape whose rounded-up rows cost least is 18 %
 // slower (68 %), because how many blocks share a small pass counts for more than its padding.  (Double precision is bound by the pipes throughout.)
 struct TileRate {
   int nph, bm, bn;
@@ -921,16 +922,16 @@ TileChoice choose_tile(int M, const std::vector<long long> &phase_npos, int min_
   for (int ci = 0; ci < ncfgs; ++ci)
     forced_fits |= cfgs[ci].bm == forced.bm && cfgs[ci].bn == forced.bn && (!cfgs[ci].tap_only || tap_major) &&
                    !(tap_major && elem == 8 && cfgs[ci].bn * cfgs[ci].bm >= 128 * 128);  // (no such double-precision tile)
-  const int bm = forced_fits ? forced.bm : tap_major ? 0 : table_driven_rows(M, phase_npos, tiny);  // 0: whichever costs least
+  const int bm = forced_fits ? forced.bm : tap_major ? 0 : table_driven_rows(M, phase_npos, tiny, elem == 8);  // 0: whichever costs least
   const int cus = runtime().props.multiProcessorCount;
   struct Candidate {
     TileChoice tile;
     double time, chain;
   };
   std::vector<Candidate> candidates;
-  // A sum's rounding errors grow with the number of terms that one accumulator takes, and how often K is
-  // cut differs between the shapes of a small pass: none is taken whose chain is longer than that of
-  // the height of little waste, at the width that wastes least of the rounds.  (Without this limit single
+  // A sum's rounding errors grow with the square root of the terms that one accumulator takes, and how
+  // often K is cut differs between the shapes of a small pass: none is taken whose chain is more than a
+  // fifth longer than that of the height of little waste, at the width that wastes least of the rounds.  (Without this limit single
   // errors against 64 bits were 2.4 times as large, in single precision: (353,777) @ (777,2631) 2.4e-7
   // on 128 rows, 5.0e-7 on 32.)
   const int usual = std::min(rows_of_little_waste(M), nph == 4 ? 64 : 128);
@@ -1060,7 +1061,7 @@ TileChoice choose_tile(int M, const std::vector<long long> &phase_npos, int min_
   }
   const Candidate *chosen = nullptr;
   for (const Candidate &c : candidates)
-    if ((longest == 0 || c.chain <= 1.05 * longest) && (!chosen || c.time < chosen->time)) chosen = &c;
+    if ((longest == 0 || c.chain <= 1.2 * longest) && (!chosen || c.time < chosen->time)) chosen = &c;
   return chosen ? chosen->tile : TileChoice{};
 }
 
