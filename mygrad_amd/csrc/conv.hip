@@ -661,6 +661,7 @@ struct Plan {
   // wgrad
   int splits = 1;
   int kchunk = 0;
+  int run_tiles = 0;  // WgradParams::run_tiles
   char note[200] = "";  // what mg_last_plan() reports after a call that ran this plan
 };
 
@@ -1950,35 +1951,14 @@ int build_dgrad_plan(const Geometry &g, Plan &pl) {
   X(T, 32, 64, (sizeof(T) == 8 ? 32 : 64), 32, 16)                                     \
   X(T, 16, 64, (sizeof(T) == 8 ? 32 : 64), 16, 16)
 
-// Blocks of the filter-gradient kernel that fit on one compute unit at a time.
-// Row tile of the filter gradient for F filters, at most `limit` rows: the one whose rounded-up rows
-// cost least at the relative cost of a row (the last tile is moved back to end with the last filter, so
-// a tile has no more rows than there are filters).  The costs are the tiles' rates on filter counts
-// that they divide: single precision 122 / 125 / 117 / 109 / 80 TFLOP/s with 128 / 64 / 48 / 32 / 16 rows, double
-// 50 / 50 / 45 / 45 / 36 (83 filters: 71 TFLOP/s on 16 rows, 94 on 32; 80 filters: 78 and 91).
-int wgrad_rows(int F, int limit) {
-  struct Rows {
-    int bm;
-    double cost;
-  };
-  static const Rows cands[] = {{128, 1.00}, {64, 1.00}, {48, 1.06}, {32, 1.12}, {16, 1.50}};
-  int best = 0;
-  double least = 0;
-  for (const Rows &c : cands) {
-    if (F < c.bm || c.bm > limit) continue;
-    const double cost = (double)(ceil_div(F, c.bm) * c.bm) * c.cost;
-    if (least == 0 || cost < least) best = c.bm, least = cost;
-  }
-  return best;
-}
-
 // Tile shapes that only the table-row mode of the tap-major filter-gradient kernel has.
 #define MG_WGRAD_TABLE_SHAPES(T, X)                \
   X(T, 64, 80, (sizeof(T) == 8 ? 32 : 64), 16, 80) \
   X(T, 64, 32, (sizeof(T) == 8 ? 32 : 64), 32, 16)
 
+// Blocks of the filter-gradient kernel that fit on one compute unit at a time.
 template <typename T>
-int wgrad_blocks_per_cu(int bm, int bn, bool tap_major) {
+int ask_wgrad_blocks_per_cu(int bm, int bn, bool tap_major) {
 #define MG_OCC_TABLE(TT, BM, BN, BK, WM, WN) \
   if (bm == BM && bn == BN && tap_major) return resident_blocks(tap_wgrad_kernel<TT, BM, BN, BK, WM, WN, true, true>, 512);
   MG_WGRAD_TABLE_SHAPES(T, MG_OCC_TABLE)
@@ -1991,6 +1971,14 @@ int wgrad_blocks_per_cu(int bm, int bn, bool tap_major) {
   MG_WGRAD_SHAPES(T, MG_OCC)
 #undef MG_OCC
   return 1;
+}
+// (the runtime's answer, asked for once per kernel)
+template <typename T>
+int wgrad_blocks_per_cu(int bm, int bn, bool tap_major) {
+  static std::map<std::array<int, 3>, int> known;
+  int &n = known[{bm, bn, tap_major}];
+  if (n == 0) n = ask_wgrad_blocks_per_cu<T>(bm, bn, tap_major);
+  return n;
 }
 
 // The position table of the tap-major filter-gradient kernel: row idx describes position
@@ -2091,52 +2079,82 @@ int build_wgrad_plan(const Geometry &g, Plan &pl) {
     }
     return std::max<long long>(1, std::min(slots / tiles, max_splits));
   };
-  // Tap-major candidates in the order of preference: the first shape wins that has the row tile for F
-  // filters (wgrad_rows), wastes
-  // little on padding the columns to whole tiles and still fills most block slots of the device
-  // with tiles x K splits.  128 x 128 re-reads grad and x least.  With 64 filters the tile is square
-  // with the K tile 64 deep (half the barriers, one column group per gathering thread): tiles of
-  // 64 x 192 and 64 x 128 with K tiles of 32, forced in turn on four layers with 64 filters, were
-  // 3 - 13 % slower (3x3 at 56x56: 240 / 250 / 294 us; 5x5 dilated: 173 / 192 / 197 us) and are
-  // no longer built.
+  // Tap-major candidates: rows x columns x K tile, and what a block of the shape is bound by, as for the
+  // gather-GEMM (TileRate): `step` microseconds per K tile of a block's chain, `rate` of the peak of the
+  // matrix pipes.  Fitted to 6130 timed (filter gradient, shape, K splits) of 142 layers and products;
+  // shape and splits that cost least are 2.4 % slower than the best on average (10 % at the 95th
+  // percentile).  Fixing the rows by their padding and the splits afterwards, to what fits in one round
+  // of blocks, is 10 % slower (37 %): between half a round and a whole one the empty slots stay empty.
+  // Tiles of 64 x 192 and 64 x 128 with K tiles of 32, forced in turn on four layers with 64 filters,
+  // were 3 - 13 % slower than 64 x 64 with its K tile 64 deep (3x3 at 56x56: 240 / 250 / 294 us; 5x5
+  // dilated: 173 / 192 / 197 us) and are not built.  32 x 64 double-precision tiles are bound by LDS
+  // reads (the 4x4x4 MFMA takes an operand per 512 flops), which 32 x 128 halves; in single precision
+  // that shape measured slower.
   struct Cand {
     int bm, bn, bk;
+    double step, rate;
   };
-  const Cand cands[] = {{128, 128, f64 ? 16 : 32}, {64, 64, f64 ? 32 : 64}, {48, 64, f64 ? 32 : 64}, {32, 128, f64 ? 16 : 32},
-                        {32, 64, f64 ? 32 : 64},   {16, 64, f64 ? 32 : 64}};
+  static const Cand cands32[] = {{128, 128, 32, 0.01, 0.78}, {64, 64, 64, 0.01, 0.69}, {48, 64, 64, 0.01, 0.64}, {32, 64, 64, 0.59, 0.585}, {16, 64, 64, 0.33, 0.405}};
+  static const Cand cands64[] = {{128, 128, 16, 0.82, 0.76}, {64, 64, 32, 0.73, 0.71}, {48, 64, 32, 0.71, 0.67}, {32, 128, 16, 0.60, 0.71}, {32, 64, 32, 0.51, 0.64},
+                                 {16, 64, 32, 0.42, 0.49}};
+  const Cand *first = f64 ? cands64 : cands32, *last = f64 ? cands64 + 6 : cands32 + 5;
+  auto per_cu = [&](const Cand &c) { return f64 ? wgrad_blocks_per_cu<double>(c.bm, c.bn, true) : wgrad_blocks_per_cu<float>(c.bm, c.bn, true); };
+  // (Filters that fill no whole tiles: the last tile is moved back to end with the last filter, or, where the
+  // only one has up to 15 rows beyond them, those are computed and not stored.)
+  auto fits = [&](const Cand &c) { return c.bm - g.F < 16; };
+  auto chunk_of = [&](const Cand &c, long long sp) { return ceil_div(ceil_div(kpos, c.bk), sp) * c.bk; };
   long long best_splits = 1;
   pl.bm = 0;
   // MYGRAD_HIP_WGRAD_TILE="rows,columns" (diagnostics and the tests of every tile shape; part of the
   // plan's key): that candidate or, where it does not apply, the usual choice
   int forced_bm = 0, forced_bn = 0;
   if (const char *v = getenv("MYGRAD_HIP_WGRAD_TILE")) sscanf(v, "%d,%d", &forced_bm, &forced_bn);
-  bool forced = false;
-  for (const Cand &c : cands)
-    forced |= c.bm == forced_bm && c.bn == forced_bn && g.F >= c.bm && !(c.bm == 32 && c.bn == 128 && !f64);
   if (whole_c && fits_buffer_loads(g)) {
-    int limit = 128;
-    for (const Cand &c : cands) {
-      if (forced && (c.bm != forced_bm || c.bn != forced_bn)) continue;
-      if (!forced && wgrad_rows(g.F, limit) != c.bm) continue;
-      // 32x64 double-precision tiles are bound by LDS reads (the 4x4x4 MFMA takes an operand
-      // per 512 flops); the wider tile halves them per flop and is worth more padding.
-      // In single precision 32x128 measured slower than 32x64.
-      if (c.bm == 32 && c.bn == 128 && !f64) continue;
-      const long long col_tiles = ceil_div(ct, c.bn), row_tiles = ceil_div(g.F, c.bm);
-      const long long splits = splits_for(c.bm, c.bn, c.bk, true);
-      if (c.bn > 64 && !forced) {
-        const int per_cu = f64 ? wgrad_blocks_per_cu<double>(c.bm, c.bn, true) : wgrad_blocks_per_cu<float>(c.bm, c.bn, true);
-        const double waste = (double)(col_tiles * c.bn - ct) / (double)ct;
-        const double filled = (double)(col_tiles * row_tiles * splits) / ((double)per_cu * cus);
-        if (waste > (c.bm == 32 ? 0.15 : 0.12) || filled < 0.75) {
-          limit = std::min(limit, c.bm == 128 ? 64 : limit);
-          continue;
-        }
-      }
-      best_splits = splits;
-      pl.bm = c.bm, pl.bn = c.bn, pl.bk = c.bk;
-      break;
+    // The usual plan: the largest row tile that divides the filters (rounded up as below), with little
+    // padding of its columns and most slots of one round filled.  No accumulator sums up a K chunk more
+    // than a fifth longer than its, in double precision and on 128 x 128 tiles: a sum's rounding errors
+    // grow with the square root of its terms.  The other single-precision tiles add up runs that are no
+    // longer than that (WgradParams::run_tiles), and no longer than 1024 positions.
+    const int unit = g.wvol != 1 || g.F < 256 ? 16 : g.F < 1024 ? 64 : 128;
+    const int rows = (int)ceil_div(g.F, unit) * unit;
+    const Cand *usual = nullptr;
+    long long usual_splits = 1;
+    for (const Cand *c = first; c != last && !usual; ++c) {
+      if (c->bm == 48 || rows % c->bm != 0 || !fits(*c)) continue;
+      usual_splits = splits_for(c->bm, c->bn, c->bk, true);
+      const long long columns = ceil_div(ct, c->bn) * c->bn;
+      const double waste = (double)(columns - ct) / (double)ct;
+      const double filled = (double)(columns / c->bn * ceil_div(g.F, c->bm) * usual_splits) / ((double)per_cu(*c) * cus);
+      if (c->bn <= 64 || (waste <= (c->bm == 32 ? 0.15 : 0.12) && filled >= 0.75)) usual = c;
     }
+    double least = 0;
+    for (const Cand *c = first; c != last; ++c) {
+      if (!fits(*c)) continue;
+      if (c->bm == forced_bm && c->bn == forced_bn) {
+        best_splits = splits_for(c->bm, c->bn, c->bk, true);
+        pl.bm = c->bm, pl.bn = c->bn, pl.bk = c->bk;
+        break;
+      }
+      const long long ktiles = ceil_div(kpos, c->bk), tiles = ceil_div(ct, c->bn) * ceil_div(g.F, c->bm), slots = (long long)per_cu(*c) * cus;
+      const long long most = std::max<long long>(1, std::min<long long>(ktiles / 4, 1024));
+      const double peak = (f64 ? 78.6e6 : 157.3e6) / cus;  // flops per microsecond of a unit
+      auto consider = [&](long long sp) {
+        if (sp < 1 || sp > most) return;
+        if ((f64 || c->bm == 128) && !(c == usual && sp == usual_splits) && 5 * chunk_of(*c, sp) > 6 * chunk_of(*usual, usual_splits)) return;
+        const double share = (double)ceil_div(ktiles, sp), blocks = (double)(tiles * sp);
+        const double a = std::ceil(blocks / (double)slots) * share * c->step;
+        const double b = std::ceil(blocks / cus) * share * 2.0 * c->bm * c->bn * c->bk / (peak * c->rate);
+        double time = std::sqrt(std::sqrt(a * a * a * a + b * b * b * b));
+        if (sp > 1 || g.wvol > 1) time += (f64 ? 2.7 : 4.6) + (double)g.F * (double)ct * (double)(sp + 1) * (f64 ? 8 : 4) / 4.0e6;
+        // (the usual plan stays unless another is 3 % cheaper: below that the fit does not tell them apart)
+        if (c == usual && sp == usual_splits) time *= 0.97;
+        if (pl.bm == 0 || time < least) least = time, best_splits = sp, pl.bm = c->bm, pl.bn = c->bn, pl.bk = c->bk;
+      };
+      for (long long sp = 1; sp <= 16; ++sp) consider(sp);
+      for (long long rounds = 1; rounds <= 4; ++rounds) consider(rounds * slots / tiles);
+      if (c == usual) consider(usual_splits);
+    }
+    pl.run_tiles = (int)std::max<long long>(1, std::min<long long>(1024, chunk_of(*usual, usual_splits)) / pl.bk);
   }
   pl.tap_major = pl.bm != 0;
   if (!pl.tap_major) {
@@ -2149,8 +2167,8 @@ int build_wgrad_plan(const Geometry &g, Plan &pl) {
       const char *flag = getenv("MYGRAD_HIP_TABLE_ROWS");
       return !(flag && flag[0] == '0');
     }();
-    // filters in row tiles of 16, 32 or 64, the last one possibly short: its rows beyond F read
-    // whatever follows in grad (or zeros past its end) and are not stored
+    // filters in row tiles of 16, 32 or 64, the last one moved back to end with the last filter (with fewer
+    // filters than rows, those beyond read whatever follows in grad, or zeros past its end, and are not stored)
     const int row_tile = g.F <= 16 ? 16 : g.F <= 32 ? 32 : g.F <= 48 ? 16 : 64;
     if (rows_on && fits_buffer_loads(g)) {
       pl.tap_major = pl.table_rows = true;
@@ -2716,6 +2734,7 @@ int conv_wgrad_impl(const Geometry &g, const Plan &pl, const void *grad, const v
   wp.by_g2 = make_fastdiv((unsigned)g.G[2]);
   wp.pos_tab = pl.pos_tab;
   wp.wvol = (int)g.wvol;
+  wp.run_tiles = pl.run_tiles;
   wp.shift_from = staged || pl.depth == g.C ? 1 << 30 : pl.depth - 16;
   wp.col_shift = pl.depth - g.C;
   {
@@ -2744,8 +2763,11 @@ int conv_wgrad_impl(const Geometry &g, const Plan &pl, const void *grad, const v
     const int count = g.F * ct;
     ScopedTiming timed(TAG_WGRAD_REDUCE);
     if (pl.tap_major && !pl.table_rows) {
-      // four runs of splits per element when one thread per element would leave units idle
-      if (ceil_div(count, 256) < runtime().props.multiProcessorCount && pl.splits >= 16)
+      // four or sixteen runs of splits per element when one thread per element would leave units idle
+      if (ceil_div(count, 256) < runtime().props.multiProcessorCount / 8 && pl.splits >= 64)
+        hipLaunchKernelGGL((tap_reduce_kernel<T, 16>), dim3((unsigned)ceil_div(count, 16)), dim3(256), 0, s,
+                           static_cast<const T *>(target), static_cast<T *>(dw), g.F, g.C, (int)g.wvol, pl.splits, ct);
+      else if (ceil_div(count, 256) < runtime().props.multiProcessorCount && pl.splits >= 16)
         hipLaunchKernelGGL((tap_reduce_kernel<T, 4>), dim3((unsigned)ceil_div(count, 64)), dim3(256), 0, s,
                            static_cast<const T *>(target), static_cast<T *>(dw), g.F, g.C, (int)g.wvol, pl.splits, ct);
       else

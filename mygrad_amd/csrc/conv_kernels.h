@@ -240,6 +240,7 @@ struct WgradParams {
   // One tap and channels that are no multiple of 16 (out is in dw's own layout): columns from
   // shift_from on are the last, shifted channel block; column col there is channel col - col_shift.
   int shift_from, col_shift;
+  int run_tiles;  // K tiles that an accumulator sums up before they are added to the total (tap-major, single precision)
 };
 
 }  // namespace mg

@@ -1383,12 +1383,27 @@ __global__ void __launch_bounds__(512) tap_wgrad_kernel(const WgradParams p) {
 #pragma unroll
     for (int j = 0; j < TN; ++j) acc[i][j] = typename Mma<T>::Acc{0, 0, 0, 0};
 
+  // Runs of WgradParams::run_tiles K tiles are summed up apart and added to `total`: what an accumulator
+  // takes without a break bounds a single-precision sum's error, and K is long here.  ((329,2639) @
+  // (2639,1862), da, K not cut: 7.7e-7 against 64 bits in one run, 2.9e-7 in runs of 256 positions.)  A
+  // break waits for the matrix pipes; every 1024 positions that is not to be seen (64 channels, 3x3 at
+  // 56x56: 261.4 us, 261.2 without; the error 1.5e-6 -> 5.8e-7).  128 x 128 tiles have no registers for
+  // it (two blocks per unit), table rows keep the chunks they have.
+  constexpr bool RUNS = !TABLE && TM * TN <= 4;
+  typename Mma<T>::Acc total[RUNS ? TM : 1][RUNS ? TN : 1];
+  if constexpr (RUNS) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) total[i][j] = typename Mma<T>::Acc{0, 0, 0, 0};
+  }
+
   // The order in which the K tile is contracted is free: quarter-wave lk takes the
   // K indices lk*KQ .. lk*KQ+KQ-1, one per MFMA step, so that four steps' operands
   // of a lane are adjacent in LDS and come in one read.
   __syncthreads();
   int buf = 0;
-  for (int kt = 0; kt < ktiles; ++kt) {
+  auto contract = [&] {
 #pragma unroll
     for (int s4 = 0; s4 < KQ / 4; ++s4) {
       T a[TM][4], b[TN][4];
@@ -1425,6 +1440,21 @@ __global__ void __launch_bounds__(512) tap_wgrad_kernel(const WgradParams p) {
     }
     __syncthreads();
     buf ^= 1;
+  };
+  if constexpr (RUNS) {
+    for (int kt = 0; kt < ktiles;) {
+      for (const int stop = min(kt + p.run_tiles, ktiles); kt < stop; ++kt) contract();
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) total[i][j] += acc[i][j], acc[i][j] = typename Mma<T>::Acc{0, 0, 0, 0};
+    }
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] = total[i][j];
+  } else {
+    for (int kt = 0; kt < ktiles; ++kt) contract();
   }
 
   // partial sums [split][f][column]
@@ -1447,7 +1477,7 @@ __global__ void __launch_bounds__(512) tap_wgrad_kernel(const WgradParams p) {
 // channel blocks of 16, then taps, then the channel inside the block:
 // col = ((c/16) * wvol + t) * 16 + c%16; `ct` columns in all.  With C no multiple of 16 the last
 // block holds channels C-16..C-1, of which those of the block before it are passed over.
-// The splits are cut into RUNS runs (1 or 4); wave q of the block adds run q in split
+// The splits are cut into RUNS runs (1, 4 or 16); part q of the block adds run q in split
 // order for 256 / RUNS consecutive elements, and the run sums are added in run order:
 // always the same association for a given plan, so the result repeats exactly.  Four
 // runs put four times the loads in flight, which pays when dw is too small to fill
@@ -1456,7 +1486,7 @@ template <typename T, int RUNS>
 __global__ void __launch_bounds__(256) tap_reduce_kernel(const T *__restrict__ part, T *__restrict__ dw, int F, int C,
                                                          int wvol, int splits, int ct) {
   constexpr int WIDTH = 256 / RUNS;
-  __shared__ T runs[4][64];
+  __shared__ T runs[RUNS][WIDTH];
   const int count = F * ct;
   const int q = threadIdx.x / WIDTH, lane = threadIdx.x % WIDTH;
   // Threads run through the partial sums' own layout, so a wave reads consecutive
@@ -1485,7 +1515,10 @@ __global__ void __launch_bounds__(256) tap_reduce_kernel(const T *__restrict__ p
     // runs past the last split are empty and hold +0.0; adding them changes nothing
     // except that a total of -0.0 would read +0.0, which a sum of products starting
     // from +0.0 accumulators cannot be
-    dw[i] = ((runs[0][lane] + runs[1][lane]) + runs[2][lane]) + runs[3][lane];
+    T all = runs[0][lane];
+#pragma unroll
+    for (int r = 1; r < RUNS; ++r) all += runs[r][lane];
+    dw[i] = all;
   }
 }
 

@@ -1082,6 +1082,48 @@ def test_small_products_add_up_no_longer_chains(abi, m, k, n):
     assert np.linalg.norm(got - want) <= 3.3e-7 * np.linalg.norm(want)
 
 
+@pytest.mark.parametrize("x_shape,w_shape,bound", [
+    ((1, 2639, 1862), (329, 2639, 1), 3.5e-7),   # what these showed against 64 bits with their K cut into 8, 7, 5
+    ((1, 2294, 1235), (473, 2294, 1), 3.1e-7),   # splits (2.9e-7, 2.5e-7, 2.5e-7, ...), a fifth above it; in one run
+    ((1, 747, 877), (1947, 747, 1), 3.1e-7),     # 7.7e-7, 6.3e-7, 5.3e-7
+    ((1, 693, 664), (2112, 693, 1), 2.8e-7),
+    ((15, 51, 12603), (24, 51, 5), 7.8e-7),      # 6.5e-7; 8.9e-7 with half as many splits
+    ((32, 24, 56, 56), (24, 24, 3, 3), 5.7e-7),  # 4.7e-7; 6.3e-7
+])
+def test_filter_gradient_adds_up_runs_of_a_bounded_length(abi, x_shape, w_shape, bound):
+    rng = np.random.default_rng(w_shape[0])
+    pad = (w_shape[2] // 2 if len(x_shape) == 4 else 0,) * (len(x_shape) - 2)
+    ones = (1,) * len(pad)
+    grid = tuple(a + 2 * q - t + 1 for a, q, t in zip(x_shape[2:], pad, w_shape[2:]))
+    x = rng.standard_normal(x_shape).astype(np.float32)
+    g = rng.standard_normal((x_shape[0], w_shape[0], *grid)).astype(np.float32)
+    got = abi.conv_wgrad(g, x, w_shape, 1, pad, 1)
+    g64, x64 = g.astype(np.float64), np.pad(x.astype(np.float64), [(0, 0), (0, 0)] + [(q, q) for q in pad])
+    want = np.empty(w_shape)
+    for tap in np.ndindex(*w_shape[2:]):
+        part = x64[(slice(None), slice(None), *(slice(t, t + n) for t, n in zip(tap, grid)))]
+        want[(slice(None), slice(None), *tap)] = sum(a.reshape(a.shape[0], -1) @ b.reshape(b.shape[0], -1).T for a, b in zip(g64, part))
+    assert np.linalg.norm(got - want) <= bound * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("filters", [1, 5, 12, 15, 17, 33, 60])
+def test_filter_gradient_of_filters_that_fill_no_row_tile(abi, dtype, filters):
+    """The rows beyond the last filter are computed from whatever follows in grad, or zeros, and not stored."""
+    from mygrad_amd import _hip
+
+    for x_shape, w_shape in (((7, 32, 23, 21), (filters, 32, 3, 3)), ((1, 16, 999), (filters, 16, 1)), ((1, 48, 40, 41), (filters, 48, 1, 3))):
+        nd = len(x_shape) - 2
+        rng = np.random.default_rng(filters)
+        x = rng.integers(-3, 4, x_shape).astype(dtype)
+        grid = tuple(a - t + 1 for a, t in zip(x_shape[2:], w_shape[2:]))
+        g = rng.integers(-2, 3, (x_shape[0], filters, *grid)).astype(dtype)
+        conf = (1,) * nd, (0,) * nd, (1,) * nd
+        print("few filters", np.dtype(dtype).name, x_shape, w_shape, flush=True)
+        assert np.array_equal(abi.conv_wgrad(g, x, w_shape, *conf), direct.conv_backward_w(g, x, w_shape, *conf).astype(dtype))
+        assert "tap-major tile" in _hip.last_plan()
+
+
 KERNEL_VARIANT_CASES = [
     # x shape, w shape, stride, padding, dilation
     ((8, 128, 28, 28), (128, 128, 3, 3), (1, 1), (1, 1), (1, 1)),   # 128-row tiles, wgrad 128x128
