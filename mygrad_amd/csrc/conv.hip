@@ -591,20 +591,26 @@ double conv_flops(const Geometry &g) {
   return 2.0 * (double)g.N * (double)g.F * (double)g.gvol * (double)g.C * (double)g.wvol;
 }
 
+// Whether a count rounded up to whole K tiles of 16 has at most a quarter of dead rows.
+bool mostly_live(int channels) { return 3 * ((channels + 15) / 16 * 16) <= 4 * channels; }
+
 // Channels that the tap-major kernels contract per tap (filters, for the data gradient) for a count
 // of `channels`: the count itself where it fills whole K tiles, else rounded up to whole tiles of 16
 // whose last one has fewer live rows; 0 where the table of rows is the better form: a small problem,
-// or more than a third of dead rows (a product has one tap, and its table rows no structure to use:
-// any count).  MYGRAD_HIP_PAD=0 leaves every awkward count to the table of rows.
+// or more than a quarter of dead rows.  With one tap that form has no structure to use, and dead rows are
+// the better ones for any count: (64,8,112,112) * (16,8,1,1) 26.8 us against 31.6 on table rows, 5 x 3000
+// rows of a product's contraction 28.6 against 56; the two are alike in double precision, where K tiles of 8
+// leave eight channels whole (43.8 us with dead rows, 40.8 without).  MYGRAD_HIP_PAD=0 leaves every
+// awkward count to the table of rows.
 int whole_channels(const Geometry &g, int channels) {
   if (channels % 16 == 0) return channels;
   static const bool on = [] {
     const char *flag = getenv("MYGRAD_HIP_PAD");
     return !(flag && flag[0] == '0');
   }();
-  const int up = (channels + 15) / 16 * 16;
-  if (on && conv_flops(g) >= 2.0e8 && (3 * up <= 4 * channels || g.wvol == 1)) return up;
-  return channels % gemm_bk(g.dtype) == 0 ? channels : 0;
+  const bool whole = channels % gemm_bk(g.dtype) == 0;
+  if (on && conv_flops(g) >= 2.0e8 && (mostly_live(channels) || (g.wvol == 1 && !whole))) return (channels + 15) / 16 * 16;
+  return whole ? channels : 0;
 }
 // K tile of a tap-major plan that contracts `channels` channels per tap.  Double precision: 16
 // where the channels allow it -- a K tile of 8 is 64 MFMAs per wave between two barriers, and
@@ -1430,7 +1436,10 @@ void thin_tables(Plan &pl, Tables &t, const std::vector<ThinUse> &uses, int nph,
 
 int build_fwd_plan(const Geometry &g, Plan &pl) {
   Tables t;
-  if ((g.F <= 4 || (g.F <= 1024 && whole_channels(g, g.C) == 0)) && thin_applies(g, g.F, (long long)g.N * g.gvol, (long long)g.C * g.wvol, 1)) {
+  // (one tap and few channels: one position per lane takes 34.7 - 40.3 us for (64,C,112,112) * (64,C,1,1), C = 2 -
+  // 11, whole K tiles of 16 with dead rows 41.9 - 44.3)
+  const int whole = whole_channels(g, g.C);
+  if ((g.F <= 4 || (g.F <= 1024 && (whole == 0 || (whole > g.C && !mostly_live(g.C))))) && thin_applies(g, g.F, (long long)g.N * g.gvol, (long long)g.C * g.wvol, 1)) {
     // up to four filters, or a first layer (channels that fill no K tile; passes of 64 filters), in
     // single precision: one output position per lane
     const int qs[3] = {g.X[1] * g.X[2], g.X[2], 1};

@@ -131,9 +131,12 @@ struct Quad {
 // ------------------------------------------------------------------------------------------
 // Whether the kernel for channels that are no multiple of BK is an instance of its own (DEAD): in the
 // others the test of KTile::dead costs nothing measurable (64 x 256: 260 -> 251 us on 64 channels
-// at 56x56), but the 128 x 128 float tile loses 1.2 % with it (4096^3: 991 -> 1003 us) and the four
-// fused phases 1 %.
-constexpr bool tap_gemm_dead_apart(int bm, int bn, int nph, int elem) { return elem == 4 && (nph == 4 || (bm == 128 && bn == 128)); }
+// at 56x56), but the 128 x 128 float tile loses 1.2 % with it (4096^3: 991 -> 1003 us), the four
+// fused phases 1 %, and 16 rows, which wait for their gathers, 5 % ((64,64,112,112) * (9,64,1,1) 48.4 ->
+// 51.0 us).
+constexpr bool tap_gemm_dead_apart(int bm, int bn, int nph, int elem) {
+  return elem == 4 && (nph == 4 || (bm == 128 && bn == 128) || (bm == 16 && bn == 256 && nph == 1));
+}
 
 template <typename T, int BM, int BN, int BK, int WM, int WN, int NPH = 1, bool FOLD = false, bool ROWS = false, bool DEAD = false>
 __global__ void __launch_bounds__(512) tap_gemm_kernel(const GemmParams p) {

@@ -1124,6 +1124,21 @@ def test_filter_gradient_of_filters_that_fill_no_row_tile(abi, dtype, filters):
         assert "tap-major tile" in _hip.last_plan()
 
 
+@pytest.mark.parametrize("dtype,channels,has", [(np.float32, 5, "one position per lane"), (np.float32, 11, "one position per lane"),
+                                                (np.float32, 13, "tap-major tile"), (np.float64, 8, "x8, 1 phase")])
+def test_single_taps_of_few_channels(abi, dtype, channels, has):
+    """1x1 convolutions whose channels fill no K tile of 16 mostly: no dead rows where a kernel without them is faster."""
+    from mygrad_amd import _hip
+
+    rng = np.random.default_rng(channels)
+    x_shape, w_shape = (24, channels, 56, 56), (1600 // channels, channels, 1, 1)
+    x, w = rng.integers(-3, 4, x_shape).astype(dtype), rng.integers(-2, 3, w_shape).astype(dtype)
+    want = direct.conv_forward(x, w, (1, 1), (0, 0), (1, 1)).astype(dtype)
+    got = abi.conv_fwd(x, w, 1, 0, 1)
+    assert np.array_equal(got, want)
+    assert 2 * want.size * channels >= 2e8 and has in _hip.last_plan(), _hip.last_plan()
+
+
 KERNEL_VARIANT_CASES = [
     # x shape, w shape, stride, padding, dilation
     ((8, 128, 28, 28), (128, 128, 3, 3), (1, 1), (1, 1), (1, 1)),   # 128-row tiles, wgrad 128x128
