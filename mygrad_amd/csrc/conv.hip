@@ -2053,9 +2053,10 @@ int build_pos_table(const Geometry &g, Plan &pl) {
 int build_wgrad_plan(const Geometry &g, Plan &pl) {
   Tables t;
   const bool f64 = g.dtype == MG_F64;
-  // tap-major columns: whole groups of 16 channels per tap (the last group moved back, see WGroup),
-  // which takes 16 channels to move in
-  const bool ragged_c = g.C % 16 != 0 && g.C >= 16 && whole_channels(g, g.C) % 16 == 0 && whole_channels(g, g.C) != 0;
+  // tap-major columns: whole groups of 16 channels per tap (the last group moved back, see WGroup), which
+  // takes 16 channels to move in, unless most of that group would be computed twice: table rows come
+  // in narrower tiles ((8,17,112,112) * (256,17,1,1), double precision: 43 us, 67 on whole groups)
+  const bool ragged_c = g.C % 16 != 0 && g.C >= 16 && mostly_live(g.C) && whole_channels(g, g.C) % 16 == 0 && whole_channels(g, g.C) != 0;
   const bool whole_c = g.C % 16 == 0 || ragged_c;
   pl.depth = ragged_c ? whole_channels(g, g.C) : g.C;
   long long ct = (long long)pl.depth * g.wvol;

@@ -1139,6 +1139,18 @@ def test_single_taps_of_few_channels(abi, dtype, channels, has):
     assert 2 * want.size * channels >= 2e8 and has in _hip.last_plan(), _hip.last_plan()
 
 
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_filter_gradient_of_a_tap_with_one_channel_beyond_a_group(abi, dtype):
+    """17 channels are 32 columns of two groups, fifteen of them computed twice: on table rows they are 17 of 32."""
+    from mygrad_amd import _hip
+
+    rng = np.random.default_rng(17)
+    x, g = rng.integers(-3, 4, (2, 17, 61, 63)).astype(dtype), rng.integers(-2, 3, (2, 800, 61, 63)).astype(dtype)
+    conf = (1, 1), (0, 0), (1, 1)
+    assert np.array_equal(abi.conv_wgrad(g, x, (800, 17, 1, 1), *conf), direct.conv_backward_w(g, x, (800, 17, 1, 1), *conf).astype(dtype))
+    assert "table rows tile 64x32" in _hip.last_plan(), _hip.last_plan()
+
+
 KERNEL_VARIANT_CASES = [
     # x shape, w shape, stride, padding, dilation
     ((8, 128, 28, 28), (128, 128, 3, 3), (1, 1), (1, 1), (1, 1)),   # 128-row tiles, wgrad 128x128
