@@ -4,13 +4,15 @@
 // the result carry) is bound by launches, not arithmetic, when each pair gets a launch of the
 // convolution kernels; here a wavefront makes one 16x16 tile of one product on the matrix cores,
 // reading its operands where they lie (a transposed operand is a pair of swapped strides), so the
-// whole stack is one grid.  Results larger than 32 x 32 go through a second kernel, where a
-// block of four wavefronts makes a tile of one product from operands it has copied to
+// whole stack is one grid.  Where it costs less (stack_time) it goes through a second kernel, where
+// a block of four wavefronts makes a tile of one product from operands it has copied to
 // LDS once (16 bytes per lane, coalesced) instead of every wavefront fetching its own rows and
 // columns through L1.  Large pairs stay with the tiled convolution kernels.
 #include "internal.h"
 
 #include <algorithm>
+#include <cmath>
+#include <cstdio>
 #include <cstdlib>
 #include <type_traits>
 
@@ -137,17 +139,15 @@ __global__ void __launch_bounds__(256) batched_product_kernel(BatchedParams p, c
 // matrix's edge cuts goes element by element).  Each of the four wavefronts makes a 32 x 32 part.
 //
 // What bounds it: the trips of a chunk from memory to LDS to registers, not the matrix pipes, so
-// the loads of the next chunk are issued before this one is multiplied, chunks are short (128 bytes
-// of k: six or seven blocks on a unit cover for one another; 256 bytes: 794 x (86,117,322) 117 us
-// instead of 103), and the LDS reads are wide.  Measured, single precision, forward / da / db: 96 x
-// (197,64,197) 14.1 / 13.8 / 13.7 us (34 TFLOP/s; 19.9 / 17.3 / 20.4 with element loads and
-// element LDS reads, which rows that are no whole pieces and every row took before), 794 x
-// (86,117,322) 103 / 91 / 104 us (147 / 130 / 139), 8 x 512^3 29 / 28 / 30 us.
+// the loads of the next chunk are issued before this one is multiplied, and the LDS reads are wide.
+// Chunks of 128 bytes of k where there are many blocks (six or seven on a unit cover for one another:
+// 794 x (86,117,322) 103 us, 117 with 256 bytes), of 64 values where there are few, whose trips
+// follow one another (24 x (64,64,64) in double precision, forward: 6.4 -> 5.5 us).
 // The sum over k may run in any order that both operands share: in a block of 4 * VEC values of k
 // (VEC = 16 bytes) the lane groups (lane / 16 = q) take k = VEC * q + s at step s, so an operand
 // that lies along k gives a lane VEC steps per LDS read; of one that lies along its rows or columns
 // a lane takes two neighbours, the two MFMA fragments it feeds, per read.
-template <typename T, bool TA, bool TB, int BM, int BN>
+template <typename T, bool TA, bool TB, int BM, int BN, int KC>
 __global__ void __launch_bounds__(256) batched_staged_kernel(BatchedParams p, const T *__restrict__ a, const T *__restrict__ b,
                                                              T *__restrict__ out) {
   constexpr int VEC = 16 / sizeof(T);
@@ -156,7 +156,6 @@ __global__ void __launch_bounds__(256) batched_staged_kernel(BatchedParams p, co
   typedef T Pair __attribute__((ext_vector_type(2)));
   typedef T PairU __attribute__((ext_vector_type(2), aligned(sizeof(T))));
   static_assert((BM / 32) * (BN / 32) == 4, "four wavefronts of 32 x 32");
-  constexpr int KC = 128 / sizeof(T);  // depth of a chunk
   // The stored pieces: rows x columns as in memory, rows 16-byte aligned in LDS.  Of pieces with k down
   // their rows the lane groups read rows VEC apart: 8 floats of padding put two groups' 32 banks
   // side by side.
@@ -190,29 +189,51 @@ __global__ void __launch_bounds__(256) batched_staged_kernel(BatchedParams p, co
   const T *pb = b + (long long)pair * p.b_pair;
 
   // R x C elements of a stored matrix (`rows` x `cols`, row-major) from (r0, c0): through registers
-  // (zeros outside the matrix) into LDS; the loads of both operands are issued before either is
-  // parked, so that a chunk costs one trip to memory, not two
+  // into LDS; the loads of both operands are issued before either is parked, so that a chunk costs
+  // one trip to memory, not two.  Loads are unconditional, from addresses clamped to the matrix (a
+  // branch per piece is most of a short product's time); at its edges, a branch of the whole block,
+  // pieces are put right before they are parked: the last one of a row was moved back to end with it.
   auto fetch = [&](auto rc, auto cc, const T *src, int rows, int cols, int r0, int c0, auto &reg) {
     constexpr int R = decltype(rc)::value, C = decltype(cc)::value, PIECES = C / VEC, PASS = 256 / PIECES;
-    const int c = c0 + (tid % PIECES) * VEC;
-    const T *at = src + (long long)(r0 + tid / PIECES) * cols + c;
+    const int from = max(min(c0 + (tid % PIECES) * VEC, cols - VEC), 0);
 #pragma unroll
     for (int i = 0; i < R / PASS; ++i) {
-      reg[i] = V{};
-      if (r0 + tid / PIECES + i * PASS < rows) {
-        const T *piece = at + (long long)(i * PASS) * cols;
-        if (c + VEC <= cols) {
-          reg[i] = *reinterpret_cast<const VU *>(piece);
-        } else {
+      const T *at = src + (long long)min(r0 + tid / PIECES + i * PASS, rows - 1) * cols + from;
+      if (cols >= VEC) {
+        reg[i] = *reinterpret_cast<const VU *>(at);
+      } else {
 #pragma unroll
-          for (int s = 0; s < VEC - 1; ++s)
-            if (c + s < cols) reg[i][s] = piece[s];
-        }
+        for (int s = 0; s < VEC; ++s) reg[i][s] = at[min(s, cols - 1)];
       }
     }
   };
-  auto park = [&](auto rc, auto cc, T *dst, auto ld, const auto &reg) {
+  // (k: whether the rows, or else the columns, run along K.  What lies outside the matrix along M or N makes
+  // results that are not stored, so only the columns of a row that is no whole pieces have to be put
+  // back in place there; along K both operands are zero outside.)
+  auto park = [&](auto rc, auto cc, auto k, int rows, int cols, int r0, int c0, T *dst, auto ld, auto &reg) {
     constexpr int R = decltype(rc)::value, C = decltype(cc)::value, PIECES = C / VEC, PASS = 256 / PIECES;
+    constexpr bool K_ROWS = decltype(k)::value;
+    const int c = c0 + (tid % PIECES) * VEC;
+    if (c0 + C > cols && cols % VEC != 0) {
+      const int moved = c - max(min(c, cols - VEC), 0);
+#pragma unroll
+      for (int i = 0; i < R / PASS; ++i) {
+        V v = reg[i];
+        if constexpr (VEC == 4)
+          if (moved & 2) v = V{v[2], v[3], T(0), T(0)};
+        if (moved & 1) {
+#pragma unroll
+          for (int s = 0; s + 1 < VEC; ++s) v[s] = v[s + 1];
+        }
+#pragma unroll
+        for (int s = 0; s < VEC; ++s) reg[i][s] = K_ROWS || c + s < cols ? v[s] : T(0);
+      }
+    }
+    if (K_ROWS ? r0 + R > rows : c0 + C > cols) {
+#pragma unroll
+      for (int i = 0; i < R / PASS; ++i)
+        if (K_ROWS ? r0 + tid / PIECES + i * PASS >= rows : c >= cols) reg[i] = V{};
+    }
 #pragma unroll
     for (int i = 0; i < R / PASS; ++i)
       *reinterpret_cast<V *>(dst + (tid / PIECES + i * PASS) * decltype(ld)::value + (tid % PIECES) * VEC) = reg[i];
@@ -225,6 +246,10 @@ __global__ void __launch_bounds__(256) batched_staged_kernel(BatchedParams p, co
   auto fetch_chunk = [&](int k0) {
     fetch(ar, ac, pa, TA ? p.K : p.M, TA ? p.M : p.K, TA ? k0 : row0, TA ? row0 : k0, ra);
     fetch(br, bc, pb, TB ? p.N : p.K, TB ? p.K : p.N, TB ? col0 : k0, TB ? k0 : col0, rb);
+  };
+  auto park_chunk = [&](int k0) {
+    park(ar, ac, std::integral_constant<bool, TA>{}, TA ? p.K : p.M, TA ? p.M : p.K, TA ? k0 : row0, TA ? row0 : k0, As, std::integral_constant<int, LDA>{}, ra);
+    park(br, bc, std::integral_constant<bool, !TB>{}, TB ? p.N : p.K, TB ? p.K : p.N, TB ? col0 : k0, TB ? k0 : col0, Bs, std::integral_constant<int, LDB>{}, rb);
   };
 
   constexpr int WAVES_N = BN / 32;
@@ -239,12 +264,11 @@ __global__ void __launch_bounds__(256) batched_staged_kernel(BatchedParams p, co
   fetch_chunk(0);
   for (int k0 = 0; k0 < p.K; k0 += KC) {
     if (k0 > 0) __syncthreads();  // everyone has finished with the previous chunk
-    park(ar, ac, As, std::integral_constant<int, LDA>{}, ra);
-    park(br, bc, Bs, std::integral_constant<int, LDB>{}, rb);
+    park_chunk(k0);
     __syncthreads();
     if (k0 + KC < p.K) fetch_chunk(k0 + KC);  // on its way while this chunk is multiplied
-    const int blocks = live ? (min(KC, p.K - k0) + 4 * VEC - 1) / (4 * VEC) : 0;
-    for (int kb = 0; kb < blocks; ++kb) {
+    constexpr int BLOCKS = KC / (4 * VEC);
+    auto multiply = [&](int kb) {
       const int k = kb * (4 * VEC) + lk * VEC;
       T av[2][VEC], bv[2][VEC];
       // rows of the tile: fragment i's are wr + 16 i + l16, or (op(a) along its rows) wr + 2 l16 + i
@@ -283,6 +307,13 @@ __global__ void __launch_bounds__(256) batched_staged_kernel(BatchedParams p, co
         for (int i = 0; i < 2; ++i)
 #pragma unroll
           for (int j = 0; j < 2; ++j) acc[i][j] = Tile<T>::run(av[i][s], bv[j][s], acc[i][j]);
+    };
+    const int blocks = live ? (min(KC, p.K - k0) + 4 * VEC - 1) / (4 * VEC) : 0;
+    if (blocks == BLOCKS) {  // (unrolled: the next block's LDS reads under this one's products)
+#pragma unroll
+      for (int kb = 0; kb < BLOCKS; ++kb) multiply(kb);
+    } else {
+      for (int kb = 0; kb < blocks; ++kb) multiply(kb);
     }
   }
 
@@ -306,21 +337,40 @@ __global__ void __launch_bounds__(256) batched_staged_kernel(BatchedParams p, co
     }
 }
 
-// Rows of the tile: of 128 x 32, 64 x 64 and 32 x 128, all four wavefronts of 32 x 32, the one that covers
-// M x N with the least area (the squarer one where they come out the same: it loads less).
-inline int staged_rows(int64_t M, int64_t N) {
-  int best = 64;
-  int64_t least = ceil_div(M, 64) * ceil_div(N, 64);
-  for (int bm : {128, 32})
-    if (ceil_div(M, bm) * ceil_div(N, 4096 / bm) < least) best = bm, least = ceil_div(M, bm) * ceil_div(N, 4096 / bm);
-  return best;
+// What a stack costs, in microseconds, on each kernel: the chain of a block's trips (`step` for one chunk of
+// K, or for 4 values of k of the kernel that reads in place) or the work of the busiest unit (`work` for a
+// block's trip), whichever is longer, on top of `base`.  Fitted to 6720 timed pairs of a product (960,
+// 2 to 1000 pairs of 16 to 512 rows and columns, both precisions, forward, da and db) and a kernel.
+// The one that costs least is 1.7 % slower than the best on average (9 % at the 95th percentile);
+// staging every result larger than 32 x 32 in the tile of least area is 9 % slower, 64 x 64 tiles
+// where they are half full 18 %.
+struct StackRate {
+  double step, work, base;
+};
+constexpr int kTileRows[3] = {32, 64, 128};  // x 128, 64, 32 columns
+// [double precision][chunk of 64 values of k, or of 128 bytes][tile]
+constexpr StackRate kStaged[2][2][3] = {{{{0.84, 0.74, 2.96}, {0.82, 0.76, 2.95}, {0.90, 0.74, 2.96}}, {{1.42, 1.50, 2.78}, {1.34, 1.40, 2.75}, {1.56, 1.53, 2.74}}},
+                                        {{{0.81, 0.69, 2.94}, {0.76, 0.71, 2.87}, {0.92, 0.74, 2.86}}, {{0.06, 3.87, 1.89}, {0.07, 2.84, 2.67}, {0.06, 3.91, 1.95}}}};
+// [double precision][forward; op(a) in 16-byte pieces; da; both in pieces; op(a) transposed]
+constexpr StackRate kInPlace[2][5] = {{{0.172, 0.087, 2.39}, {0.054, 0.053, 2.76}, {0.129, 0.141, 2.19}, {0.002, 0.051, 2.88}, {0.131, 0.072, 2.61}},
+                                      {{0.208, 0.125, 2.38}, {0.134, 0.096, 2.53}, {0.174, 0.167, 2.43}, {0.094, 0.106, 2.43}, {0.186, 0.108, 2.59}}};
+
+double stack_time(const StackRate &r, double trips, double per_unit, double memory) {
+  const double a = trips * r.step, b = trips * per_unit * r.work;
+  return r.base + std::sqrt(std::sqrt(a * a * a * a + b * b * b * b + memory * memory * memory * memory));
 }
 
 template <typename T>
-void launch_staged(const BatchedParams &p, int bm, unsigned blocks, bool ta, bool tb, const void *a, const void *b, void *out, hipStream_t s) {
-#define MG_STAGED(TA, TB, BM)                    \
-  if (ta == TA && tb == TB && bm == BM)          \
-    hipLaunchKernelGGL((batched_staged_kernel<T, TA, TB, BM, 4096 / BM>), dim3(blocks), dim3(256), 0, s, p, (const T *)a, (const T *)b, (T *)out);
+void launch_staged(const BatchedParams &p, int bm, bool deep, unsigned blocks, bool ta, bool tb, const void *a, const void *b, void *out, hipStream_t s) {
+#define MG_STAGED_KC(TA, TB, BM, KC) \
+  hipLaunchKernelGGL((batched_staged_kernel<T, TA, TB, BM, 4096 / BM, KC>), dim3(blocks), dim3(256), 0, s, p, (const T *)a, (const T *)b, (T *)out)
+#define MG_STAGED(TA, TB, BM)                              \
+  if (ta == TA && tb == TB && bm == BM) {                  \
+    if (deep)                                              \
+      MG_STAGED_KC(TA, TB, BM, 64);                        \
+    else                                                   \
+      MG_STAGED_KC(TA, TB, BM, 128 / (int)sizeof(T));      \
+  }
 #define MG_STAGED_BM(TA, TB) MG_STAGED(TA, TB, 64) MG_STAGED(TA, TB, 128) MG_STAGED(TA, TB, 32)
   MG_STAGED_BM(false, false)
   MG_STAGED_BM(false, true)
@@ -328,6 +378,7 @@ void launch_staged(const BatchedParams &p, int bm, unsigned blocks, bool ta, boo
   MG_STAGED_BM(true, true)
 #undef MG_STAGED_BM
 #undef MG_STAGED
+#undef MG_STAGED_KC
 }
 
 }  // namespace
@@ -364,32 +415,58 @@ int mg_matmul_batched(int dtype, int64_t batch, int64_t M, int64_t K, int64_t N,
     const char *flag = getenv("MYGRAD_HIP_BMM_STAGED");
     return !(flag && flag[0] == '0');
   }();
-  const int bm = staged_rows(M, N);
-  p.dealt = batch >= 64;
-  const long long blocks = (p.dealt ? ceil_div(batch, 8) * 8 : batch) * ceil_div(M, bm) * ceil_div(N, 4096 / bm);
+  // 16-byte pieces along K: the operand is contiguous there, K is a whole number of pieces (so
+  // every row starts on one) and the stack itself is aligned
+  const bool f64 = dtype == MG_F64;
+  const int vec = f64 ? 2 : 4;
+  const bool av = p.a_col == 1 && K % vec == 0 && reinterpret_cast<uintptr_t>(a) % 16 == 0;
+  const bool bv = p.b_row == 1 && K % vec == 0 && reinterpret_cast<uintptr_t>(b) % 16 == 0;
+  // Results of 16 rows or columns at most stay in place.  Of the others those whose 64 x 64 tiles are half
+  // full leave it to an operand without pieces: what its strided reads cost depends on more than is fitted
+  // here (16 x (197,64,197), db in double precision: 20.7 us in place, 14.1 staged, 11.9 expected).
+  const double cus = runtime().props.multiProcessorCount;
+  const double memory = (double)batch * (double)(M * K + K * N + M * N) * (f64 ? 8.0 : 4.0) / 6.0e6;
+  int tile = -1, deep = 0;
+  if (staged_on && K > 0 && M > 16 && N > 16) {
+    const StackRate &in_place = kInPlace[f64][trans_a ? 4 : trans_b ? (av && bv ? 3 : 2) : av ? 1 : 0];
+    double least = stack_time(in_place, (double)ceil_div(K, 4), std::ceil((double)ceil_div(p.tiles, 4) / cus), memory);
+    const bool half_full = M >= 32 && N >= 32 && 2 * M * N >= ceil_div(M, 64) * ceil_div(N, 64) * 4096;
+    if (half_full && !av && !bv) least = 1e30;
+    for (int d = 0; d < 2; ++d)
+      for (int t = 0; t < 3; ++t) {
+        const double blocks = (double)batch * (double)ceil_div(M, kTileRows[t]) * (double)ceil_div(N, 4096 / kTileRows[t]);
+        const double time = stack_time(kStaged[f64][d][t], (double)ceil_div(K, d ? 64 : 128 / (f64 ? 8 : 4)), std::max(blocks / cus, 1.0), memory);
+        if (time < least) least = time, tile = t, deep = d;
+      }
+    // MYGRAD_HIP_BMM_TILE="rows,deep" (read at every call, for the tests of every tile): that one
+    int rows = 0, chunk = 0;
+    if (const char *v = getenv("MYGRAD_HIP_BMM_TILE"))
+      if (sscanf(v, "%d,%d", &rows, &chunk) == 2)
+        for (int t = 0; t < 3; ++t)
+          if (kTileRows[t] == rows) tile = t, deep = chunk != 0;
+  }
+  static const char *const notes[3][2] = {{"batched: 32 x 128 tiles, short chunks", "batched: 32 x 128 tiles, deep chunks"},
+                                          {"batched: 64 x 64 tiles, short chunks", "batched: 64 x 64 tiles, deep chunks"},
+                                          {"batched: 128 x 32 tiles, short chunks", "batched: 128 x 32 tiles, deep chunks"}};
+  note_plan(tile < 0 ? "batched: operands read in place" : notes[tile][deep]);
+  const int bm = tile < 0 ? 64 : kTileRows[tile];
+  const long long tiles = batch * ceil_div(M, bm) * ceil_div(N, 4096 / bm);
+  // (dealing pairs out to the XCDs pays where each has many: with 100 pairs of five tiles some units get a
+  // third block, 25 -> 37 us)
+  p.dealt = batch >= 64 && tiles >= 8 * cus;
+  const long long blocks = p.dealt ? ceil_div(batch, 8) * 8 * (tiles / batch) : tiles;
   p.pairs = (int)batch;
-  // A result of one wavefront's 32 x 32 or of 16 rows or columns stays with the kernel above (300 x
-  // (20,100,20): 5.6 us there, 8.0 staged).  In double precision, whose 16x16x4 MFMA takes three
-  // times as long, 32 x 32 parts that are less than 0.6 full lose too (64 x (300,400,18): 48 / 57 us;
-  // 34 x (310,259,31): 31 / 21) unless 64 x 64 tiles are half full.
-  const long long parts = ceil_div(M, 32) * ceil_div(N, 32) * 1024, t64 = ceil_div(M, 64) * ceil_div(N, 64) * 4096;
-  const bool full = dtype == MG_F32 || 10 * M * N >= 6 * parts || (M >= 32 && N >= 32 && 2 * M * N >= t64);
-  if (staged_on && K > 0 && M > 16 && N > 16 && (M > 32 || N > 32) && full && blocks < (1ll << 31)) {
+  if (tile >= 0 && blocks < (1ll << 31)) {
     p.row_tiles = (int)ceil_div(M, bm);
     p.col_tiles = (int)ceil_div(N, 4096 / bm);
     if (dtype == MG_F32)
-      launch_staged<float>(p, bm, (unsigned)blocks, trans_a != 0, trans_b != 0, a, b, out, s);
+      launch_staged<float>(p, bm, deep != 0, (unsigned)blocks, trans_a != 0, trans_b != 0, a, b, out, s);
     else
-      launch_staged<double>(p, bm, (unsigned)blocks, trans_a != 0, trans_b != 0, a, b, out, s);
+      launch_staged<double>(p, bm, deep != 0, (unsigned)blocks, trans_a != 0, trans_b != 0, a, b, out, s);
     MG_HIP(hipGetLastError());
     return MG_OK;
   }
   const dim3 grid((unsigned)ceil_div(p.tiles, 4)), block(256);
-  // 16-byte pieces along K: the operand is contiguous there, K is a whole number of pieces (so
-  // every row starts on one) and the stack itself is aligned
-  const int vec = dtype == MG_F32 ? 4 : 2;
-  const bool av = p.a_col == 1 && K % vec == 0 && reinterpret_cast<uintptr_t>(a) % 16 == 0;
-  const bool bv = p.b_row == 1 && K % vec == 0 && reinterpret_cast<uintptr_t>(b) % 16 == 0;
 #define MG_BATCHED(T, AV, BV) \
   hipLaunchKernelGGL((batched_product_kernel<T, AV, BV>), grid, block, 0, s, p, (const T *)a, (const T *)b, (T *)out)
 #define MG_BATCHED_T(T)                 \

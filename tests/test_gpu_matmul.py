@@ -108,6 +108,40 @@ def test_batched_product_with_and_without_transposed_operands(abi, batch, M, K, 
         assert np.array_equal(abi.matmul_batched(ai, bi), np.matmul(ai, bi))
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("tile", ["32,0", "64,0", "128,0", "32,1", "64,1", "128,1"])
+def test_every_staged_tile_of_a_batched_product(abi, monkeypatch, tile, dtype):
+    """Edges of the tiles and of the chunks (16, 32 or 64 values of k), rows shorter than a 16-byte piece and of every
+    remainder; what lies beside a pair in its stack stays out of its product, NaN and all."""
+    from mygrad_amd import _hip
+
+    monkeypatch.setenv("MYGRAD_HIP_BMM_TILE", tile)
+    for batch, M, K, N in ((3, 17, 1, 18), (2, 33, 3, 31), (2, 65, 2, 129), (3, 129, 17, 66), (2, 64, 64, 64), (2, 63, 65, 33), (9, 35, 130, 37), (64, 40, 19, 21)):
+        rng = np.random.default_rng([batch, M, K, N])
+        a, b = rng.integers(-4, 5, (batch, M, K)).astype(dtype), rng.integers(-4, 5, (batch, K, N)).astype(dtype)
+        want = np.matmul(a, b)
+        a[1::2], b[1::2] = np.nan, np.inf
+        at, bt = np.ascontiguousarray(a.transpose(0, 2, 1)), np.ascontiguousarray(b.transpose(0, 2, 1))
+        print("tile", tile, np.dtype(dtype).name, batch, M, K, N, flush=True)
+        for ta, tb in ((False, False), (True, False), (False, True), (True, True)):
+            got = abi.matmul_batched(at if ta else a, bt if tb else b, ta, tb)
+            assert f"{tile.split(',')[0]} x" in _hip.last_plan()
+            assert np.array_equal(got[::2], want[::2]), (M, K, N, ta, tb)
+
+
+@pytest.mark.parametrize("dtype,batch,M,K,N,short", [
+    (np.float64, 24, 64, 64, 64, False), (np.float32, 4, 200, 100, 60, False), (np.float32, 9, 300, 500, 40, False), (np.float64, 16, 64, 197, 197, False),
+    (np.float32, 500, 86, 117, 322, True), (np.float32, 300, 20, 100, 20, False),
+])
+def test_small_stacks_take_few_trips(abi, dtype, batch, M, K, N, short):
+    """A stack of few blocks is bound by the trips of one block's chain, a large one by the work of a unit."""
+    from mygrad_amd import _hip
+
+    a, b = np.ones((batch, M, K), dtype=dtype), np.ones((batch, K, N), dtype=dtype)
+    assert np.array_equal(abi.matmul_batched(a, b), np.full((batch, M, N), K, dtype=dtype))
+    assert _hip.last_plan().startswith("batched") and ("short" in _hip.last_plan()) == short, _hip.last_plan()
+
+
 def test_batched_product_bad_arguments(abi):
     from mygrad_amd import _device, _hip
 
