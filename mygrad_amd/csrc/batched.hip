@@ -454,21 +454,32 @@ int mg_matmul_batched(int dtype, int64_t batch, int64_t M, int64_t K, int64_t N,
   // (dealing pairs out to the XCDs pays where each has many: with 100 pairs of five tiles some units get a
   // third block, 25 -> 37 us)
   p.dealt = batch >= 64 && tiles >= 8 * cus;
-  const long long blocks = p.dealt ? ceil_div(batch, 8) * 8 * (tiles / batch) : tiles;
-  p.pairs = (int)batch;
-  if (tile >= 0 && blocks < (1ll << 31)) {
-    p.row_tiles = (int)ceil_div(M, bm);
-    p.col_tiles = (int)ceil_div(N, 4096 / bm);
-    if (dtype == MG_F32)
-      launch_staged<float>(p, bm, deep != 0, (unsigned)blocks, trans_a != 0, trans_b != 0, a, b, out, s);
-    else
-      launch_staged<double>(p, bm, deep != 0, (unsigned)blocks, trans_a != 0, trans_b != 0, a, b, out, s);
-    MG_HIP(hipGetLastError());
-    return MG_OK;
-  }
-  const dim3 grid((unsigned)ceil_div(p.tiles, 4)), block(256);
+  // A launch has fewer than 2^32 threads along x, which is 2^24 - 1 blocks: a longer stack goes in runs of pairs.
+  const long long most = (1ll << 24) - 1, per_pair = tile < 0 ? (long long)p.row_tiles * p.col_tiles : tiles / batch;
+  long long at_once = (tile < 0 ? 4 * most : most) / per_pair;
+  if (at_once < 1) return fail(MG_ERR_UNSUPPORTED, "mg_matmul_batched: a product of 2^24 tiles or more");
+  if (at_once < 8) p.dealt = 0;
+  if (p.dealt) at_once = at_once / 8 * 8;
+  const size_t elem = f64 ? 8 : 4;
+  for (long long first = 0; first < batch; first += at_once) {
+    const long long count = std::min(at_once, batch - first);
+    const void *pa = static_cast<const char *>(a) + first * p.a_pair * elem, *pb = static_cast<const char *>(b) + first * p.b_pair * elem;
+    void *po = static_cast<char *>(out) + first * M * N * elem;
+    p.pairs = (int)count;
+    p.tiles = count * per_pair;
+    if (tile >= 0) {
+      p.row_tiles = (int)ceil_div(M, bm);
+      p.col_tiles = (int)ceil_div(N, 4096 / bm);
+      const unsigned blocks = (unsigned)(p.dealt ? ceil_div(count, 8) * 8 * per_pair : p.tiles);
+      if (f64)
+        launch_staged<double>(p, bm, deep != 0, blocks, trans_a != 0, trans_b != 0, pa, pb, po, s);
+      else
+        launch_staged<float>(p, bm, deep != 0, blocks, trans_a != 0, trans_b != 0, pa, pb, po, s);
+      continue;
+    }
+    const dim3 grid((unsigned)ceil_div(p.tiles, 4)), block(256);
 #define MG_BATCHED(T, AV, BV) \
-  hipLaunchKernelGGL((batched_product_kernel<T, AV, BV>), grid, block, 0, s, p, (const T *)a, (const T *)b, (T *)out)
+  hipLaunchKernelGGL((batched_product_kernel<T, AV, BV>), grid, block, 0, s, p, (const T *)pa, (const T *)pb, (T *)po)
 #define MG_BATCHED_T(T)                 \
   do {                                  \
     if (av && bv) MG_BATCHED(T, true, true);        \
@@ -476,9 +487,10 @@ int mg_matmul_batched(int dtype, int64_t batch, int64_t M, int64_t K, int64_t N,
     else if (bv) MG_BATCHED(T, false, true);        \
     else MG_BATCHED(T, false, false);               \
   } while (0)
-  if (dtype == MG_F32) MG_BATCHED_T(float); else MG_BATCHED_T(double);
+    if (f64) MG_BATCHED_T(double); else MG_BATCHED_T(float);
 #undef MG_BATCHED_T
 #undef MG_BATCHED
+  }
   MG_HIP(hipGetLastError());
   return MG_OK;
 }

@@ -142,6 +142,14 @@ def test_small_stacks_take_few_trips(abi, dtype, batch, M, K, N, short):
     assert _hip.last_plan().startswith("batched") and ("short" in _hip.last_plan()) == short, _hip.last_plan()
 
 
+def test_batched_product_of_more_blocks_than_a_launch_has(abi):
+    """2^26 + 5 products of one element are 2^24 + 2 blocks of four; a launch is limited to fewer than 2^32 threads."""
+    batch = 2**26 + 5
+    a = (np.arange(batch) % 251).astype(np.float32).reshape(batch, 1, 1)
+    b = (np.arange(batch) % 127).astype(np.float32).reshape(batch, 1, 1)
+    assert np.array_equal(abi.matmul_batched(a, b), a * b)
+
+
 def test_batched_product_bad_arguments(abi):
     from mygrad_amd import _device, _hip
 
