@@ -309,7 +309,7 @@ int mg_fill_value(int dtype, int64_t n, double value, void *out);
 /* mean[c], var[c] = mean and (biased) variance of x[:, c, ...]; y = (x - mean) /
  * sqrt(var + eps) [* gamma] [+ beta].  The sums run over a fixed partition in double and
  * are rounded once; the element-wise steps are rounded in dtype in the reference's order.
- * mean and var, (C,) each, are outputs the caller keeps for mg_batchnorm_bwd.
+ * mean and var, (C,) each, are outputs the caller keeps for mg_batchnorm_bwd.  y may be x.
  * Replaces BatchNorm.__call__, src/mygrad/nnet/layers/batchnorm.py:26-74. */
 int mg_batchnorm_fwd(const mg_bn_desc *desc, const void *x, const void *gamma, const void *beta, void *y, void *mean,
                      void *var);
@@ -320,7 +320,7 @@ int mg_batchnorm_fwd(const mg_bn_desc *desc, const void *x, const void *gamma, c
  *            (BatchNorm.backward_var index 0, batchnorm.py:78-99)
  *   dgamma = sum_c(grad * xn)   (index 1 with gamma, batchnorm.py:101-102)
  *   dbeta  = sum_c(grad)        (index 2, or 1 without gamma, batchnorm.py:104-106)
- * Any of dx, dgamma, dbeta may be null (not wanted), not all three. */
+ * Any of dx, dgamma, dbeta may be null (not wanted), not all three.  dx may be x or grad. */
 int mg_batchnorm_bwd(const mg_bn_desc *desc, const void *x, const void *grad, const void *gamma, const void *mean,
                      const void *var, void *dx, void *dgamma, void *dbeta);
 

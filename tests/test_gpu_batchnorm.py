@@ -286,3 +286,42 @@ def test_rows_that_are_no_whole_16_byte_pieces(abi, shape, dtype):
     assert np.array_equal(dbeta, grad.sum(axes).astype(dtype))
     one = np.ones(shape[1])
     assert err(dx, ora.batchnorm_backward(grad.astype(np.float64), x.astype(np.float64), one, eps=1e-5)[0]) <= TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("shape", [(3, 2, 65), (40, 3, 11, 11), (5, 2, 68), (33, 5, 9), (7, 2, 5003)])
+def test_in_place(abi, dtype, shape):
+    """The result may take the place of x, and dx that of x or of the gradient, for rows of any length: every
+    element is read before it is written, and written once."""
+    import ctypes
+
+    from mygrad_amd import _device, _hip
+
+    rng = np.random.default_rng(list(shape))
+    dtype = np.dtype(dtype)
+    x, g = rng.standard_normal(shape).astype(dtype), rng.standard_normal(shape).astype(dtype)
+    c = shape[1]
+    desc = _hip.BnDesc(dtype=_hip.dtype_code(dtype), has_gamma=0, has_beta=0, reserved=0, N=shape[0], C=c, S=x.size // shape[0] // c, eps=1e-5)
+    lib, ref = _hip.lib(), ctypes.byref(desc)
+
+    def buffer(arr):
+        buf = _device.DeviceBuffer(max(arr.nbytes, 16))
+        buf.upload(arr)
+        return buf
+
+    def values(buf):
+        out = np.empty(shape, dtype)
+        buf.download_into(out)
+        return out
+
+    mean, var = (buffer(np.zeros(c, dtype)) for _ in range(2))
+    apart, place, kept = buffer(np.zeros_like(x)), buffer(x), (buffer(x), buffer(g))
+    _hip.check(lib.mg_batchnorm_fwd(ref, kept[0].ptr, None, None, apart.ptr, mean.ptr, var.ptr))
+    _hip.check(lib.mg_batchnorm_fwd(ref, place.ptr, None, None, place.ptr, mean.ptr, var.ptr))
+    assert np.array_equal(values(apart), values(place))
+    _hip.check(lib.mg_batchnorm_bwd(ref, kept[0].ptr, kept[1].ptr, None, mean.ptr, var.ptr, apart.ptr, None, None))
+    for over_x in (True, False):
+        xb, gb = buffer(x), buffer(g)
+        dx = xb if over_x else gb
+        _hip.check(lib.mg_batchnorm_bwd(ref, xb.ptr, gb.ptr, None, mean.ptr, var.ptr, dx.ptr, None, None))
+        assert np.array_equal(values(apart), values(dx))
