@@ -284,6 +284,21 @@ void staging_release() {
     if (e) (void)hipEventDestroy(e);
   st = Staging{};
 }
+// Whether there are staging memory and its events; all of them or none.
+bool staging_prepare() {
+  Staging &st = staging();
+  bool ok = hipHostMalloc(reinterpret_cast<void **>(&st.base), Staging::kSegment * Staging::kSegments, hipHostMallocDefault) == hipSuccess;
+  if (!ok) st.base = nullptr;
+  for (hipEvent_t &e : st.left) {
+    ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+    if (!ok) e = nullptr;
+  }
+  if (!ok) {
+    staging_release();
+    (void)hipGetLastError();
+  }
+  return ok;
+}
 // Copies of at most this many bytes between device and pinned memory are a kernel of this library: a
 // launch and the link's latency, where the runtime's copy costs about twice that.  Larger ones leave
 // the link to the runtime's copy.
@@ -527,14 +542,7 @@ int mg_upload(void *dst_dev, const void *src_host, size_t nbytes) {
   if (nbytes > Staging::kSegment / 4) return mg_memcpy_h2d(dst_dev, src_host, nbytes);
   Runtime &rt = runtime();
   Staging &st = staging();
-  if (!st.base) {
-    if (hipHostMalloc(reinterpret_cast<void **>(&st.base), Staging::kSegment * Staging::kSegments, hipHostMallocDefault) != hipSuccess) {
-      (void)hipGetLastError();
-      st.base = nullptr;
-      return mg_memcpy_h2d(dst_dev, src_host, nbytes);
-    }
-    for (hipEvent_t &e : st.left) MG_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-  }
+  if (!st.base && !staging_prepare()) return mg_memcpy_h2d(dst_dev, src_host, nbytes);
   if (st.offset + nbytes > Staging::kSegment) {
     MG_HIP(hipEventRecord(st.left[st.segment], rt.stream));
     st.pending[st.segment] = true;

@@ -713,3 +713,36 @@ def test_reused_checks_refuse_what_the_checks_refuse():
         for _ in range(2):
             with pytest.raises(ValueError):
                 _probe_shape(a, b)
+
+
+@pytest.mark.parametrize("fail", ["0", "1", "3"])
+def test_uploads_without_staging_memory_still_arrive(tmp_path, fail):
+    """If an event of the staging memory cannot be made, uploads take the copy that is waited for (host stand-ins
+    for the runtime; more bytes than the staging memory holds)."""
+    import shutil
+    import subprocess
+    import sys
+
+    from mygrad_amd import _hip
+
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    if not shutil.which("g++") or not os.path.exists(os.path.join(rocm, "include", "hip")) or not os.path.exists(_hip.library_path()):
+        pytest.skip("needs g++, the HIP headers and the built library")
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    shim = tmp_path / "standins.so"
+    subprocess.run(["g++", "-shared", "-fPIC", "-w", f"-I{rocm}/include", os.path.join(root, "tests", "hip_standins.cpp"), "-o", str(shim)], check=True)
+    program = """
+import numpy as np
+from mygrad_amd import _device, _hip
+for i in range(30):
+    source = np.full(200003, i + 1, dtype=np.uint8)
+    buf = _device.DeviceBuffer(source.nbytes)
+    buf.stage(source)
+    back = np.zeros_like(source)
+    buf.download_into(back)
+    assert np.array_equal(back, source), i
+print("arrived")
+"""
+    env = {**os.environ, "LD_PRELOAD": str(shim), "STANDIN_FAIL_EVENT": fail}
+    done = subprocess.run([sys.executable, "-c", program], cwd=root, env=env, capture_output=True, text=True, timeout=300)
+    assert done.returncode == 0 and "arrived" in done.stdout, done.stderr[-2000:]
