@@ -715,15 +715,11 @@ def test_reused_checks_refuse_what_the_checks_refuse():
                 _probe_shape(a, b)
 
 
-@pytest.mark.parametrize("fail", ["0", "1", "3"])
-def test_uploads_without_staging_memory_still_arrive(tmp_path, fail):
-    """If an event of the staging memory cannot be made, uploads take the copy that is waited for (host stand-ins
-    for the runtime; more bytes than the staging memory holds)."""
+def run_on_standins(tmp_path, program, **variables):
+    """Runs a program on host stand-ins for the HIP runtime (kernels are not run); its output."""
     import shutil
     import subprocess
     import sys
-
-    from mygrad_amd import _hip
 
     rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
     if not shutil.which("g++") or not os.path.exists(os.path.join(rocm, "include", "hip")) or not os.path.exists(_hip.library_path()):
@@ -731,6 +727,16 @@ def test_uploads_without_staging_memory_still_arrive(tmp_path, fail):
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
     shim = tmp_path / "standins.so"
     subprocess.run(["g++", "-shared", "-fPIC", "-w", f"-I{rocm}/include", os.path.join(root, "tests", "hip_standins.cpp"), "-o", str(shim)], check=True)
+    done = subprocess.run([sys.executable, "-c", program], cwd=root, env={**os.environ, "LD_PRELOAD": str(shim), **variables},
+                          capture_output=True, text=True, timeout=300)
+    assert done.returncode == 0, done.stderr[-2000:]
+    return done.stdout
+
+
+@pytest.mark.parametrize("fail", ["0", "1", "3"])
+def test_uploads_without_staging_memory_still_arrive(tmp_path, fail):
+    """If an event of the staging memory cannot be made, uploads take the copy that is waited for (more bytes than
+    the staging memory holds)."""
     program = """
 import numpy as np
 from mygrad_amd import _device, _hip
@@ -743,6 +749,29 @@ for i in range(30):
     assert np.array_equal(back, source), i
 print("arrived")
 """
-    env = {**os.environ, "LD_PRELOAD": str(shim), "STANDIN_FAIL_EVENT": fail}
-    done = subprocess.run([sys.executable, "-c", program], cwd=root, env=env, capture_output=True, text=True, timeout=300)
-    assert done.returncode == 0 and "arrived" in done.stdout, done.stderr[-2000:]
+    assert "arrived" in run_on_standins(tmp_path, program, STANDIN_FAIL_EVENT=fail)
+
+
+def test_copies_beyond_a_block_are_refused(tmp_path):
+    """What is copied by a kernel is checked on the host first: both blocks hold that many bytes.  Addresses inside
+    a block, or of no pool, are left to the runtime's copy."""
+    program = """
+import ctypes, numpy as np
+from mygrad_amd import _device, _hip
+lib = _hip.lib()
+small, large = _device.DeviceBuffer(512), _device.DeviceBuffer(8192)
+pin_small, pin_large = ctypes.c_void_p(), ctypes.c_void_p()
+assert lib.mg_host_alloc(ctypes.byref(pin_small), 512) == lib.mg_host_alloc(ctypes.byref(pin_large), 8192) == _hip.MG_OK
+host = np.arange(8192, dtype=np.uint8)
+bad, ok = _hip.MG_ERR_BAD_ARG, _hip.MG_OK
+assert lib.mg_upload(small.ptr, host.ctypes.data, 513) == bad
+assert lib.mg_upload(small.ptr, host.ctypes.data, 512) == lib.mg_upload(large.ptr, host.ctypes.data, 8192) == ok
+assert lib.mg_memcpy_d2h(pin_small, large.ptr, 513) == lib.mg_memcpy_d2h(pin_large, small.ptr, 513) == bad
+assert lib.mg_memcpy_d2h(pin_small, large.ptr, 512) == lib.mg_memcpy_d2h(pin_large, large.ptr, 8192) == ok
+# the runtime's copy (memcpy here) moves what starts inside a block
+assert lib.mg_upload(large.ptr + 16, host.ctypes.data, 4096) == ok
+back = np.zeros(4096, np.uint8)
+assert lib.mg_memcpy_d2h(back.ctypes.data, large.ptr + 16, 4096) == ok and np.array_equal(back, host[:4096])
+print("refused")
+"""
+    assert "refused" in run_on_standins(tmp_path, program)
