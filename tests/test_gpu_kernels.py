@@ -936,15 +936,8 @@ def test_random_problems_with_few_rows(abi, m, which):
         done += 1
 
 
-# Shapes picked so that, between them, every tile shape and code path of the tap-major
-# kernels runs: all gather-GEMM tiles (rows 16..128), persistent blocks that stream
-# through several tiles and K slices, strided dgrad phases, filter counts that are not a
-# multiple of four (padded packed rows), the 128x128 / 64x192 / 64x128 / 64x64 / 32x64 /
-# 16x64 filter-gradient tiles, and an odd number of positions per sample (grad tile
-# loaded element by element instead of 16 bytes per lane).
-PADDED_CHANNEL_CASES = [
-    # (x shape, w shape, stride, pad, dilation): large enough, channel / filter counts that are no
-    # multiple of 16 but within a third of one: run on zero-padded copies by the tap-major kernels
+AWKWARD_CHANNEL_CASES = [
+    # (x shape, w shape, stride, pad, dilation): channel / filter counts that are no multiple of 16
     ((8, 24, 48, 48), (40, 24, 3, 3), (1, 1), (1, 1), (1, 1)),
     ((6, 40, 40, 40), (32, 40, 3, 3), (2, 2), (1, 1), (1, 1)),
     ((4, 32, 64, 64), (56, 32, 3, 3), (1, 1), (0, 0), (2, 2)),
@@ -954,9 +947,9 @@ PADDED_CHANNEL_CASES = [
 
 
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
-@pytest.mark.parametrize("case", range(len(PADDED_CHANNEL_CASES)))
-def test_conv_awkward_channel_counts_on_padded_copies(abi, dtype, case):
-    x_shape, w_shape, s, p, d = PADDED_CHANNEL_CASES[case]
+@pytest.mark.parametrize("case", range(len(AWKWARD_CHANNEL_CASES)))
+def test_conv_awkward_channel_counts(abi, dtype, case):
+    x_shape, w_shape, s, p, d = AWKWARD_CHANNEL_CASES[case]
     rng = np.random.default_rng(700 + case)
     tol = TOL[np.dtype(dtype)]
     x = rng.standard_normal(x_shape).astype(dtype)
@@ -969,34 +962,45 @@ def test_conv_awkward_channel_counts_on_padded_copies(abi, dtype, case):
 
 
 # Counts that fill no K tile (channels forward, filters in the data gradient) or no row tile, read where they lie:
-# one row short of and one beyond a K tile, of each row tile and of a group of 16 columns; strides (fused
-# phases, phases as rows), folded taps, one tap (the filter gradient written without a pass over
-# partial sums), an odd number of positions.
+# one row short of and one beyond a K tile, of each row tile and of a group of 16 columns; an odd number of
+# positions.  From 2e8 flops on such counts are contracted in K tiles with dead rows; which kernel a pass
+# takes is part of the case: (x, w, stride, padding, dilation, forward, data gradient in float32, in float64).
 RAGGED_CASES = [
-    # x shape, w shape, stride, padding, dilation
-    ((2, 47, 41, 37), (83, 47, 3, 3), (1, 1), (1, 1), (1, 1)),
-    ((2, 33, 47, 43), (65, 33, 3, 3), (2, 2), (1, 1), (1, 1)),
-    ((3, 45, 30, 64), (31, 45, 3, 3), (1, 1), (1, 1), (1, 1)),
-    ((2, 4, 113, 113), (95, 4, 5, 5), (2, 2), (2, 2), (1, 1)),
-    ((2, 49, 1501), (129, 49, 9), (1,), (4,), (1,)),
-    ((1, 81, 9001), (161, 81, 1), (1,), (0,), (1,)),
-    ((4, 18, 6, 25, 25), (47, 18, 3, 3, 1), (1, 2, 2), (1, 0, 0), (1, 1, 1)),
+    ((2, 47, 41, 37), (83, 47, 3, 3), (1, 1), (1, 1), (1, 1), "tap-major tile", "tap-major tile", "tap-major tile"),
+    # four fused stride phases, K tiles 16 and 32 deep; two
+    ((12, 45, 47, 43), (65, 45, 3, 3), (2, 2), (1, 1), (1, 1), "tap-major tile", "x16, 1 phase(s) (4 fused", "4 phase(s) (1 fused"),
+    ((12, 31, 47, 43), (93, 31, 3, 3), (2, 2), (1, 1), (1, 1), "tap-major tile", "x32, 1 phase(s) (4 fused", "4 phase(s) (1 fused"),
+    ((6, 45, 33, 41), (61, 45, 3, 3), (1, 2), (1, 1), (1, 1), "tap-major tile", "(2 fused", "2 phase(s) (1 fused"),
+    # the taps of the last axis folded into the rows: forward (96 x 128), data gradient (48 x 256)
+    ((6, 45, 30, 64), (31, 45, 3, 3), (1, 1), (1, 1), (1, 1), "folded taps tile 96x128", "tap-major tile", "tap-major tile"),
+    ((12, 13, 30, 64), (45, 13, 3, 3), (1, 1), (1, 1), (1, 1), "tap-major tile", "folded taps tile 48x256", "folded taps tile 48x256"),
+    # the stride phases of a few channels as rows
+    ((4, 4, 113, 113), (95, 4, 5, 5), (2, 2), (2, 2), (1, 1), "fwd", "stride phases as rows", "stride phases as rows"),
+    ((2, 49, 1501), (129, 49, 9), (1,), (4,), (1,), "tap-major tile", "tap-major tile", "tap-major tile"),
+    # one tap: the filter gradient written without a pass over partial sums
+    ((1, 81, 9001), (161, 81, 1), (1,), (0,), (1,), "tap-major tile", "tap-major tile", "tap-major tile"),
+    ((10, 29, 6, 25, 25), (47, 29, 3, 3, 1), (1, 2, 2), (1, 0, 0), (1, 1, 1), "tap-major tile", "(4 fused", "4 phase(s) (1 fused"),
 ]
 
 
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 @pytest.mark.parametrize("case", range(len(RAGGED_CASES)))
 def test_conv_counts_that_fill_no_tile_in_place(abi, dtype, case):
-    x_shape, w_shape, s, p, d = RAGGED_CASES[case]
+    from mygrad_amd import _hip
+
+    x_shape, w_shape, s, p, d, fwd, dx32, dx64 = RAGGED_CASES[case]
     rng = np.random.default_rng(1700 + case)
     print("ragged", np.dtype(dtype).name, x_shape, w_shape, s, p, d, flush=True)
     # small integers: every sum is exact in both precisions, so the results are compared as they are
     x = rng.integers(-3, 4, x_shape).astype(dtype)
     w = rng.integers(-2, 3, w_shape).astype(dtype)
     want = direct.conv_forward(x, w, s, p, d).astype(dtype)
+    assert 2.0 * want.size * w[0].size >= 2e8
     g = rng.integers(-2, 3, want.shape).astype(dtype)
     assert np.array_equal(abi.conv_fwd(x, w, s, p, d), want)
+    assert fwd in _hip.last_plan(), _hip.last_plan()
     assert np.array_equal(abi.conv_dgrad(g, x_shape, w, s, p, d), direct.conv_backward_x(g, x_shape, w, s, p, d).astype(dtype))
+    assert (dx32 if dtype == np.float32 else dx64) in _hip.last_plan(), _hip.last_plan()
     assert np.array_equal(abi.conv_wgrad(g, x, w_shape, s, p, d), direct.conv_backward_w(g, x, w_shape, s, p, d).astype(dtype))
     # what lies behind a sample's channels (the next sample's first ones) stays out of its sums, NaN and all
     if x_shape[0] > 1:
@@ -1005,6 +1009,24 @@ def test_conv_counts_that_fill_no_tile_in_place(abi, dtype, case):
         assert np.array_equal(abi.conv_fwd(xn, w, s, p, d)[0], want[0])
         dx = direct.conv_backward_x(g[:1], (1, *x_shape[1:]), w, s, p, d).astype(dtype)
         assert np.array_equal(abi.conv_dgrad(gn, x_shape, w, s, p, d)[0], dx[0])
+
+
+@pytest.mark.parametrize("tile", ["128,128", "128,64", "96,128", "64,256", "64,128", "48,256", "32,256", "32,128", "16,256"])
+def test_dead_rows_in_every_tile(abi, monkeypatch, tile):
+    """float32, one K tile of dead rows per tap, in every tile shape of the forward and data-gradient kernels (some
+    have an instance of their own for it)."""
+    from mygrad_amd import _hip
+
+    monkeypatch.setenv("MYGRAD_HIP_TILE", tile)
+    rng = np.random.default_rng(45)
+    x_shape, w_shape, conf = (3, 45, 41, 37), (61, 45, 3, 3), ((1, 1), (1, 1), (1, 1))
+    x, w = rng.integers(-3, 4, x_shape).astype(np.float32), rng.integers(-2, 3, w_shape).astype(np.float32)
+    want = direct.conv_forward(x, w, *conf).astype(np.float32)
+    g = rng.integers(-2, 3, want.shape).astype(np.float32)
+    print("dead rows", tile, flush=True)
+    for got, ref in ((abi.conv_fwd(x, w, *conf), want), (abi.conv_dgrad(g, x_shape, w, *conf), direct.conv_backward_x(g, x_shape, w, *conf).astype(np.float32))):
+        assert f"tap-major tile {tile.replace(',', 'x')}x" in _hip.last_plan(), _hip.last_plan()
+        assert np.array_equal(got, ref)
 
 
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
@@ -1151,12 +1173,17 @@ def test_filter_gradient_of_a_tap_with_one_channel_beyond_a_group(abi, dtype):
     assert "table rows tile 64x32" in _hip.last_plan(), _hip.last_plan()
 
 
+# Shapes picked so that, between them, the code paths of the tap-major kernels run: persistent blocks that
+# stream through several tiles and K slices, strided dgrad phases, filter counts that are not a multiple of
+# four (padded packed rows), wide and square filter-gradient tiles, and an odd number of positions per
+# sample (grad tile loaded element by element instead of 16 bytes per lane).  (Every tile shape is
+# forced in tests of its own, above.)
 KERNEL_VARIANT_CASES = [
     # x shape, w shape, stride, padding, dilation
-    ((8, 128, 28, 28), (128, 128, 3, 3), (1, 1), (1, 1), (1, 1)),   # 128-row tiles, wgrad 128x128
-    ((32, 64, 28, 28), (64, 64, 3, 3), (1, 1), (1, 1), (1, 1)),     # 64x256, wgrad 64x192
-    ((64, 64, 28, 28), (64, 64, 2, 2), (1, 1), (0, 0), (1, 1)),     # wgrad 64x128
-    ((16, 128, 29, 29), (256, 128, 3, 3), (2, 2), (1, 1), (1, 1)),  # four dgrad phases, 128x64 tiles, tail slices
+    ((8, 128, 28, 28), (128, 128, 3, 3), (1, 1), (1, 1), (1, 1)),   # wgrad 128x128
+    ((32, 64, 28, 28), (64, 64, 3, 3), (1, 1), (1, 1), (1, 1)),     # wgrad 64x64
+    ((64, 64, 28, 28), (64, 64, 2, 2), (1, 1), (0, 0), (1, 1)),
+    ((16, 128, 29, 29), (256, 128, 3, 3), (2, 2), (1, 1), (1, 1)),  # four dgrad phases
     ((4, 16, 15, 15), (32, 16, 3, 3), (1, 1), (1, 1), (1, 1)),      # 225 positions per sample (odd)
     ((6, 16, 20, 20), (10, 16, 3, 3), (1, 1), (1, 1), (1, 1)),      # F = 10: packed rows padded to 12
     ((5, 48, 9, 33), (16, 48, 3, 5), (1, 2), (1, 0), (1, 2)),       # 16-row tiles, dilation, mixed strides
