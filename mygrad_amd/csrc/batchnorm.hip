@@ -435,7 +435,7 @@ __device__ __forceinline__ void axis_sum_body(const BnParams &p, const T *__rest
   __shared__ double slots[8];
   bool active;
   const int c = my_channel<WALK>(p, &active);
-  double even = 0.0, odd = 0.0;  // two running sums, added at the end
+  double even = 0.0, odd = 0.0;  // two running sums, added at the end of the thread's share
   if (active)
     visit<T, WALK>(p, [&](long long at, int seen) {
 #pragma clang fp contract(off)  // the product is rounded to T, like a product formed first: no fused multiply-add
@@ -453,7 +453,9 @@ __device__ __forceinline__ void axis_sum_body(const BnParams &p, const T *__rest
         even += (double)v;
       }
     });
-  put_partial<WALK>(p, c, active, even, odd, partial, slots);
+  // one sum over the block, not two: a channel of few elements takes little but the exchanges of that
+  // sum.  (3, 40000, 77), single precision: 55.6 us with both, 33.7 with one
+  put_partial<WALK>(p, c, active, even + odd, 0.0, partial, slots);
 }
 
 template <typename T, int WALK>
@@ -473,9 +475,9 @@ template <typename T>
 __global__ void __launch_bounds__(256) axis_sum_finish_kernel(BnParams p, const double *__restrict__ partial, T *__restrict__ out) {
   const int c = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (c >= p.C) return;
-  double even, odd;
-  channel_totals(p, c, partial, &even, &odd);
-  if ((threadIdx.x & 63) == 0) out[c] = (T)(even + odd);
+  double sum, none;
+  channel_totals(p, c, partial, &sum, &none);
+  if ((threadIdx.x & 63) == 0) out[c] = (T)sum;
 }
 
 // out[o, i] = sum over m of x[o, m, i] for x:(outer, n, inner).  A thread owns VEC consecutive
