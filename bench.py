@@ -165,6 +165,15 @@ def _sweep_shapes():
     pool("p2x2s2@14-f64", "f64", (128, 256, 14, 14), (2, 2), 2)
     pool("p3x3x3s2@33x65x65-f32", "f32", (8, 32, 33, 65, 65), (3, 3, 3), 2)
     pool("p2x2x2s2@32x64x64-f32", "f32", (8, 32, 32, 64, 64), (2, 2, 2), 2)
+    # channel and filter counts that fill no tile, and passes with fewer tiles than the device has block slots
+    conv("c9-45to83@16001", "f32", (16, 45, 16001), (83, 45, 9), 1, 4, 1)
+    conv("c5-51to24@12603", "f32", (15, 51, 12603), (24, 51, 5), 1, 0, 1)
+    conv("c3x3s21-156to424@107x43", "f32", (2, 156, 107, 43), (424, 156, 3, 3), (2, 1), 0, 1)
+    conv("c3x2x3-171to326@5x25x45", "f32", (1, 171, 5, 25, 45), (326, 171, 3, 2, 3), 1, 0, 1)
+    conv("c3x3-259to27@26x31-f64", "f64", (8, 259, 26, 31), (27, 259, 3, 3), 1, 0, 1)
+    conv("c3x3-7to37@17x28", "f32", (1, 7, 17, 28), (37, 7, 3, 3), 1, 0, 1)
+    conv("c1x1-8to64@112", "f32", (64, 8, 112, 112), (64, 8, 1, 1), 1, 0, 1)
+    conv("c1x1-17to64@112", "f32", (64, 17, 112, 112), (64, 17, 1, 1), 1, 0, 1)
     return shapes
 
 
