@@ -120,7 +120,9 @@ int mg_host_free(void *hptr);
 int mg_memcpy_h2d(void *dst_dev, const void *src_host, size_t nbytes); /* stream-ordered, returns when src may be reused */
 int mg_upload(void *dst_dev, const void *src_host, size_t nbytes);     /* the same for memory that only this library's stream
                                                                           reads: arrays of up to 256 KiB go through pinned
-                                                                          staging memory and are not waited for */
+                                                                          staging memory and are not waited for.  Here and in
+                                                                          mg_memcpy_d2h more bytes than a block of mg_malloc
+                                                                          (mg_host_alloc) holds, from its start, are refused */
 int mg_memcpy_d2h(void *dst_host, const void *src_dev, size_t nbytes); /* returns when dst holds the data */
 int mg_memcpy_d2d(void *dst_dev, const void *src_dev, size_t nbytes);  /* stream-ordered; a plain 16-byte-per-lane
                                                                           copy kernel when everything is 16-byte aligned */

@@ -2060,7 +2060,8 @@ int build_wgrad_plan(const Geometry &g, Plan &pl) {
   const bool f64 = g.dtype == MG_F64;
   // tap-major columns: whole groups of 16 channels per tap (the last group moved back, see WGroup), which
   // takes 16 channels to move in, unless most of that group would be computed twice: table rows come
-  // in narrower tiles ((8,17,112,112) * (256,17,1,1), double precision: 43 us, 67 on whole groups)
+  // in narrower tiles ((8,17,112,112) * (256,17,1,1), double precision: 43 us, 67 on whole groups).  So do
+  // 12 to 15 channels: (32,C,56,56) * (64,C,3,3) 28.5 - 40.3 us, 40.1 on copies padded to 16.
   const bool ragged_c = g.C % 16 != 0 && g.C >= 16 && mostly_live(g.C) && whole_channels(g, g.C) % 16 == 0 && whole_channels(g, g.C) != 0;
   const bool whole_c = g.C % 16 == 0 || ragged_c;
   pl.depth = ragged_c ? whole_channels(g, g.C) : g.C;
