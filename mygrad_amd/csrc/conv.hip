@@ -13,6 +13,7 @@
 //   wgrad     M = F, N = (c, tap),        K = (n, g)     gathers grad and x; the
 //             long K is split over blocks, partial sums are added in a fixed
 //             order by a second kernel (no atomics, run-to-run identical)
+#include "conv_device.h"
 #include "conv_kernels.h"
 #include "internal.h"
 
@@ -23,55 +24,11 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <memory>
 #include <string>
 #include <vector>
 
 namespace mg {
-
-// Tables that every lane of a wavefront reads at the same index are addressed
-// through the constant address space, which lets the compiler fetch them with
-// scalar loads (one request per wavefront, no vector-memory wait) instead of 64
-// identical vector loads.
-#define MG_CONSTANT __attribute__((address_space(4)))
-typedef int int4v __attribute__((ext_vector_type(4)));
-static_assert(sizeof(TabEntry) == sizeof(int4v), "a table row is read as one 16-byte vector");
-__device__ __forceinline__ const int4v MG_CONSTANT *as_constant(const TabEntry *p) {
-  return (const int4v MG_CONSTANT *)(p);
-}
-__device__ __forceinline__ const int MG_CONSTANT *as_constant(const int *p) { return (const int MG_CONSTANT *)(p); }
-__device__ __forceinline__ TabEntry table_row(const int4v MG_CONSTANT *tab, int i) {
-  const int4v v = tab[i];
-  return TabEntry{v.x, v.y, v.z, v.w};
-}
-// The wavefront-uniform value of x as a scalar register.
-__device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
-
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef double f64x4 __attribute__((ext_vector_type(4)));
-
-// D(16x16) += A(16x4) * B(4x16) on one wavefront.  Lane l supplies A[l%16][l/16]
-// and B[l/16][l%16].  Lane l receives four elements of column l%16 of D; their
-// rows are row_of(l, r), r = 0..3, which differs between the two instructions.
-template <typename T>
-struct Mma;
-
-template <>
-struct Mma<float> {
-  using Acc = f32x4;
-  static __device__ __forceinline__ Acc run(float a, float b, Acc c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ int row_of(int lane, int r) { return 4 * (lane >> 4) + r; }
-};
-
-template <>
-struct Mma<double> {
-  using Acc = f64x4;
-  static __device__ __forceinline__ Acc run(double a, double b, Acc c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ int row_of(int lane, int r) { return 4 * r + (lane >> 4); }
-};
 
 // ------------------------------------------------------------------------------------------
 // filter packing: the tap-major GEMMs want the filter operand with M contiguous
@@ -131,7 +88,11 @@ __global__ void __launch_bounds__(256) pack_phase_rows_kernel(const T *__restric
 
 template <typename T>
 __global__ void __launch_bounds__(256) pack_filters_kernel(const T *__restrict__ w, T *__restrict__ ap, int F, int C,
-                                                           int wvol, int mode, int ld, int depth) {
+                                                           int wvol, int mode, int ld, int depth, SplitFlags *gate) {
+  if (gate != nullptr) {  // behind a pass of conv_split.hip
+    if (blockIdx.x == 0 && threadIdx.x == 0) gate->filters = 0;
+    if (gate->rerun == 0) return;
+  }
   const int M = (mode == 2 || mode == 6) ? F : mode == 3 ? C : mode == 4 ? 3 * C : 3 * F;
   const int total = (mode == 4 || mode == 5 ? wvol / 3 : wvol) * depth * ld;
   for (int idx = blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += gridDim.x * blockDim.x) {
@@ -495,34 +456,6 @@ __global__ void __launch_bounds__(256) wgrad_kernel(const WgradParams p) {
   }
 }
 
-// ((p[0] + p[stride]) + p[2*stride]) + ... over `terms` terms: always this order, so
-// the result does not change from run to run; sixteen loads are in flight at a time
-// (the partial sums were written by other XCDs a moment ago: every load is a trip
-// past this XCD's L2).
-template <typename T>
-__device__ __forceinline__ T sum_in_order(const T *__restrict__ p, long long stride, int terms) {
-  constexpr int BATCH = 16;
-  T s = p[0];
-  int k = 1;
-  for (; k + BATCH <= terms; k += BATCH) {
-    T v[BATCH];
-#pragma unroll
-    for (int u = 0; u < BATCH; ++u) v[u] = p[(long long)(k + u) * stride];
-#pragma unroll
-    for (int u = 0; u < BATCH; ++u) s += v[u];
-  }
-  if (k < terms) {
-    // the rest in one more batch: loads past the end repeat the last term and are not added
-    T v[BATCH];
-#pragma unroll
-    for (int u = 0; u < BATCH; ++u) v[u] = p[(long long)min(k + u, terms - 1) * stride];
-#pragma unroll
-    for (int u = 0; u < BATCH; ++u)
-      if (k + u < terms) s += v[u];
-  }
-  return s;
-}
-
 // dw[i] = ((part[0][i] + part[1][i]) + part[2][i]) + ...   (fixed order)
 // RUNS > 1: the splits are cut into RUNS consecutive runs, each summed in order by its own
 // thread, and the runs' totals are added in order (for a small dw, where one thread per
@@ -632,7 +565,7 @@ struct Plan {
   int pos_blocks = 0;  // position blocks of the gather-GEMM (all phases)
   int bm = 0, bn = 0;
   int bk = 0;           // depth of a K tile of the kernel chosen for this plan
-  void *pos_tab = nullptr;  // filter gradient: one row per position (WgradParams::pos_tab), its own allocation
+  void *pos_tab = nullptr;  // filter gradient: one row per position (WgradParams::pos_tab), its own allocation; so is that of a split plan
   int m_tiles = 1;     // row tiles per position block
   int full_tiles = 0;  // tiles computed whole by one block (tap-major kernel)
   int tail_split = 1;  // blocks sharing each of the remaining tiles
@@ -645,6 +578,15 @@ struct Plan {
   bool tap_major = false;  // which kernel family the tables are for
   bool ragged = false;     // tap-major: some K tile has dead rows (KTile::dead)
   int depth = 0;           // tap-major: rows of the packed filters per tap (whole_channels)
+  bool split = false;      // tap-major, single precision: operands in three bf16 parts (conv_split.hip)
+  SplitPhase *split_phases = nullptr;
+  int *split_inner = nullptr, *split_tiles = nullptr;
+  int2 *split_halves = nullptr;  // (first channel, tap) of every 16 rows of the packed filters
+  int split_half_count = 0, patch_rows = 0;
+  bool split_odd = false;        // an odd number of taps per stage
+  int split_npos = 0;            // positions (pos_tab: 8 bytes each, behind one SplitFlags)
+  std::shared_ptr<Plan> exact;   // the same pass on the single-precision kernels
+  double chain = 0;              // terms that one accumulator sums up without a break, on average
   bool single_dense_phase = false;  // positions enumerate the destination tensor in order
   bool table_rows = false;          // tap-major kernel whose K tiles are rows of the gather table (channel count no multiple of the K tile)
   int table_count = 0;              // data gradient on table rows: rows of the (padded) table = rows of the packed filters
@@ -668,7 +610,7 @@ struct Plan {
   int splits = 1;
   int kchunk = 0;
   int run_tiles = 0;  // WgradParams::run_tiles
-  char note[200] = "";  // what mg_last_plan() reports after a call that ran this plan
+  char note[256] = "";  // what mg_last_plan() reports after a call that ran this plan
 };
 
 std::map<std::string, Plan> &plans() {
@@ -854,6 +796,9 @@ struct TileRate {
   double step, rate, rate64;
 };
 constexpr TileRate kTileRates[] = {
+    // (nph 0: split_gemm_kernel)
+    {0, 16, 256, 0.50, 0.74, 0.00}, {0, 32, 256, 0.50, 0.82, 0.00}, {0, 48, 256, 0.50, 0.92, 0.00}, {0, 64, 128, 0.40, 1.05, 0.00},
+    {0, 64, 256, 0.50, 1.15, 0.00}, {0, 96, 128, 0.45, 0.95, 0.00}, {0, 128, 128, 0.50, 1.05, 0.00},
     {1, 16, 256, 0.50, 0.42, 0.42}, {1, 32, 128, 0.35, 0.59, 0.62},  {1, 32, 256, 0.55, 0.63, 0.64}, {1, 48, 256, 0.62, 0.70, 0.67},
     {1, 64, 128, 0.47, 0.77, 0.70}, {1, 64, 256, 0.78, 0.83, 0.00},  {1, 96, 128, 0.56, 0.82, 0.80}, {1, 128, 64, 0.27, 0.81, 0.87},
     {1, 128, 128, 0.63, 0.86, 0.0}, {2, 16, 256, 0.53, 0.50, 0.00},  {2, 32, 256, 0.47, 0.70, 0.00}, {2, 64, 128, 0.45, 0.82, 0.00},
@@ -882,7 +827,7 @@ double tile_time(const TileChoice &t, long long ktiles, int bk, size_t elem, int
   double a = 0, b = work * 2.0 * tile * bk * cus / (elem == 8 ? 78.6e6 * r->rate64 : 157.3e6 * r->rate);
   if (elem == 4) a = chain * r->step * bk / 16;
   if (elem == 4 && table_rows) a *= 2.1, b *= 1.2;  // (its gathers look up a row of the table per element)
-  return std::sqrt(std::sqrt(a * a * a * a + b * b * b * b)) + slices * tile * (double)elem * nph * 2.0 / 4.0e6;
+  return std::sqrt(std::sqrt(a * a * a * a + b * b * b * b)) + slices * tile * (double)elem * std::max(nph, 1) * 2.0 / 4.0e6;
 }
 
 // K tiles that one accumulator sums up without a break, on average over the results.
@@ -897,7 +842,7 @@ double mean_chain(const TileChoice &t, long long ktiles, int resident) {
 }
 
 TileChoice choose_tile(int M, const std::vector<long long> &phase_npos, int min_ktiles, bool tap_major, size_t elem, int nph, int bk, bool table_rows,
-                       bool tiny, int avg_ktiles = -1) {
+                       bool tiny, int avg_ktiles = -1, const int *patch = nullptr) {
   if (avg_ktiles < 0) avg_ktiles = min_ktiles;  // K tiles of an average tile (phases of a data gradient differ)
   struct Cfg {
     int bm, bn;
@@ -908,8 +853,10 @@ TileChoice choose_tile(int M, const std::vector<long long> &phase_npos, int min_
                               {64, 128, 1.08, true},   {48, 256, 1.00, true},  {32, 256, 1.00, false},  {32, 128, 1.10, true}, {16, 256, 1.00, false}};
   static const Cfg fused2[] = {{128, 64, 1.05, true}, {64, 128, 1.08, true}, {32, 256, 1.00, true}, {16, 256, 1.00, true}};
   static const Cfg fused4[] = {{64, 64, 1.10, true}, {32, 128, 1.10, true}, {16, 256, 1.00, true}};
-  const Cfg *cfgs = nph == 4 ? fused4 : nph == 2 ? fused2 : plain;
-  const int ncfgs = nph == 4 ? 3 : nph == 2 ? 4 : 9;
+  static const Cfg split[] = {{128, 128, 1.00, true}, {96, 128, 1.00, true}, {64, 256, 1.00, true}, {64, 128, 1.05, true},
+                              {48, 256, 1.00, true},  {32, 256, 1.00, true}, {16, 256, 1.00, true}};
+  const Cfg *cfgs = nph == 4 ? fused4 : nph == 2 ? fused2 : nph == 0 ? split : plain;
+  const int ncfgs = nph == 4 ? 3 : nph == 2 ? 4 : nph == 0 ? 7 : 9;
   // MYGRAD_HIP_TILE="rows,positions[,blocks per unit]" (diagnostics and the tests of every tile shape;
   // read whenever a plan is built, and part of the plan's key): only that tile shape, where it exists
   struct Forced {
@@ -925,10 +872,12 @@ TileChoice choose_tile(int M, const std::vector<long long> &phase_npos, int min_
     const char *flag = getenv("MYGRAD_HIP_SHARES");
     return !(flag && flag[0] == '0');
   }();
+  auto patch_fits = [&](const Cfg &c) { return patch[c.bn == 256] > 0 && patch[c.bn == 256] <= split_patch_limit(c.bm, c.bn); };
   bool forced_fits = false;
   for (int ci = 0; ci < ncfgs; ++ci)
     forced_fits |= cfgs[ci].bm == forced.bm && cfgs[ci].bn == forced.bn && (!cfgs[ci].tap_only || tap_major) &&
-                   !(tap_major && elem == 8 && cfgs[ci].bn * cfgs[ci].bm >= 128 * 128);  // (no such double-precision tile)
+                   !(tap_major && elem == 8 && cfgs[ci].bn * cfgs[ci].bm >= 128 * 128) &&  // (no such double-precision tile)
+                   !(nph == 0 && !patch_fits(cfgs[ci]));
   const int bm = forced_fits ? forced.bm : tap_major ? 0 : table_driven_rows(M, phase_npos, tiny, elem == 8);  // 0: whichever costs least
   const int cus = runtime().props.multiProcessorCount;
   struct Candidate {
@@ -949,11 +898,12 @@ TileChoice choose_tile(int M, const std::vector<long long> &phase_npos, int min_
     TileChoice best{};  // of this shape: how many blocks per unit, how the last round is shared out
     double best_cost = 0;
     if ((bm != 0 && c.bm != bm) || (c.tap_only && !tap_major) || (forced_fits && c.bn != forced.bn)) continue;
+    if (nph == 0 && !patch_fits(c)) continue;
     // 64x64 fp64 wave tiles hold 128 accumulator registers: only one 8-wave block
     // fits on a compute unit, so the tap-major kernels use the half-size shapes
     if (tap_major && elem == 8 && c.bn * c.bm >= 128 * 128) continue;
-    const bool stream = tap_major && tap_gemm_streams(c.bm, (int)elem);
-    const int per_cu = !stream ? 1 : elem == 8 ? gemm_blocks_per_cu<double>(c.bm, c.bn, 1, bk) : gemm_blocks_per_cu<float>(c.bm, c.bn, nph, bk);
+    const bool stream = nph == 0 || (tap_major && tap_gemm_streams(c.bm, (int)elem));
+    const int per_cu = !stream ? 1 : nph == 0 ? split_gemm_blocks_per_cu(c.bm, c.bn, patch[c.bn == 256]) : elem == 8 ? gemm_blocks_per_cu<double>(c.bm, c.bn, 1, bk) : gemm_blocks_per_cu<float>(c.bm, c.bn, nph, bk);
     long long pos_blocks = 0;
     for (long long n : phase_npos) pos_blocks += ceil_div(n, c.bn);
     // (most blocks first: where the rounds come out the same, more resident blocks cover more of one
@@ -999,7 +949,7 @@ TileChoice choose_tile(int M, const std::vector<long long> &phase_npos, int min_
           const double tile_seconds = 2.0 * c.bm * c.bn * depth / (0.75 * (elem == 8 ? 78.6e12 : 157.3e12) / cus);
           const long long runs = std::max<long long>(1, std::min<long long>(grid, left * (long long)std::max(avg_ktiles, 1) / kMinRun));
           const double slices = (double)(runs - 1) + (double)std::min<long long>(left, runs - 1);
-          const double fix_seconds = slices * c.bm * c.bn * (double)elem * nph * 2.0 / 4.0e12 + 4e-6;
+          const double fix_seconds = slices * c.bm * c.bn * (double)elem * std::max(nph, 1) * 2.0 / 4.0e12 + 4e-6;
           units += fix_seconds / tile_seconds;
         }
         const double cost = units * alone;
@@ -1014,7 +964,7 @@ TileChoice choose_tile(int M, const std::vector<long long> &phase_npos, int min_
         tail = (double)ceil_div(rem, cus);
         if (tap_major) {
           // slices of at least two K tiles, at most 32 MB of partial sums
-          const long long tile_bytes = (long long)c.bm * c.bn * (long long)elem * nph;
+          const long long tile_bytes = (long long)c.bm * c.bn * (long long)elem * std::max(nph, 1);
           const int smax = (int)std::max<long long>(1, std::min<long long>({(long long)min_ktiles / 2, 32ll, (32ll << 20) / (rem * tile_bytes)}));
           for (int sp = 2; sp <= smax; ++sp) {
             const double share = (double)ceil_div(rem * sp, cus) / sp + 0.01 * sp;  // + a little for the fix-up pass
@@ -1045,7 +995,7 @@ TileChoice choose_tile(int M, const std::vector<long long> &phase_npos, int min_
         u.tail_split = 1;
         if (left > 0) {
           double share = 1.0;
-          const long long tile_bytes = (long long)c.bm * c.bn * (long long)elem * nph;
+          const long long tile_bytes = (long long)c.bm * c.bn * (long long)elem * std::max(nph, 1);
           const int smax = (int)std::max<long long>(1, std::min<long long>({(long long)min_ktiles / 2, 32ll, (32ll << 20) / (left * tile_bytes)}));
           for (int sp = 2; sp <= smax; ++sp) {
             const double sh = (double)ceil_div(left * sp, cus) / sp + 0.01 * sp;
@@ -1092,6 +1042,9 @@ struct Tables {
   std::vector<int> share_first;
   std::vector<ShareSlice> share_slices;
   std::vector<ShareFix> share_fix;
+  std::vector<SplitPhase> split_phases;
+  std::vector<int> split_inner, split_tiles;
+  std::vector<int2> split_halves;
 };
 
 // Even shares of what the whole tiles leave over: the K tiles of the tiles from pl.full_tiles on,
@@ -1189,7 +1142,11 @@ int upload_plan(Plan &pl, Tables &t) {
   const size_t off_sf = off_gr + padded_bytes(t.groups);
   const size_t off_ss = off_sf + padded_bytes(t.share_first);
   const size_t off_sx = off_ss + padded_bytes(t.share_slices);
-  const size_t total = off_sx + padded_bytes(t.share_fix) + 256;
+  const size_t off_sp = off_sx + padded_bytes(t.share_fix);
+  const size_t off_si = off_sp + padded_bytes(t.split_phases);
+  const size_t off_st = off_si + padded_bytes(t.split_inner);
+  const size_t off_sh = off_st + padded_bytes(t.split_tiles);
+  const size_t total = off_sh + padded_bytes(t.split_halves) + 256;
   std::vector<char> host(total, 0);
   auto put = [&](size_t off, const void *src, size_t n) {
     if (n) memcpy(host.data() + off, src, n);
@@ -1202,6 +1159,10 @@ int upload_plan(Plan &pl, Tables &t) {
   put(off_sf, t.share_first.data(), t.share_first.size() * sizeof(int));
   put(off_ss, t.share_slices.data(), t.share_slices.size() * sizeof(ShareSlice));
   put(off_sx, t.share_fix.data(), t.share_fix.size() * sizeof(ShareFix));
+  put(off_sp, t.split_phases.data(), t.split_phases.size() * sizeof(SplitPhase));
+  put(off_si, t.split_inner.data(), t.split_inner.size() * sizeof(int));
+  put(off_st, t.split_tiles.data(), t.split_tiles.size() * sizeof(int));
+  put(off_sh, t.split_halves.data(), t.split_halves.size() * sizeof(int2));
   MG_HIP(hipMalloc(&pl.blob, host.size()));
   hipError_t err = hipMemcpy(pl.blob, host.data(), host.size(), hipMemcpyHostToDevice);
   if (err != hipSuccess) {
@@ -1216,6 +1177,10 @@ int upload_plan(Plan &pl, Tables &t) {
   pl.phases = reinterpret_cast<Phase *>(base + off_ph);
   pl.ktiles = reinterpret_cast<KTile *>(base + off_kt);
   pl.groups = reinterpret_cast<WGroup *>(base + off_gr);
+  pl.split_phases = reinterpret_cast<SplitPhase *>(base + off_sp);
+  pl.split_inner = reinterpret_cast<int *>(base + off_si);
+  pl.split_tiles = reinterpret_cast<int *>(base + off_st);
+  pl.split_halves = reinterpret_cast<int2 *>(base + off_sh);
   if (pl.share_grid > 0) {
     pl.share_first = reinterpret_cast<int *>(base + off_sf);
     pl.share_slices = reinterpret_cast<ShareSlice *>(base + off_ss);
@@ -1439,7 +1404,133 @@ void thin_tables(Plan &pl, Tables &t, const std::vector<ThinUse> &uses, int nph,
   pl.thin_w_mstride = (int)w_mstride;
 }
 
-int build_fwd_plan(const Geometry &g, Plan &pl) {
+// MYGRAD_HIP_SPLIT=0: single precision stays on the single-precision matrix instruction (part of the plan key).
+bool split_on() {
+  const char *flag = getenv("MYGRAD_HIP_SPLIT");
+  return !(flag && flag[0] == '0');
+}
+
+// Flops from which a pass runs there, for a bank of `filters` values: below, what the kernel takes per stage, the packing
+// and the gated launches behind it count for more than its products.  Against the single-precision kernels, everything included,
+// over some 1400 drawn passes of unit strides: 0.7 - 1.2 of their speed at 4 - 6 GFLOP, 0.97 - 1.8 from 8 GFLOP on ((128,64,56,56) *
+// (64,64,3,3), 29.6 GFLOP: forward 270 -> 178 us, dx 259 -> 171; (16,45,16001) * (83,45,9): 178 -> 138 and 175 -> 121;
+// (64,512,7,7) * (512,512,3,3): 156 -> 114 and 141 -> 109), but (25,316,118) * (424,316,15), 9 GFLOP against two million values: 117 ->
+// 108 and 130 -> 135.  Strided forward passes touch the more rows per position: 0.4 - 1.1 of the speed in most.
+// MYGRAD_HIP_SPLIT_MIN=flops replaces the line, and takes away the rules on speed and accuracy below (tests; part of the plan key).
+double split_min_flops(double filters) {
+  const char *v = getenv("MYGRAD_HIP_SPLIT_MIN");
+  return v ? atof(v) : 8.0e9 + 2.0e3 * filters;
+}
+
+// How a pass would run on conv_split.hip: its phase, its stages' window and the rows of src that a tile of 128 or 256
+// positions touches (0: more than the kernel has room for, with any tile of that width).
+inline long long up4(long long n) { return (n + 3) / 4 * 4; }
+struct SplitLayout {
+  SplitPhase sp{};
+  int offs[31] = {};
+  int taps = 0;
+  int patch[2] = {0, 0};
+  std::vector<int> first[2];  // see GemmParams::split_tiles
+};
+
+// The rows of src that `bn` consecutive positions touch at most, and each block's first one, when axes `inner` .. 2 are a stage's
+// window and the others' taps shift it as a whole.  A tap outside src touches nothing: along an axis of the window a position spans
+// from its first tap that may lie inside to the last.  (Positions need not ascend in rows: the data gradient has more of them
+// along an axis than the gradient has elements.)
+long long touched_rows(const SplitPhase &sp, const Phase &ph, int samples, const int *Q, int inner, int bn, std::vector<int> &first) {
+  const int qs[3] = {Q[1] * Q[2], Q[2], 1};
+  std::vector<int> low[3], high[3];
+  for (int k = 0; k < 3; ++k)
+    for (int j = 0; j < ph.J[k]; ++j) {
+      const int a = j + sp.d[k], b = a + (sp.count[k] - 1) * sp.step[k];
+      low[k].push_back((k < inner ? a : std::clamp(std::min(a, b), 0, Q[k] - 1)) * qs[k]);
+      high[k].push_back((k < inner ? a : std::clamp(std::max(a, b), 0, Q[k] - 1)) * qs[k]);
+    }
+  const long long sample_rows = up4((long long)Q[0] * qs[0]), blocks = ceil_div(ph.npos, bn);
+  std::vector<long long> from(blocks, 1ll << 60), to(blocks, -(1ll << 60));
+  long long pos = 0;
+  for (int n = 0; n < samples; ++n)
+    for (int j0 = 0; j0 < ph.J[0]; ++j0)
+      for (int j1 = 0; j1 < ph.J[1]; ++j1)
+        for (int j2 = 0; j2 < ph.J[2];) {
+          const long long block = pos / bn;
+          const int run = (int)std::min<long long>(ph.J[2] - j2, (block + 1) * bn - pos);  // low and high ascend along an axis
+          from[block] = std::min(from[block], n * sample_rows + low[0][j0] + low[1][j1] + low[2][j2]);
+          to[block] = std::max(to[block], n * sample_rows + high[0][j0] + high[1][j1] + high[2][j2 + run - 1]);
+          j2 += run, pos += run;
+        }
+  long long most = 0;
+  for (long long b = 0; b < blocks; ++b) most = std::max(most, to[b] - from[b] + 1);
+  first.assign(from.begin(), from.end());
+  return most;
+}
+
+// Whether a tap-major pass (positions of `ph`, sources at j * sj + the taps' offsets in Q) can run on operands in three
+// bf16 parts, and how.
+bool split_applies(const Geometry &g, const Plan &pl, int rows, const Phase &ph, const int *Q, SplitLayout &lay) {
+  const long long f = g.F + 31, c = g.C + 31;  // (the packed filters of either pass: 6 bytes a value, whole octets of 16 filters)
+  if (g.dtype != MG_F32 || !pl.tap_major || pl.table_rows || g.S[0] * g.S[1] * g.S[2] != 1 || conv_flops(g) < split_min_flops((double)g.F * g.C * g.wvol) || g.wvol < 3 ||
+      g.wvol > 31 || g.xvol < 2 || g.gvol < 2 || (long long)ph.npos * 8 > (32ll << 20) || f * c * g.wvol * 6 >= 1ll << 31 ||
+      (getenv("MYGRAD_HIP_TILE") && !getenv("MYGRAD_HIP_SPLIT_MIN")) || fold_applies(g, rows, pl.depth) || !split_on())
+    return false;
+  SplitPhase &sp = lay.sp;
+  const int qs[3] = {Q[1] * Q[2], Q[2], 1};
+  lay.taps = (int)g.wvol;
+  for (int a = 0, t = 0; a < sp.count[0]; ++a)
+    for (int b = 0; b < sp.count[1]; ++b)
+      for (int e = 0; e < sp.count[2]; ++e, ++t)
+        lay.offs[t] = (sp.d[0] + a * sp.step[0]) * qs[0] + (sp.d[1] + b * sp.step[1]) * qs[1] + (sp.d[2] + e * sp.step[2]);
+  // the largest inner window whose rows fit
+  for (int inner = 0; inner < 3; ++inner) {
+    int window = 1;
+    for (int k = inner; k < 3; ++k) window *= sp.count[k];
+    // (a stage's elements are loaded, split and parked for its taps' products: with three taps that is what bounds it, (59,56,930) *
+    // (443,56,3), dx, 101 us on the other kernel, 145 here; the kernel itself takes three and more)
+    if (window < (getenv("MYGRAD_HIP_SPLIT_MIN") ? 3 : 5)) break;
+    for (int wide = 0; wide < 2; ++wide) {
+      const long long rows = (touched_rows(sp, ph, g.N, Q, inner, wide ? 256 : 128, lay.first[wide]) + 3 + 15) / 16 * 16;
+      lay.patch[wide] = rows <= split_patch_limit(wide ? 64 : 96, wide ? 256 : 128) ? (int)rows : 0;
+    }
+    sp.window = window;
+    if (lay.patch[0] > 0 || lay.patch[1] > 0) return true;
+  }
+  return false;
+}
+
+// The tables of a pass on conv_split.hip that contracts `channels` channels (pl.depth of them, with dead rows), `cstride` elements apart.
+// The table of positions is filled, and the flags before it cleared, on the library's stream.
+int split_tables(Plan &pl, Tables &t, const SplitLayout &lay, const Phase &ph, const int *Q, int channels, long long cstride) {
+  const int window = lay.sp.window;
+  MG_HIP(hipMalloc(&pl.pos_tab, sizeof(SplitFlags) + (size_t)ph.npos * 8));
+  SplitPositions p{};
+  p.npos = ph.npos, p.sp = lay.sp, p.sample_rows = (int)up4((long long)Q[0] * Q[1] * Q[2]);
+  for (int k = 0; k < 3; ++k) p.J[k] = ph.J[k], p.Q[k] = Q[k];
+  launch_split_positions(p, pl.pos_tab, runtime().stream);
+  MG_HIP(hipGetLastError());
+  for (int c0 = 0; c0 < pl.depth; c0 += 16)
+    for (int tap = 0; tap < lay.taps; ++tap) {
+      if (tap % window == 0) {
+        KTile e{};  // a stage
+        e.a_row0 = (int)t.split_halves.size();
+        e.coff = (int)(c0 * cstride);
+        e.d0 = lay.offs[tap] - lay.offs[0];
+        e.d1 = tap;
+        e.dead = dead_rows(16, channels - c0);
+        t.ktiles.push_back(e);
+      }
+      t.split_halves.push_back(int2{c0, tap});
+    }
+  t.split_inner.assign(lay.offs, lay.offs + window);
+  t.split_tiles = lay.first[pl.bn == 256];
+  t.split_phases.push_back(lay.sp);
+  pl.split_half_count = (int)t.split_halves.size();
+  pl.split_odd = window % 2 != 0;
+  pl.split_npos = ph.npos;
+  pl.patch_rows = lay.patch[pl.bn == 256];
+  return MG_OK;
+}
+
+int build_fwd_plan(const Geometry &g, Plan &pl, bool may_split) {
   Tables t;
   // (one tap and few channels: one position per lane takes 34.7 - 40.3 us for (64,C,112,112) * (64,C,1,1), C = 2 -
   // 11, whole K tiles of 16 with dead rows 41.9 - 44.3)
@@ -1481,14 +1572,6 @@ int build_fwd_plan(const Geometry &g, Plan &pl) {
   if (pl.table_rows) pl.tap_major = true;
   const int bk = pl.table_rows ? 16 : pl.tap_major ? tap_bk(g.dtype, pl.depth) : gemm_bk(g.dtype);
   pl.bk = bk;
-  pl.single_dense_phase = true;
-  {
-    const long long ktiles = pl.table_rows ? ceil_div((long long)g.C * g.wvol, bk)
-                             : pl.tap_major ? g.wvol * (pl.depth / bk) : ceil_div((long long)g.C * g.wvol, bk);
-    const TileChoice tc = choose_tile(g.F, {(long long)g.N * g.gvol}, (int)ktiles, pl.tap_major, g.dtype == MG_F64 ? 8 : 4, 1, bk, pl.table_rows, is_tiny(g));
-    pl.bm = tc.bm, pl.bn = tc.bn, pl.m_tiles = tc.m_tiles, pl.full_tiles = tc.full_tiles, pl.tail_split = tc.tail_split, pl.blocks_per_cu = tc.blocks_per_cu;
-    deepen_if_tiny(g, pl);
-  }
   Phase ph{};
   for (int k = 0; k < 3; ++k) {
     ph.J[k] = g.G[k];
@@ -1498,6 +1581,19 @@ int build_fwd_plan(const Geometry &g, Plan &pl) {
   ph.blk_begin = 0;
   ph.npos = (int)((long long)g.N * g.gvol);
   set_divisors(ph);
+  pl.single_dense_phase = true;
+  SplitLayout lay;
+  for (int k = 0; k < 3; ++k) lay.sp.count[k] = g.W[k], lay.sp.d[k] = -g.P[k], lay.sp.step[k] = g.D[k];
+  pl.split = may_split && split_applies(g, pl, g.F, ph, g.X, lay);
+  {
+    const long long ktiles = pl.table_rows ? ceil_div((long long)g.C * g.wvol, bk)
+                             : pl.split     ? pl.depth / 16 * (g.wvol / lay.sp.window)
+                             : pl.tap_major ? g.wvol * (pl.depth / bk) : ceil_div((long long)g.C * g.wvol, bk);
+    const TileChoice tc = choose_tile(g.F, {(long long)g.N * g.gvol}, (int)ktiles, pl.tap_major, g.dtype == MG_F64 ? 8 : 4, pl.split ? 0 : 1, pl.split ? 16 * lay.sp.window : bk, pl.table_rows, is_tiny(g), -1, lay.patch);
+    pl.chain = mean_chain(tc, ktiles, tc.blocks_per_cu) * (pl.split ? 16 * lay.sp.window : bk);
+    pl.bm = tc.bm, pl.bn = tc.bn, pl.m_tiles = tc.m_tiles, pl.full_tiles = tc.full_tiles, pl.tail_split = tc.tail_split, pl.blocks_per_cu = tc.blocks_per_cu;
+    deepen_if_tiny(g, pl);
+  }
   if (pl.table_rows) {
     // the table in the filter's own row order (c, taps), padded to whole K tiles with rows that
     // lie outside every input (and meet rows of A beyond its end: zeros)
@@ -1512,6 +1608,13 @@ int build_fwd_plan(const Geometry &g, Plan &pl) {
     TabEntry outside{};
     outside.d0 = outside.d1 = outside.d2 = 1 << 29;
     while (t.tab.size() % bk != 0) t.tab.push_back(outside);
+    ph.k_count = (int)t.ktiles.size();
+    t.phases.push_back(ph);
+    pl.pos_blocks = (int)ceil_div(ph.npos, pl.bn);
+    return upload_plan(pl, t);
+  }
+  if (pl.split) {
+    if (int rc = split_tables(pl, t, lay, ph, g.X, g.C, g.xvol)) return rc;
     ph.k_count = (int)t.ktiles.size();
     t.phases.push_back(ph);
     pl.pos_blocks = (int)ceil_div(ph.npos, pl.bn);
@@ -1579,7 +1682,7 @@ bool deep_fused_on() {
   return on;
 }
 
-int build_dgrad_plan(const Geometry &g, Plan &pl) {
+int build_dgrad_plan(const Geometry &g, Plan &pl, bool may_split) {
   Tables t;
   // a tiny problem with a handful of channels is bound by its launches: the table-driven kernel
   // with its deep K tiles needs neither packed filters nor a pass over partial sums.  (Measured,
@@ -1679,6 +1782,32 @@ int build_dgrad_plan(const Geometry &g, Plan &pl) {
   // matrix pipes -- and the epilogue adds the three rows of a channel, shifted along the last
   // axis, into dx.  A wave's 64 positions must be whole rows: rows of up to 64 positions, padded
   // to a power of two.
+  // ---- unit strides: the kernel on operands in three bf16 parts, where it applies (phases with different numbers of taps would need stages of
+  // their own each)
+  if (may_split && nphase == 1 && found.size() == 1) {
+    const PhaseTaps &pt = found[0];
+    SplitLayout lay;
+    for (int k = 0; k < 3; ++k) {
+      lay.sp.count[k] = (int)pt.offs[k].size();
+      lay.sp.d[k] = pt.offs[k][0];
+      lay.sp.step[k] = lay.sp.count[k] > 1 ? pt.offs[k][1] - pt.offs[k][0] : 0;
+    }
+    pl.split = split_applies(g, pl, g.C, pt.ph, g.G, lay);
+    if (pl.split) {
+      const int stages = (int)(pl.depth / 16 * (g.wvol / lay.sp.window));
+      const TileChoice tc = choose_tile(g.C, {(long long)pt.ph.npos}, stages, true, 4, 0, 16 * lay.sp.window, false, false, -1, lay.patch);
+      pl.chain = mean_chain(tc, stages, tc.blocks_per_cu) * 16 * lay.sp.window;
+      pl.bm = tc.bm, pl.bn = tc.bn, pl.m_tiles = tc.m_tiles, pl.full_tiles = tc.full_tiles, pl.tail_split = tc.tail_split, pl.blocks_per_cu = tc.blocks_per_cu;
+      if (int rc = split_tables(pl, t, lay, pt.ph, g.G, g.F, g.gvol)) return rc;
+      Phase ph = pt.ph;
+      ph.k_begin = 0, ph.blk_begin = 0;
+      ph.k_count = (int)t.ktiles.size();
+      t.phases.push_back(ph);
+      pl.pos_blocks = (int)ceil_div(ph.npos, pl.bn);
+      return upload_plan(pl, t);
+    }
+  }
+
   if (fold_applies(g, g.C, pl.depth) && pl.tap_major && !pl.table_rows && nphase == 1 && found.size() == 1) {
     const PhaseTaps &pt = found[0];
     Phase ph = pt.ph;
@@ -1877,6 +2006,7 @@ int build_dgrad_plan(const Geometry &g, Plan &pl) {
     }
     const TileChoice tc = choose_tile(g.C, npos, (int)std::max<long long>(min_ktiles, 0), pl.tap_major, g.dtype == MG_F64 ? 8 : 4, 1, bk, pl.table_rows,
                                       is_tiny(g), (int)(all_ktiles / std::max<long long>(all_pos, 1)));
+    pl.chain = mean_chain(tc, std::max<long long>(min_ktiles, 0), tc.blocks_per_cu) * bk;
     pl.bm = tc.bm, pl.bn = tc.bn, pl.m_tiles = tc.m_tiles, pl.full_tiles = tc.full_tiles, pl.tail_split = tc.tail_split, pl.blocks_per_cu = tc.blocks_per_cu;
     deepen_if_tiny(g, pl);
   }
@@ -2239,6 +2369,12 @@ int build_wgrad_plan(const Geometry &g, Plan &pl) {
   return build_pos_table(g, pl);
 }
 
+void free_tables(Plan &pl) {
+  if (pl.blob) (void)hipFree(pl.blob);
+  if (pl.pos_tab) (void)hipFree(pl.pos_tab);
+  pl.blob = pl.pos_tab = nullptr;
+}
+
 int get_plan(ConvOp op, const mg_conv_desc *d, const Geometry &g, Plan **out) {
   std::string key(reinterpret_cast<const char *>(d), sizeof *d);
   key.push_back((char)op);
@@ -2246,6 +2382,8 @@ int get_plan(ConvOp op, const mg_conv_desc *d, const Geometry &g, Plan **out) {
   key.push_back(thin_on() ? 'n' : 'N');
   key.push_back(phase_rows_enabled() ? 'p' : 'P');
   key.push_back(pos_table_enabled() ? 'q' : 'Q');
+  key.push_back(split_on() ? 's' : 'S');
+  if (const char *least = getenv("MYGRAD_HIP_SPLIT_MIN")) key.append("m").append(least);
   if (const char *tile = getenv("MYGRAD_HIP_TILE")) key.append(tile);
   if (const char *tile = getenv("MYGRAD_HIP_WGRAD_TILE")) key.append("w").append(tile);
   if (const char *row = getenv("MYGRAD_HIP_FUSE_MIN_ROW")) key.append("r").append(row);
@@ -2258,7 +2396,32 @@ int get_plan(ConvOp op, const mg_conv_desc *d, const Geometry &g, Plan **out) {
       release_conv_plans();
     }
     Plan pl;
-    int rc = op == OP_FWD ? build_fwd_plan(g, pl) : op == OP_DGRAD ? build_dgrad_plan(g, pl) : build_wgrad_plan(g, pl);
+    auto build = [&](Plan &into, bool may_split) {
+      return op == OP_FWD ? build_fwd_plan(g, into, may_split) : op == OP_DGRAD ? build_dgrad_plan(g, into, may_split) : build_wgrad_plan(g, into);
+    };
+    int rc = build(pl, true);
+    if (pl.split) {
+      // the single-precision plan stands behind one on split operands, and alone where there is no memory for the latter's tables
+      Plan exact;
+      if (const int failed = build(exact, false)) {
+        free_tables(pl);
+        return failed;
+      }
+      // Six roundings into an accumulator for 32 terms here, eight there: no less accurate as long as there is no more than
+      // a third more to sum up without a break (the single-precision plan cuts K into more slices where it has few tiles: (2,57,16936) *
+      // (125,57,15), dx, error against 64 bits 6.8e-7 here, 3.8e-7 there).
+      const bool as_accurate = pl.chain <= 1.25 * exact.chain || getenv("MYGRAD_HIP_SPLIT_MIN") != nullptr;
+      // Nor on tiles of many more rows, where the patches of 256 positions do not fit: (98,110,69,63) * (15,110,3,3) 181 us on
+      // tiles of 16 x 256, 436 here on 96 x 128.
+      const bool as_full = 4ll * pl.m_tiles * pl.bm <= 5ll * exact.m_tiles * exact.bm || getenv("MYGRAD_HIP_SPLIT_MIN") != nullptr;
+      if (rc == MG_OK && as_accurate && as_full) {
+        pl.exact = std::make_shared<Plan>(exact);
+      } else {
+        (void)hipGetLastError();
+        free_tables(pl);
+        pl = exact, rc = MG_OK;
+      }
+    }
     if (rc) return rc;
     char tail[64];
     if (pl.share_grid > 0)
@@ -2267,11 +2430,11 @@ int get_plan(ConvOp op, const mg_conv_desc *d, const Geometry &g, Plan **out) {
       snprintf(tail, sizeof tail, "tail split %d", pl.tail_split);
     snprintf(pl.note, sizeof pl.note,
              "%s: %s%s%s tile %dx%dx%d, %d phase(s) (%d fused per tile), %d position blocks x %d row tiles, %d whole tiles + %s, "
-             "%d block(s) per unit, K splits %d",
+             "%d block(s) per unit, K splits %d%s",
              op == OP_FWD ? "fwd" : op == OP_DGRAD ? "dgrad" : "wgrad",
              pl.thin ? "one position per lane" : pl.tap_major ? "tap-major" : "table-driven", pl.table_rows ? ", table rows" : pl.phase_rows ? ", stride phases as rows" : "",
-             pl.fold_row ? ", folded taps" : "", pl.bm, pl.bn, pl.bk, pl.nphases, pl.nph, pl.pos_blocks, pl.m_tiles, pl.full_tiles, tail,
-             pl.blocks_per_cu, pl.splits);
+             pl.fold_row ? ", folded taps" : "", pl.bm, pl.bn, pl.split ? 32 : pl.bk, pl.nphases, pl.nph, pl.pos_blocks, pl.m_tiles, pl.full_tiles, tail,
+             pl.blocks_per_cu, pl.splits, pl.split ? ", three bf16 parts" : "");
     // MYGRAD_HIP_TRACE=1 reports, once per new descriptor, what was planned
     static const bool trace = getenv("MYGRAD_HIP_TRACE") != nullptr;
     if (trace) fprintf(stderr, "[mygrad_hip] plan %s (K chunk %d)\n", pl.note, pl.kchunk);
@@ -2323,6 +2486,32 @@ bool launch_gemm(GemmParams &gp, const Plan &pl, hipStream_t s) {
   return false;
 }
 
+// A plan on split operands: the grid and the fix-up pass are those of the streaming tap-major kernel.
+bool launch_split(GemmParams &gp, const Plan &pl, hipStream_t s) {
+  const long long tail_tiles = (long long)pl.pos_blocks * pl.m_tiles - pl.full_tiles;
+  const long long slots = (long long)pl.blocks_per_cu * runtime().props.multiProcessorCount;
+  gp.share_first = pl.share_first, gp.share_slices = pl.share_slices, gp.share_fix = pl.share_fix;
+  long long grid = pl.share_grid, fixes = pl.share_fixes;
+  if (pl.share_grid > 0) {
+    gp.items = pl.full_tiles;
+  } else {
+    gp.items = (int)(pl.full_tiles + tail_tiles * pl.tail_split);
+    grid = std::min<long long>(gp.items, slots);
+    fixes = tail_tiles;
+    const int c = pl.m_tiles;
+    gp.xcd_chunk = grid == slots && (c == 2 || c == 4 || c == 8) && grid % (8 * c) == 0 ? c : 1;
+  }
+  if (!launch_split_gemm(gp, pl.bm, pl.bn, pl.split_odd, (unsigned)grid, s)) return false;
+  if (fixes > 0) {
+#define MG_FIXUP(TT, BM, BN, WM, WN)                                                                                                     \
+  if (pl.bm == BM && pl.bn == BN)                                                                                                        \
+    hipLaunchKernelGGL((tail_fixup_kernel<TT, BM, BN, 1>), dim3((unsigned)ceil_div(BM * BN, 256), (unsigned)fixes), dim3(256), 0, s, gp);
+    MG_GEMM_SHAPES(float, MG_FIXUP)
+#undef MG_FIXUP
+  }
+  return true;
+}
+
 // Bytes of partial sums the shared tail tiles of this plan need.
 size_t tail_bytes(const Plan &pl, size_t elem) {
   const long long tail_tiles = (long long)pl.pos_blocks * pl.m_tiles - pl.full_tiles;
@@ -2369,6 +2558,7 @@ int run_gemm(GemmParams &gp, const Plan &pl, int tag, hipStream_t s) {
   }
   ScopedTiming timed(tag);
   bool launched = false;
+  if (pl.split) launched = launch_split(gp, pl, s);
   if (pl.deep_k) {
     launched = launch_gemm<T, 16, 64, 4 * BK, 16, 16>(gp, pl, s);
   }
@@ -2436,7 +2626,7 @@ int run_gemm(GemmParams &gp, const Plan &pl, int tag, hipStream_t s) {
       MG_FUSED4_SHAPES(T, MG_LAUNCH4)
     }
   }
-  if (pl.nph == 1) {
+  if (pl.nph == 1 && !pl.split) {
     MG_GEMM_SHAPES(T, MG_LAUNCH)
   }
 #undef MG_LAUNCH
@@ -2460,7 +2650,7 @@ int folded_ld(int n) {
 }
 
 template <typename T>
-int pack_filters(const Geometry &g, const void *w, int mode, int depth, void **packed, size_t extra = 0, void **behind = nullptr) {
+int pack_filters(const Geometry &g, const void *w, int mode, int depth, void **packed, size_t extra = 0, void **behind = nullptr, SplitFlags *gate = nullptr) {
   const int M = (mode == 2 || mode == 6) ? g.F : mode == 3 ? g.C : mode == 4 ? 3 * g.C : 3 * g.F;
   const int ld = mode == 4 || mode == 5 ? folded_ld<T>(M / 3) : packed_ld(M, true);
   const size_t count = (size_t)(mode == 4 || mode == 5 ? g.wvol / 3 : g.wvol) * depth * ld;
@@ -2483,10 +2673,35 @@ int pack_filters(const Geometry &g, const void *w, int mode, int depth, void **p
     MG_HIP(hipGetLastError());
     return MG_OK;
   }
-  const unsigned blocks = (unsigned)std::min<long long>(ceil_div((long long)count, 256), 4096);
+  // (behind a gate most passes have nothing to do: few blocks)
+  const unsigned blocks = (unsigned)std::min<long long>(ceil_div((long long)count, 256), gate ? 256 : 4096);
   ScopedTiming timed(TAG_PACK_FILTERS);
   hipLaunchKernelGGL(pack_filters_kernel<T>, dim3(blocks), dim3(256), 0, runtime().stream, static_cast<const T *>(w),
-                     static_cast<T *>(*packed), g.F, g.C, (int)g.wvol, mode, ld, depth);
+                     static_cast<T *>(*packed), g.F, g.C, (int)g.wvol, mode, ld, depth, gate);
+  MG_HIP(hipGetLastError());
+  return MG_OK;
+}
+
+// The filters of a plan on split operands (M rows of the product, `channels` channels contracted; row m's value under tap t of
+// channel c is w[m * m_stride + c * c_stride + t]) in the workspace; what the partial sums need follows.
+int pack_split(GemmParams &gp, const Plan &pl, const void *w, int M, int channels, long long m_stride, long long c_stride, void **partial) {
+  gp.a_ld = (int)ceil_div(M, 16) * 16;
+  gp.split_phases = pl.split_phases;
+  gp.split_inner = pl.split_inner;
+  gp.split_tiles = pl.split_tiles;
+  gp.patch_rows = pl.patch_rows;
+  gp.split_flags = static_cast<SplitFlags *>(pl.pos_tab);
+  gp.positions = gp.split_flags + 1;
+  gp.npos = pl.split_npos;
+  const size_t packed_bytes = (size_t)pl.split_half_count * 16 * gp.a_ld * 6;
+  void *scratch = nullptr;
+  if (int rc = workspace(packed_bytes + tail_bytes(pl, 4), &scratch)) return rc;
+  gp.A = scratch;
+  gp.a_bytes = (unsigned)packed_bytes;
+  *partial = static_cast<char *>(scratch) + packed_bytes;
+  ScopedTiming timed(TAG_PACK_FILTERS);
+  launch_split_pack(static_cast<const float *>(w), scratch, pl.split_halves, pl.split_half_count, gp.split_flags, M, channels, m_stride, c_stride, gp.a_ld,
+                    runtime().stream);
   MG_HIP(hipGetLastError());
   return MG_OK;
 }
@@ -2536,7 +2751,7 @@ int run_thin(const Plan &pl, ThinParams &tp, const void *w, int tag) {
 }
 
 template <typename T>
-int conv_fwd_impl(const Geometry &g, const Plan &pl, const void *x, const void *w, void *out) {
+int conv_fwd_impl(const Geometry &g, const Plan &pl, const void *x, const void *w, void *out, SplitFlags *gate = nullptr) {
   if (pl.thin) {
     ThinParams tp{};
     tp.src = static_cast<const float *>(x);
@@ -2559,14 +2774,17 @@ int conv_fwd_impl(const Geometry &g, const Plan &pl, const void *x, const void *
   }
   void *packed = nullptr;
   void *partial = nullptr;
-  if (!pl.tap_major) {
+  GemmParams gp{};
+  if (pl.split) {
+    if (int rc = pack_split(gp, pl, w, g.F, g.C, g.C * g.wvol, g.wvol, &partial)) return rc;
+  } else if (!pl.tap_major) {
     packed = const_cast<void *>(w);  // read in place: row k = (c, taps) of filter m lies at w[m * C*taps + k]
-  } else if (int rc = pack_filters<T>(g, w, pl.table_rows ? 6 : pl.fold_row ? 5 : 2, pl.table_rows ? g.C : pl.depth, &packed, tail_bytes(pl, sizeof(T)), &partial)) {
+  } else if (int rc = pack_filters<T>(g, w, pl.table_rows ? 6 : pl.fold_row ? 5 : 2, pl.table_rows ? g.C : pl.depth, &packed, tail_bytes(pl, sizeof(T)), &partial, gate)) {
     return rc;
   }
-  GemmParams gp{};
   gp.partial = partial;
-  gp.A = packed;
+  if (!pl.split) gp.A = packed;
+  if (gate) gp.gate = &gate->rerun;
   gp.a_mstride = (int)(g.C * g.wvol);
   gp.src = x;
   gp.dst = out;
@@ -2584,6 +2802,14 @@ int conv_fwd_impl(const Geometry &g, const Plan &pl, const void *x, const void *
   gp.src_cstride = (int)g.xvol;
   gp.src_nstride = (long long)g.C * g.xvol;
   gp.dst_nstride = (long long)g.F * g.gvol;
+  if (pl.split) {
+    gp.src_bytes = (unsigned)((size_t)g.N * g.C * g.xvol * sizeof(T));
+    gp.samples = g.N;
+    gp.sample_rows = (int)up4(g.xvol);
+    gp.by_sample = make_fastdiv((unsigned)gp.sample_rows);
+    if (int rc = run_gemm<T>(gp, pl, TAG_CONV_FWD, runtime().stream)) return rc;
+    return conv_fwd_impl<T>(g, *pl.exact, x, w, out, gp.split_flags);
+  }
   gp.a_ld = pl.fold_row ? folded_ld<T>(g.F) : packed_ld(g.F, pl.tap_major);
   gp.a_bytes = (unsigned)((size_t)(pl.tap_major && !pl.table_rows ? pl.depth : g.C) * (pl.fold_row ? g.wvol / 3 : g.wvol) * gp.a_ld * sizeof(T));
   gp.src_bytes = pl.tap_major ? (unsigned)((size_t)g.N * g.C * g.xvol * sizeof(T)) : 0;
@@ -2591,7 +2817,7 @@ int conv_fwd_impl(const Geometry &g, const Plan &pl, const void *x, const void *
 }
 
 template <typename T>
-int conv_dgrad_impl(const Geometry &g, const Plan &pl, const void *grad, const void *w, void *dx) {
+int conv_dgrad_impl(const Geometry &g, const Plan &pl, const void *grad, const void *w, void *dx, SplitFlags *gate = nullptr) {
   if (pl.thin) {
     ThinParams tp{};
     tp.src = static_cast<const float *>(grad);
@@ -2614,7 +2840,10 @@ int conv_dgrad_impl(const Geometry &g, const Plan &pl, const void *grad, const v
   }
   void *packed = nullptr;
   void *partial = nullptr;
-  if (!pl.tap_major) {
+  GemmParams gp{};
+  if (pl.split) {
+    if (int rc = pack_split(gp, pl, w, g.C, g.F, g.wvol, g.C * g.wvol, &partial)) return rc;
+  } else if (!pl.tap_major) {
     packed = const_cast<void *>(w);  // read in place: row k = (f, tap) of channel m lies at w[(f * C + m) * taps + tap]
   } else if (pl.table_rows) {
     const int ld = packed_ld(g.C, true);
@@ -2638,12 +2867,12 @@ int conv_dgrad_impl(const Geometry &g, const Plan &pl, const void *grad, const v
     hipLaunchKernelGGL(pack_phase_rows_kernel<T>, dim3(blocks), dim3(256), 0, runtime().stream, static_cast<const T *>(w),
                        static_cast<T *>(packed), pl.arow, pl.table_count, pl.phase_count, (int)g.F, pl.depth, (int)g.C, (int)g.wvol, ld);
     MG_HIP(hipGetLastError());
-  } else if (int rc = pack_filters<T>(g, w, pl.fold_row ? 4 : 3, pl.depth, &packed, tail_bytes(pl, sizeof(T)), &partial)) {
+  } else if (int rc = pack_filters<T>(g, w, pl.fold_row ? 4 : 3, pl.depth, &packed, tail_bytes(pl, sizeof(T)), &partial, gate)) {
     return rc;
   }
-  GemmParams gp{};
   gp.partial = partial;
-  gp.A = packed;
+  if (!pl.split) gp.A = packed;
+  if (gate) gp.gate = &gate->rerun;
   gp.a_mstride = (int)g.wvol;
   gp.src = grad;
   gp.dst = dx;
@@ -2661,6 +2890,14 @@ int conv_dgrad_impl(const Geometry &g, const Plan &pl, const void *grad, const v
   gp.src_cstride = (int)g.gvol;
   gp.src_nstride = (long long)g.F * g.gvol;
   gp.dst_nstride = (long long)g.C * g.xvol;
+  if (pl.split) {
+    gp.src_bytes = (unsigned)((size_t)g.N * g.F * g.gvol * sizeof(T));
+    gp.samples = g.N;
+    gp.sample_rows = (int)up4(g.gvol);
+    gp.by_sample = make_fastdiv((unsigned)gp.sample_rows);
+    if (int rc = run_gemm<T>(gp, pl, TAG_CONV_DGRAD, runtime().stream)) return rc;
+    return conv_dgrad_impl<T>(g, *pl.exact, grad, w, dx, gp.split_flags);
+  }
   gp.a_ld = pl.fold_row ? folded_ld<T>(g.C) : packed_ld(g.C, pl.tap_major);
   gp.a_bytes = pl.table_rows ? (unsigned)((size_t)pl.table_count * gp.a_ld * sizeof(T))
                              : (unsigned)((size_t)(pl.tap_major ? pl.depth : g.F) * (pl.fold_row ? g.wvol / 3 : g.wvol) * gp.a_ld * sizeof(T));
@@ -2807,8 +3044,8 @@ int conv_wgrad_impl(const Geometry &g, const Plan &pl, const void *grad, const v
 void release_conv_plans() {
   note_plan("");  // it may point into a plan
   for (auto &kv : plans()) {
-    if (kv.second.blob) (void)hipFree(kv.second.blob);
-    if (kv.second.pos_tab) (void)hipFree(kv.second.pos_tab);
+    if (kv.second.exact) free_tables(*kv.second.exact);
+    free_tables(kv.second);
   }
   plans().clear();
 }

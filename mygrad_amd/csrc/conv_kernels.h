@@ -91,6 +91,22 @@ struct ShareFix {
   int tile, first_slot, slots, pad_;
 };
 
+// A phase of conv_split.hip.  Tap (a * count[1] + b) * count[2] + c reads at coordinate offsets d[0] + a * step[0],
+// d[1] + b * step[1], d[2] + c * step[2]; at most 31 of them.  A stage is 16 channels under `window` consecutive taps; tap t of the
+// window reads inner[t] rows (elements of a channel's plane) from the position's own, counted from the stage's row offset.
+struct SplitPhase {
+  int count[3], d[3], step[3];
+  int window, inner_begin;  // inner_begin: into GemmParams::split_inner
+  int pad_[5];
+};
+static_assert(sizeof(SplitPhase) == 64, "read as one 64-byte row");
+
+// What a pass of conv_split.hip finds out about its operands.
+struct SplitFlags {
+  int rerun;    // the single-precision kernels have to do the pass; cleared when a pass packs its filters
+  int filters;  // of the filters being packed; cleared by the gated pack_filters_kernel at the end of a pass
+};
+
 // Gather-GEMM:  dst[n, m, pos] = sum_k A(k, m) * src[n, row k, pos]
 // The tap-major kernels read A from packed filters, [rows][a_ld] with the M values of a row
 // contiguous; the table-driven kernel reads the filter bank where it lies:
@@ -163,7 +179,35 @@ struct GemmParams {
   int xcd_chunk;
   int phase_count;      // 0: off; else the number of stride phases (2 or 4)
   int phase_pairs;      // phases 2q, 2q + 1 are neighbours along the last axis of dst
+  // conv_split.hip: A is split into bf16 parts, a_ld a multiple of 16; ktiles holds stages, the names of KTile's fields aside:
+  // first half (tap of 16 channels) in A, channel offset, row offset, first tap, -, dead rows
+  const SplitPhase *split_phases;  // one per phase
+  const int *split_inner;
+  const int *split_tiles;  // per block of positions: the lowest row that any of its windows touches, a stage's row offset aside
+  int patch_rows;       // rows of LDS for a stage's elements
+  int samples;          // of src
+  int sample_rows;      // rows that a sample of src is numbered with: its elements per channel rounded up to a multiple of four
+  const void *positions;  // row of src and taps of every position, 8 bytes each
+  int npos;
+  FastDiv by_sample;    // row -> sample
+  SplitFlags *split_flags;
+  const int *gate;      // not null: the kernels return at once while *gate is zero
 };
+
+// The table of positions of conv_split.hip (GemmParams::positions): positions (n, j) of J, sources at j + the taps' offsets in Q.
+struct SplitPositions {
+  int npos, J[3], Q[3];
+  int sample_rows;
+  SplitPhase sp;
+};
+
+// conv_split.hip
+int split_patch_limit(int bm, int bn);
+int split_gemm_blocks_per_cu(int bm, int bn, int patch_rows);
+bool launch_split_gemm(const GemmParams &p, int bm, int bn, bool odd, unsigned grid, hipStream_t s);
+void launch_split_pack(const float *w, void *packed, const void *halves, int count, SplitFlags *flags, int M, int channels, long long m_stride,
+                       long long c_stride, int ld, hipStream_t s);
+void launch_split_positions(const SplitPositions &p, void *out, hipStream_t s);
 
 // Gather-GEMM with one position per lane, for few rows (the data gradient of a layer with a
 // handful of channels, the forward pass of one with a handful of filters or of a first layer):

@@ -1,0 +1,631 @@
+// Gather-GEMM in single precision on the bf16 matrix instructions, for the forward pass and the
+// data gradient of large problems.
+//
+// v_mfma_f32_16x16x4_f32 does 157 TFLOP/s at best on this device and shares its issue with the vector
+// ALU (44 vector instructions next to 16 of them: 154 -> 110 TFLOP/s); v_mfma_f32_16x16x32_bf16 does
+// 1800 - 2000 and does not.  A float is the sum of three bf16 numbers exactly (8 + 8 + 8 bits of its
+// significand), x = x0 + x1 + x2, and
+//   x * w = x0 w0 + (x0 w1 + x1 w0) + (x0 w2 + x1 w1 + x2 w0) + terms below 2^-25 |x w|,
+// six products, each exact in single precision and added up in single-precision accumulators: an
+// effective peak of 300 - 330 TFLOP/s.  The error against 64 bits is no larger than that of the single-precision
+// instruction, whose every step of four terms rounds into the accumulator where this one rounds six times per
+// 32 terms (K = 64 / 576 / 4096, normal values: 9.8e-8 / 3.7e-7 / 1.0e-6 here, 1.4e-7 / 4.6e-7 / 1.1e-6 there).  (The five small
+// products summed apart and added once per step halve it, 1.7e-7 at K = 576, but need registers that 64-row
+// wave tiles do not have: they spill, and 178 us become 224.)
+//
+// What bounds it: (128,64,56,56) * (64,64,3,3), 29.6 GFLOP, takes 178 us with its packing and gated passes, about 160 by itself: 185
+// TFLOP/s of the 300.  The rest is the turn between stages, where the waves of a block wait for the patch to be split and
+// parked, and the first stage of a tile; loads are hidden.
+//
+// What the split cannot represent is left to the single-precision kernels.  An infinite operand leaves Inf - Inf in
+// its second part and makes every sum that it takes part in a NaN, as an infinite or NaN operand or an overflow makes
+// it something not finite in any arithmetic.  The low parts of operands below 2^-102 may fall under the smallest
+// numbers that the instruction takes, 2^-126: against a sum of 2^-70 or more, K terms of at most 2^16 * 2^-126 are less
+// than its last bit for every K up to 2^16.  So a flag is set by a wave that holds a sum that is not finite, or not
+// zero and below 2^-70; where a filter value is above 2^16; and where one is below 2^-100 and an element of src above
+// 2^16.  The single-precision kernels are launched behind this one and return at once unless it is set: they then
+// do the whole pass, and its result is theirs.
+#include "conv_device.h"
+#include "conv_kernels.h"
+#include "internal.h"
+
+#include <algorithm>
+#include <array>
+#include <map>
+#include <type_traits>
+
+namespace mg {
+
+namespace {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+typedef int int8v __attribute__((ext_vector_type(8)));
+typedef int int16v __attribute__((ext_vector_type(16)));
+static_assert(sizeof(KTile) == sizeof(int8v) && sizeof(SplitPhase) == sizeof(int16v), "table rows");
+
+constexpr unsigned kOutside = 0x80000000u;  // a byte offset past the end of any tensor (each below 2 GiB): reads as zero
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void *base, unsigned bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)bytes, 0x00020000);
+}
+
+__device__ __forceinline__ unsigned bits_of(float v) { return __builtin_bit_cast(unsigned, v); }
+__device__ __forceinline__ float float_of(unsigned v) { return __builtin_bit_cast(float, v); }
+
+// a = h[0] + m[0] + l[0] and b likewise, exactly.  The first part is cut off, not rounded (rounding could
+// overflow); the rest, at most 16 bits, is rounded to nearest, so that what the six products leave
+// out has no sign of its own.  Eleven vector instructions for two values.
+__device__ __forceinline__ void split_pair(float a, float b, unsigned &h, unsigned &m, unsigned &l) {
+  h = __builtin_amdgcn_perm(bits_of(b), bits_of(a), 0x07060302u);
+  const float ra = a - float_of(bits_of(a) & 0xffff0000u), rb = b - float_of(bits_of(b) & 0xffff0000u);
+  m = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{ra, rb}), bf16x2));
+  const float qa = ra - float_of(m << 16), qb = rb - float_of(m & 0xffff0000u);
+  l = __builtin_amdgcn_perm(bits_of(qb), bits_of(qa), 0x07060302u);
+}
+
+__device__ __forceinline__ void split_eight(const float (&v)[8], bf16x8 (&parts)[3]) {
+  u32x4 h, m, l;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    unsigned a, b, c;
+    split_pair(v[2 * e], v[2 * e + 1], a, b, c);
+    h[e] = a, m[e] = b, l[e] = c;
+  }
+  parts[0] = __builtin_bit_cast(bf16x8, h);
+  parts[1] = __builtin_bit_cast(bf16x8, m);
+  parts[2] = __builtin_bit_cast(bf16x8, l);
+}
+
+// (see the head of the file) not finite, or not zero and below 2^-70
+__device__ __forceinline__ bool suspect(float v) {
+  constexpr unsigned low = 2u * (57u << 23), high = 2u * (255u << 23);  // 2^-70 and Inf, without their sign bit
+  const unsigned u = bits_of(v) << 1;
+  return u != 0 && u - low >= high - low;
+}
+constexpr float kWide = 0x1p16f, kTiny = 0x1p-100f;  // operands: see the head of the file
+enum : int { kTinyFilter = 1, kWideFilter = 2 };     // SplitFlags::filters
+
+__device__ __forceinline__ Phase load_phase(const Phase *phases, int i) {
+  const int8v MG_CONSTANT *q = (const int8v MG_CONSTANT *)(phases + uniform(i));
+  const int8v a = q[0], b = q[1], c = q[2];
+  Phase ph;
+  ph.J[0] = a[0], ph.J[1] = a[1], ph.J[2] = a[2];
+  ph.o0[0] = a[3], ph.o0[1] = a[4], ph.o0[2] = a[5];
+  ph.k_begin = a[6], ph.k_count = a[7];
+  ph.blk_begin = b[0], ph.npos = b[1];
+  ph.by_jvol = FastDiv{(unsigned)b[2], (unsigned)b[3], (unsigned)b[4], 0u};
+  ph.by_j12 = FastDiv{(unsigned)b[6], (unsigned)b[7], (unsigned)c[0], 0u};
+  ph.by_j2 = FastDiv{(unsigned)c[2], (unsigned)c[3], (unsigned)c[4], 0u};
+  return ph;
+}
+__device__ __forceinline__ int phase_first_block(const Phase *phases, int i) {
+  return ((const int MG_CONSTANT *)(phases + uniform(i)))[8];
+}
+
+// One tile is MW * WM rows (filters) by NW * 64 positions, a wave of the block for each WM x 64 of it.  The contraction
+// runs in stages: 16 channels under the taps of one inner window (all taps, or those of the last axes where the
+// others reach too far).  A stage's elements of src -- every row (position of src) that the tile's windows touch, 16
+// channels of each -- are loaded and split once, parked in LDS, and serve all taps of the window from there: operand
+// position n under tap t is row base(n) + offset(t), 16 bytes a lane.  (Split anew for every tap, as the waves
+// gather them for the single-precision instruction, the vector ALU and the vector cache are the bound: 64 channels, 3x3, 56x56
+// 180 us.)  A position without the tap (padding) reads a row of zeros.
+//
+// A K step is 32 deep: two taps, lanes 0 - 31 hold the first one's 16 channels, lanes 32 - 63 the second one's.  An
+// odd last tap (ODD) makes a step of three products instead of six: lanes 0 - 31 and 32 - 63 hold different parts of the one tap.
+//
+// The positions are the rows of D, so that a lane holds four consecutive positions of one filter and stores them as a vector.  The filters,
+// split and laid out in the order of the stages beforehand (split_pack_kernel), pass through LDS two steps ahead of their use.
+// Blocks are persistent, as in tap_gemm_kernel.
+template <int WM, int MW, int NW, bool ODD>
+__global__ void __launch_bounds__(64 * MW * NW, 2) split_gemm_kernel(const GemmParams p) {
+  constexpr int BM = WM * MW, BN = 64 * NW, TM = WM / 16, THREADS = 64 * MW * NW;
+  static_assert(WM % 16 == 0, "16 x 16 tiles");
+  constexpr int PIECES = 12 * BM;  // of 16 bytes: a step's filters, [part][octet of K rows][row]
+  constexpr int ALOADS = (PIECES + THREADS - 1) / THREADS;
+  // [2][PIECES] filters, then the patch: [octet of channels][row][part], p.patch_rows + 1 rows, the last one zeros
+  extern __shared__ __attribute__((aligned(16))) u32x4 lds[];
+  u32x4 *const patch = lds + 2 * PIECES;
+
+  const int lane = threadIdx.x & 63;
+  const int wave = uniform((threadIdx.x >> 6) % NW), wm0 = uniform((threadIdx.x >> 6) / NW) * WM;  // the wave's positions and rows
+  const int l16 = lane & 15, lk = lane >> 4;
+  const bool second = lk >= 2;  // this lane holds channels under the second tap of a step
+
+  struct Item {
+    int tile, pos0, m0, kt_begin, kt_end, slot;
+    bool partial;
+    Phase ph;
+  };
+  float widest = 0.0f;  // |element of src| among those this lane has split
+  const bool shares = p.share_first != nullptr;
+  const int share_begin = shares ? ((const int MG_CONSTANT *)p.share_first)[uniform((int)blockIdx.x)] : 0;
+  const int share_end = shares ? ((const int MG_CONSTANT *)p.share_first)[uniform((int)blockIdx.x) + 1] : 0;
+  const int item_end = shares ? p.full_tiles + share_end : p.items;
+  const int chunk = p.xcd_chunk;
+  const int place = chunk > 1 ? (((int)blockIdx.x >> 3) / chunk * 8 + ((int)blockIdx.x & 7)) * chunk + ((int)blockIdx.x >> 3) % chunk
+                              : (int)blockIdx.x;
+  const int item_first = (!shares || place < p.full_tiles) ? place : p.full_tiles + share_begin;
+  auto next_item = [&](int item) -> int {
+    if (!shares) return item + (int)gridDim.x;
+    if (item >= p.full_tiles) return item + 1;
+    return item + (int)gridDim.x < p.full_tiles ? item + (int)gridDim.x : p.full_tiles + share_begin;
+  };
+  auto locate = [&](int item, int &pi, Item &it) {  // pi: phase of the previous item of this cursor (tiles ascend)
+    it.tile = item;
+    it.slot = 0;
+    it.partial = item >= p.full_tiles;
+    int4v row = {0, 0, 0, 0};
+    int piece = 0;
+    if (it.partial) {
+      if (shares) {
+        row = ((const int4v MG_CONSTANT *)p.share_slices)[uniform(item - p.full_tiles)];
+        it.tile = row[0];
+        it.slot = row[3];
+        it.partial = row[3] >= 0;
+      } else {
+        const int j = item - p.full_tiles;
+        it.tile = p.full_tiles + j / p.tail_split;
+        piece = j % p.tail_split;
+        it.slot = j;
+      }
+    }
+    const int pblk = it.tile / p.m_tiles;
+    while (pi + 1 < p.nphases && pblk >= phase_first_block(p.phases, pi + 1)) ++pi;
+    it.ph = load_phase(p.phases, pi);
+    it.pos0 = (pblk - it.ph.blk_begin) * BN;
+    it.m0 = (it.tile % p.m_tiles) * BM;
+    it.kt_begin = 0;
+    it.kt_end = it.ph.k_count;
+    if (shares && item >= p.full_tiles) {
+      it.kt_begin = row[1];
+      it.kt_end = row[2];
+    } else if (it.partial) {
+      const int per = (it.ph.k_count + p.tail_split - 1) / p.tail_split;
+      it.kt_begin = min(piece * per, it.ph.k_count);
+      it.kt_end = min(it.kt_begin + per, it.ph.k_count);
+    }
+  };
+
+  const __amdgpu_buffer_rsrc_t a_buf = buffer_of(p.A, p.a_bytes);
+  const __amdgpu_buffer_rsrc_t src_buf = buffer_of(p.src, p.src_bytes);
+  const __amdgpu_buffer_rsrc_t table_buf = buffer_of(p.positions, (unsigned)p.npos * 8u);  // (row, taps) of every position
+  const unsigned piece_row = (unsigned)p.a_ld * 16u;  // bytes of one part of one octet of packed filters
+  const unsigned c_step = (unsigned)p.src_cstride * 4u;
+  const int octet_rows = p.patch_rows + 1;
+  if (threadIdx.x < 6) patch[((int)threadIdx.x / 3 * octet_rows + p.patch_rows) * 3 + (int)threadIdx.x % 3] = u32x4{0, 0, 0, 0};
+  float *__restrict__ dst = static_cast<float *>(p.dst);
+  int pi = 0;
+  Item me;
+  u32x4 raw[8];        // elements on their way to the patch: [channel][row of four]
+  bool ahead = false;  // those of the item's first stage were requested by the item before it
+  // the patch being requested: its first row, its stage's row of the table, whether there is one
+  int patch_row = 0;
+  int8v patch_e = {0, 0, 0, 0, 0, 0, 0, 0};  // first half, channel offset, row offset, first tap, -, dead rows
+  bool patch_real = false;
+  auto first_of = [&](const Item &it) -> int { return ((const int MG_CONSTANT *)p.split_tiles)[uniform(it.pos0 / BN)]; };
+  // A quarter of the patch's loads.  A thread takes four rows, which begin on a multiple of four and therefore lie in one sample
+  // (a sample's rows are numbered up to a multiple of four; what is loaded for those beyond its last is of no use to anyone), and
+  // loads them as one vector, whatever its alignment: 16 bytes a lane take the vector cache 16 cycles, 4 bytes 8 - 11.
+  auto request_part = [&](int k) {
+    const int quads = p.patch_rows / 4, octet = (int)threadIdx.x >= quads ? 1 : 0;
+    const int row = ((patch_row + patch_e[2]) & ~3) + ((int)threadIdx.x - octet * quads) * 4;
+    const unsigned n = __umulhi((unsigned)max(row, 0), p.by_sample.mul) >> p.by_sample.shr;  // (more than one row to a sample)
+    unsigned at = (n * (unsigned)p.src_nstride + (unsigned)(row - (int)n * p.sample_rows + patch_e[1] + octet * 8 * p.src_cstride)) * 4u;
+    at = ((int)threadIdx.x < 2 * quads) & (row >= 0) & ((int)n < p.samples) & patch_real ? at : kOutside;
+    const unsigned dead = (unsigned)patch_e[5] >> (octet * 8);
+#pragma unroll
+    for (int r = 2 * k; r < 2 * k + 2; ++r)
+      raw[r] = __builtin_amdgcn_raw_buffer_load_b128(src_buf, (int)(at | ((dead << (31 - r)) & kOutside)), (int)((unsigned)r * c_step), 0);
+  };
+  auto park_patch = [&] {
+    const int quads = p.patch_rows / 4, octet = (int)threadIdx.x >= quads ? 1 : 0;
+    u32x4 *const out = patch + (octet * octet_rows + ((int)threadIdx.x - octet * quads) * 4) * 3;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      float v[8];
+#pragma unroll
+      for (int r = 0; r < 8; ++r) v[r] = float_of(raw[r][u]);
+#pragma unroll
+      for (int r = 0; r < 8; r += 2) widest = __builtin_fmaxf(__builtin_fmaxf(widest, __builtin_fabsf(v[r])), __builtin_fabsf(v[r + 1]));
+      bf16x8 parts[3];
+      split_eight(v, parts);
+      if ((int)threadIdx.x < 2 * quads) {
+#pragma unroll
+        for (int part = 0; part < 3; ++part) out[u * 3 + part] = __builtin_bit_cast(u32x4, parts[part]);
+      }
+    }
+  };
+  for (int item = item_first; item < item_end; item = next_item(item)) {
+    locate(item, pi, me);
+    f32x4 acc[4][TM];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int i = 0; i < TM; ++i) acc[j][i] = f32x4{0, 0, 0, 0};
+    const int stages = me.kt_end - me.kt_begin;
+    const int16v sp = ((const int16v MG_CONSTANT *)p.split_phases)[uniform(pi)];  // see SplitPhase
+    const int window = sp[9];  // taps of the inner window
+    const int inner = p.split_inner[sp[10] + min(lane, window - 1)];  // lane t: row offset of the window's tap t
+
+    // ---- this lane's positions: their row in the patch and the taps they have (bit by bit; none beyond the last position)
+    const int first_row = first_of(me);
+    int row_at[4];
+    unsigned taps[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      typedef int int2v __attribute__((ext_vector_type(2)));
+      const int ipos = me.pos0 + wave * 64 + j * 16 + l16;
+      const int2v at = __builtin_bit_cast(int2v, __builtin_amdgcn_raw_buffer_load_b64(table_buf, (int)((unsigned)ipos * 8u), 0, 0));
+      row_at[j] = at[0] - first_row;
+      taps[j] = (unsigned)at[1];
+    }
+    unsigned a_at[ALOADS];
+#pragma unroll
+    for (int u = 0; u < ALOADS; ++u) {
+      const int q = (int)threadIdx.x + THREADS * u;
+      const int m = me.m0 + q % BM, oct = q / BM % 4, part = q / (4 * BM);
+      a_at[u] = q < PIECES && m < p.a_ld ? (unsigned)(oct * 3 + part) * piece_row + (unsigned)m * 16u : kOutside;
+    }
+
+    // ---- filters: `half` counts taps of 16 channels in the order of the stages
+    u32x4 areg[ALOADS];
+    auto request_filters = [&](int half) {
+      const unsigned at = (unsigned)half * 6u * piece_row;
+#pragma unroll
+      for (int u = 0; u < ALOADS; ++u) areg[u] = __builtin_amdgcn_raw_buffer_load_b128(a_buf, (int)(a_at[u] + at), 0, 0);
+    };
+    auto park_filters = [&](int buf) {
+#pragma unroll
+      for (int u = 0; u < ALOADS; ++u) {
+        const int q = (int)threadIdx.x + THREADS * u;
+        if (PIECES % THREADS == 0 || q < PIECES) lds[buf * PIECES + q] = areg[u];
+      }
+    };
+    bf16x8 w[TM][3];
+    auto read_filters = [&](int buf, int i, bool single) {
+      // (a single tap: parts 0 | 2 and 1 | 0 of its two octets)
+      const u32x4 *mine = lds + buf * PIECES + (single ? lk & 1 : lk) * BM + wm0 + l16 + i * 16;
+      if (single) {
+        w[i][0] = __builtin_bit_cast(bf16x8, mine[(second ? 2 : 0) * 4 * BM]);
+        w[i][1] = __builtin_bit_cast(bf16x8, mine[(second ? 0 : 1) * 4 * BM]);
+      } else {
+#pragma unroll
+        for (int part = 0; part < 3; ++part) w[i][part] = __builtin_bit_cast(bf16x8, mine[part * 4 * BM]);
+      }
+    };
+
+    // ---- the patch
+    const int8v MG_CONSTANT *table = (const int8v MG_CONSTANT *)p.ktiles + (me.ph.k_begin + me.kt_begin);
+    // what the steps of stage `stage` request: the next stage's patch, or the first one of the block's next item
+    auto aim = [&](int stage) {
+      patch_row = first_row;
+      patch_real = stage + 1 < stages;
+      if (patch_real) {
+        patch_e = table[stage + 1];
+      } else {
+        const int then = next_item(item);
+        if (then < item_end) {
+          Item nx;
+          int npi = pi;
+          locate(then, npi, nx);
+          if (nx.kt_begin < nx.kt_end) {
+            patch_row = first_of(nx);
+            patch_e = ((const int8v MG_CONSTANT *)p.ktiles)[uniform(nx.ph.k_begin + nx.kt_begin)];
+            patch_real = true;
+          }
+        }
+      }
+    };
+    int x_at[4], x_next[4];  // of the step under way and the one after it: 16-byte pieces from the start of the patch
+    // tap0: number of the window's first tap; q: first tap of the step within it; lead: rows of the patch ahead of the tile's first one
+    auto place = [&](int tap0, int q, bool single, int lead) {
+      const int off0 = __builtin_amdgcn_readlane(inner, q), off1 = __builtin_amdgcn_readlane(inner, single ? q : q + 1);
+      const int off = (second ? off1 : off0) + lead;
+      const unsigned tap = (unsigned)(tap0 + q + (!single && second ? 1 : 0));
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int keep = __builtin_amdgcn_sbfe((int)taps[j], tap, 1u);  // all ones where the position has the tap
+        x_next[j] = (((row_at[j] + off - p.patch_rows) & keep) + p.patch_rows + (lk & 1) * octet_rows) * 3;
+      }
+    };
+    auto enter_step = [&] {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x_at[j] = x_next[j];
+    };
+    auto read_position = [&](int j, bool single, bf16x8(&x)[3]) {
+      const u32x4 *mine = patch + x_at[j];
+      if (single) {  // parts 2 | 0, 1 | 1, 0 | 0
+        x[0] = __builtin_bit_cast(bf16x8, mine[second ? 0 : 2]);
+        x[1] = __builtin_bit_cast(bf16x8, mine[1]);
+        x[2] = __builtin_bit_cast(bf16x8, mine[0]);
+      } else {
+#pragma unroll
+        for (int part = 0; part < 3; ++part) x[part] = __builtin_bit_cast(bf16x8, mine[part]);
+      }
+    };
+
+    // One K step (`step_no` of the item) whose operands' first position is in x[0] and whose filters are in w; the next step
+    // starts at tap `q_next` of its window, `single_next`: it is a window's odd last tap.  `turn`: the stage ends here.
+    bf16x8 x[2][3];
+    int step_no = 0;
+    auto step = [&](auto single_c, auto turn_c, auto single_next_c, int half_after, int tap0_next, int q_next, int lead_next, int stage, int parts) {
+      constexpr bool SINGLE = decltype(single_c)::value, TURN = decltype(turn_c)::value, NEXT = decltype(single_next_c)::value;
+      constexpr int PRODUCTS = SINGLE ? 3 : 6;
+      constexpr int PX[6] = {SINGLE ? 0 : 2, SINGLE ? 1 : 0, SINGLE ? 2 : 1, 1, 0, 0}, PW[6] = {0, SINGLE ? 1 : 2, 1, 0, 1, 0};  // smallest first
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (j < 3) {
+          read_position(j + 1, SINGLE, x[(j + 1) % 2]);
+          if (j == 2) place(tap0_next, q_next, NEXT, lead_next);
+        } else {
+          park_filters((step_no + 1) & 1);
+          __syncthreads();  // the next step's filters are there; nobody reads this one's patch any more
+          // the patch's loads are spread over the steps (all at once they fill the vector cache's queue, and every wave waits for
+          // memory there: 8000 cycles), ahead of the filters' so that parking those waits for nothing younger
+          if constexpr (!SINGLE) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+              if ((parts >> k) & 1) request_part(k);
+          }
+          request_filters(half_after);
+          if constexpr (TURN) {
+            if (stage + 1 < stages) park_patch();
+          } else {
+            enter_step();
+            read_position(0, NEXT, x[0]);
+          }
+        }
+#pragma unroll
+        for (int i0 = 0; i0 < TM; i0 += 2) {
+#pragma unroll
+          for (int t = 0; t < PRODUCTS; ++t)
+#pragma unroll
+            for (int i = i0; i < TM && i < i0 + 2; ++i)
+              acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[j % 2][PX[t]], w[i][PW[t]], acc[j][i], 0, 0, 0);
+          if (j == 3) {
+#pragma unroll
+            for (int i = i0; i < TM && i < i0 + 2; ++i) read_filters((step_no + 1) & 1, i, NEXT);
+          }
+        }
+        if (j < 3) __builtin_amdgcn_sched_barrier(0);
+      }
+      if constexpr (TURN) {
+        __syncthreads();
+        enter_step();
+        read_position(0, NEXT, x[0]);
+        if (stage + 1 < stages) aim(stage + 1);
+      }
+      ++step_no;
+    };
+    if (stages > 0) {
+      const std::true_type yes;
+      const std::false_type no;
+      const int half0 = table[0][0];
+      __syncthreads();  // (the last item's operands have been read)
+      request_filters(half0);
+      if (!ahead) {
+        patch_row = first_row, patch_e = table[0], patch_real = true;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) request_part(k);
+      }
+      park_patch();
+      park_filters(0);
+      request_filters(half0 + 2);
+      aim(0);
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < TM; ++i) read_filters(0, i, false);
+      place(table[0][3], 0, false, (first_row + table[0][2]) & 3);
+      enter_step();
+      read_position(0, false, x[0]);
+      for (int stage = 0; stage < stages; ++stage) {
+        const int8v here = table[stage], there = table[min(stage + 1, stages - 1)];
+        const int tap0 = here[3], tap0_next = there[3], lead = (first_row + here[2]) & 3, lead_next = (first_row + there[2]) & 3;
+        const int half = half0 + stage * window;  // (stages follow each other in the packed filters)
+        // the quarters of the next patch (bits) that pair s of `pairs` requests: all but the last pair share them
+        const int pairs = window / 2, spread = max(pairs - 1, 1);
+        auto parts_of = [&](int s) -> int {
+          const int from = min(4, (4 * s + spread - 1) / spread), to = min(4, (4 * s + 4 + spread - 1) / spread);
+          return (1 << to) - (1 << from);
+        };
+        if constexpr (ODD) {
+          // window = 2 n + 1 >= 3: n pairs, then the single tap; filters are requested two steps ahead
+          int q = 0;
+          for (; q + 4 < window; q += 2) step(no, no, no, half + q + 4, tap0, q + 2, lead, stage, parts_of(q / 2));
+          step(no, no, yes, half + window, tap0, q + 2, lead, stage, parts_of(q / 2));
+          step(yes, yes, no, half + window + 2, tap0_next, 0, lead_next, stage, 0);
+        } else {
+          int q = 0;
+          for (; q + 2 < window; q += 2) step(no, no, no, half + q + 4, tap0, q + 2, lead, stage, parts_of(q / 2));
+          step(no, yes, no, half + window + 2, tap0_next, 0, lead_next, stage, parts_of(q / 2));
+        }
+      }
+      ahead = patch_real;
+    }
+
+    // ---- epilogue: acc[j][i][q] is row m0 + wm0 + 16 i + l16 at position pos0 + 64 wave + 16 j + 4 lk + q
+    bool odd = false;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) odd |= suspect(acc[j][i][q]);
+    const int filters = p.split_flags->filters;
+    odd |= (filters & kWideFilter) != 0 || ((filters & kTinyFilter) != 0 && widest > kWide);
+    if (odd) p.split_flags->rerun = 1;
+
+    const Phase &ph = me.ph;
+    const int first = me.pos0 + wave * 64 + lk * 4;
+    if (me.partial) {
+      float *slot = static_cast<float *>(p.partial) + (long long)me.slot * (BM * BN) + wave * 64 + lk * 4;
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) *reinterpret_cast<f32x4 *>(slot + (wm0 + i * 16 + l16) * BN + j * 16) = acc[j][i];
+      continue;
+    }
+    const int j12 = ph.J[1] * ph.J[2];
+    const int jvol = ph.J[0] * j12;
+    auto dst_of = [&](int ipos) -> float * {
+      const unsigned pos = (unsigned)ipos;
+      const unsigned n = ph.by_jvol.div(pos);
+      unsigned r = pos - n * (unsigned)jvol;
+      const int j0 = (int)ph.by_j12.div(r);
+      r -= (unsigned)j0 * (unsigned)j12;
+      const int j1 = (int)ph.by_j2.div(r);
+      const int j2 = (int)r - j1 * ph.J[2];
+      return dst + (long long)n * p.dst_nstride + (long long)(ph.o0[0] + j0 * p.oj[0]) * p.os[0] +
+             (long long)(ph.o0[1] + j1 * p.oj[1]) * p.os[1] + (long long)(ph.o0[2] + j2 * p.oj[2]) * p.os[2];
+    };
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int four = first + j * 16;
+      if (four >= ph.npos) continue;
+      // four positions that are adjacent in dst leave as one vector, aligned or not (see GemmParams::run_store)
+      bool together = p.vec_store;
+      if (p.run_store && four + 4 <= ph.npos) {
+        const unsigned n = ph.by_jvol.div((unsigned)four);
+        together = (unsigned)four - n * (unsigned)jvol + 4u <= (unsigned)jvol;
+      }
+      if (together) {
+        typedef float OutVec __attribute__((ext_vector_type(4), aligned(4)));
+        float *out = dst_of(four);
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+          const int m = me.m0 + wm0 + i * 16 + l16;
+          if (m < p.M) *reinterpret_cast<OutVec *>(out + (long long)m * p.dst_mstride) = acc[j][i];
+        }
+      } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          if (four + q >= ph.npos) continue;
+          float *out = dst_of(four + q);
+#pragma unroll
+          for (int i = 0; i < TM; ++i) {
+            const int m = me.m0 + wm0 + i * 16 + l16;
+            if (m < p.M) out[(long long)m * p.dst_mstride] = acc[j][i][q];
+          }
+        }
+      }
+    }
+  }
+}
+
+// The filters of split_gemm_kernel, in three parts: piece [octet of K rows][part][m] holds the eight bf16
+// values of K rows 8 * octet .. + 7 of row m of the product, `ld` (a multiple of 16) pieces to a row.  Sixteen K rows
+// are 16 channels from c0 on under one tap, named by halves[K row / 16] = (c0, tap): row m's value is w[m * m_stride + c * c_stride + tap],
+// zero for c >= channels and m >= M.  Also clears
+// the flag that split_gemm_kernel may set, and notes filters out of the range it can represent.
+__global__ void __launch_bounds__(256) split_pack_kernel(const float *__restrict__ w, u32x4 *__restrict__ packed, const int2 *__restrict__ halves,
+                                                         int count, SplitFlags *flags, int M, int channels, long long m_stride, long long c_stride, int ld) {
+  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) flags->rerun = 0;
+  const int oct = blockIdx.x * 16 + (int)(threadIdx.x >> 4), m = blockIdx.y * 16 + (int)(threadIdx.x & 15);
+  if (oct >= 2 * count) return;
+  const int2 h = halves[oct / 2];
+  const int c0 = h.x + oct % 2 * 8;
+  float v[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e)
+    v[e] = m < M && c0 + e < channels ? w[(long long)m * m_stride + (long long)(c0 + e) * c_stride + h.y] : 0.0f;
+  int found = 0;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float a = __builtin_fabsf(v[e]);
+    found |= a > kWide ? kWideFilter : a < kTiny && a != 0.0f ? kTinyFilter : 0;
+  }
+  if (found != 0) atomicOr(&flags->filters, found);
+  bf16x8 parts[3];
+  split_eight(v, parts);
+#pragma unroll
+  for (int part = 0; part < 3; ++part) packed[((long long)oct * 3 + part) * ld + m] = __builtin_bit_cast(u32x4, parts[part]);
+}
+
+// (row, taps) of every position: the row of src (sample * sample_rows + element of a channel's plane) that its window starts
+// from, padding aside, and which taps have an element there, bit by bit; and cleared flags before them.
+__global__ void __launch_bounds__(256) split_positions_kernel(const SplitPositions p, SplitFlags *flags) {
+  int2 *const out = reinterpret_cast<int2 *>(flags + 1);
+  const int idx = blockIdx.x * 256 + threadIdx.x;
+  if (idx == 0) flags->rerun = flags->filters = 0;
+  if (idx >= p.npos) return;
+  const int j12 = p.J[1] * p.J[2], n = idx / (p.J[0] * j12), r = idx - n * p.J[0] * j12;
+  const int q0 = r / j12, q1 = r / p.J[2] % p.J[1], q2 = r % p.J[2];
+  unsigned taps = 0;
+  int t = 0;
+  for (int a = 0; a < p.sp.count[0]; ++a)
+    for (int b = 0; b < p.sp.count[1]; ++b)
+      for (int c = 0; c < p.sp.count[2]; ++c, ++t) {
+        const int i0 = q0 + p.sp.d[0] + a * p.sp.step[0], i1 = q1 + p.sp.d[1] + b * p.sp.step[1], i2 = q2 + p.sp.d[2] + c * p.sp.step[2];
+        if ((unsigned)i0 < (unsigned)p.Q[0] && (unsigned)i1 < (unsigned)p.Q[1] && (unsigned)i2 < (unsigned)p.Q[2]) taps |= 1u << t;
+      }
+  out[idx] = int2{n * p.sample_rows + (q0 * p.Q[1] + q1) * p.Q[2] + q2, (int)taps};
+}
+
+// rows of a wave; waves along the rows and the positions of a tile
+#define MG_SPLIT_SHAPES(X) X(64, 2, 2) X(48, 2, 2) X(64, 1, 4) X(64, 1, 2) X(48, 1, 4) X(32, 1, 4) X(16, 1, 4)
+
+template <int WM, int MW, int NW>
+size_t lds_bytes(int patch_rows) {
+  return (size_t)(2 * 12 * WM * MW + 2 * (patch_rows + 1) * 3) * 16;
+}
+
+}  // namespace
+
+// Rows of a patch that a tile has room for: a thread takes eight channels of four rows, and two blocks share a unit's LDS (alone on
+// it, a block's waves wait for their barriers: 256 filters, 3x3, stride 2, 27x27 161 us on patches of 540 rows, 134 on the other kernel).
+int split_patch_limit(int bm, int bn) {
+#define MG_LIMIT(WM, MW, NW) \
+  if (bm == WM * MW && bn == 64 * NW) return std::min(64 * MW * NW * 2, (int)(80 * 1024 / 16 - 24 * WM * MW) / 6 - 1);
+  MG_SPLIT_SHAPES(MG_LIMIT)
+#undef MG_LIMIT
+  return 0;
+}
+
+int split_gemm_blocks_per_cu(int bm, int bn, int patch_rows) {
+  static std::map<std::array<int, 3>, int> known;  // (behind the lock of the entry points)
+  int &n = known[{bm, bn, patch_rows}];
+  if (n > 0) return n;
+#define MG_OCC(WM, MW, NW)                                                                                                              \
+  if (bm == WM * MW && bn == 64 * NW) {                                                                                                 \
+    const size_t bytes = lds_bytes<WM, MW, NW>(patch_rows);                                                                             \
+    (void)hipFuncSetAttribute((const void *)split_gemm_kernel<WM, MW, NW, true>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);  \
+    (void)hipFuncSetAttribute((const void *)split_gemm_kernel<WM, MW, NW, false>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); \
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, split_gemm_kernel<WM, MW, NW, true>, 64 * MW * NW, bytes) != hipSuccess) n = 0; \
+  }
+  MG_SPLIT_SHAPES(MG_OCC)
+#undef MG_OCC
+  if (n < 1) {
+    (void)hipGetLastError();
+    n = 1;
+  }
+  return n;
+}
+
+bool launch_split_gemm(const GemmParams &p, int bm, int bn, bool odd, unsigned grid, hipStream_t s) {
+#define MG_LAUNCH(WM, MW, NW)                                                                                                                  \
+  if (bm == WM * MW && bn == 64 * NW) {                                                                                                        \
+    if (odd)                                                                                                                                   \
+      hipLaunchKernelGGL((split_gemm_kernel<WM, MW, NW, true>), dim3(grid), dim3(64 * MW * NW), (lds_bytes<WM, MW, NW>(p.patch_rows)), s, p);  \
+    else                                                                                                                                       \
+      hipLaunchKernelGGL((split_gemm_kernel<WM, MW, NW, false>), dim3(grid), dim3(64 * MW * NW), (lds_bytes<WM, MW, NW>(p.patch_rows)), s, p); \
+    return true;                                                                                                                               \
+  }
+  MG_SPLIT_SHAPES(MG_LAUNCH)
+#undef MG_LAUNCH
+  return false;
+}
+
+void launch_split_pack(const float *w, void *packed, const void *halves, int count, SplitFlags *flags, int M, int channels, long long m_stride,
+                       long long c_stride, int ld, hipStream_t s) {
+  hipLaunchKernelGGL(split_pack_kernel, dim3((unsigned)ceil_div(2 * count, 16), (unsigned)(ld / 16)), dim3(256), 0, s, w,
+                     static_cast<u32x4 *>(packed), static_cast<const int2 *>(halves), count, flags, M, channels, m_stride, c_stride, ld);
+}
+
+void launch_split_positions(const SplitPositions &p, void *out, hipStream_t s) {
+  hipLaunchKernelGGL(split_positions_kernel, dim3((unsigned)ceil_div(p.npos, 256)), dim3(256), 0, s, p, static_cast<SplitFlags *>(out));
+}
+
+}  // namespace mg

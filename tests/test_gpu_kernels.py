@@ -1421,3 +1421,84 @@ def test_per_launch_timing_records_chains_and_pauses():
         assert _hip.timing_read() == []
     finally:
         _hip.timing_enable(False)
+
+
+# float32 on operands split into three bf16 parts: (x, w, padding, dilation, tile; "" leaves the tile to the plan).  Odd
+# extents, so that row ends and sample ends fall inside tiles; channels and filters that fill no 16.
+SPLIT_PROBLEMS = [
+    ((3, 32, 29, 27), (160, 32, 3, 3), (1, 1), (1, 1), "128,128"),           # odd window; a quarter row tile
+    ((9, 45, 31, 33), (101, 45, 2, 3), (1, 2), (1, 1), "96,128"),            # even window, ragged counts
+    ((2, 16, 23, 300), (64, 16, 3, 3), (1, 1), (1, 1), "64,256"),            # rows longer than a tile: stages of one row of taps
+    ((17, 61, 13, 13), (64, 61, 5, 5), (2, 2), (1, 2), "64,128"),             # the tiles of several samples; dilation
+    ((2, 48, 5000), (48, 48, 8), (3,), (2,), "48,256"),                      # one axis, even window
+    ((310, 24, 7, 7), (32, 24, 3, 3), (2, 2), (2, 2), "32,256"),              # planes of 49: samples rounded up to whole loads
+    ((1, 16, 4099), (16, 16, 31), (15,), (1,), "16,256"),                    # as many taps as a position's bits
+    ((4, 45, 9, 11, 13), (76, 45, 2, 3, 3), (1, 0, 1), (1, 2, 1), ""),       # three axes
+    ((11, 32, 19, 21), (48, 32, 5, 3), (0, 0), (1, 1), ""),                  # no padding: the data gradient's positions outnumber
+    ((37, 32, 61), (80, 32, 9), (0,), (2,), ""),                             # its rows along every axis, and samples overlap in them
+    ((3, 32, 9, 11, 12), (48, 32, 3, 3, 3), (1, 0, 0), (1, 1, 2), ""),
+    ((2, 512, 6, 5), (512, 512, 3, 3), (1, 1), (1, 1), ""),                  # every tile shared out
+]
+
+
+@pytest.mark.parametrize("problem", range(len(SPLIT_PROBLEMS)))
+def test_products_of_three_bf16_parts(abi, monkeypatch, problem):
+    from mygrad_amd import _hip
+
+    x_shape, w_shape, p, d, tile = SPLIT_PROBLEMS[problem]
+    s = (1,) * len(p)
+    rng = np.random.default_rng(3100 + problem)
+
+    def passes(x, w, g, split=True):
+        """Forward pass and data gradient, and whether both ran on split operands."""
+        with monkeypatch.context() as m:
+            m.setenv("MYGRAD_HIP_TINY", "0")
+            m.setenv("MYGRAD_HIP_SPLIT_MIN", "0")
+            m.setenv("MYGRAD_HIP_SPLIT", "1" if split else "0")
+            if tile:
+                m.setenv("MYGRAD_HIP_TILE", tile)
+            out = abi.conv_fwd(x, w, s, p, d)
+            plans = [_hip.last_plan()]
+            dx = abi.conv_dgrad(g, x_shape, w, s, p, d)
+            plans.append(_hip.last_plan())
+        print(*plans, sep="\n", flush=True)
+        for plan in plans:
+            assert plan.endswith("three bf16 parts") == split and tile.replace(",", "x") in plan
+        return out, dx
+
+    # small integers: every sum is exact
+    xi, wi = rng.integers(-3, 4, x_shape).astype(np.float32), rng.integers(-2, 3, w_shape).astype(np.float32)
+    want = direct.conv_forward(xi, wi, s, p, d).astype(np.float32)
+    gi = rng.integers(-2, 3, want.shape).astype(np.float32)
+    out, dx = passes(xi, wi, gi)
+    assert np.array_equal(out, want)
+    assert np.array_equal(dx, direct.conv_backward_x(gi, x_shape, wi, s, p, d).astype(np.float32))
+    # against 64 bits: a sum of K terms takes six roundings into its accumulator for every 32 of them (three for 16).  Rounded off towards
+    # zero, a number is off by 2^-23 * E[m^-2]^1/2 / 3^1/2 = 5.06e-8 of itself on average (significands m of 1 to 2, evenly in
+    # their logarithm), and after a share of its roundings a sum of normal terms has that share of its variance: together 5.06e-8 *
+    # (6 K / 32 / 2)^1/2 of the result; a quarter for the spread of a sample, K in whole blocks of 16 channels
+    x, w, g = (rng.standard_normal(shape).astype(np.float32) for shape in (x_shape, w_shape, want.shape))
+    x64, w64, g64 = (a.astype(np.float64) for a in (x, w, g))
+    exact = direct.conv_forward(x64, w64, s, p, d), direct.conv_backward_x(g64, x_shape, w64, s, p, d)
+    for got, plain, ref, count in zip(passes(x, w, g), passes(x, w, g, split=False), exact, (w_shape[1], w_shape[0])):
+        assert not np.array_equal(got, plain)  # (nothing was left to the single-precision kernels)
+        terms = -(-count // 16) * 16 * np.prod(w_shape[2:])
+        assert np.linalg.norm(got - ref) <= 1.25 * 5.06e-8 * np.sqrt(6 * terms / 64) * np.linalg.norm(ref)
+    # what the parts cannot hold is left to the single-precision kernels: infinite and NaN operands, sums that overflow, operands and sums
+    # near the smallest numbers; and the pass after it is none of that
+    at = tuple(n // 2 for n in x_shape)
+    for value in (np.inf, np.nan, 3e38):
+        xs, gs = x.copy(), g.copy()
+        xs[at] = value
+        gs[tuple(n // 2 for n in g.shape)] = value
+        with np.errstate(all="ignore"):
+            ws = w * np.float32(4)
+        for got, plain in zip(passes(xs, ws, gs), passes(xs, ws, gs, split=False)):
+            assert np.array_equal(bits(got), bits(plain))
+    scales = (1e-30, 1.0, 1e-30), (1e-36, 1e9, 1e-36), (1e9, 1e-36, 1e9), (1e-20, 1e-20, 1e-20)
+    for a, b, c in scales:
+        xs, ws, gs = x * np.float32(a), w * np.float32(b), g * np.float32(c)
+        for got, plain in zip(passes(xs, ws, gs), passes(xs, ws, gs, split=False)):
+            assert np.array_equal(bits(got), bits(plain))
+    again = passes(xi, wi, gi)
+    assert np.array_equal(bits(again[0]), bits(out)) and np.array_equal(bits(again[1]), bits(dx))
