@@ -2556,7 +2556,7 @@ int run_gemm(GemmParams &gp, const Plan &pl, int tag, hipStream_t s) {
     gp.vec_store = pl.pJ[0][2] == pl.pJ[1][2] && gp.os[1] % 4 == 0 && gp.os[0] % 4 == 0 && gp.dst_mstride % 4 == 0 &&
                    gp.dst_nstride % 4 == 0 && reinterpret_cast<uintptr_t>(gp.dst) % 16 == 0;
   }
-  ScopedTiming timed(tag);
+  ScopedTiming timed(gp.gate != nullptr ? TAG_GATED : tag);
   bool launched = false;
   if (pl.split) launched = launch_split(gp, pl, s);
   if (pl.deep_k) {
@@ -2675,7 +2675,7 @@ int pack_filters(const Geometry &g, const void *w, int mode, int depth, void **p
   }
   // (behind a gate most passes have nothing to do: few blocks)
   const unsigned blocks = (unsigned)std::min<long long>(ceil_div((long long)count, 256), gate ? 256 : 4096);
-  ScopedTiming timed(TAG_PACK_FILTERS);
+  ScopedTiming timed(gate ? TAG_GATED : TAG_PACK_FILTERS);
   hipLaunchKernelGGL(pack_filters_kernel<T>, dim3(blocks), dim3(256), 0, runtime().stream, static_cast<const T *>(w),
                      static_cast<T *>(*packed), g.F, g.C, (int)g.wvol, mode, ld, depth, gate);
   MG_HIP(hipGetLastError());
