@@ -797,8 +797,8 @@ struct TileRate {
 };
 constexpr TileRate kTileRates[] = {
     // (nph 0: split_gemm_kernel)
-    {0, 16, 256, 0.50, 0.74, 0.00}, {0, 32, 256, 0.50, 0.82, 0.00}, {0, 48, 256, 0.50, 0.92, 0.00}, {0, 64, 128, 0.40, 1.05, 0.00},
-    {0, 64, 256, 0.50, 1.15, 0.00}, {0, 96, 128, 0.45, 0.95, 0.00}, {0, 128, 128, 0.50, 1.05, 0.00},
+    {0, 16, 256, 0.50, 0.74, 0.00}, {0, 32, 256, 0.50, 0.90, 0.00}, {0, 48, 256, 0.50, 1.14, 0.00}, {0, 64, 128, 0.40, 1.00, 0.00},
+    {0, 64, 192, 0.45, 1.22, 0.00}, {0, 128, 128, 0.50, 1.00, 0.00},
     {1, 16, 256, 0.50, 0.42, 0.42}, {1, 32, 128, 0.35, 0.59, 0.62},  {1, 32, 256, 0.55, 0.63, 0.64}, {1, 48, 256, 0.62, 0.70, 0.67},
     {1, 64, 128, 0.47, 0.77, 0.70}, {1, 64, 256, 0.78, 0.83, 0.00},  {1, 96, 128, 0.56, 0.82, 0.80}, {1, 128, 64, 0.27, 0.81, 0.87},
     {1, 128, 128, 0.63, 0.86, 0.0}, {2, 16, 256, 0.53, 0.50, 0.00},  {2, 32, 256, 0.47, 0.70, 0.00}, {2, 64, 128, 0.45, 0.82, 0.00},
@@ -853,10 +853,10 @@ TileChoice choose_tile(int M, const std::vector<long long> &phase_npos, int min_
                               {64, 128, 1.08, true},   {48, 256, 1.00, true},  {32, 256, 1.00, false},  {32, 128, 1.10, true}, {16, 256, 1.00, false}};
   static const Cfg fused2[] = {{128, 64, 1.05, true}, {64, 128, 1.08, true}, {32, 256, 1.00, true}, {16, 256, 1.00, true}};
   static const Cfg fused4[] = {{64, 64, 1.10, true}, {32, 128, 1.10, true}, {16, 256, 1.00, true}};
-  static const Cfg split[] = {{128, 128, 1.00, true}, {96, 128, 1.00, true}, {64, 256, 1.00, true}, {64, 128, 1.05, true},
+  static const Cfg split[] = {{128, 128, 1.00, true}, {64, 192, 1.00, true}, {64, 128, 1.05, true},
                               {48, 256, 1.00, true},  {32, 256, 1.00, true}, {16, 256, 1.00, true}};
   const Cfg *cfgs = nph == 4 ? fused4 : nph == 2 ? fused2 : nph == 0 ? split : plain;
-  const int ncfgs = nph == 4 ? 3 : nph == 2 ? 4 : nph == 0 ? 7 : 9;
+  const int ncfgs = nph == 4 ? 3 : nph == 2 ? 4 : nph == 0 ? 6 : 9;
   // MYGRAD_HIP_TILE="rows,positions[,blocks per unit]" (diagnostics and the tests of every tile shape;
   // read whenever a plan is built, and part of the plan's key): only that tile shape, where it exists
   struct Forced {
@@ -872,7 +872,7 @@ TileChoice choose_tile(int M, const std::vector<long long> &phase_npos, int min_
     const char *flag = getenv("MYGRAD_HIP_SHARES");
     return !(flag && flag[0] == '0');
   }();
-  auto patch_fits = [&](const Cfg &c) { return patch[c.bn == 256] > 0 && patch[c.bn == 256] <= split_patch_limit(c.bm, c.bn); };
+  auto patch_fits = [&](const Cfg &c) { return patch[split_width(c.bn)] > 0 && patch[split_width(c.bn)] <= split_patch_limit(c.bm, c.bn); };
   bool forced_fits = false;
   for (int ci = 0; ci < ncfgs; ++ci)
     forced_fits |= cfgs[ci].bm == forced.bm && cfgs[ci].bn == forced.bn && (!cfgs[ci].tap_only || tap_major) &&
@@ -903,7 +903,7 @@ TileChoice choose_tile(int M, const std::vector<long long> &phase_npos, int min_
     // fits on a compute unit, so the tap-major kernels use the half-size shapes
     if (tap_major && elem == 8 && c.bn * c.bm >= 128 * 128) continue;
     const bool stream = nph == 0 || (tap_major && tap_gemm_streams(c.bm, (int)elem));
-    const int per_cu = !stream ? 1 : nph == 0 ? split_gemm_blocks_per_cu(c.bm, c.bn, patch[c.bn == 256]) : elem == 8 ? gemm_blocks_per_cu<double>(c.bm, c.bn, 1, bk) : gemm_blocks_per_cu<float>(c.bm, c.bn, nph, bk);
+    const int per_cu = !stream ? 1 : nph == 0 ? split_gemm_blocks_per_cu(c.bm, c.bn, patch[split_width(c.bn)]) : elem == 8 ? gemm_blocks_per_cu<double>(c.bm, c.bn, 1, bk) : gemm_blocks_per_cu<float>(c.bm, c.bn, nph, bk);
     long long pos_blocks = 0;
     for (long long n : phase_npos) pos_blocks += ceil_div(n, c.bn);
     // (most blocks first: where the rounds come out the same, more resident blocks cover more of one
@@ -1422,15 +1422,15 @@ double split_min_flops(double filters) {
   return v ? atof(v) : 8.0e9 + 2.0e3 * filters;
 }
 
-// How a pass would run on conv_split.hip: its phase, its stages' window and the rows of src that a tile of 128 or 256
+// How a pass would run on conv_split.hip: its phase, its stages' window and the rows of src that a tile of 128, 192 or 256
 // positions touches (0: more than the kernel has room for, with any tile of that width).
 inline long long up4(long long n) { return (n + 3) / 4 * 4; }
 struct SplitLayout {
   SplitPhase sp{};
   int offs[31] = {};
   int taps = 0;
-  int patch[2] = {0, 0};
-  std::vector<int> first[2];  // see GemmParams::split_tiles
+  int patch[3] = {0, 0, 0};
+  std::vector<int> first[3];  // see GemmParams::split_tiles
 };
 
 // The rows of src that `bn` consecutive positions touch at most, and each block's first one, when axes `inner` .. 2 are a stage's
@@ -1487,12 +1487,14 @@ bool split_applies(const Geometry &g, const Plan &pl, int rows, const Phase &ph,
     // (a stage's elements are loaded, split and parked for its taps' products: with three taps that is what bounds it, (59,56,930) *
     // (443,56,3), dx, 101 us on the other kernel, 145 here; the kernel itself takes three and more)
     if (window < (getenv("MYGRAD_HIP_SPLIT_MIN") ? 3 : 5)) break;
-    for (int wide = 0; wide < 2; ++wide) {
-      const long long rows = (touched_rows(sp, ph, g.N, Q, inner, wide ? 256 : 128, lay.first[wide]) + 3 + 15) / 16 * 16;
-      lay.patch[wide] = rows <= split_patch_limit(wide ? 64 : 96, wide ? 256 : 128) ? (int)rows : 0;
+    bool fits = false;
+    for (int bn : {128, 192, 256}) {
+      const int width = split_width(bn), rows = (int)std::min(1ll << 20, (touched_rows(sp, ph, g.N, Q, inner, bn, lay.first[width]) + 3 + 15) / 16 * 16);
+      lay.patch[width] = rows <= split_patch_limit(bn == 256 ? 16 : 64, bn) ? rows : 0;
+      fits |= lay.patch[width] > 0;
     }
     sp.window = window;
-    if (lay.patch[0] > 0 || lay.patch[1] > 0) return true;
+    if (fits) return true;
   }
   return false;
 }
@@ -1521,12 +1523,12 @@ int split_tables(Plan &pl, Tables &t, const SplitLayout &lay, const Phase &ph, c
       t.split_halves.push_back(int2{c0, tap});
     }
   t.split_inner.assign(lay.offs, lay.offs + window);
-  t.split_tiles = lay.first[pl.bn == 256];
+  t.split_tiles = lay.first[split_width(pl.bn)];
   t.split_phases.push_back(lay.sp);
   pl.split_half_count = (int)t.split_halves.size();
   pl.split_odd = window % 2 != 0;
   pl.split_npos = ph.npos;
-  pl.patch_rows = lay.patch[pl.bn == 256];
+  pl.patch_rows = lay.patch[split_width(pl.bn)];
   return MG_OK;
 }
 
@@ -2407,9 +2409,8 @@ int get_plan(ConvOp op, const mg_conv_desc *d, const Geometry &g, Plan **out) {
         free_tables(pl);
         return failed;
       }
-      // Six roundings into an accumulator for 32 terms here, eight there: no less accurate as long as there is no more than
-      // a third more to sum up without a break (the single-precision plan cuts K into more slices where it has few tiles: (2,57,16936) *
-      // (125,57,15), dx, error against 64 bits 6.8e-7 here, 3.8e-7 there).
+      // One rounding of a sum for 32 terms here, eight there: a third of the error on sums cut alike.  The single-precision plan cuts K into
+      // more slices where it has few tiles; where that would leave more than a quarter more to sum up without a break here, it stays.
       const bool as_accurate = pl.chain <= 1.25 * exact.chain || getenv("MYGRAD_HIP_SPLIT_MIN") != nullptr;
       // Nor on tiles of many more rows, where the patches of 256 positions do not fit: (98,110,69,63) * (15,110,3,3) 181 us on
       // tiles of 16 x 256, 436 here on 96 x 128.
@@ -2503,10 +2504,15 @@ bool launch_split(GemmParams &gp, const Plan &pl, hipStream_t s) {
   }
   if (!launch_split_gemm(gp, pl.bm, pl.bn, pl.split_odd, (unsigned)grid, s)) return false;
   if (fixes > 0) {
-#define MG_FIXUP(TT, BM, BN, WM, WN)                                                                                                     \
-  if (pl.bm == BM && pl.bn == BN)                                                                                                        \
-    hipLaunchKernelGGL((tail_fixup_kernel<TT, BM, BN, 1>), dim3((unsigned)ceil_div(BM * BN, 256), (unsigned)fixes), dim3(256), 0, s, gp);
-    MG_GEMM_SHAPES(float, MG_FIXUP)
+#define MG_FIXUP(BM, BN)             \
+  if (pl.bm == BM && pl.bn == BN)    \
+    hipLaunchKernelGGL((tail_fixup_kernel<float, BM, BN, 1>), dim3((unsigned)ceil_div(BM * BN, 256), (unsigned)fixes), dim3(256), 0, s, gp);
+    MG_FIXUP(128, 128)
+    MG_FIXUP(64, 192)
+    MG_FIXUP(64, 128)
+    MG_FIXUP(48, 256)
+    MG_FIXUP(32, 256)
+    MG_FIXUP(16, 256)
 #undef MG_FIXUP
   }
   return true;

@@ -202,6 +202,7 @@ struct SplitPositions {
 };
 
 // conv_split.hip
+inline int split_width(int bn) { return bn / 64 - 2; }  // numbers the widths of its tiles: 128, 192, 256 positions
 int split_patch_limit(int bm, int bn);
 int split_gemm_blocks_per_cu(int bm, int bn, int patch_rows);
 bool launch_split_gemm(const GemmParams &p, int bm, int bn, bool odd, unsigned grid, hipStream_t s);

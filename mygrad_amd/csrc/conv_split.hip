@@ -5,17 +5,24 @@
 // ALU (44 vector instructions next to 16 of them: 154 -> 110 TFLOP/s); v_mfma_f32_16x16x32_bf16 does
 // 1800 - 2000 and does not.  A float is the sum of three bf16 numbers exactly (8 + 8 + 8 bits of its
 // significand), x = x0 + x1 + x2, and
-//   x * w = x0 w0 + (x0 w1 + x1 w0) + (x0 w2 + x1 w1 + x2 w0) + terms below 2^-25 |x w|,
-// six products, each exact in single precision and added up in single-precision accumulators: an
-// effective peak of 300 - 330 TFLOP/s.  The error against 64 bits is no larger than that of the single-precision
-// instruction, whose every step of four terms rounds into the accumulator where this one rounds six times per
-// 32 terms (K = 64 / 576 / 4096, normal values: 9.8e-8 / 3.7e-7 / 1.0e-6 here, 1.4e-7 / 4.6e-7 / 1.1e-6 there).  (The five small
-// products summed apart and added once per step halve it, 1.7e-7 at K = 576, but need registers that 64-row
-// wave tiles do not have: they spill, and 178 us become 224.)
+//   x * w = x0 w0 + (x0 w1 + x1 w0) + (x0 w2 + x1 w1 + x2 w0) + at most 2^-24 |x w|,
+// six products, each exact in single precision: an effective peak of 300 - 330 TFLOP/s.
 //
-// What bounds it: (128,64,56,56) * (64,64,3,3), 29.6 GFLOP, takes 178 us with its packing and gated passes, about 160 by itself: 185
-// TFLOP/s of the 300.  The rest is the turn between stages, where the waves of a block wait for the patch to be split and
-// parked, and the first stage of a tile; loads are hidden.
+// Precision.  The large product and the five small ones have an accumulator each, added at the end.  An accumulator rounds once per
+// 32 terms of a product, whatever the terms are, and loses some bits of what it adds; in one accumulator for all six that
+// made sums of few terms less accurate than the single-precision instruction, which rounds only where a term is not zero.
+// Error against 64 bits (2-norm), one accumulator / two / single precision, (128,64,56,56) * (64,64,3,3):
+//   normal values 3.5e-7 / 1.4e-7 / 4.2e-7; behind a relu 3.4e-7 / 1.2e-7 / 3.0e-7; one element in 100 not zero 9.8e-8 / 3.7e-8 /
+//   4.9e-8; one product a sum 4.2e-8 / 2.6e-8 / 2.5e-8 (there what the six products leave out shows: no result is off by more than
+//   2^-23 of itself, where one rounding is 2^-24).
+// Two accumulators of 64 x 64 wave tiles do not fit 256 registers (70 - 85 of them spill: 186 us below become 246), those of 64 x 48 do but for
+// a dozen values that no step needs.
+//
+// What bounds it: (128,64,56,56) * (64,64,3,3), 29.6 GFLOP, takes 186 us with its packing and gated passes (single precision 234), about
+// 170 by itself: 174 TFLOP/s of the 300.  Operands from LDS (64 x 48 and 48 x 64 waves: 21 reads of 16 bytes a lane for 72 matrix
+// instructions, 58 % of its bandwidth; 32 x 64 ones 18 for 48, 75 %: 201 us), and the turn between stages, where the waves of a block wait for
+// the patch to be split and parked; loads are hidden.  Smaller planes have smaller patches: (128,128,28,28) * (128,128,3,3), 29.6 GFLOP,
+// 230 -> 161 us; (16,96,16001) * (48,96,9), 21.2 GFLOP, 172 -> 130.
 //
 // What the split cannot represent is left to the single-precision kernels.  An infinite operand leaves Inf - Inf in
 // its second part and makes every sum that it takes part in a NaN, as an infinite or NaN operand or an overflow makes
@@ -41,6 +48,7 @@ namespace {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 typedef int int8v __attribute__((ext_vector_type(8)));
 typedef int int16v __attribute__((ext_vector_type(16)));
@@ -55,12 +63,13 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void *base, un
 __device__ __forceinline__ unsigned bits_of(float v) { return __builtin_bit_cast(unsigned, v); }
 __device__ __forceinline__ float float_of(unsigned v) { return __builtin_bit_cast(float, v); }
 
-// a = h[0] + m[0] + l[0] and b likewise, exactly.  The first part is cut off, not rounded (rounding could
-// overflow); the rest, at most 16 bits, is rounded to nearest, so that what the six products leave
-// out has no sign of its own.  Eleven vector instructions for two values.
+// a = h[0] + m[0] + l[0] and b likewise, exactly.  Every part is rounded to nearest (the last one, of at most eight bits, needs
+// none): x1 is at most 2^-8 of x and x2 2^-17, so what the six products leave out, x1 w2 + x2 w1 + x2 w2, is at most 2^-24 of x w and
+// has no sign of its own (with the first part cut off instead it was up to 2^-22).  A value that rounds to infinity leaves a
+// NaN in its second part.  Eleven vector instructions for two values.
 __device__ __forceinline__ void split_pair(float a, float b, unsigned &h, unsigned &m, unsigned &l) {
-  h = __builtin_amdgcn_perm(bits_of(b), bits_of(a), 0x07060302u);
-  const float ra = a - float_of(bits_of(a) & 0xffff0000u), rb = b - float_of(bits_of(b) & 0xffff0000u);
+  h = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{a, b}), bf16x2));
+  const float ra = a - float_of(h << 16), rb = b - float_of(h & 0xffff0000u);
   m = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{ra, rb}), bf16x2));
   const float qa = ra - float_of(m << 16), qb = rb - float_of(m & 0xffff0000u);
   l = __builtin_amdgcn_perm(bits_of(qb), bits_of(qa), 0x07060302u);
@@ -105,7 +114,7 @@ __device__ __forceinline__ int phase_first_block(const Phase *phases, int i) {
   return ((const int MG_CONSTANT *)(phases + uniform(i)))[8];
 }
 
-// One tile is MW * WM rows (filters) by NW * 64 positions, a wave of the block for each WM x 64 of it.  The contraction
+// One tile is MW * WM rows (filters) by NW * 16 TN positions, a wave of the block for each WM x 16 TN of it.  The contraction
 // runs in stages: 16 channels under the taps of one inner window (all taps, or those of the last axes where the
 // others reach too far).  A stage's elements of src -- every row (position of src) that the tile's windows touch, 16
 // channels of each -- are loaded and split once, parked in LDS, and serve all taps of the window from there: operand
@@ -114,14 +123,15 @@ __device__ __forceinline__ int phase_first_block(const Phase *phases, int i) {
 // 180 us.)  A position without the tap (padding) reads a row of zeros.
 //
 // A K step is 32 deep: two taps, lanes 0 - 31 hold the first one's 16 channels, lanes 32 - 63 the second one's.  An
-// odd last tap (ODD) makes a step of three products instead of six: lanes 0 - 31 and 32 - 63 hold different parts of the one tap.
+// odd last tap (ODD) makes a step of four products instead of six: lanes 0 - 31 and 32 - 63 hold different parts of the one tap, and
+// nothing beside x0 w0.
 //
 // The positions are the rows of D, so that a lane holds four consecutive positions of one filter and stores them as a vector.  The filters,
 // split and laid out in the order of the stages beforehand (split_pack_kernel), pass through LDS two steps ahead of their use.
 // Blocks are persistent, as in tap_gemm_kernel.
-template <int WM, int MW, int NW, bool ODD>
+template <int WM, int MW, int TN, int NW, int ROUNDS, bool ODD>
 __global__ void __launch_bounds__(64 * MW * NW, 2) split_gemm_kernel(const GemmParams p) {
-  constexpr int BM = WM * MW, BN = 64 * NW, TM = WM / 16, THREADS = 64 * MW * NW;
+  constexpr int BM = WM * MW, WN = 16 * TN, BN = WN * NW, TM = WM / 16, THREADS = 64 * MW * NW;
   static_assert(WM % 16 == 0, "16 x 16 tiles");
   constexpr int PIECES = 12 * BM;  // of 16 bytes: a step's filters, [part][octet of K rows][row]
   constexpr int ALOADS = (PIECES + THREADS - 1) / THREADS;
@@ -199,52 +209,64 @@ __global__ void __launch_bounds__(64 * MW * NW, 2) split_gemm_kernel(const GemmP
   float *__restrict__ dst = static_cast<float *>(p.dst);
   int pi = 0;
   Item me;
-  u32x4 raw[8];        // elements on their way to the patch: [channel][row of four]
-  bool ahead = false;  // those of the item's first stage were requested by the item before it
+  u32x4 raw[ROUNDS][4];  // elements on their way to the patch: [round][channel][row of four]
+  bool ahead = false;    // those of the item's first stage were requested by the item before it
   // the patch being requested: its first row, its stage's row of the table, whether there is one
   int patch_row = 0;
   int8v patch_e = {0, 0, 0, 0, 0, 0, 0, 0};  // first half, channel offset, row offset, first tap, -, dead rows
   bool patch_real = false;
   auto first_of = [&](const Item &it) -> int { return ((const int MG_CONSTANT *)p.split_tiles)[uniform(it.pos0 / BN)]; };
-  // A quarter of the patch's loads.  A thread takes four rows, which begin on a multiple of four and therefore lie in one sample
-  // (a sample's rows are numbered up to a multiple of four; what is loaded for those beyond its last is of no use to anyone), and
-  // loads them as one vector, whatever its alignment: 16 bytes a lane take the vector cache 16 cycles, 4 bytes 8 - 11.
+  // A part of the patch's loads.  A thread takes four rows of four channels in each round; the rows begin on a multiple of four and therefore
+  // lie in one sample (a sample's rows are numbered up to a multiple of four; what is loaded for those beyond its last is of no use to
+  // anyone), and are loaded as one vector, whatever its alignment: 16 bytes a lane take the vector cache 16 cycles, 4 bytes 8 - 11.
+  const int quads = p.patch_rows / 4;
+  auto quarter_of = [&](int idx) -> int { return (idx >= quads) + (idx >= 2 * quads) + (idx >= 3 * quads); };  // of the stage's channels
   auto request_part = [&](int k) {
-    const int quads = p.patch_rows / 4, octet = (int)threadIdx.x >= quads ? 1 : 0;
-    const int row = ((patch_row + patch_e[2]) & ~3) + ((int)threadIdx.x - octet * quads) * 4;
+    constexpr int CHANNELS = ROUNDS;  // a part is a round's four channels, a quarter or a half of them at a time
+    const int round = k * ROUNDS / 4;
+    if (round * THREADS >= p.patch_rows) return;
+    const int idx = (int)threadIdx.x + round * THREADS, quarter = quarter_of(idx);
+    const int row = ((patch_row + patch_e[2]) & ~3) + (idx - quarter * quads) * 4;
     const unsigned n = __umulhi((unsigned)max(row, 0), p.by_sample.mul) >> p.by_sample.shr;  // (more than one row to a sample)
-    unsigned at = (n * (unsigned)p.src_nstride + (unsigned)(row - (int)n * p.sample_rows + patch_e[1] + octet * 8 * p.src_cstride)) * 4u;
-    at = ((int)threadIdx.x < 2 * quads) & (row >= 0) & ((int)n < p.samples) & patch_real ? at : kOutside;
-    const unsigned dead = (unsigned)patch_e[5] >> (octet * 8);
+    unsigned at = (n * (unsigned)p.src_nstride + (unsigned)(row - (int)n * p.sample_rows + patch_e[1] + quarter * 4 * p.src_cstride)) * 4u;
+    at = (idx < p.patch_rows) & (row >= 0) & ((int)n < p.samples) & patch_real ? at : kOutside;
+    const unsigned dead = (unsigned)patch_e[5] >> (quarter * 4);
 #pragma unroll
-    for (int r = 2 * k; r < 2 * k + 2; ++r)
-      raw[r] = __builtin_amdgcn_raw_buffer_load_b128(src_buf, (int)(at | ((dead << (31 - r)) & kOutside)), (int)((unsigned)r * c_step), 0);
+    for (int u = 0; u < CHANNELS; ++u) {
+      const int r = k * CHANNELS % 4 + u;
+      raw[round][r] = __builtin_amdgcn_raw_buffer_load_b128(src_buf, (int)(at | ((dead << (31 - r)) & kOutside)), (int)((unsigned)r * c_step), 0);
+    }
   };
   auto park_patch = [&] {
-    const int quads = p.patch_rows / 4, octet = (int)threadIdx.x >= quads ? 1 : 0;
-    u32x4 *const out = patch + (octet * octet_rows + ((int)threadIdx.x - octet * quads) * 4) * 3;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      float v[8];
+    for (int round = 0; round < ROUNDS; ++round) {
+      if (round * THREADS >= p.patch_rows) break;
+      const int idx = (int)threadIdx.x + round * THREADS, quarter = quarter_of(idx);
+      u32x2 *const out = reinterpret_cast<u32x2 *>(patch + (quarter / 2 * octet_rows + (idx - quarter * quads) * 4) * 3) + quarter % 2;
 #pragma unroll
-      for (int r = 0; r < 8; ++r) v[r] = float_of(raw[r][u]);
+      for (int u = 0; u < 4; ++u) {
+        float v[4];
 #pragma unroll
-      for (int r = 0; r < 8; r += 2) widest = __builtin_fmaxf(__builtin_fmaxf(widest, __builtin_fabsf(v[r])), __builtin_fabsf(v[r + 1]));
-      bf16x8 parts[3];
-      split_eight(v, parts);
-      if ((int)threadIdx.x < 2 * quads) {
+        for (int r = 0; r < 4; ++r) v[r] = float_of(raw[round][r][u]);
 #pragma unroll
-        for (int part = 0; part < 3; ++part) out[u * 3 + part] = __builtin_bit_cast(u32x4, parts[part]);
+        for (int r = 0; r < 4; r += 2) widest = __builtin_fmaxf(__builtin_fmaxf(widest, __builtin_fabsf(v[r])), __builtin_fabsf(v[r + 1]));
+        unsigned parts[3][2];
+        split_pair(v[0], v[1], parts[0][0], parts[1][0], parts[2][0]);
+        split_pair(v[2], v[3], parts[0][1], parts[1][1], parts[2][1]);
+        if (idx < p.patch_rows) {
+#pragma unroll
+          for (int part = 0; part < 3; ++part) out[(u * 3 + part) * 2] = u32x2{parts[part][0], parts[part][1]};
+        }
       }
     }
   };
   for (int item = item_first; item < item_end; item = next_item(item)) {
     locate(item, pi, me);
-    f32x4 acc[4][TM];
+    f32x4 acc[TN][TM], low[TN][TM];  // sums of x0 w0 and of the five small products
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < TN; ++j)
 #pragma unroll
-      for (int i = 0; i < TM; ++i) acc[j][i] = f32x4{0, 0, 0, 0};
+      for (int i = 0; i < TM; ++i) acc[j][i] = low[j][i] = f32x4{0, 0, 0, 0};
     const int stages = me.kt_end - me.kt_begin;
     const int16v sp = ((const int16v MG_CONSTANT *)p.split_phases)[uniform(pi)];  // see SplitPhase
     const int window = sp[9];  // taps of the inner window
@@ -252,12 +274,12 @@ __global__ void __launch_bounds__(64 * MW * NW, 2) split_gemm_kernel(const GemmP
 
     // ---- this lane's positions: their row in the patch and the taps they have (bit by bit; none beyond the last position)
     const int first_row = first_of(me);
-    int row_at[4];
-    unsigned taps[4];
+    int row_at[TN];
+    unsigned taps[TN];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < TN; ++j) {
       typedef int int2v __attribute__((ext_vector_type(2)));
-      const int ipos = me.pos0 + wave * 64 + j * 16 + l16;
+      const int ipos = me.pos0 + wave * WN + j * 16 + l16;
       const int2v at = __builtin_bit_cast(int2v, __builtin_amdgcn_raw_buffer_load_b64(table_buf, (int)((unsigned)ipos * 8u), 0, 0));
       row_at[j] = at[0] - first_row;
       taps[j] = (unsigned)at[1];
@@ -319,28 +341,28 @@ __global__ void __launch_bounds__(64 * MW * NW, 2) split_gemm_kernel(const GemmP
         }
       }
     };
-    int x_at[4], x_next[4];  // of the step under way and the one after it: 16-byte pieces from the start of the patch
+    int x_at[TN], x_next[TN];  // of the step under way and the one after it: 16-byte pieces from the start of the patch
     // tap0: number of the window's first tap; q: first tap of the step within it; lead: rows of the patch ahead of the tile's first one
     auto place = [&](int tap0, int q, bool single, int lead) {
       const int off0 = __builtin_amdgcn_readlane(inner, q), off1 = __builtin_amdgcn_readlane(inner, single ? q : q + 1);
       const int off = (second ? off1 : off0) + lead;
       const unsigned tap = (unsigned)(tap0 + q + (!single && second ? 1 : 0));
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int j = 0; j < TN; ++j) {
         const int keep = __builtin_amdgcn_sbfe((int)taps[j], tap, 1u);  // all ones where the position has the tap
         x_next[j] = (((row_at[j] + off - p.patch_rows) & keep) + p.patch_rows + (lk & 1) * octet_rows) * 3;
       }
     };
     auto enter_step = [&] {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) x_at[j] = x_next[j];
+      for (int j = 0; j < TN; ++j) x_at[j] = x_next[j];
     };
     auto read_position = [&](int j, bool single, bf16x8(&x)[3]) {
       const u32x4 *mine = patch + x_at[j];
-      if (single) {  // parts 2 | 0, 1 | 1, 0 | 0
+      if (single) {  // parts 2 | 0, 1 | 1, 0 | nothing
         x[0] = __builtin_bit_cast(bf16x8, mine[second ? 0 : 2]);
         x[1] = __builtin_bit_cast(bf16x8, mine[1]);
-        x[2] = __builtin_bit_cast(bf16x8, mine[0]);
+        x[2] = __builtin_bit_cast(bf16x8, *(second ? patch + p.patch_rows * 3 : mine));
       } else {
 #pragma unroll
         for (int part = 0; part < 3; ++part) x[part] = __builtin_bit_cast(bf16x8, mine[part]);
@@ -353,13 +375,14 @@ __global__ void __launch_bounds__(64 * MW * NW, 2) split_gemm_kernel(const GemmP
     int step_no = 0;
     auto step = [&](auto single_c, auto turn_c, auto single_next_c, int half_after, int tap0_next, int q_next, int lead_next, int stage, int parts) {
       constexpr bool SINGLE = decltype(single_c)::value, TURN = decltype(turn_c)::value, NEXT = decltype(single_next_c)::value;
-      constexpr int PRODUCTS = SINGLE ? 3 : 6;
-      constexpr int PX[6] = {SINGLE ? 0 : 2, SINGLE ? 1 : 0, SINGLE ? 2 : 1, 1, 0, 0}, PW[6] = {0, SINGLE ? 1 : 2, 1, 0, 1, 0};  // smallest first
+      // smallest first; x0 w0 alone into the sum of large products, for a sum of a few of those is exact
+      constexpr int PRODUCTS = SINGLE ? 4 : 6;
+      constexpr int PX[6] = {SINGLE ? 0 : 2, SINGLE ? 1 : 0, SINGLE ? 2 : 1, SINGLE ? 2 : 1, 0, 0}, PW[6] = {0, SINGLE ? 1 : 2, 1, 0, 1, 0};
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if (j < 3) {
+      for (int j = 0; j < TN; ++j) {
+        if (j + 1 < TN) {
           read_position(j + 1, SINGLE, x[(j + 1) % 2]);
-          if (j == 2) place(tap0_next, q_next, NEXT, lead_next);
+          if (j + 2 == TN) place(tap0_next, q_next, NEXT, lead_next);
         } else {
           park_filters((step_no + 1) & 1);
           __syncthreads();  // the next step's filters are there; nobody reads this one's patch any more
@@ -375,7 +398,7 @@ __global__ void __launch_bounds__(64 * MW * NW, 2) split_gemm_kernel(const GemmP
             if (stage + 1 < stages) park_patch();
           } else {
             enter_step();
-            read_position(0, NEXT, x[0]);
+            read_position(0, NEXT, x[TN % 2]);
           }
         }
 #pragma unroll
@@ -383,20 +406,25 @@ __global__ void __launch_bounds__(64 * MW * NW, 2) split_gemm_kernel(const GemmP
 #pragma unroll
           for (int t = 0; t < PRODUCTS; ++t)
 #pragma unroll
-            for (int i = i0; i < TM && i < i0 + 2; ++i)
-              acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[j % 2][PX[t]], w[i][PW[t]], acc[j][i], 0, 0, 0);
-          if (j == 3) {
+            for (int i = i0; i < TM && i < i0 + 2; ++i) {
+              f32x4 &into = t + 1 < PRODUCTS ? low[j][i] : acc[j][i];
+              into = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[j % 2][PX[t]], w[i][PW[t]], into, 0, 0, 0);
+            }
+          if (j + 1 == TN) {
 #pragma unroll
             for (int i = i0; i < TM && i < i0 + 2; ++i) read_filters((step_no + 1) & 1, i, NEXT);
           }
         }
-        if (j < 3) __builtin_amdgcn_sched_barrier(0);
+        if (j + 1 < TN) __builtin_amdgcn_sched_barrier(0);
       }
       if constexpr (TURN) {
         __syncthreads();
         enter_step();
         read_position(0, NEXT, x[0]);
         if (stage + 1 < stages) aim(stage + 1);
+      } else if constexpr (TN % 2 != 0) {
+#pragma unroll
+        for (int part = 0; part < 3; ++part) x[0][part] = x[1][part];
       }
       ++step_no;
     };
@@ -449,7 +477,11 @@ __global__ void __launch_bounds__(64 * MW * NW, 2) split_gemm_kernel(const GemmP
     // ---- epilogue: acc[j][i][q] is row m0 + wm0 + 16 i + l16 at position pos0 + 64 wave + 16 j + 4 lk + q
     bool odd = false;
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int i = 0; i < TM; ++i) acc[j][i] += low[j][i];
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -459,13 +491,13 @@ __global__ void __launch_bounds__(64 * MW * NW, 2) split_gemm_kernel(const GemmP
     if (odd) p.split_flags->rerun = 1;
 
     const Phase &ph = me.ph;
-    const int first = me.pos0 + wave * 64 + lk * 4;
+    const int first = me.pos0 + wave * WN + lk * 4;
     if (me.partial) {
-      float *slot = static_cast<float *>(p.partial) + (long long)me.slot * (BM * BN) + wave * 64 + lk * 4;
+      float *slot = static_cast<float *>(p.partial) + (long long)me.slot * (BM * BN) + wave * WN + lk * 4;
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) *reinterpret_cast<f32x4 *>(slot + (wm0 + i * 16 + l16) * BN + j * 16) = acc[j][i];
+        for (int j = 0; j < TN; ++j) *reinterpret_cast<f32x4 *>(slot + (wm0 + i * 16 + l16) * BN + j * 16) = acc[j][i];
       continue;
     }
     const int j12 = ph.J[1] * ph.J[2];
@@ -482,7 +514,7 @@ __global__ void __launch_bounds__(64 * MW * NW, 2) split_gemm_kernel(const GemmP
              (long long)(ph.o0[1] + j1 * p.oj[1]) * p.os[1] + (long long)(ph.o0[2] + j2 * p.oj[2]) * p.os[2];
     };
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < TN; ++j) {
       const int four = first + j * 16;
       if (four >= ph.npos) continue;
       // four positions that are adjacent in dst leave as one vector, aligned or not (see GemmParams::run_store)
@@ -564,36 +596,40 @@ __global__ void __launch_bounds__(256) split_positions_kernel(const SplitPositio
   out[idx] = int2{n * p.sample_rows + (q0 * p.Q[1] + q1) * p.Q[2] + q2, (int)taps};
 }
 
-// rows of a wave; waves along the rows and the positions of a tile
-#define MG_SPLIT_SHAPES(X) X(64, 2, 2) X(48, 2, 2) X(64, 1, 4) X(64, 1, 2) X(48, 1, 4) X(32, 1, 4) X(16, 1, 4)
+// rows of a wave; waves along the rows of a tile; 16 positions of a wave; waves along the positions; rounds of a patch (the fewest that hold it)
+#define MG_SPLIT_SHAPES(X) \
+  X(32, 4, 4, 2, 1) X(64, 1, 3, 4, 2) X(32, 2, 4, 2, 1) X(32, 2, 4, 2, 2) X(48, 1, 4, 4, 2) X(32, 1, 4, 4, 2) X(16, 1, 4, 4, 2)
 
-template <int WM, int MW, int NW>
-size_t lds_bytes(int patch_rows) {
-  return (size_t)(2 * 12 * WM * MW + 2 * (patch_rows + 1) * 3) * 16;
+// Rows of a patch that a tile has room for: those of its threads' rounds, and two blocks share a unit's LDS (alone on
+// it, a block's waves wait for their barriers: 256 filters, 3x3, stride 2, 27x27 161 us on patches of 540 rows, 134 on the other kernel).
+constexpr int patch_limit(int bm, int threads, int rounds) {
+  const int held = threads * rounds, room = (80 * 1024 / 16 - 24 * bm) / 6 - 1;
+  return held < room ? held : room;
 }
+
+size_t lds_bytes(int bm, int patch_rows) { return (size_t)(2 * 12 * bm + 2 * (patch_rows + 1) * 3) * 16; }
 
 }  // namespace
 
-// Rows of a patch that a tile has room for: a thread takes eight channels of four rows, and two blocks share a unit's LDS (alone on
-// it, a block's waves wait for their barriers: 256 filters, 3x3, stride 2, 27x27 161 us on patches of 540 rows, 134 on the other kernel).
 int split_patch_limit(int bm, int bn) {
-#define MG_LIMIT(WM, MW, NW) \
-  if (bm == WM * MW && bn == 64 * NW) return std::min(64 * MW * NW * 2, (int)(80 * 1024 / 16 - 24 * WM * MW) / 6 - 1);
+  int most = 0;
+#define MG_LIMIT(WM, MW, TN, NW, ROUNDS) \
+  if (bm == WM * MW && bn == 16 * TN * NW) most = std::max(most, patch_limit(bm, 64 * MW * NW, ROUNDS));
   MG_SPLIT_SHAPES(MG_LIMIT)
 #undef MG_LIMIT
-  return 0;
+  return most;
 }
 
 int split_gemm_blocks_per_cu(int bm, int bn, int patch_rows) {
   static std::map<std::array<int, 3>, int> known;  // (behind the lock of the entry points)
   int &n = known[{bm, bn, patch_rows}];
   if (n > 0) return n;
-#define MG_OCC(WM, MW, NW)                                                                                                              \
-  if (bm == WM * MW && bn == 64 * NW) {                                                                                                 \
-    const size_t bytes = lds_bytes<WM, MW, NW>(patch_rows);                                                                             \
-    (void)hipFuncSetAttribute((const void *)split_gemm_kernel<WM, MW, NW, true>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);  \
-    (void)hipFuncSetAttribute((const void *)split_gemm_kernel<WM, MW, NW, false>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); \
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, split_gemm_kernel<WM, MW, NW, true>, 64 * MW * NW, bytes) != hipSuccess) n = 0; \
+#define MG_OCC(WM, MW, TN, NW, ROUNDS)                                                                                     \
+  if (n == 0 && bm == WM * MW && bn == 16 * TN * NW && patch_rows <= patch_limit(bm, 64 * MW * NW, ROUNDS)) {              \
+    const auto odd = split_gemm_kernel<WM, MW, TN, NW, ROUNDS, true>, even = split_gemm_kernel<WM, MW, TN, NW, ROUNDS, false>; \
+    for (const auto kernel : {odd, even})                                                                                  \
+      (void)hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);             \
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, odd, 64 * MW * NW, lds_bytes(bm, patch_rows)) != hipSuccess) n = 0; \
   }
   MG_SPLIT_SHAPES(MG_OCC)
 #undef MG_OCC
@@ -605,13 +641,11 @@ int split_gemm_blocks_per_cu(int bm, int bn, int patch_rows) {
 }
 
 bool launch_split_gemm(const GemmParams &p, int bm, int bn, bool odd, unsigned grid, hipStream_t s) {
-#define MG_LAUNCH(WM, MW, NW)                                                                                                                  \
-  if (bm == WM * MW && bn == 64 * NW) {                                                                                                        \
-    if (odd)                                                                                                                                   \
-      hipLaunchKernelGGL((split_gemm_kernel<WM, MW, NW, true>), dim3(grid), dim3(64 * MW * NW), (lds_bytes<WM, MW, NW>(p.patch_rows)), s, p);  \
-    else                                                                                                                                       \
-      hipLaunchKernelGGL((split_gemm_kernel<WM, MW, NW, false>), dim3(grid), dim3(64 * MW * NW), (lds_bytes<WM, MW, NW>(p.patch_rows)), s, p); \
-    return true;                                                                                                                               \
+#define MG_LAUNCH(WM, MW, TN, NW, ROUNDS)                                                                                              \
+  if (bm == WM * MW && bn == 16 * TN * NW && p.patch_rows <= patch_limit(bm, 64 * MW * NW, ROUNDS)) {                                  \
+    const auto kernel = odd ? split_gemm_kernel<WM, MW, TN, NW, ROUNDS, true> : split_gemm_kernel<WM, MW, TN, NW, ROUNDS, false>;      \
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * MW * NW), lds_bytes(bm, p.patch_rows), s, p);                                     \
+    return true;                                                                                                                       \
   }
   MG_SPLIT_SHAPES(MG_LAUNCH)
 #undef MG_LAUNCH

@@ -1427,8 +1427,8 @@ def test_per_launch_timing_records_chains_and_pauses():
 # extents, so that row ends and sample ends fall inside tiles; channels and filters that fill no 16.
 SPLIT_PROBLEMS = [
     ((3, 32, 29, 27), (160, 32, 3, 3), (1, 1), (1, 1), "128,128"),           # odd window; a quarter row tile
-    ((9, 45, 31, 33), (101, 45, 2, 3), (1, 2), (1, 1), "96,128"),            # even window, ragged counts
-    ((2, 16, 23, 300), (64, 16, 3, 3), (1, 1), (1, 1), "64,256"),            # rows longer than a tile: stages of one row of taps
+    ((9, 45, 31, 33), (101, 45, 2, 3), (1, 2), (1, 1), "64,192"),            # even window, ragged counts
+    ((2, 16, 23, 300), (64, 16, 3, 3), (1, 1), (1, 1), "48,256"),            # rows longer than a tile: stages of one row of taps
     ((17, 61, 13, 13), (64, 61, 5, 5), (2, 2), (1, 2), "64,128"),             # the tiles of several samples; dilation
     ((2, 48, 5000), (48, 48, 8), (3,), (2,), "48,256"),                      # one axis, even window
     ((310, 24, 7, 7), (32, 24, 3, 3), (2, 2), (2, 2), "32,256"),              # planes of 49: samples rounded up to whole loads
@@ -1438,19 +1438,19 @@ SPLIT_PROBLEMS = [
     ((37, 32, 61), (80, 32, 9), (0,), (2,), ""),                             # its rows along every axis, and samples overlap in them
     ((3, 32, 9, 11, 12), (48, 32, 3, 3, 3), (1, 0, 0), (1, 1, 2), ""),
     ((2, 512, 6, 5), (512, 512, 3, 3), (1, 1), (1, 1), ""),                  # every tile shared out
+    ((7, 45, 27, 31), (70, 45, 3, 3), (1, 1), (1, 1), "64,192"),             # odd window
+    ((2, 32, 70, 75), (64, 32, 3, 3), (1, 1), (1, 1), "64,128"),             # patches of more rows than threads
 ]
 
 
-@pytest.mark.parametrize("problem", range(len(SPLIT_PROBLEMS)))
-def test_products_of_three_bf16_parts(abi, monkeypatch, problem):
+def _split_passes(abi, monkeypatch, problem):
+    """passes(x, w, g, split=True): forward pass and data gradient of a problem, on split operands or without."""
     from mygrad_amd import _hip
 
-    x_shape, w_shape, p, d, tile = SPLIT_PROBLEMS[problem]
+    x_shape, _, p, d, tile = SPLIT_PROBLEMS[problem]
     s = (1,) * len(p)
-    rng = np.random.default_rng(3100 + problem)
 
     def passes(x, w, g, split=True):
-        """Forward pass and data gradient, and whether both ran on split operands."""
         with monkeypatch.context() as m:
             m.setenv("MYGRAD_HIP_TINY", "0")
             m.setenv("MYGRAD_HIP_SPLIT_MIN", "0")
@@ -1463,8 +1463,19 @@ def test_products_of_three_bf16_parts(abi, monkeypatch, problem):
             plans.append(_hip.last_plan())
         print(*plans, sep="\n", flush=True)
         for plan in plans:
-            assert plan.endswith("three bf16 parts") == split and tile.replace(",", "x") in plan
+            assert plan.endswith("three bf16 parts") == split
+            assert not split or tile.replace(",", "x") in plan
         return out, dx
+
+    return passes
+
+
+@pytest.mark.parametrize("problem", range(len(SPLIT_PROBLEMS)))
+def test_products_of_three_bf16_parts(abi, monkeypatch, problem):
+    x_shape, w_shape, p, d, _ = SPLIT_PROBLEMS[problem]
+    s = (1,) * len(p)
+    rng = np.random.default_rng(3100 + problem)
+    passes = _split_passes(abi, monkeypatch, problem)
 
     # small integers: every sum is exact
     xi, wi = rng.integers(-3, 4, x_shape).astype(np.float32), rng.integers(-2, 3, w_shape).astype(np.float32)
@@ -1502,3 +1513,36 @@ def test_products_of_three_bf16_parts(abi, monkeypatch, problem):
             assert np.array_equal(bits(got), bits(plain))
     again = passes(xi, wi, gi)
     assert np.array_equal(bits(again[0]), bits(out)) and np.array_equal(bits(again[1]), bits(dx))
+
+
+@pytest.mark.parametrize("problem", [0, 1, 3, 5, 8, 11, 12])
+def test_products_of_three_bf16_parts_keep_single_precision(abi, monkeypatch, problem):
+    """Sums of few terms, where an error that long dense sums hide would show."""
+    x_shape, w_shape, p, d, _ = SPLIT_PROBLEMS[problem]
+    s = (1,) * len(p)
+    rng = np.random.default_rng(3200 + problem)
+    passes = _split_passes(abi, monkeypatch, problem)
+    normal = lambda shape: rng.standard_normal(shape).astype(np.float32)
+    x, w = normal(x_shape), normal(w_shape)
+    g = normal(direct.conv_forward(x, w, s, p, d).shape)
+
+    def exact(x, w, g):
+        x, w, g = (a.astype(np.float64) for a in (x, w, g))
+        return direct.conv_forward(x, w, s, p, d), direct.conv_backward_x(g, x_shape, w, s, p, d)
+
+    # one tap of one channel per filter, and no channel twice: every sum is one product.  What the six products leave out is at
+    # most 2^-24 of it (second parts of at most 2^-8 and third ones of 2^-17 of their values), x0 w0 is exact, the five small products
+    # round off 2^-29 each and their sum with x0 w0 2^-24
+    few = np.zeros_like(w)
+    for f in range(min(w_shape[:2])):
+        at = np.unravel_index(f * 7 % np.prod(w_shape[2:]), w_shape[2:])
+        few[(f, f, *at)] = w[(f, f, *at)]
+    for got, ref in zip(passes(x, few, g), exact(x, few, g)):
+        assert np.all(np.abs(got - ref) <= (2 + 5 / 32) * 2.0**-24 * np.abs(ref))
+    # dense, behind a relu, and few values not zero: a sum of large products rounds off once in a step, of 32 terms or of 16 under an odd
+    # tap, 5.06e-8 of itself each time (see above), the rest 3.5e-8.  (All six products in one sum: twice as much.)
+    for share in (1.0, 0.5, 0.02):
+        xs, gs = (np.where(rng.random(a.shape) < share, a if share == 1.0 else np.abs(a), np.float32(0)) for a in (x, g))
+        for got, ref, count in zip(passes(xs, w, gs), exact(xs, w, gs), (w_shape[1], w_shape[0])):
+            steps = -(-count // 16) * (np.prod(w_shape[2:]) + 1) / 2
+            assert np.linalg.norm(got - ref) <= (1.25 * 5.06e-8 * np.sqrt(steps / 2) + 3.5e-8) * np.linalg.norm(ref)
