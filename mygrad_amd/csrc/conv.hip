@@ -89,10 +89,7 @@ __global__ void __launch_bounds__(256) pack_phase_rows_kernel(const T *__restric
 template <typename T>
 __global__ void __launch_bounds__(256) pack_filters_kernel(const T *__restrict__ w, T *__restrict__ ap, int F, int C,
                                                            int wvol, int mode, int ld, int depth, SplitFlags *gate) {
-  if (gate != nullptr) {  // behind a pass of conv_split.hip
-    if (blockIdx.x == 0 && threadIdx.x == 0) gate->filters = 0;
-    if (gate->rerun == 0) return;
-  }
+  if (gate != nullptr && gate->rerun == 0) return;  // behind a pass of conv_split.hip
   const int M = (mode == 2 || mode == 6) ? F : mode == 3 ? C : mode == 4 ? 3 * C : 3 * F;
   const int total = (mode == 4 || mode == 5 ? wvol / 3 : wvol) * depth * ld;
   for (int idx = blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += gridDim.x * blockDim.x) {

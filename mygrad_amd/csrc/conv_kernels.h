@@ -103,8 +103,8 @@ static_assert(sizeof(SplitPhase) == 64, "read as one 64-byte row");
 
 // What a pass of conv_split.hip finds out about its operands.
 struct SplitFlags {
-  int rerun;    // the single-precision kernels have to do the pass; cleared when a pass packs its filters
-  int filters;  // of the filters being packed; cleared by the gated pack_filters_kernel at the end of a pass
+  int rerun;  // the single-precision kernels have to do the pass; cleared when a pass packs its filters
+  int pad_;
 };
 
 // Gather-GEMM:  dst[n, m, pos] = sum_k A(k, m) * src[n, row k, pos]

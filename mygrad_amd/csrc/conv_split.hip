@@ -26,11 +26,11 @@
 //
 // What the split cannot represent is left to the single-precision kernels.  An infinite operand leaves Inf - Inf in
 // its second part and makes every sum that it takes part in a NaN, as an infinite or NaN operand or an overflow makes
-// it something not finite in any arithmetic.  The low parts of operands below 2^-102 may fall under the smallest
-// numbers that the instruction takes, 2^-126: against a sum of 2^-70 or more, K terms of at most 2^16 * 2^-126 are less
-// than its last bit for every K up to 2^16.  So a flag is set by a wave that holds a sum that is not finite, or not
-// zero and below 2^-70; where a filter value is above 2^16; and where one is below 2^-100 and an element of src above
-// 2^16.  The single-precision kernels are launched behind this one and return at once unless it is set: they then
+// it something not finite in any arithmetic.  And parts are multiples of 2^-133, the smallest number of bf16 (which the instruction takes as
+// it is, like every product and sum below 2^-126): of an operand below 2^-110 bits may be lost, below 2^-134 all of them.  K such losses
+// times the largest value of the other operand are less than the last bit of a sum of K * 2^-109 times that value.  So a block that has
+// a sum that is not finite, or has lost bits of an element or seen a filter value below 2^-109 and has a sum, zero included, below that bound, sets
+// a flag.  The single-precision kernels are launched behind this one and return at once unless it is set: they then
 // do the whole pass, and its result is theirs.
 #include "conv_device.h"
 #include "conv_kernels.h"
@@ -47,6 +47,7 @@ namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
@@ -67,35 +68,19 @@ __device__ __forceinline__ float float_of(unsigned v) { return __builtin_bit_cas
 // none): x1 is at most 2^-8 of x and x2 2^-17, so what the six products leave out, x1 w2 + x2 w1 + x2 w2, is at most 2^-24 of x w and
 // has no sign of its own (with the first part cut off instead it was up to 2^-22).  A value that rounds to infinity leaves a
 // NaN in its second part.  Eleven vector instructions for two values.
-__device__ __forceinline__ void split_pair(float a, float b, unsigned &h, unsigned &m, unsigned &l) {
+// The low sixteen bits of `lost` are set where the last part has lost some (see the head of the file).
+__device__ __forceinline__ void split_pair(float a, float b, unsigned &h, unsigned &m, unsigned &l, unsigned &lost) {
   h = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{a, b}), bf16x2));
   const float ra = a - float_of(h << 16), rb = b - float_of(h & 0xffff0000u);
   m = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{ra, rb}), bf16x2));
   const float qa = ra - float_of(m << 16), qb = rb - float_of(m & 0xffff0000u);
   l = __builtin_amdgcn_perm(bits_of(qb), bits_of(qa), 0x07060302u);
+  lost |= bits_of(qa) | bits_of(qb);
 }
 
-__device__ __forceinline__ void split_eight(const float (&v)[8], bf16x8 (&parts)[3]) {
-  u32x4 h, m, l;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    unsigned a, b, c;
-    split_pair(v[2 * e], v[2 * e + 1], a, b, c);
-    h[e] = a, m[e] = b, l[e] = c;
-  }
-  parts[0] = __builtin_bit_cast(bf16x8, h);
-  parts[1] = __builtin_bit_cast(bf16x8, m);
-  parts[2] = __builtin_bit_cast(bf16x8, l);
-}
-
-// (see the head of the file) not finite, or not zero and below 2^-70
-__device__ __forceinline__ bool suspect(float v) {
-  constexpr unsigned low = 2u * (57u << 23), high = 2u * (255u << 23);  // 2^-70 and Inf, without their sign bit
-  const unsigned u = bits_of(v) << 1;
-  return u != 0 && u - low >= high - low;
-}
-constexpr float kWide = 0x1p16f, kTiny = 0x1p-100f;  // operands: see the head of the file
-enum : int { kTinyFilter = 1, kWideFilter = 2 };     // SplitFlags::filters
+// What a block finds out about an item's operands and sums, bit by bit.
+enum : unsigned { kNotFinite = 1, kLostElement = 2, kTinyFilter = 4, kLostSum = 8 };
+constexpr unsigned short kTinyBits = 18 << 7;  // 2^-109 in bf16
 
 __device__ __forceinline__ Phase load_phase(const Phase *phases, int i) {
   const int8v MG_CONSTANT *q = (const int8v MG_CONSTANT *)(phases + uniform(i));
@@ -130,12 +115,12 @@ __device__ __forceinline__ int phase_first_block(const Phase *phases, int i) {
 // split and laid out in the order of the stages beforehand (split_pack_kernel), pass through LDS two steps ahead of their use.
 // Blocks are persistent, as in tap_gemm_kernel.
 template <int WM, int MW, int TN, int NW, int ROUNDS, bool ODD>
-__global__ void __launch_bounds__(64 * MW * NW, 2) split_gemm_kernel(const GemmParams p) {
+__global__ void __launch_bounds__(64 * MW * NW, WM == 16 ? 3 : 2) split_gemm_kernel(const GemmParams p) {
   constexpr int BM = WM * MW, WN = 16 * TN, BN = WN * NW, TM = WM / 16, THREADS = 64 * MW * NW;
   static_assert(WM % 16 == 0, "16 x 16 tiles");
   constexpr int PIECES = 12 * BM;  // of 16 bytes: a step's filters, [part][octet of K rows][row]
   constexpr int ALOADS = (PIECES + THREADS - 1) / THREADS;
-  // [2][PIECES] filters, then the patch: [octet of channels][row][part], p.patch_rows + 1 rows, the last one zeros
+  // [2][PIECES] filters, then the patch: [octet of channels][row][part], p.patch_rows + 1 rows, the last one zeros; and three words (note)
   extern __shared__ __attribute__((aligned(16))) u32x4 lds[];
   u32x4 *const patch = lds + 2 * PIECES;
 
@@ -149,7 +134,9 @@ __global__ void __launch_bounds__(64 * MW * NW, 2) split_gemm_kernel(const GemmP
     bool partial;
     Phase ph;
   };
-  float widest = 0.0f;  // |element of src| among those this lane has split
+  // of the item, this lane's: bits lost of the elements that it has split, the smallest |filter value| that it has parked, less one (zeros aside)
+  unsigned lost = 0;
+  u16x2 tiniest = {0xffff, 0xffff};
   const bool shares = p.share_first != nullptr;
   const int share_begin = shares ? ((const int MG_CONSTANT *)p.share_first)[uniform((int)blockIdx.x)] : 0;
   const int share_end = shares ? ((const int MG_CONSTANT *)p.share_first)[uniform((int)blockIdx.x) + 1] : 0;
@@ -205,6 +192,7 @@ __global__ void __launch_bounds__(64 * MW * NW, 2) split_gemm_kernel(const GemmP
   const unsigned piece_row = (unsigned)p.a_ld * 16u;  // bytes of one part of one octet of packed filters
   const unsigned c_step = (unsigned)p.src_cstride * 4u;
   const int octet_rows = p.patch_rows + 1;
+  unsigned *const note = reinterpret_cast<unsigned *>(patch + 2 * octet_rows * 3);  // what was found, the widest filter value, the widest element
   if (threadIdx.x < 6) patch[((int)threadIdx.x / 3 * octet_rows + p.patch_rows) * 3 + (int)threadIdx.x % 3] = u32x4{0, 0, 0, 0};
   float *__restrict__ dst = static_cast<float *>(p.dst);
   int pi = 0;
@@ -229,7 +217,7 @@ __global__ void __launch_bounds__(64 * MW * NW, 2) split_gemm_kernel(const GemmP
     const int row = ((patch_row + patch_e[2]) & ~3) + (idx - quarter * quads) * 4;
     const unsigned n = __umulhi((unsigned)max(row, 0), p.by_sample.mul) >> p.by_sample.shr;  // (more than one row to a sample)
     unsigned at = (n * (unsigned)p.src_nstride + (unsigned)(row - (int)n * p.sample_rows + patch_e[1] + quarter * 4 * p.src_cstride)) * 4u;
-    at = (idx < p.patch_rows) & (row >= 0) & ((int)n < p.samples) & patch_real ? at : kOutside;
+    at = ((idx < p.patch_rows) & (row >= 0) & ((int)n < p.samples) & patch_real) ? at : kOutside;
     const unsigned dead = (unsigned)patch_e[5] >> (quarter * 4);
 #pragma unroll
     for (int u = 0; u < CHANNELS; ++u) {
@@ -248,11 +236,9 @@ __global__ void __launch_bounds__(64 * MW * NW, 2) split_gemm_kernel(const GemmP
         float v[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) v[r] = float_of(raw[round][r][u]);
-#pragma unroll
-        for (int r = 0; r < 4; r += 2) widest = __builtin_fmaxf(__builtin_fmaxf(widest, __builtin_fabsf(v[r])), __builtin_fabsf(v[r + 1]));
         unsigned parts[3][2];
-        split_pair(v[0], v[1], parts[0][0], parts[1][0], parts[2][0]);
-        split_pair(v[2], v[3], parts[0][1], parts[1][1], parts[2][1]);
+        split_pair(v[0], v[1], parts[0][0], parts[1][0], parts[2][0], lost);
+        split_pair(v[2], v[3], parts[0][1], parts[1][1], parts[2][1], lost);
         if (idx < p.patch_rows) {
 #pragma unroll
           for (int part = 0; part < 3; ++part) out[(u * 3 + part) * 2] = u32x2{parts[part][0], parts[part][1]};
@@ -304,6 +290,12 @@ __global__ void __launch_bounds__(64 * MW * NW, 2) split_gemm_kernel(const GemmP
       for (int u = 0; u < ALOADS; ++u) {
         const int q = (int)threadIdx.x + THREADS * u;
         if (PIECES % THREADS == 0 || q < PIECES) lds[buf * PIECES + q] = areg[u];
+      }
+      static_assert(4 * BM <= THREADS, "first parts: the first piece of a thread");
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const u16x2 size = __builtin_bit_cast(u16x2, areg[0][e] & 0x7fff7fffu);
+        tiniest = __builtin_elementwise_min(tiniest, (u16x2)(size - u16x2{1, 1}));
       }
     };
     bf16x8 w[TM][3];
@@ -432,7 +424,9 @@ __global__ void __launch_bounds__(64 * MW * NW, 2) split_gemm_kernel(const GemmP
       const std::true_type yes;
       const std::false_type no;
       const int half0 = table[0][0];
-      __syncthreads();  // (the last item's operands have been read)
+      __syncthreads();  // (the last item's operands and notes have been read)
+      if (threadIdx.x < 3) note[threadIdx.x] = 0;
+      lost = 0, tiniest = u16x2{0xffff, 0xffff};
       request_filters(half0);
       if (!ahead) {
         patch_row = first_row, patch_e = table[0], patch_real = true;
@@ -475,23 +469,71 @@ __global__ void __launch_bounds__(64 * MW * NW, 2) split_gemm_kernel(const GemmP
     }
 
     // ---- epilogue: acc[j][i][q] is row m0 + wm0 + 16 i + l16 at position pos0 + 64 wave + 16 j + 4 lk + q
-    bool odd = false;
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
       for (int i = 0; i < TM; ++i) acc[j][i] += low[j][i];
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) odd |= suspect(acc[j][i][q]);
-    const int filters = p.split_flags->filters;
-    odd |= (filters & kWideFilter) != 0 || ((filters & kTinyFilter) != 0 && widest > kWide);
-    if (odd) p.split_flags->rerun = 1;
-
     const Phase &ph = me.ph;
     const int first = me.pos0 + wave * WN + lk * 4;
+    if (stages > 0) {
+      unsigned largest = 0;
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) largest = max(largest, bits_of(acc[j][i][q]) << 1);
+      const unsigned mine = (largest >= 2u * (255u << 23) ? kNotFinite : 0u) | ((lost & 0xffffu) != 0 ? kLostElement : 0u) |
+                            ((int)threadIdx.x < 4 * BM && min(tiniest[0], tiniest[1]) < kTinyBits - 1 ? kTinyFilter : 0u);
+      if (mine != 0) atomicOr(&note[0], mine);
+      __syncthreads();
+      unsigned found = (unsigned)uniform((int)note[0]);
+      if ((found & (kLostElement | kTinyFilter)) != 0 && (found & kNotFinite) == 0) {
+        // seldom: the largest value that meets one that has lost bits
+        unsigned widest = 0;
+        if ((found & kLostElement) != 0) {
+          for (int at = (int)threadIdx.x; at < stages * window * 2 * BM; at += THREADS) {
+            const u32x4 firsts = __builtin_amdgcn_raw_buffer_load_b128(
+                a_buf, me.m0 + at % BM < p.a_ld ? (int)((unsigned)((table[0][0] * 2 + at / BM) * 3) * piece_row + (unsigned)(me.m0 + at % BM) * 16u) : (int)kOutside, 0, 0);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) widest = max(widest, max((firsts[e] & 0x7fffu) << 16, firsts[e] & 0x7fff0000u));
+          }
+          atomicMax(&note[1], widest);
+        }
+        if ((found & kTinyFilter) != 0) {
+          widest = 0;
+          patch_row = first_row, patch_real = true;
+          for (int stage = 0; stage < stages; ++stage) {
+            patch_e = table[stage];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) request_part(k);
+#pragma unroll
+            for (int round = 0; round < ROUNDS; ++round)
+              if (round * THREADS < p.patch_rows) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) widest = max(widest, raw[round][r / 4][r % 4] & 0x7fffffffu);
+              }
+          }
+          ahead = false;  // (the next item's first patch was there)
+          atomicMax(&note[2], widest);
+        }
+        __syncthreads();
+        const float bound = (float_of(note[1]) + float_of(note[2])) * (float)(stages * window * 16) * 0x1.02p-109f;  // (first parts are rounded)
+        bool below = false;
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+              below |= me.m0 + wm0 + i * 16 + l16 < p.M && first + j * 16 + q < ph.npos && __builtin_fabsf(acc[j][i][q]) < bound;
+        if (below) atomicOr(&note[0], (unsigned)kLostSum);
+        __syncthreads();
+        found = (unsigned)uniform((int)note[0]);
+      }
+      if ((found & (kNotFinite | kLostSum)) != 0) p.split_flags->rerun = 1;
+    }
+
     if (me.partial) {
       float *slot = static_cast<float *>(p.partial) + (long long)me.slot * (BM * BN) + wave * WN + lk * 4;
 #pragma unroll
@@ -550,8 +592,8 @@ __global__ void __launch_bounds__(64 * MW * NW, 2) split_gemm_kernel(const GemmP
 // The filters of split_gemm_kernel, in three parts: piece [octet of K rows][part][m] holds the eight bf16
 // values of K rows 8 * octet .. + 7 of row m of the product, `ld` (a multiple of 16) pieces to a row.  Sixteen K rows
 // are 16 channels from c0 on under one tap, named by halves[K row / 16] = (c0, tap): row m's value is w[m * m_stride + c * c_stride + tap],
-// zero for c >= channels and m >= M.  Also clears
-// the flag that split_gemm_kernel may set, and notes filters out of the range it can represent.
+// zero for c >= channels and m >= M.  A value that is not zero has a first part that is not, the smallest number of bf16 at least: that is how
+// split_gemm_kernel knows of those that have lost bits.  Also clears the flag that it may set.
 __global__ void __launch_bounds__(256) split_pack_kernel(const float *__restrict__ w, u32x4 *__restrict__ packed, const int2 *__restrict__ halves,
                                                          int count, SplitFlags *flags, int M, int channels, long long m_stride, long long c_stride, int ld) {
   if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) flags->rerun = 0;
@@ -559,21 +601,23 @@ __global__ void __launch_bounds__(256) split_pack_kernel(const float *__restrict
   if (oct >= 2 * count) return;
   const int2 h = halves[oct / 2];
   const int c0 = h.x + oct % 2 * 8;
-  float v[8];
+  u32x4 parts[3];
 #pragma unroll
-  for (int e = 0; e < 8; ++e)
-    v[e] = m < M && c0 + e < channels ? w[(long long)m * m_stride + (long long)(c0 + e) * c_stride + h.y] : 0.0f;
-  int found = 0;
+  for (int e = 0; e < 4; ++e) {
+    float v[2];
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const float a = __builtin_fabsf(v[e]);
-    found |= a > kWide ? kWideFilter : a < kTiny && a != 0.0f ? kTinyFilter : 0;
+    for (int u = 0; u < 2; ++u) {
+      const int c = c0 + 2 * e + u;
+      v[u] = m < M && c < channels ? w[(long long)m * m_stride + (long long)c * c_stride + h.y] : 0.0f;
+    }
+    unsigned first, second, third, lost = 0;
+    split_pair(v[0], v[1], first, second, third, lost);
+    if (v[0] != 0.0f && (first & 0x7fffu) == 0) first |= 1u;
+    if (v[1] != 0.0f && (first & 0x7fff0000u) == 0) first |= 1u << 16;
+    parts[0][e] = first, parts[1][e] = second, parts[2][e] = third;
   }
-  if (found != 0) atomicOr(&flags->filters, found);
-  bf16x8 parts[3];
-  split_eight(v, parts);
 #pragma unroll
-  for (int part = 0; part < 3; ++part) packed[((long long)oct * 3 + part) * ld + m] = __builtin_bit_cast(u32x4, parts[part]);
+  for (int part = 0; part < 3; ++part) packed[((long long)oct * 3 + part) * ld + m] = parts[part];
 }
 
 // (row, taps) of every position: the row of src (sample * sample_rows + element of a channel's plane) that its window starts
@@ -581,7 +625,7 @@ __global__ void __launch_bounds__(256) split_pack_kernel(const float *__restrict
 __global__ void __launch_bounds__(256) split_positions_kernel(const SplitPositions p, SplitFlags *flags) {
   int2 *const out = reinterpret_cast<int2 *>(flags + 1);
   const int idx = blockIdx.x * 256 + threadIdx.x;
-  if (idx == 0) flags->rerun = flags->filters = 0;
+  if (idx == 0) flags->rerun = 0;
   if (idx >= p.npos) return;
   const int j12 = p.J[1] * p.J[2], n = idx / (p.J[0] * j12), r = idx - n * p.J[0] * j12;
   const int q0 = r / j12, q1 = r / p.J[2] % p.J[1], q2 = r % p.J[2];
@@ -603,11 +647,11 @@ __global__ void __launch_bounds__(256) split_positions_kernel(const SplitPositio
 // Rows of a patch that a tile has room for: those of its threads' rounds, and two blocks share a unit's LDS (alone on
 // it, a block's waves wait for their barriers: 256 filters, 3x3, stride 2, 27x27 161 us on patches of 540 rows, 134 on the other kernel).
 constexpr int patch_limit(int bm, int threads, int rounds) {
-  const int held = threads * rounds, room = (80 * 1024 / 16 - 24 * bm) / 6 - 1;
+  const int held = threads * rounds, room = (80 * 1024 / 16 - 24 * bm - 1) / 6 - 1;
   return held < room ? held : room;
 }
 
-size_t lds_bytes(int bm, int patch_rows) { return (size_t)(2 * 12 * bm + 2 * (patch_rows + 1) * 3) * 16; }
+size_t lds_bytes(int bm, int patch_rows) { return (size_t)(2 * 12 * bm + 2 * (patch_rows + 1) * 3 + 1) * 16; }
 
 }  // namespace
 
