@@ -24,7 +24,6 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
-#include <memory>
 #include <string>
 #include <vector>
 
@@ -88,8 +87,7 @@ __global__ void __launch_bounds__(256) pack_phase_rows_kernel(const T *__restric
 
 template <typename T>
 __global__ void __launch_bounds__(256) pack_filters_kernel(const T *__restrict__ w, T *__restrict__ ap, int F, int C,
-                                                           int wvol, int mode, int ld, int depth, SplitFlags *gate) {
-  if (gate != nullptr && gate->rerun == 0) return;  // behind a pass of conv_split.hip
+                                                           int wvol, int mode, int ld, int depth) {
   const int M = (mode == 2 || mode == 6) ? F : mode == 3 ? C : mode == 4 ? 3 * C : 3 * F;
   const int total = (mode == 4 || mode == 5 ? wvol / 3 : wvol) * depth * ld;
   for (int idx = blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += gridDim.x * blockDim.x) {
@@ -581,9 +579,7 @@ struct Plan {
   int2 *split_halves = nullptr;  // (first channel, tap) of every 16 rows of the packed filters
   int split_half_count = 0, patch_rows = 0;
   bool split_odd = false;        // an odd number of taps per stage
-  int split_npos = 0;            // positions (pos_tab: 8 bytes each, behind one SplitFlags)
-  std::shared_ptr<Plan> exact;   // the same pass on the single-precision kernels
-  double chain = 0;              // terms that one accumulator sums up without a break, on average
+  int split_npos = 0;            // positions (pos_tab: 8 bytes each)
   bool single_dense_phase = false;  // positions enumerate the destination tensor in order
   bool table_rows = false;          // tap-major kernel whose K tiles are rows of the gather table (channel count no multiple of the K tile)
   int table_count = 0;              // data gradient on table rows: rows of the (padded) table = rows of the packed filters
@@ -1496,16 +1492,31 @@ bool split_applies(const Geometry &g, const Plan &pl, int rows, const Phase &ph,
   return false;
 }
 
+// Whether such a pass on tiles `split` (`stages` stages) is to be had, or the single-precision kernels stay with tiles `single` (`ktiles` K tiles of `bk`).
+bool split_pays(const SplitLayout &lay, const TileChoice &split, long long stages, const TileChoice &single, long long ktiles, int bk) {
+  if (getenv("MYGRAD_HIP_SPLIT_MIN")) return true;
+  // One rounding of a sum for 32 terms here, eight there: a third of the error on sums cut alike.  The single-precision plan cuts K into
+  // more slices where it has few tiles; where that would leave more than a quarter more to sum up without a break here, it stays.
+  if (mean_chain(split, stages, split.blocks_per_cu) * 16 * lay.sp.window > 1.25 * mean_chain(single, ktiles, single.blocks_per_cu) * bk) return false;
+  // Nor on tiles of many more rows, where the patches of 256 positions do not fit: (98,110,69,63) * (15,110,3,3) 181 us on
+  // tiles of 16 x 256, 436 here on 96 x 128.
+  return 4ll * split.m_tiles * split.bm <= 5ll * single.m_tiles * single.bm;
+}
+
 // The tables of a pass on conv_split.hip that contracts `channels` channels (pl.depth of them, with dead rows), `cstride` elements apart.
-// The table of positions is filled, and the flags before it cleared, on the library's stream.
-int split_tables(Plan &pl, Tables &t, const SplitLayout &lay, const Phase &ph, const int *Q, int channels, long long cstride) {
+// The table of positions is filled on the library's stream.
+// False where there is no memory for that table: such a pass stays on the single-precision kernels.
+bool split_tables(Plan &pl, Tables &t, const SplitLayout &lay, int bn, const Phase &ph, const int *Q, int channels, long long cstride) {
   const int window = lay.sp.window;
-  MG_HIP(hipMalloc(&pl.pos_tab, sizeof(SplitFlags) + (size_t)ph.npos * 8));
+  if (hipMalloc(&pl.pos_tab, (size_t)ph.npos * 8) != hipSuccess) {
+    (void)hipGetLastError();
+    pl.pos_tab = nullptr;
+    return false;
+  }
   SplitPositions p{};
   p.npos = ph.npos, p.sp = lay.sp, p.sample_rows = (int)up4((long long)Q[0] * Q[1] * Q[2]);
   for (int k = 0; k < 3; ++k) p.J[k] = ph.J[k], p.Q[k] = Q[k];
   launch_split_positions(p, pl.pos_tab, runtime().stream);
-  MG_HIP(hipGetLastError());
   for (int c0 = 0; c0 < pl.depth; c0 += 16)
     for (int tap = 0; tap < lay.taps; ++tap) {
       if (tap % window == 0) {
@@ -1514,22 +1525,23 @@ int split_tables(Plan &pl, Tables &t, const SplitLayout &lay, const Phase &ph, c
         e.coff = (int)(c0 * cstride);
         e.d0 = lay.offs[tap] - lay.offs[0];
         e.d1 = tap;
+        e.d2 = c0;
         e.dead = dead_rows(16, channels - c0);
         t.ktiles.push_back(e);
       }
       t.split_halves.push_back(int2{c0, tap});
     }
   t.split_inner.assign(lay.offs, lay.offs + window);
-  t.split_tiles = lay.first[split_width(pl.bn)];
+  t.split_tiles = lay.first[split_width(bn)];
   t.split_phases.push_back(lay.sp);
   pl.split_half_count = (int)t.split_halves.size();
   pl.split_odd = window % 2 != 0;
   pl.split_npos = ph.npos;
-  pl.patch_rows = lay.patch[split_width(pl.bn)];
-  return MG_OK;
+  pl.patch_rows = lay.patch[split_width(bn)];
+  return true;
 }
 
-int build_fwd_plan(const Geometry &g, Plan &pl, bool may_split) {
+int build_fwd_plan(const Geometry &g, Plan &pl) {
   Tables t;
   // (one tap and few channels: one position per lane takes 34.7 - 40.3 us for (64,C,112,112) * (64,C,1,1), C = 2 -
   // 11, whole K tiles of 16 with dead rows 41.9 - 44.3)
@@ -1583,13 +1595,15 @@ int build_fwd_plan(const Geometry &g, Plan &pl, bool may_split) {
   pl.single_dense_phase = true;
   SplitLayout lay;
   for (int k = 0; k < 3; ++k) lay.sp.count[k] = g.W[k], lay.sp.d[k] = -g.P[k], lay.sp.step[k] = g.D[k];
-  pl.split = may_split && split_applies(g, pl, g.F, ph, g.X, lay);
   {
-    const long long ktiles = pl.table_rows ? ceil_div((long long)g.C * g.wvol, bk)
-                             : pl.split     ? pl.depth / 16 * (g.wvol / lay.sp.window)
-                             : pl.tap_major ? g.wvol * (pl.depth / bk) : ceil_div((long long)g.C * g.wvol, bk);
-    const TileChoice tc = choose_tile(g.F, {(long long)g.N * g.gvol}, (int)ktiles, pl.tap_major, g.dtype == MG_F64 ? 8 : 4, pl.split ? 0 : 1, pl.split ? 16 * lay.sp.window : bk, pl.table_rows, is_tiny(g), -1, lay.patch);
-    pl.chain = mean_chain(tc, ktiles, tc.blocks_per_cu) * (pl.split ? 16 * lay.sp.window : bk);
+    const long long ktiles = pl.tap_major && !pl.table_rows ? g.wvol * (pl.depth / bk) : ceil_div((long long)g.C * g.wvol, bk);
+    TileChoice tc = choose_tile(g.F, {(long long)ph.npos}, (int)ktiles, pl.tap_major, g.dtype == MG_F64 ? 8 : 4, 1, bk, pl.table_rows, is_tiny(g));
+    if (split_applies(g, pl, g.F, ph, g.X, lay)) {
+      const int stages = (int)(pl.depth / 16 * (g.wvol / lay.sp.window));
+      const TileChoice split = choose_tile(g.F, {(long long)ph.npos}, stages, true, 4, 0, 16 * lay.sp.window, false, false, -1, lay.patch);
+      pl.split = split_pays(lay, split, stages, tc, ktiles, bk) && split_tables(pl, t, lay, split.bn, ph, g.X, g.C, g.xvol);
+      if (pl.split) tc = split;
+    }
     pl.bm = tc.bm, pl.bn = tc.bn, pl.m_tiles = tc.m_tiles, pl.full_tiles = tc.full_tiles, pl.tail_split = tc.tail_split, pl.blocks_per_cu = tc.blocks_per_cu;
     deepen_if_tiny(g, pl);
   }
@@ -1613,7 +1627,6 @@ int build_fwd_plan(const Geometry &g, Plan &pl, bool may_split) {
     return upload_plan(pl, t);
   }
   if (pl.split) {
-    if (int rc = split_tables(pl, t, lay, ph, g.X, g.C, g.xvol)) return rc;
     ph.k_count = (int)t.ktiles.size();
     t.phases.push_back(ph);
     pl.pos_blocks = (int)ceil_div(ph.npos, pl.bn);
@@ -1681,7 +1694,7 @@ bool deep_fused_on() {
   return on;
 }
 
-int build_dgrad_plan(const Geometry &g, Plan &pl, bool may_split) {
+int build_dgrad_plan(const Geometry &g, Plan &pl) {
   Tables t;
   // a tiny problem with a handful of channels is bound by its launches: the table-driven kernel
   // with its deep K tiles needs neither packed filters nor a pass over partial sums.  (Measured,
@@ -1774,16 +1787,9 @@ int build_dgrad_plan(const Geometry &g, Plan &pl, bool may_split) {
     }
   }
 
-  // ---- few channels, unit strides, a 3-tap "same" last axis (float): the rows of the GEMM are
-  // (channel, tap of the last axis), three times as many as there are channels, and the K tiles
-  // run over the taps of the other axes only.  A gathered element of grad then feeds three
-  // times the MFMAs -- with 16 channels the plain tiles are bound by the gather, not by the
-  // matrix pipes -- and the epilogue adds the three rows of a channel, shifted along the last
-  // axis, into dx.  A wave's 64 positions must be whole rows: rows of up to 64 positions, padded
-  // to a power of two.
   // ---- unit strides: the kernel on operands in three bf16 parts, where it applies (phases with different numbers of taps would need stages of
   // their own each)
-  if (may_split && nphase == 1 && found.size() == 1) {
+  if (nphase == 1 && found.size() == 1) {
     const PhaseTaps &pt = found[0];
     SplitLayout lay;
     for (int k = 0; k < 3; ++k) {
@@ -1791,22 +1797,31 @@ int build_dgrad_plan(const Geometry &g, Plan &pl, bool may_split) {
       lay.sp.d[k] = pt.offs[k][0];
       lay.sp.step[k] = lay.sp.count[k] > 1 ? pt.offs[k][1] - pt.offs[k][0] : 0;
     }
-    pl.split = split_applies(g, pl, g.C, pt.ph, g.G, lay);
-    if (pl.split) {
+    if (split_applies(g, pl, g.C, pt.ph, g.G, lay)) {
+      const long long ktiles = g.wvol * (pl.depth / bk), npos = pt.ph.npos;
       const int stages = (int)(pl.depth / 16 * (g.wvol / lay.sp.window));
-      const TileChoice tc = choose_tile(g.C, {(long long)pt.ph.npos}, stages, true, 4, 0, 16 * lay.sp.window, false, false, -1, lay.patch);
-      pl.chain = mean_chain(tc, stages, tc.blocks_per_cu) * 16 * lay.sp.window;
-      pl.bm = tc.bm, pl.bn = tc.bn, pl.m_tiles = tc.m_tiles, pl.full_tiles = tc.full_tiles, pl.tail_split = tc.tail_split, pl.blocks_per_cu = tc.blocks_per_cu;
-      if (int rc = split_tables(pl, t, lay, pt.ph, g.G, g.F, g.gvol)) return rc;
-      Phase ph = pt.ph;
-      ph.k_begin = 0, ph.blk_begin = 0;
-      ph.k_count = (int)t.ktiles.size();
-      t.phases.push_back(ph);
-      pl.pos_blocks = (int)ceil_div(ph.npos, pl.bn);
-      return upload_plan(pl, t);
+      const TileChoice single = choose_tile(g.C, {npos}, (int)ktiles, true, 4, 1, bk, false, is_tiny(g));
+      const TileChoice tc = choose_tile(g.C, {npos}, stages, true, 4, 0, 16 * lay.sp.window, false, false, -1, lay.patch);
+      pl.split = split_pays(lay, tc, stages, single, ktiles, bk) && split_tables(pl, t, lay, tc.bn, pt.ph, g.G, g.F, g.gvol);
+      if (pl.split) {
+        pl.bm = tc.bm, pl.bn = tc.bn, pl.m_tiles = tc.m_tiles, pl.full_tiles = tc.full_tiles, pl.tail_split = tc.tail_split, pl.blocks_per_cu = tc.blocks_per_cu;
+        Phase ph = pt.ph;
+        ph.k_begin = 0, ph.blk_begin = 0;
+        ph.k_count = (int)t.ktiles.size();
+        t.phases.push_back(ph);
+        pl.pos_blocks = (int)ceil_div(ph.npos, pl.bn);
+        return upload_plan(pl, t);
+      }
     }
   }
 
+  // ---- few channels, unit strides, a 3-tap "same" last axis (float): the rows of the GEMM are
+  // (channel, tap of the last axis), three times as many as there are channels, and the K tiles
+  // run over the taps of the other axes only.  A gathered element of grad then feeds three
+  // times the MFMAs -- with 16 channels the plain tiles are bound by the gather, not by the
+  // matrix pipes -- and the epilogue adds the three rows of a channel, shifted along the last
+  // axis, into dx.  A wave's 64 positions must be whole rows: rows of up to 64 positions, padded
+  // to a power of two.
   if (fold_applies(g, g.C, pl.depth) && pl.tap_major && !pl.table_rows && nphase == 1 && found.size() == 1) {
     const PhaseTaps &pt = found[0];
     Phase ph = pt.ph;
@@ -2005,7 +2020,6 @@ int build_dgrad_plan(const Geometry &g, Plan &pl, bool may_split) {
     }
     const TileChoice tc = choose_tile(g.C, npos, (int)std::max<long long>(min_ktiles, 0), pl.tap_major, g.dtype == MG_F64 ? 8 : 4, 1, bk, pl.table_rows,
                                       is_tiny(g), (int)(all_ktiles / std::max<long long>(all_pos, 1)));
-    pl.chain = mean_chain(tc, std::max<long long>(min_ktiles, 0), tc.blocks_per_cu) * bk;
     pl.bm = tc.bm, pl.bn = tc.bn, pl.m_tiles = tc.m_tiles, pl.full_tiles = tc.full_tiles, pl.tail_split = tc.tail_split, pl.blocks_per_cu = tc.blocks_per_cu;
     deepen_if_tiny(g, pl);
   }
@@ -2395,32 +2409,11 @@ int get_plan(ConvOp op, const mg_conv_desc *d, const Geometry &g, Plan **out) {
       release_conv_plans();
     }
     Plan pl;
-    auto build = [&](Plan &into, bool may_split) {
-      return op == OP_FWD ? build_fwd_plan(g, into, may_split) : op == OP_DGRAD ? build_dgrad_plan(g, into, may_split) : build_wgrad_plan(g, into);
-    };
-    int rc = build(pl, true);
-    if (pl.split) {
-      // the single-precision plan stands behind one on split operands, and alone where there is no memory for the latter's tables
-      Plan exact;
-      if (const int failed = build(exact, false)) {
-        free_tables(pl);
-        return failed;
-      }
-      // One rounding of a sum for 32 terms here, eight there: a third of the error on sums cut alike.  The single-precision plan cuts K into
-      // more slices where it has few tiles; where that would leave more than a quarter more to sum up without a break here, it stays.
-      const bool as_accurate = pl.chain <= 1.25 * exact.chain || getenv("MYGRAD_HIP_SPLIT_MIN") != nullptr;
-      // Nor on tiles of many more rows, where the patches of 256 positions do not fit: (98,110,69,63) * (15,110,3,3) 181 us on
-      // tiles of 16 x 256, 436 here on 96 x 128.
-      const bool as_full = 4ll * pl.m_tiles * pl.bm <= 5ll * exact.m_tiles * exact.bm || getenv("MYGRAD_HIP_SPLIT_MIN") != nullptr;
-      if (rc == MG_OK && as_accurate && as_full) {
-        pl.exact = std::make_shared<Plan>(exact);
-      } else {
-        (void)hipGetLastError();
-        free_tables(pl);
-        pl = exact, rc = MG_OK;
-      }
+    int rc = op == OP_FWD ? build_fwd_plan(g, pl) : op == OP_DGRAD ? build_dgrad_plan(g, pl) : build_wgrad_plan(g, pl);
+    if (rc) {
+      free_tables(pl);
+      return rc;
     }
-    if (rc) return rc;
     char tail[64];
     if (pl.share_grid > 0)
       snprintf(tail, sizeof tail, "even shares of the rest (%d partial slices)", pl.share_slots);
@@ -2512,6 +2505,7 @@ bool launch_split(GemmParams &gp, const Plan &pl, hipStream_t s) {
     MG_FIXUP(16, 256)
 #undef MG_FIXUP
   }
+  launch_split_redo(gp, pl.bm, pl.bn, pl.pos_blocks * pl.m_tiles, s);
   return true;
 }
 
@@ -2559,7 +2553,7 @@ int run_gemm(GemmParams &gp, const Plan &pl, int tag, hipStream_t s) {
     gp.vec_store = pl.pJ[0][2] == pl.pJ[1][2] && gp.os[1] % 4 == 0 && gp.os[0] % 4 == 0 && gp.dst_mstride % 4 == 0 &&
                    gp.dst_nstride % 4 == 0 && reinterpret_cast<uintptr_t>(gp.dst) % 16 == 0;
   }
-  ScopedTiming timed(gp.gate != nullptr ? TAG_GATED : tag);
+  ScopedTiming timed(tag);
   bool launched = false;
   if (pl.split) launched = launch_split(gp, pl, s);
   if (pl.deep_k) {
@@ -2653,7 +2647,7 @@ int folded_ld(int n) {
 }
 
 template <typename T>
-int pack_filters(const Geometry &g, const void *w, int mode, int depth, void **packed, size_t extra = 0, void **behind = nullptr, SplitFlags *gate = nullptr) {
+int pack_filters(const Geometry &g, const void *w, int mode, int depth, void **packed, size_t extra = 0, void **behind = nullptr) {
   const int M = (mode == 2 || mode == 6) ? g.F : mode == 3 ? g.C : mode == 4 ? 3 * g.C : 3 * g.F;
   const int ld = mode == 4 || mode == 5 ? folded_ld<T>(M / 3) : packed_ld(M, true);
   const size_t count = (size_t)(mode == 4 || mode == 5 ? g.wvol / 3 : g.wvol) * depth * ld;
@@ -2676,11 +2670,10 @@ int pack_filters(const Geometry &g, const void *w, int mode, int depth, void **p
     MG_HIP(hipGetLastError());
     return MG_OK;
   }
-  // (behind a gate most passes have nothing to do: few blocks)
-  const unsigned blocks = (unsigned)std::min<long long>(ceil_div((long long)count, 256), gate ? 256 : 4096);
-  ScopedTiming timed(gate ? TAG_GATED : TAG_PACK_FILTERS);
+  const unsigned blocks = (unsigned)std::min<long long>(ceil_div((long long)count, 256), 4096);
+  ScopedTiming timed(TAG_PACK_FILTERS);
   hipLaunchKernelGGL(pack_filters_kernel<T>, dim3(blocks), dim3(256), 0, runtime().stream, static_cast<const T *>(w),
-                     static_cast<T *>(*packed), g.F, g.C, (int)g.wvol, mode, ld, depth, gate);
+                     static_cast<T *>(*packed), g.F, g.C, (int)g.wvol, mode, ld, depth);
   MG_HIP(hipGetLastError());
   return MG_OK;
 }
@@ -2693,17 +2686,22 @@ int pack_split(GemmParams &gp, const Plan &pl, const void *w, int M, int channel
   gp.split_inner = pl.split_inner;
   gp.split_tiles = pl.split_tiles;
   gp.patch_rows = pl.patch_rows;
-  gp.split_flags = static_cast<SplitFlags *>(pl.pos_tab);
-  gp.positions = gp.split_flags + 1;
+  gp.positions = pl.pos_tab;
   gp.npos = pl.split_npos;
   const size_t packed_bytes = (size_t)pl.split_half_count * 16 * gp.a_ld * 6;
+  const int marks = 1 + (int)ceil_div((long long)pl.pos_blocks * pl.m_tiles, 32);
+  const size_t mark_bytes = (size_t)ceil_div(marks, 64) * 256;
   void *scratch = nullptr;
-  if (int rc = workspace(packed_bytes + tail_bytes(pl, 4), &scratch)) return rc;
+  if (int rc = workspace(packed_bytes + mark_bytes + tail_bytes(pl, 4), &scratch)) return rc;
   gp.A = scratch;
   gp.a_bytes = (unsigned)packed_bytes;
-  *partial = static_cast<char *>(scratch) + packed_bytes;
+  gp.redo = reinterpret_cast<unsigned *>(static_cast<char *>(scratch) + packed_bytes);
+  *partial = static_cast<char *>(scratch) + packed_bytes + mark_bytes;
+  gp.split_w = w;
+  gp.split_w_bytes = (unsigned)((std::max(m_stride * M, c_stride * channels)) * sizeof(float));
+  gp.split_w_mstride = (int)m_stride, gp.split_w_cstride = (int)c_stride;
   ScopedTiming timed(TAG_PACK_FILTERS);
-  launch_split_pack(static_cast<const float *>(w), scratch, pl.split_halves, pl.split_half_count, gp.split_flags, M, channels, m_stride, c_stride, gp.a_ld,
+  launch_split_pack(static_cast<const float *>(w), scratch, pl.split_halves, pl.split_half_count, gp.redo, marks, M, channels, m_stride, c_stride, gp.a_ld,
                     runtime().stream);
   MG_HIP(hipGetLastError());
   return MG_OK;
@@ -2754,7 +2752,7 @@ int run_thin(const Plan &pl, ThinParams &tp, const void *w, int tag) {
 }
 
 template <typename T>
-int conv_fwd_impl(const Geometry &g, const Plan &pl, const void *x, const void *w, void *out, SplitFlags *gate = nullptr) {
+int conv_fwd_impl(const Geometry &g, const Plan &pl, const void *x, const void *w, void *out) {
   if (pl.thin) {
     ThinParams tp{};
     tp.src = static_cast<const float *>(x);
@@ -2782,12 +2780,11 @@ int conv_fwd_impl(const Geometry &g, const Plan &pl, const void *x, const void *
     if (int rc = pack_split(gp, pl, w, g.F, g.C, g.C * g.wvol, g.wvol, &partial)) return rc;
   } else if (!pl.tap_major) {
     packed = const_cast<void *>(w);  // read in place: row k = (c, taps) of filter m lies at w[m * C*taps + k]
-  } else if (int rc = pack_filters<T>(g, w, pl.table_rows ? 6 : pl.fold_row ? 5 : 2, pl.table_rows ? g.C : pl.depth, &packed, tail_bytes(pl, sizeof(T)), &partial, gate)) {
+  } else if (int rc = pack_filters<T>(g, w, pl.table_rows ? 6 : pl.fold_row ? 5 : 2, pl.table_rows ? g.C : pl.depth, &packed, tail_bytes(pl, sizeof(T)), &partial)) {
     return rc;
   }
   gp.partial = partial;
   if (!pl.split) gp.A = packed;
-  if (gate) gp.gate = &gate->rerun;
   gp.a_mstride = (int)(g.C * g.wvol);
   gp.src = x;
   gp.dst = out;
@@ -2810,8 +2807,7 @@ int conv_fwd_impl(const Geometry &g, const Plan &pl, const void *x, const void *
     gp.samples = g.N;
     gp.sample_rows = (int)up4(g.xvol);
     gp.by_sample = make_fastdiv((unsigned)gp.sample_rows);
-    if (int rc = run_gemm<T>(gp, pl, TAG_CONV_FWD, runtime().stream)) return rc;
-    return conv_fwd_impl<T>(g, *pl.exact, x, w, out, gp.split_flags);
+    return run_gemm<T>(gp, pl, TAG_CONV_FWD, runtime().stream);
   }
   gp.a_ld = pl.fold_row ? folded_ld<T>(g.F) : packed_ld(g.F, pl.tap_major);
   gp.a_bytes = (unsigned)((size_t)(pl.tap_major && !pl.table_rows ? pl.depth : g.C) * (pl.fold_row ? g.wvol / 3 : g.wvol) * gp.a_ld * sizeof(T));
@@ -2820,7 +2816,7 @@ int conv_fwd_impl(const Geometry &g, const Plan &pl, const void *x, const void *
 }
 
 template <typename T>
-int conv_dgrad_impl(const Geometry &g, const Plan &pl, const void *grad, const void *w, void *dx, SplitFlags *gate = nullptr) {
+int conv_dgrad_impl(const Geometry &g, const Plan &pl, const void *grad, const void *w, void *dx) {
   if (pl.thin) {
     ThinParams tp{};
     tp.src = static_cast<const float *>(grad);
@@ -2870,12 +2866,11 @@ int conv_dgrad_impl(const Geometry &g, const Plan &pl, const void *grad, const v
     hipLaunchKernelGGL(pack_phase_rows_kernel<T>, dim3(blocks), dim3(256), 0, runtime().stream, static_cast<const T *>(w),
                        static_cast<T *>(packed), pl.arow, pl.table_count, pl.phase_count, (int)g.F, pl.depth, (int)g.C, (int)g.wvol, ld);
     MG_HIP(hipGetLastError());
-  } else if (int rc = pack_filters<T>(g, w, pl.fold_row ? 4 : 3, pl.depth, &packed, tail_bytes(pl, sizeof(T)), &partial, gate)) {
+  } else if (int rc = pack_filters<T>(g, w, pl.fold_row ? 4 : 3, pl.depth, &packed, tail_bytes(pl, sizeof(T)), &partial)) {
     return rc;
   }
   gp.partial = partial;
   if (!pl.split) gp.A = packed;
-  if (gate) gp.gate = &gate->rerun;
   gp.a_mstride = (int)g.wvol;
   gp.src = grad;
   gp.dst = dx;
@@ -2898,8 +2893,7 @@ int conv_dgrad_impl(const Geometry &g, const Plan &pl, const void *grad, const v
     gp.samples = g.N;
     gp.sample_rows = (int)up4(g.gvol);
     gp.by_sample = make_fastdiv((unsigned)gp.sample_rows);
-    if (int rc = run_gemm<T>(gp, pl, TAG_CONV_DGRAD, runtime().stream)) return rc;
-    return conv_dgrad_impl<T>(g, *pl.exact, grad, w, dx, gp.split_flags);
+    return run_gemm<T>(gp, pl, TAG_CONV_DGRAD, runtime().stream);
   }
   gp.a_ld = pl.fold_row ? folded_ld<T>(g.C) : packed_ld(g.C, pl.tap_major);
   gp.a_bytes = pl.table_rows ? (unsigned)((size_t)pl.table_count * gp.a_ld * sizeof(T))
@@ -3047,7 +3041,6 @@ int conv_wgrad_impl(const Geometry &g, const Plan &pl, const void *grad, const v
 void release_conv_plans() {
   note_plan("");  // it may point into a plan
   for (auto &kv : plans()) {
-    if (kv.second.exact) free_tables(*kv.second.exact);
     free_tables(kv.second);
   }
   plans().clear();

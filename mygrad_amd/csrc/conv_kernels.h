@@ -101,12 +101,6 @@ struct SplitPhase {
 };
 static_assert(sizeof(SplitPhase) == 64, "read as one 64-byte row");
 
-// What a pass of conv_split.hip finds out about its operands.
-struct SplitFlags {
-  int rerun;  // the single-precision kernels have to do the pass; cleared when a pass packs its filters
-  int pad_;
-};
-
 // Gather-GEMM:  dst[n, m, pos] = sum_k A(k, m) * src[n, row k, pos]
 // The tap-major kernels read A from packed filters, [rows][a_ld] with the M values of a row
 // contiguous; the table-driven kernel reads the filter bank where it lies:
@@ -180,7 +174,7 @@ struct GemmParams {
   int phase_count;      // 0: off; else the number of stride phases (2 or 4)
   int phase_pairs;      // phases 2q, 2q + 1 are neighbours along the last axis of dst
   // conv_split.hip: A is split into bf16 parts, a_ld a multiple of 16; ktiles holds stages, the names of KTile's fields aside:
-  // first half (tap of 16 channels) in A, channel offset, row offset, first tap, -, dead rows
+  // first half (tap of 16 channels) in A, channel offset, row offset, first tap, first channel, dead rows
   const SplitPhase *split_phases;  // one per phase
   const int *split_inner;
   const int *split_tiles;  // per block of positions: the lowest row that any of its windows touches, a stage's row offset aside
@@ -190,8 +184,10 @@ struct GemmParams {
   const void *positions;  // row of src and taps of every position, 8 bytes each
   int npos;
   FastDiv by_sample;    // row -> sample
-  SplitFlags *split_flags;
-  const int *gate;      // not null: the kernels return at once while *gate is zero
+  const void *split_w;  // the filter bank where it lies: row m's value under tap t of channel c at m * split_w_mstride + c * split_w_cstride + t
+  unsigned split_w_bytes;
+  unsigned *redo;  // whether there is a marked tile, then the marks, a bit each: see split_redo_kernel; cleared as the filters are packed
+  int split_w_mstride, split_w_cstride;
 };
 
 // The table of positions of conv_split.hip (GemmParams::positions): positions (n, j) of J, sources at j + the taps' offsets in Q.
@@ -205,8 +201,9 @@ struct SplitPositions {
 inline int split_width(int bn) { return bn / 64 - 2; }  // numbers the widths of its tiles: 128, 192, 256 positions
 int split_patch_limit(int bm, int bn);
 int split_gemm_blocks_per_cu(int bm, int bn, int patch_rows);
+void launch_split_redo(const GemmParams &p, int bm, int bn, int tiles, hipStream_t s);
 bool launch_split_gemm(const GemmParams &p, int bm, int bn, bool odd, unsigned grid, hipStream_t s);
-void launch_split_pack(const float *w, void *packed, const void *halves, int count, SplitFlags *flags, int M, int channels, long long m_stride,
+void launch_split_pack(const float *w, void *packed, const void *halves, int count, unsigned *redo, int marks, int M, int channels, long long m_stride,
                        long long c_stride, int ld, hipStream_t s);
 void launch_split_positions(const SplitPositions &p, void *out, hipStream_t s);
 

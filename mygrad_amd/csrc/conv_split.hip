@@ -18,20 +18,22 @@
 // Two accumulators of 64 x 64 wave tiles do not fit 256 registers (70 - 85 of them spill: 186 us below become 246), those of 64 x 48 do but for
 // a dozen values that no step needs.
 //
-// What bounds it: (128,64,56,56) * (64,64,3,3), 29.6 GFLOP, takes 186 us with its packing and gated passes (single precision 234), about
-// 170 by itself: 174 TFLOP/s of the 300.  Operands from LDS (64 x 48 and 48 x 64 waves: 21 reads of 16 bytes a lane for 72 matrix
+// What bounds it: (128,64,56,56) * (64,64,3,3), 29.6 GFLOP, takes 178 - 194 us with its packing and the pass over marked tiles, from device to device
+// (single precision 232), some 165 - 180 by itself: 165 - 180 TFLOP/s of the 300.  Operands from LDS (64 x 48 and 48 x 64 waves: 21 reads of 16 bytes a lane for 72 matrix
 // instructions, 58 % of its bandwidth; 32 x 64 ones 18 for 48, 75 %: 201 us), and the turn between stages, where the waves of a block wait for
 // the patch to be split and parked; loads are hidden.  Smaller planes have smaller patches: (128,128,28,28) * (128,128,3,3), 29.6 GFLOP,
 // 230 -> 161 us; (16,96,16001) * (48,96,9), 21.2 GFLOP, 172 -> 130.
 //
-// What the split cannot represent is left to the single-precision kernels.  An infinite operand leaves Inf - Inf in
+// What the split cannot represent.  An infinite operand leaves Inf - Inf in
 // its second part and makes every sum that it takes part in a NaN, as an infinite or NaN operand or an overflow makes
 // it something not finite in any arithmetic.  And parts are multiples of 2^-133, the smallest number of bf16 (which the instruction takes as
 // it is, like every product and sum below 2^-126): of an operand below 2^-110 bits may be lost, below 2^-134 all of them.  K such losses
-// times the largest value of the other operand are less than the last bit of a sum of K * 2^-109 times that value.  So a block that has
-// a sum that is not finite, or has lost bits of an element or seen a filter value below 2^-109 and has a sum, zero included, below that bound, sets
-// a flag.  The single-precision kernels are launched behind this one and return at once unless it is set: they then
-// do the whole pass, and its result is theirs.
+// times the largest value of the other operand are less than the last bit of a sum of K * 2^-109 times that value.  So where a block has
+// a sum that is not finite, or has lost bits of an element or seen a filter value below 2^-109 and has a sum, zero included, below that bound,
+// it marks its tile, and split_redo_kernel computes marked tiles again on the single-precision instruction.  The bits of other
+// tiles do not depend on it, and few marked tiles cost little: the forward pass below 194 us as it is, 205 with one NaN, 252 with one sample in 20 of
+// values about 1e-38, 811 where every tile is marked (single precision 232).  (The whole pass on the single-precision kernels, three launches that
+// returned at once otherwise, took 381 for the first odd value and 9 more for none.)
 #include "conv_device.h"
 #include "conv_kernels.h"
 #include "internal.h"
@@ -97,6 +99,19 @@ __device__ __forceinline__ Phase load_phase(const Phase *phases, int i) {
 }
 __device__ __forceinline__ int phase_first_block(const Phase *phases, int i) {
   return ((const int MG_CONSTANT *)(phases + uniform(i)))[8];
+}
+
+// the element of dst at position ipos of the phase, row 0
+__device__ __forceinline__ float *dst_of(const GemmParams &p, const Phase &ph, int ipos) {
+  const int j12 = ph.J[1] * ph.J[2];
+  const unsigned n = ph.by_jvol.div((unsigned)ipos);
+  unsigned r = (unsigned)ipos - n * (unsigned)(ph.J[0] * j12);
+  const int j0 = (int)ph.by_j12.div(r);
+  r -= (unsigned)j0 * (unsigned)j12;
+  const int j1 = (int)ph.by_j2.div(r);
+  const int j2 = (int)r - j1 * ph.J[2];
+  return static_cast<float *>(p.dst) + (long long)n * p.dst_nstride + (long long)(ph.o0[0] + j0 * p.oj[0]) * p.os[0] +
+         (long long)(ph.o0[1] + j1 * p.oj[1]) * p.os[1] + (long long)(ph.o0[2] + j2 * p.oj[2]) * p.os[2];
 }
 
 // One tile is MW * WM rows (filters) by NW * 16 TN positions, a wave of the block for each WM x 16 TN of it.  The contraction
@@ -194,14 +209,13 @@ __global__ void __launch_bounds__(64 * MW * NW, WM == 16 ? 3 : 2) split_gemm_ker
   const int octet_rows = p.patch_rows + 1;
   unsigned *const note = reinterpret_cast<unsigned *>(patch + 2 * octet_rows * 3);  // what was found, the widest filter value, the widest element
   if (threadIdx.x < 6) patch[((int)threadIdx.x / 3 * octet_rows + p.patch_rows) * 3 + (int)threadIdx.x % 3] = u32x4{0, 0, 0, 0};
-  float *__restrict__ dst = static_cast<float *>(p.dst);
   int pi = 0;
   Item me;
   u32x4 raw[ROUNDS][4];  // elements on their way to the patch: [round][channel][row of four]
   bool ahead = false;    // those of the item's first stage were requested by the item before it
   // the patch being requested: its first row, its stage's row of the table, whether there is one
   int patch_row = 0;
-  int8v patch_e = {0, 0, 0, 0, 0, 0, 0, 0};  // first half, channel offset, row offset, first tap, -, dead rows
+  int8v patch_e = {0, 0, 0, 0, 0, 0, 0, 0};  // first half, channel offset, row offset, first tap, first channel, dead rows
   bool patch_real = false;
   auto first_of = [&](const Item &it) -> int { return ((const int MG_CONSTANT *)p.split_tiles)[uniform(it.pos0 / BN)]; };
   // A part of the patch's loads.  A thread takes four rows of four channels in each round; the rows begin on a multiple of four and therefore
@@ -531,7 +545,10 @@ __global__ void __launch_bounds__(64 * MW * NW, WM == 16 ? 3 : 2) split_gemm_ker
         __syncthreads();
         found = (unsigned)uniform((int)note[0]);
       }
-      if ((found & (kNotFinite | kLostSum)) != 0) p.split_flags->rerun = 1;
+      if ((found & (kNotFinite | kLostSum)) != 0 && threadIdx.x == 0) {
+        p.redo[0] = 1;
+        atomicOr(&p.redo[1 + me.tile / 32], 1u << (me.tile % 32));
+      }
     }
 
     if (me.partial) {
@@ -542,19 +559,7 @@ __global__ void __launch_bounds__(64 * MW * NW, WM == 16 ? 3 : 2) split_gemm_ker
         for (int j = 0; j < TN; ++j) *reinterpret_cast<f32x4 *>(slot + (wm0 + i * 16 + l16) * BN + j * 16) = acc[j][i];
       continue;
     }
-    const int j12 = ph.J[1] * ph.J[2];
-    const int jvol = ph.J[0] * j12;
-    auto dst_of = [&](int ipos) -> float * {
-      const unsigned pos = (unsigned)ipos;
-      const unsigned n = ph.by_jvol.div(pos);
-      unsigned r = pos - n * (unsigned)jvol;
-      const int j0 = (int)ph.by_j12.div(r);
-      r -= (unsigned)j0 * (unsigned)j12;
-      const int j1 = (int)ph.by_j2.div(r);
-      const int j2 = (int)r - j1 * ph.J[2];
-      return dst + (long long)n * p.dst_nstride + (long long)(ph.o0[0] + j0 * p.oj[0]) * p.os[0] +
-             (long long)(ph.o0[1] + j1 * p.oj[1]) * p.os[1] + (long long)(ph.o0[2] + j2 * p.oj[2]) * p.os[2];
-    };
+    const int jvol = ph.J[0] * ph.J[1] * ph.J[2];
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
       const int four = first + j * 16;
@@ -567,7 +572,7 @@ __global__ void __launch_bounds__(64 * MW * NW, WM == 16 ? 3 : 2) split_gemm_ker
       }
       if (together) {
         typedef float OutVec __attribute__((ext_vector_type(4), aligned(4)));
-        float *out = dst_of(four);
+        float *out = dst_of(p, ph, four);
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
           const int m = me.m0 + wm0 + i * 16 + l16;
@@ -577,7 +582,7 @@ __global__ void __launch_bounds__(64 * MW * NW, WM == 16 ? 3 : 2) split_gemm_ker
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           if (four + q >= ph.npos) continue;
-          float *out = dst_of(four + q);
+          float *out = dst_of(p, ph, four + q);
 #pragma unroll
           for (int i = 0; i < TM; ++i) {
             const int m = me.m0 + wm0 + i * 16 + l16;
@@ -589,14 +594,172 @@ __global__ void __launch_bounds__(64 * MW * NW, WM == 16 ? 3 : 2) split_gemm_ker
   }
 }
 
+// The marked tiles (bm x bn, of one phase) of split_gemm_kernel again, on the single-precision instruction.  Where few are marked a block takes up
+// to 32 rows by 32 positions of one at a time, its waves a share of K each, which they add up in order: one marked tile is the work of
+// twelve blocks.  Where many are, a wave takes 16 TM rows by 64 positions over the whole of K.  Elements are gathered one by one (a tap that a
+// position does not have reads zero, as in the patch).  Filter values are the sums of their parts, which lie together as lanes want them,
+// but for lanes that find one among theirs which the parts do not hold.  Seldom anything to do: 4.5 us behind every pass.  Not built for the last
+// bit of speed: a step waits for its own loads (four parts of some 16 us a block is where the one way meets the other).
+constexpr int kRedoWaves = 8, kRedoBlocks = 512;  // a power of two
+
+template <int TM>
+__global__ void __launch_bounds__(64 * kRedoWaves, 2) split_redo_kernel(const GemmParams p, int bm, int bn, int tiles) {
+  const unsigned *const redo = p.redo;
+  if (redo[0] == 0) return;
+  constexpr int FEW = TM < 4 ? TM : 2;  // 16-row tiles of a block's part where few tiles are marked
+  __shared__ f32x4 shares[kRedoWaves - 1][2 * FEW][64];
+  const int lane = threadIdx.x & 63, l16 = lane & 15, lk = lane >> 4, wave = uniform((int)threadIdx.x >> 6);
+  const __amdgpu_buffer_rsrc_t a_buf = buffer_of(p.A, p.a_bytes);
+  const __amdgpu_buffer_rsrc_t w_buf = buffer_of(p.split_w, p.split_w_bytes);
+  const __amdgpu_buffer_rsrc_t src_buf = buffer_of(p.src, p.src_bytes);
+  const __amdgpu_buffer_rsrc_t table_buf = buffer_of(p.positions, (unsigned)p.npos * 8u);
+  const Phase ph = load_phase(p.phases, 0);
+  const int16v sp = ((const int16v MG_CONSTANT *)p.split_phases)[0];
+  const int window = sp[9], pairs = (window + 1) / 2;
+  const unsigned piece_row = (unsigned)p.a_ld * 16u;
+  const bool second = lk >= 2;  // as in split_gemm_kernel: this lane's are eight channels under the second tap of a step
+  const int words = (tiles + 31) / 32;
+  const int MG_CONSTANT *const inner = as_constant(p.split_inner) + sp[10];
+  const int8v MG_CONSTANT *const table = (const int8v MG_CONSTANT *)p.ktiles + ph.k_begin;
+
+  // part `part` of a tile: 16 ROWS rows by 16 COLS positions, by the block or (ALONE) by the wave
+  auto compute = [&](auto rows_c, auto cols_c, auto alone_c, int tile, int part) {
+    constexpr int ROWS = decltype(rows_c)::value, COLS = decltype(cols_c)::value;
+    constexpr bool ALONE = decltype(alone_c)::value;
+    const int across = bn / (16 * COLS);
+    const int m0 = tile % p.m_tiles * bm + part / across * 16 * ROWS, pos0 = tile / p.m_tiles * bn + part % across * 16 * COLS;
+    int row_at[COLS];
+    unsigned taps[COLS];
+#pragma unroll
+    for (int j = 0; j < COLS; ++j) {
+      typedef int int2v __attribute__((ext_vector_type(2)));
+      const int2v at = __builtin_bit_cast(int2v, __builtin_amdgcn_raw_buffer_load_b64(table_buf, (int)((unsigned)(pos0 + j * 16 + l16) * 8u), 0, 0));
+      row_at[j] = at[0];
+      taps[j] = (unsigned)at[1];
+    }
+    f32x4 acc[COLS][ROWS];
+#pragma unroll
+    for (int j = 0; j < COLS; ++j)
+#pragma unroll
+      for (int i = 0; i < ROWS; ++i) acc[j][i] = f32x4{0, 0, 0, 0};
+    for (int step = ALONE ? 0 : wave; step < ph.k_count * pairs; step += ALONE ? 1 : kRedoWaves) {  // 16 channels under two taps
+      const int8v here = table[step / pairs];  // see GemmParams
+      const int q = step % pairs * 2 + (second ? 1 : 0), octet = lk & 1;
+      const bool has_tap = q < window;
+      const unsigned dead = (unsigned)here[5] >> (octet * 8);
+      float xs[COLS][8];
+#pragma unroll
+      for (int j = 0; j < COLS; ++j) {
+        const int row = row_at[j] + here[2] + inner[has_tap ? q : 0];
+        const unsigned n = __umulhi((unsigned)max(row, 0), p.by_sample.mul) >> p.by_sample.shr;
+        const unsigned at = (n * (unsigned)p.src_nstride + (unsigned)(row - (int)n * p.sample_rows + here[1] + octet * 8 * p.src_cstride)) * 4u;
+        const unsigned from = has_tap && ((taps[j] >> (here[3] + q)) & 1u) != 0 ? at : kOutside;
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          xs[j][e] = float_of(__builtin_amdgcn_raw_buffer_load_b32(src_buf, (int)(from | ((dead << (31 - e)) & kOutside)), (int)((unsigned)(e * p.src_cstride) * 4u), 0));
+      }
+      float ws[ROWS][8];
+#pragma unroll
+      for (int i = 0; i < ROWS; ++i) {
+        const int m = m0 + i * 16 + l16;
+        const unsigned at = has_tap && m < p.a_ld ? (unsigned)((here[0] + q) * 2 + octet) * 3u * piece_row + (unsigned)m * 16u : kOutside;
+        u32x4 parts[3];
+#pragma unroll
+        for (int part = 0; part < 3; ++part) parts[part] = __builtin_amdgcn_raw_buffer_load_b128(a_buf, (int)at, (int)((unsigned)part * piece_row), 0);
+        bool whole = true;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          float v[3];
+#pragma unroll
+          for (int part = 0; part < 3; ++part) v[part] = float_of(e % 2 != 0 ? parts[part][e / 2] & 0xffff0000u : parts[part][e / 2] << 16);
+          ws[i][e] = v[0] + (v[1] + v[2]);
+          whole &= v[0] == 0.0f || (__builtin_fabsf(v[0]) >= 0x1p-109f && __builtin_fabsf(v[0]) < __builtin_inff());
+        }
+        if (!whole) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            ws[i][e] = float_of(__builtin_amdgcn_raw_buffer_load_b32(
+                w_buf, (int)((unsigned)(m * p.split_w_mstride + (here[4] + octet * 8 + e) * p.split_w_cstride + here[3] + q) * 4u | ((dead << (31 - e)) & kOutside)), 0, 0));
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+#pragma unroll
+        for (int i = 0; i < ROWS; ++i)
+#pragma unroll
+          for (int j = 0; j < COLS; ++j) acc[j][i] = Mma<float>::run(xs[j][e], ws[i][e], acc[j][i]);
+    }
+    if constexpr (!ALONE) {
+      __syncthreads();  // (the shares of the part before have been read)
+      if (wave > 0) {
+#pragma unroll
+        for (int j = 0; j < COLS; ++j)
+#pragma unroll
+          for (int i = 0; i < ROWS; ++i) shares[wave - 1][j * ROWS + i][lane] = acc[j][i];
+      }
+      __syncthreads();
+      if (wave > 0) return;
+#pragma unroll
+      for (int j = 0; j < COLS; ++j)
+#pragma unroll
+        for (int i = 0; i < ROWS; ++i)
+          for (int other = 0; other < kRedoWaves - 1; ++other) acc[j][i] += shares[other][j * ROWS + i][lane];
+    }
+#pragma unroll
+    for (int j = 0; j < COLS; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int ipos = pos0 + j * 16 + 4 * lk + q;
+        if (ipos >= ph.npos) continue;
+        float *const out = dst_of(p, ph, ipos);
+#pragma unroll
+        for (int i = 0; i < ROWS; ++i) {
+          const int m = m0 + i * 16 + l16;
+          if (m < p.M) out[(long long)m * p.dst_mstride] = acc[j][i][q];
+        }
+      }
+  };
+
+  int count = 0;
+  for (int first = 0; first < words; first += 64) {
+    int mine = first + lane < words ? __popc(redo[1 + first + lane]) : 0;
+    for (int step = 1; step < 64; step *= 2) mine += __shfl_xor(mine, step);
+    count += mine;
+  }
+  const std::integral_constant<int, 2> two;
+  const std::integral_constant<int, 4> four;
+  const int few_parts = bn / 32 * (bm / (16 * FEW));
+  if ((long long)count * few_parts <= 4 * kRedoBlocks) {
+    // every wave finds the marked tiles in the same order, and the block's parts of them
+    for (int first = 0; first < words; first += 64) {
+      const unsigned mine = first + lane < words ? redo[1 + first + lane] : 0u;
+      for (unsigned long long some = __ballot(mine != 0); some != 0; some &= some - 1) {
+        const int from = __builtin_ctzll(some);
+        for (unsigned word = (unsigned)__builtin_amdgcn_readlane((int)mine, from); word != 0; word &= word - 1) {
+          const int tile = (first + from) * 32 + __builtin_ctz(word);
+          for (int part = (int)((blockIdx.x - (unsigned)(tile * few_parts)) & (kRedoBlocks - 1)); part < few_parts; part += kRedoBlocks)
+            compute(std::integral_constant<int, FEW>(), two, std::false_type(), tile, part);
+        }
+      }
+    }
+  } else {
+    const int parts = bn / 64 * (bm / (16 * TM));
+    for (int unit = (int)blockIdx.x * kRedoWaves + wave; unit < tiles * parts; unit += kRedoBlocks * kRedoWaves) {
+      const int tile = unit / parts;
+      if (((redo[1 + tile / 32] >> (tile % 32)) & 1u) != 0) compute(std::integral_constant<int, TM>(), four, std::true_type(), tile, unit % parts);
+    }
+  }
+}
+
 // The filters of split_gemm_kernel, in three parts: piece [octet of K rows][part][m] holds the eight bf16
 // values of K rows 8 * octet .. + 7 of row m of the product, `ld` (a multiple of 16) pieces to a row.  Sixteen K rows
 // are 16 channels from c0 on under one tap, named by halves[K row / 16] = (c0, tap): row m's value is w[m * m_stride + c * c_stride + tap],
 // zero for c >= channels and m >= M.  A value that is not zero has a first part that is not, the smallest number of bf16 at least: that is how
-// split_gemm_kernel knows of those that have lost bits.  Also clears the flag that it may set.
+// split_gemm_kernel knows of those that have lost bits.  Also clears the marks of tiles, `marks` words of them.
 __global__ void __launch_bounds__(256) split_pack_kernel(const float *__restrict__ w, u32x4 *__restrict__ packed, const int2 *__restrict__ halves,
-                                                         int count, SplitFlags *flags, int M, int channels, long long m_stride, long long c_stride, int ld) {
-  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) flags->rerun = 0;
+                                                         int count, unsigned *__restrict__ redo, int marks, int M, int channels, long long m_stride,
+                                                         long long c_stride, int ld) {
+  for (unsigned i = (blockIdx.y * gridDim.x + blockIdx.x) * 256 + threadIdx.x; i < (unsigned)marks; i += gridDim.x * gridDim.y * 256) redo[i] = 0;
   const int oct = blockIdx.x * 16 + (int)(threadIdx.x >> 4), m = blockIdx.y * 16 + (int)(threadIdx.x & 15);
   if (oct >= 2 * count) return;
   const int2 h = halves[oct / 2];
@@ -621,11 +784,9 @@ __global__ void __launch_bounds__(256) split_pack_kernel(const float *__restrict
 }
 
 // (row, taps) of every position: the row of src (sample * sample_rows + element of a channel's plane) that its window starts
-// from, padding aside, and which taps have an element there, bit by bit; and cleared flags before them.
-__global__ void __launch_bounds__(256) split_positions_kernel(const SplitPositions p, SplitFlags *flags) {
-  int2 *const out = reinterpret_cast<int2 *>(flags + 1);
+// from, padding aside, and which taps have an element there, bit by bit.
+__global__ void __launch_bounds__(256) split_positions_kernel(const SplitPositions p, int2 *__restrict__ out) {
   const int idx = blockIdx.x * 256 + threadIdx.x;
-  if (idx == 0) flags->rerun = 0;
   if (idx >= p.npos) return;
   const int j12 = p.J[1] * p.J[2], n = idx / (p.J[0] * j12), r = idx - n * p.J[0] * j12;
   const int q0 = r / j12, q1 = r / p.J[2] % p.J[1], q2 = r % p.J[2];
@@ -696,14 +857,19 @@ bool launch_split_gemm(const GemmParams &p, int bm, int bn, bool odd, unsigned g
   return false;
 }
 
-void launch_split_pack(const float *w, void *packed, const void *halves, int count, SplitFlags *flags, int M, int channels, long long m_stride,
+void launch_split_redo(const GemmParams &p, int bm, int bn, int tiles, hipStream_t s) {
+  const auto kernel = bm % 64 == 0 ? split_redo_kernel<4> : bm == 48 ? split_redo_kernel<3> : bm == 32 ? split_redo_kernel<2> : split_redo_kernel<1>;
+  hipLaunchKernelGGL(kernel, dim3(kRedoBlocks), dim3(64 * kRedoWaves), 0, s, p, bm, bn, tiles);
+}
+
+void launch_split_pack(const float *w, void *packed, const void *halves, int count, unsigned *redo, int marks, int M, int channels, long long m_stride,
                        long long c_stride, int ld, hipStream_t s) {
   hipLaunchKernelGGL(split_pack_kernel, dim3((unsigned)ceil_div(2 * count, 16), (unsigned)(ld / 16)), dim3(256), 0, s, w,
-                     static_cast<u32x4 *>(packed), static_cast<const int2 *>(halves), count, flags, M, channels, m_stride, c_stride, ld);
+                     static_cast<u32x4 *>(packed), static_cast<const int2 *>(halves), count, redo, marks, M, channels, m_stride, c_stride, ld);
 }
 
 void launch_split_positions(const SplitPositions &p, void *out, hipStream_t s) {
-  hipLaunchKernelGGL(split_positions_kernel, dim3((unsigned)ceil_div(p.npos, 256)), dim3(256), 0, s, p, static_cast<SplitFlags *>(out));
+  hipLaunchKernelGGL(split_positions_kernel, dim3((unsigned)ceil_div(p.npos, 256)), dim3(256), 0, s, p, static_cast<int2 *>(out));
 }
 
 }  // namespace mg

@@ -140,7 +140,6 @@ constexpr bool tap_gemm_dead_apart(int bm, int bn, int nph, int elem) {
 
 template <typename T, int BM, int BN, int BK, int WM, int WN, int NPH = 1, bool FOLD = false, bool ROWS = false, bool DEAD = false>
 __global__ void __launch_bounds__(512) tap_gemm_kernel(const GemmParams p) {
-  if (p.gate != nullptr && *p.gate == 0) return;
   // ROWS: the BK rows of a K tile are any rows of the gather table (GemmParams::tab: element
   // offset and coordinate offsets of one (channel, tap) each), not BK channels under one tap;
   // KTile::coff is then the index of the tile's first table row.  For channel counts that are
@@ -968,7 +967,6 @@ __global__ void __launch_bounds__(512) tap_gemm_kernel(const GemmParams p) {
 // One thread per tile element; blockIdx.y is the tail tile.
 template <typename T, int BM, int BN, int NPH = 1>
 __global__ void __launch_bounds__(256) tail_fixup_kernel(const GemmParams p) {
-  if (p.gate != nullptr && *p.gate == 0) return;
   const int e = blockIdx.x * 256 + threadIdx.x;  // element of the [BM][BN] tile
   if (e >= BM * BN) return;
   // the tile, where its slices' partial sums start and how many there are

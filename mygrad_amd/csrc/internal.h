@@ -62,7 +62,6 @@ enum KernelTag {
   TAG_SUM_OVER = 18,
   TAG_PERMUTE = 19,
   TAG_BATCHED_PRODUCT = 20,
-  TAG_GATED = 21,  // the launches behind a pass of conv_split.hip
 };
 void timing_begin(int tag);
 void timing_end();

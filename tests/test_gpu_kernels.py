@@ -1440,6 +1440,10 @@ SPLIT_PROBLEMS = [
     ((2, 512, 6, 5), (512, 512, 3, 3), (1, 1), (1, 1), ""),                  # every tile shared out
     ((7, 45, 27, 31), (70, 45, 3, 3), (1, 1), (1, 1), "64,192"),             # odd window
     ((2, 32, 70, 75), (64, 32, 3, 3), (1, 1), (1, 1), "64,128"),             # patches of more rows than threads
+    ((9, 16, 4099), (64, 16, 3), (1,), (1,), "64,192"),                      # enough tiles for a pass over marked ones to go by waves
+    ((17, 16, 4099), (48, 16, 4), (2,), (1,), "48,256"),
+    ((17, 16, 4099), (32, 16, 4), (2,), (1,), "32,256"),
+    ((17, 16, 4099), (16, 16, 3), (1,), (1,), "16,256"),
 ]
 
 
@@ -1557,7 +1561,7 @@ def test_products_of_three_bf16_parts_keep_single_precision(abi, monkeypatch, pr
             assert np.linalg.norm(got - ref) <= (1.25 * 5.06e-8 * np.sqrt(steps / 2) + 3.5e-8) * np.linalg.norm(ref)
 
 
-@pytest.mark.parametrize("problem", [0, 1, 3, 5, 8, 12])
+@pytest.mark.parametrize("problem", [0, 1, 3, 5, 8, 12, 14, 15, 16, 17])
 def test_products_of_three_bf16_parts_lose_no_operand(abi, monkeypatch, problem):
     """Operands whose low bits, or all of them, are below the smallest number of bf16: the products are normal numbers all the same."""
     x_shape, w_shape, p, d, _ = SPLIT_PROBLEMS[problem]
@@ -1579,3 +1583,26 @@ def test_products_of_three_bf16_parts_lose_no_operand(abi, monkeypatch, problem)
             exact = direct.conv_forward(x64, w64, s, p, d), direct.conv_backward_x(g64, x_shape, w64, s, p, d)
             for got, ref in zip(passes(xs, ws, gs), exact):
                 assert np.all(np.abs(got - ref) <= (2 + 5 / 32) * 2.0**-24 * np.abs(ref) + 2.0**-149)
+
+
+@pytest.mark.parametrize("problem", [0, 1, 5, 7, 10, 12])
+def test_products_of_three_bf16_parts_keep_odd_values_apart(abi, monkeypatch, problem):
+    """What the parts cannot hold in one sample leaves every bit of another one alone."""
+    x_shape, w_shape, p, d, _ = SPLIT_PROBLEMS[problem]
+    rng = np.random.default_rng(3400 + problem)
+    passes = _split_passes(abi, monkeypatch, problem)
+    x, w = (rng.standard_normal(shape).astype(np.float32) for shape in (x_shape, w_shape))
+    g = rng.standard_normal(direct.conv_forward(x, w, (1,) * len(p), p, d).shape).astype(np.float32)
+    plain = passes(x, w, g)
+    # samples that no tile of 256 positions shares with the first one
+    apart = [1 + -(-256 // np.prod(out.shape[2:])) for out in plain]
+    for value in (np.inf, np.nan, 1e-40):
+        xs, gs = x.copy(), g.copy()
+        for v in (xs, gs):
+            if value == 1e-40:
+                v[0] *= np.float32(1e-40)
+            else:
+                v[(0, *(n // 2 for n in v.shape[1:]))] = value
+        for got, was, first in zip(passes(xs, w, gs), plain, apart):
+            assert first < len(was)
+            assert np.array_equal(bits(got[first:]), bits(was[first:])) and not np.array_equal(got[0], was[0])
