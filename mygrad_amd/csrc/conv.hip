@@ -790,8 +790,8 @@ struct TileRate {
 };
 constexpr TileRate kTileRates[] = {
     // (nph 0: split_gemm_kernel)
-    {0, 16, 256, 0.50, 0.74, 0.00}, {0, 32, 256, 0.50, 0.90, 0.00}, {0, 48, 256, 0.50, 1.14, 0.00}, {0, 64, 128, 0.40, 1.00, 0.00},
-    {0, 64, 192, 0.45, 1.22, 0.00}, {0, 128, 128, 0.50, 1.00, 0.00},
+    {0, 16, 256, 0.40, 1.07, 0.00}, {0, 32, 256, 0.40, 1.16, 0.00}, {0, 48, 256, 0.40, 1.33, 0.00}, {0, 64, 128, 0.35, 1.32, 0.00},
+    {0, 64, 192, 0.40, 1.47, 0.00}, {0, 128, 128, 0.45, 1.19, 0.00},
     {1, 16, 256, 0.50, 0.42, 0.42}, {1, 32, 128, 0.35, 0.59, 0.62},  {1, 32, 256, 0.55, 0.63, 0.64}, {1, 48, 256, 0.62, 0.70, 0.67},
     {1, 64, 128, 0.47, 0.77, 0.70}, {1, 64, 256, 0.78, 0.83, 0.00},  {1, 96, 128, 0.56, 0.82, 0.80}, {1, 128, 64, 0.27, 0.81, 0.87},
     {1, 128, 128, 0.63, 0.86, 0.0}, {2, 16, 256, 0.53, 0.50, 0.00},  {2, 32, 256, 0.47, 0.70, 0.00}, {2, 64, 128, 0.45, 0.82, 0.00},
@@ -799,7 +799,7 @@ constexpr TileRate kTileRates[] = {
 
 // Microseconds of the launch described by `t` (without what every shape costs alike): `ktiles` K tiles of
 // `bk` rows per tile, `resident` blocks to a unit.
-double tile_time(const TileChoice &t, long long ktiles, int bk, size_t elem, int nph, int resident, bool table_rows) {
+double tile_time(const TileChoice &t, long long ktiles, int bk, size_t elem, int nph, int resident, bool table_rows, int patch_rows = 0) {
   const double cus = runtime().props.multiProcessorCount;
   const double left = (double)(t.tiles - t.full_tiles), kt = (double)ktiles, grid = resident * cus;
   double chain, work, slices = 0;  // K tiles one after the other in a block; K tiles of the busiest unit; tiles of partial sums
@@ -819,6 +819,11 @@ double tile_time(const TileChoice &t, long long ktiles, int bk, size_t elem, int
   const double tile = (double)t.bm * t.bn;
   double a = 0, b = work * 2.0 * tile * bk * cus / (elem == 8 ? 78.6e6 * r->rate64 : 157.3e6 * r->rate);
   if (elem == 4) a = chain * r->step * bk / 16;
+  if (nph == 0) {
+    // (splitting and parking a row of the patch takes what 75 products of a tile's position and row take, on tiles of any shape)
+    const double parked = 1.0 + 75.0 * 16.0 * patch_rows / (tile * bk);
+    a *= parked, b *= parked;
+  }
   if (elem == 4 && table_rows) a *= 2.1, b *= 1.2;  // (its gathers look up a row of the table per element)
   return std::sqrt(std::sqrt(a * a * a * a + b * b * b * b)) + slices * tile * (double)elem * std::max(nph, 1) * 2.0 / 4.0e6;
 }
@@ -1006,7 +1011,7 @@ TileChoice choose_tile(int M, const std::vector<long long> &phase_npos, int min_
     if (!tap_major) return best;
     const int resident = stream ? best.blocks_per_cu : elem == 8 ? gemm_blocks_per_cu<double>(c.bm, c.bn, 1, bk) : gemm_blocks_per_cu<float>(c.bm, c.bn, nph, bk);
     const long long ktiles = std::max(avg_ktiles, 1);
-    candidates.push_back({best, tile_time(best, ktiles, bk, elem, nph, resident, table_rows), mean_chain(best, ktiles, resident)});
+    candidates.push_back({best, tile_time(best, ktiles, bk, elem, nph, resident, table_rows, nph == 0 ? patch[split_width(c.bn)] : 0), mean_chain(best, ktiles, resident)});
     const double cost = best_cost * c.bm * c.bn * c.penalty;
     if (c.bm == usual && (longest == 0 || cost < usual_cost)) usual_cost = cost, longest = candidates.back().chain, usual_at = candidates.size() - 1;
   }
@@ -1404,11 +1409,11 @@ bool split_on() {
 }
 
 // Flops from which a pass runs there, for a bank of `filters` values: below, what the kernel takes per stage, the packing
-// and the gated launches behind it count for more than its products.  Against the single-precision kernels, everything included,
-// over some 1400 drawn passes of unit strides: 0.7 - 1.2 of their speed at 4 - 6 GFLOP, 0.97 - 1.8 from 8 GFLOP on ((128,64,56,56) *
-// (64,64,3,3), 29.6 GFLOP: forward 270 -> 178 us, dx 259 -> 171; (16,45,16001) * (83,45,9): 178 -> 138 and 175 -> 121;
-// (64,512,7,7) * (512,512,3,3): 156 -> 114 and 141 -> 109), but (25,316,118) * (424,316,15), 9 GFLOP against two million values: 117 ->
-// 108 and 130 -> 135.  Strided forward passes touch the more rows per position: 0.4 - 1.1 of the speed in most.
+// and the pass over marked tiles behind it count for more than its products.  Against the single-precision kernels, everything included,
+// over some 1400 drawn passes of unit strides: 0.7 - 1.2 of their speed at 4 - 6 GFLOP, more from 8 GFLOP on ((128,64,56,56) *
+// (64,64,3,3), 29.6 GFLOP: forward 232 -> 179 us; (16,45,16001) * (83,45,9): 180 -> 141; (64,512,7,7) * (512,512,3,3): 150 -> 114), but
+// (25,316,118) * (424,316,15), 9 GFLOP against two million values: 117 -> 108 and 130 -> 135.  Strided forward passes touch the more rows per
+// position: 0.4 - 1.1 of the speed in most.
 // MYGRAD_HIP_SPLIT_MIN=flops replaces the line, and takes away the rules on speed and accuracy below (tests; part of the plan key).
 double split_min_flops(double filters) {
   const char *v = getenv("MYGRAD_HIP_SPLIT_MIN");
@@ -1495,12 +1500,18 @@ bool split_applies(const Geometry &g, const Plan &pl, int rows, const Phase &ph,
 // Whether such a pass on tiles `split` (`stages` stages) is to be had, or the single-precision kernels stay with tiles `single` (`ktiles` K tiles of `bk`).
 bool split_pays(const SplitLayout &lay, const TileChoice &split, long long stages, const TileChoice &single, long long ktiles, int bk) {
   if (getenv("MYGRAD_HIP_SPLIT_MIN")) return true;
+  const int depth = 16 * lay.sp.window;
   // One rounding of a sum for 32 terms here, eight there: a third of the error on sums cut alike.  The single-precision plan cuts K into
   // more slices where it has few tiles; where that would leave more than a quarter more to sum up without a break here, it stays.
-  if (mean_chain(split, stages, split.blocks_per_cu) * 16 * lay.sp.window > 1.25 * mean_chain(single, ktiles, single.blocks_per_cu) * bk) return false;
-  // Nor on tiles of many more rows, where the patches of 256 positions do not fit: (98,110,69,63) * (15,110,3,3) 181 us on
-  // tiles of 16 x 256, 436 here on 96 x 128.
-  return 4ll * split.m_tiles * split.bm <= 5ll * single.m_tiles * single.bm;
+  if (mean_chain(split, stages, split.blocks_per_cu) * depth > 1.25 * mean_chain(single, ktiles, single.blocks_per_cu) * bk) return false;
+  // Nor on tiles of many more rows, where the patches of 256 positions do not fit: (98,110,69,63) * (15,110,3,3) takes 188 us on tiles of
+  // 16 x 256, 281 here on 64 x 192.
+  if (4ll * split.m_tiles * split.bm > 5ll * single.m_tiles * single.bm) return false;
+  // Nor where the patches are large for their products, as under windows of five rows: (20,285,34,55) * (36,285,3,3), 16 x 256, 0.89 of the speed of
+  // three passes.  Of 1700 drawn passes that get here, 85 fall behind this line, as fast on the one as on the other on average, and the
+  // others gain a third; 20 of those lose more than the 3 % that a measurement is good for.
+  return 1.05 * tile_time(split, stages, depth, 4, 0, split.blocks_per_cu, false, lay.patch[split_width(split.bn)]) <=
+         tile_time(single, ktiles, bk, 4, 1, single.blocks_per_cu, false);
 }
 
 // The tables of a pass on conv_split.hip that contracts `channels` channels (pl.depth of them, with dead rows), `cstride` elements apart.

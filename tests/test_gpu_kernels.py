@@ -1606,3 +1606,39 @@ def test_products_of_three_bf16_parts_keep_odd_values_apart(abi, monkeypatch, pr
         for got, was, first in zip(passes(xs, w, gs), plain, apart):
             assert first < len(was)
             assert np.array_equal(bits(got[first:]), bits(was[first:])) and not np.array_equal(got[0], was[0])
+
+
+# (x, w, padding, whether the forward pass runs on split operands, and why not)
+SPLIT_RULES = [
+    ((128, 64, 56, 56), (64, 64, 3, 3), (1, 1), True),
+    ((16, 45, 16001), (83, 45, 9), (4,), True),
+    ((28, 64, 56, 56), (64, 64, 3, 3), (1, 1), False),        # 6.5 GFLOP
+    ((2, 57, 16936), (125, 57, 15), (0,), False),             # K in fewer slices
+    ((70, 113, 38, 78), (17, 113, 3, 5), (0, 0), False),      # patches that only fit tiles of twice the rows
+    ((40, 285, 34, 55), (36, 285, 5, 1), (2, 0), False),      # large patches for their products
+    ((59, 56, 930), (443, 56, 3), (1,), False),               # three taps
+]
+
+
+@pytest.mark.parametrize("rule", range(len(SPLIT_RULES)))
+def test_which_passes_run_on_three_bf16_parts(abi, rule):
+    from mygrad_amd import _hip
+
+    x_shape, w_shape, p, split = SPLIT_RULES[rule]
+    rng = np.random.default_rng(3500 + rule)
+    x, w = (rng.standard_normal(shape, dtype=np.float32) for shape in (x_shape, w_shape))
+    out = abi.conv_fwd(x, w, (1,) * len(p), p, (1,) * len(p))
+    plan = _hip.last_plan()
+    print(plan, flush=True)
+    assert plan.endswith("three bf16 parts") == split
+    # 200 of the results, each from its window; single precision rounds once a term, 2.5e-8 of the sum as it stands on average
+    padded = np.pad(x, ((0, 0), (0, 0), *((q, q) for q in p)))
+    flat = w.reshape(w_shape[0], -1).astype(np.float64)
+    terms = flat.shape[1]
+    off = norm = 0.0
+    for _ in range(200):
+        n, *at = (rng.integers(size) for size in (x_shape[0], *out.shape[2:]))
+        window = padded[(n, slice(None), *(slice(i, i + k) for i, k in zip(at, w_shape[2:])))]
+        ref = flat @ window.reshape(-1).astype(np.float64)
+        off, norm = off + np.sum((out[(n, slice(None), *at)] - ref) ** 2), norm + np.sum(ref**2)
+    assert np.sqrt(off / norm) <= 1.25 * 2.5e-8 * np.sqrt(terms / 2)
