@@ -820,7 +820,8 @@ double tile_time(const TileChoice &t, long long ktiles, int bk, size_t elem, int
   double a = 0, b = work * 2.0 * tile * bk * cus / (elem == 8 ? 78.6e6 * r->rate64 : 157.3e6 * r->rate);
   if (elem == 4) a = chain * r->step * bk / 16;
   if (nph == 0) {
-    // (splitting and parking a row of the patch takes what 75 products of a tile's position and row take, on tiles of any shape)
+    // (splitting and parking a row of the patch takes what 75 products of a tile's position and row take, on
+    // tiles of any shape)
     const double parked = 1.0 + 75.0 * 16.0 * patch_rows / (tile * bk);
     a *= parked, b *= parked;
   }
@@ -901,7 +902,11 @@ TileChoice choose_tile(int M, const std::vector<long long> &phase_npos, int min_
     // fits on a compute unit, so the tap-major kernels use the half-size shapes
     if (tap_major && elem == 8 && c.bn * c.bm >= 128 * 128) continue;
     const bool stream = nph == 0 || (tap_major && tap_gemm_streams(c.bm, (int)elem));
-    const int per_cu = !stream ? 1 : nph == 0 ? split_gemm_blocks_per_cu(c.bm, c.bn, patch[split_width(c.bn)]) : elem == 8 ? gemm_blocks_per_cu<double>(c.bm, c.bn, 1, bk) : gemm_blocks_per_cu<float>(c.bm, c.bn, nph, bk);
+    const int patch_rows = nph == 0 ? patch[split_width(c.bn)] : 0;
+    const int per_cu = !stream     ? 1
+                       : nph == 0  ? split_gemm_blocks_per_cu(c.bm, c.bn, patch_rows)
+                       : elem == 8 ? gemm_blocks_per_cu<double>(c.bm, c.bn, 1, bk)
+                                   : gemm_blocks_per_cu<float>(c.bm, c.bn, nph, bk);
     long long pos_blocks = 0;
     for (long long n : phase_npos) pos_blocks += ceil_div(n, c.bn);
     // (most blocks first: where the rounds come out the same, more resident blocks cover more of one
@@ -1011,7 +1016,8 @@ TileChoice choose_tile(int M, const std::vector<long long> &phase_npos, int min_
     if (!tap_major) return best;
     const int resident = stream ? best.blocks_per_cu : elem == 8 ? gemm_blocks_per_cu<double>(c.bm, c.bn, 1, bk) : gemm_blocks_per_cu<float>(c.bm, c.bn, nph, bk);
     const long long ktiles = std::max(avg_ktiles, 1);
-    candidates.push_back({best, tile_time(best, ktiles, bk, elem, nph, resident, table_rows, nph == 0 ? patch[split_width(c.bn)] : 0), mean_chain(best, ktiles, resident)});
+    const double time = tile_time(best, ktiles, bk, elem, nph, resident, table_rows, patch_rows);
+    candidates.push_back({best, time, mean_chain(best, ktiles, resident)});
     const double cost = best_cost * c.bm * c.bn * c.penalty;
     if (c.bm == usual && (longest == 0 || cost < usual_cost)) usual_cost = cost, longest = candidates.back().chain, usual_at = candidates.size() - 1;
   }
@@ -1408,20 +1414,21 @@ bool split_on() {
   return !(flag && flag[0] == '0');
 }
 
-// Flops from which a pass runs there, for a bank of `filters` values: below, what the kernel takes per stage, the packing
-// and the pass over marked tiles behind it count for more than its products.  Against the single-precision kernels, everything included,
-// over some 1400 drawn passes of unit strides: 0.7 - 1.2 of their speed at 4 - 6 GFLOP, more from 8 GFLOP on ((128,64,56,56) *
-// (64,64,3,3), 29.6 GFLOP: forward 232 -> 179 us; (16,45,16001) * (83,45,9): 180 -> 141; (64,512,7,7) * (512,512,3,3): 150 -> 114), but
-// (25,316,118) * (424,316,15), 9 GFLOP against two million values: 117 -> 108 and 130 -> 135.  Strided forward passes touch the more rows per
-// position: 0.4 - 1.1 of the speed in most.
-// MYGRAD_HIP_SPLIT_MIN=flops replaces the line, and takes away the rules on speed and accuracy below (tests; part of the plan key).
+// Flops from which a pass runs there, for a bank of `filters` values: below, what the kernel takes per stage,
+// the packing and the pass over marked tiles behind it count for more than its products.  Against the
+// single-precision kernels, everything included, over some 1400 drawn passes of unit strides: 0.7 - 1.2 of
+// their speed at 4 - 6 GFLOP, more from 8 GFLOP on ((128,64,56,56) * (64,64,3,3), 29.6 GFLOP: forward 232 ->
+// 179 us; (16,45,16001) * (83,45,9): 180 -> 141; (64,512,7,7) * (512,512,3,3): 150 -> 114), but (25,316,118) *
+// (424,316,15), 9 GFLOP against two million values: 117 -> 108 and 130 -> 135.  Strided forward passes touch
+// the more rows per position: 0.4 - 1.1 of the speed in most.  MYGRAD_HIP_SPLIT_MIN=flops replaces the line,
+// and takes away the rules on speed and accuracy below (tests; part of the plan key).
 double split_min_flops(double filters) {
   const char *v = getenv("MYGRAD_HIP_SPLIT_MIN");
   return v ? atof(v) : 8.0e9 + 2.0e3 * filters;
 }
 
-// How a pass would run on conv_split.hip: its phase, its stages' window and the rows of src that a tile of 128, 192 or 256
-// positions touches (0: more than the kernel has room for, with any tile of that width).
+// How a pass would run on conv_split.hip: its phase, its stages' window and the rows of src that a tile of 128,
+// 192 or 256 positions touches (0: more than the kernel has room for, with any tile of that width).
 inline long long up4(long long n) { return (n + 3) / 4 * 4; }
 struct SplitLayout {
   SplitPhase sp{};
@@ -1431,10 +1438,10 @@ struct SplitLayout {
   std::vector<int> first[3];  // see GemmParams::split_tiles
 };
 
-// The rows of src that `bn` consecutive positions touch at most, and each block's first one, when axes `inner` .. 2 are a stage's
-// window and the others' taps shift it as a whole.  A tap outside src touches nothing: along an axis of the window a position spans
-// from its first tap that may lie inside to the last.  (Positions need not ascend in rows: the data gradient has more of them
-// along an axis than the gradient has elements.)
+// The rows of src that `bn` consecutive positions touch at most, and each block's first one, when axes `inner`
+// .. 2 are a stage's window and the others' taps shift it as a whole.  A tap outside src touches nothing: along
+// an axis of the window a position spans from its first tap that may lie inside to the last.  (Positions need
+// not ascend in rows: the data gradient has more of them along an axis than the gradient has elements.)
 long long touched_rows(const SplitPhase &sp, const Phase &ph, int samples, const int *Q, int inner, int bn, std::vector<int> &first) {
   const int qs[3] = {Q[1] * Q[2], Q[2], 1};
   std::vector<int> low[3], high[3];
@@ -1467,8 +1474,8 @@ long long touched_rows(const SplitPhase &sp, const Phase &ph, int samples, const
 // bf16 parts, and how.
 bool split_applies(const Geometry &g, const Plan &pl, int rows, const Phase &ph, const int *Q, SplitLayout &lay) {
   const long long f = g.F + 31, c = g.C + 31;  // (the packed filters of either pass: 6 bytes a value, whole octets of 16 filters)
-  if (g.dtype != MG_F32 || !pl.tap_major || pl.table_rows || g.S[0] * g.S[1] * g.S[2] != 1 || conv_flops(g) < split_min_flops((double)g.F * g.C * g.wvol) || g.wvol < 3 ||
-      g.wvol > 31 || g.xvol < 2 || g.gvol < 2 || (long long)ph.npos * 8 > (32ll << 20) || f * c * g.wvol * 6 >= 1ll << 31 ||
+  if (g.dtype != MG_F32 || !pl.tap_major || pl.table_rows || g.S[0] * g.S[1] * g.S[2] != 1 ||
+      conv_flops(g) < split_min_flops((double)g.F * g.C * g.wvol) || g.wvol < 3 || g.wvol > 31 || g.xvol < 2 || g.gvol < 2 || (long long)ph.npos * 8 > (32ll << 20) || f * c * g.wvol * 6 >= 1ll << 31 ||
       (getenv("MYGRAD_HIP_TILE") && !getenv("MYGRAD_HIP_SPLIT_MIN")) || fold_applies(g, rows, pl.depth) || !split_on())
     return false;
   SplitPhase &sp = lay.sp;
@@ -1482,12 +1489,15 @@ bool split_applies(const Geometry &g, const Plan &pl, int rows, const Phase &ph,
   for (int inner = 0; inner < 3; ++inner) {
     int window = 1;
     for (int k = inner; k < 3; ++k) window *= sp.count[k];
-    // (a stage's elements are loaded, split and parked for its taps' products: with three taps that is what bounds it, (59,56,930) *
-    // (443,56,3), dx, 101 us on the other kernel, 145 here; the kernel itself takes three and more)
+    // (a stage's elements are loaded, split and parked for its taps' products: with three taps that is what
+    // bounds it, (59,56,930) * (443,56,3), dx, 101 us on the other kernel, 145 here; the kernel itself takes
+    // three and more)
     if (window < (getenv("MYGRAD_HIP_SPLIT_MIN") ? 3 : 5)) break;
     bool fits = false;
     for (int bn : {128, 192, 256}) {
-      const int width = split_width(bn), rows = (int)std::min(1ll << 20, (touched_rows(sp, ph, g.N, Q, inner, bn, lay.first[width]) + 3 + 15) / 16 * 16);
+      const int width = split_width(bn);
+      const long long touched = touched_rows(sp, ph, g.N, Q, inner, bn, lay.first[width]);
+      const int rows = (int)std::min(1ll << 20, (touched + 3 + 15) / 16 * 16);
       lay.patch[width] = rows <= split_patch_limit(bn == 256 ? 16 : 64, bn) ? rows : 0;
       fits |= lay.patch[width] > 0;
     }
@@ -1497,26 +1507,29 @@ bool split_applies(const Geometry &g, const Plan &pl, int rows, const Phase &ph,
   return false;
 }
 
-// Whether such a pass on tiles `split` (`stages` stages) is to be had, or the single-precision kernels stay with tiles `single` (`ktiles` K tiles of `bk`).
+// Whether such a pass on tiles `split` (`stages` stages) is to be had, or the single-precision kernels stay
+// with tiles `single` (`ktiles` K tiles of `bk`).
 bool split_pays(const SplitLayout &lay, const TileChoice &split, long long stages, const TileChoice &single, long long ktiles, int bk) {
   if (getenv("MYGRAD_HIP_SPLIT_MIN")) return true;
   const int depth = 16 * lay.sp.window;
-  // One rounding of a sum for 32 terms here, eight there: a third of the error on sums cut alike.  The single-precision plan cuts K into
-  // more slices where it has few tiles; where that would leave more than a quarter more to sum up without a break here, it stays.
+  // One rounding of a sum for 32 terms here, eight there: a third of the error on sums cut alike.  The
+  // single-precision plan cuts K into more slices where it has few tiles; where that would leave more than a
+  // quarter more to sum up without a break here, it stays.
   if (mean_chain(split, stages, split.blocks_per_cu) * depth > 1.25 * mean_chain(single, ktiles, single.blocks_per_cu) * bk) return false;
-  // Nor on tiles of many more rows, where the patches of 256 positions do not fit: (98,110,69,63) * (15,110,3,3) takes 188 us on tiles of
-  // 16 x 256, 281 here on 64 x 192.
+  // Nor on tiles of many more rows, where the patches of 256 positions do not fit: (98,110,69,63) *
+  // (15,110,3,3) takes 188 us on tiles of 16 x 256, 281 here on 64 x 192.
   if (4ll * split.m_tiles * split.bm > 5ll * single.m_tiles * single.bm) return false;
-  // Nor where the patches are large for their products, as under windows of five rows: (20,285,34,55) * (36,285,3,3), 16 x 256, 0.89 of the speed of
-  // three passes.  Of 1700 drawn passes that get here, 85 fall behind this line, as fast on the one as on the other on average, and the
-  // others gain a third; 20 of those lose more than the 3 % that a measurement is good for.
+  // Nor where the patches are large for their products, as under windows of five rows: (20,285,34,55) *
+  // (36,285,3,3), 16 x 256, 0.89 of the speed of three passes.  Of 1700 drawn passes that get here, 85 fall
+  // behind this line, as fast on the one as on the other on average, and the others gain a third; 20 of those
+  // lose more than the 3 % that a measurement is good for.
   return 1.05 * tile_time(split, stages, depth, 4, 0, split.blocks_per_cu, false, lay.patch[split_width(split.bn)]) <=
          tile_time(single, ktiles, bk, 4, 1, single.blocks_per_cu, false);
 }
 
-// The tables of a pass on conv_split.hip that contracts `channels` channels (pl.depth of them, with dead rows), `cstride` elements apart.
-// The table of positions is filled on the library's stream.
-// False where there is no memory for that table: such a pass stays on the single-precision kernels.
+// The tables of a pass on conv_split.hip that contracts `channels` channels (pl.depth of them, with dead rows),
+// `cstride` elements apart.  The table of positions is filled on the library's stream.  False where there is no
+// memory for that table: such a pass stays on the single-precision kernels.
 bool split_tables(Plan &pl, Tables &t, const SplitLayout &lay, int bn, const Phase &ph, const int *Q, int channels, long long cstride) {
   const int window = lay.sp.window;
   if (hipMalloc(&pl.pos_tab, (size_t)ph.npos * 8) != hipSuccess) {
@@ -1608,14 +1621,16 @@ int build_fwd_plan(const Geometry &g, Plan &pl) {
   for (int k = 0; k < 3; ++k) lay.sp.count[k] = g.W[k], lay.sp.d[k] = -g.P[k], lay.sp.step[k] = g.D[k];
   {
     const long long ktiles = pl.tap_major && !pl.table_rows ? g.wvol * (pl.depth / bk) : ceil_div((long long)g.C * g.wvol, bk);
-    TileChoice tc = choose_tile(g.F, {(long long)ph.npos}, (int)ktiles, pl.tap_major, g.dtype == MG_F64 ? 8 : 4, 1, bk, pl.table_rows, is_tiny(g));
+    TileChoice tc =
+        choose_tile(g.F, {(long long)ph.npos}, (int)ktiles, pl.tap_major, g.dtype == MG_F64 ? 8 : 4, 1, bk, pl.table_rows, is_tiny(g));
     if (split_applies(g, pl, g.F, ph, g.X, lay)) {
       const int stages = (int)(pl.depth / 16 * (g.wvol / lay.sp.window));
       const TileChoice split = choose_tile(g.F, {(long long)ph.npos}, stages, true, 4, 0, 16 * lay.sp.window, false, false, -1, lay.patch);
       pl.split = split_pays(lay, split, stages, tc, ktiles, bk) && split_tables(pl, t, lay, split.bn, ph, g.X, g.C, g.xvol);
       if (pl.split) tc = split;
     }
-    pl.bm = tc.bm, pl.bn = tc.bn, pl.m_tiles = tc.m_tiles, pl.full_tiles = tc.full_tiles, pl.tail_split = tc.tail_split, pl.blocks_per_cu = tc.blocks_per_cu;
+    pl.bm = tc.bm, pl.bn = tc.bn, pl.m_tiles = tc.m_tiles, pl.full_tiles = tc.full_tiles;
+    pl.tail_split = tc.tail_split, pl.blocks_per_cu = tc.blocks_per_cu;
     deepen_if_tiny(g, pl);
   }
   if (pl.table_rows) {
@@ -1798,8 +1813,8 @@ int build_dgrad_plan(const Geometry &g, Plan &pl) {
     }
   }
 
-  // ---- unit strides: the kernel on operands in three bf16 parts, where it applies (phases with different numbers of taps would need stages of
-  // their own each)
+  // ---- unit strides: the kernel on operands in three bf16 parts, where it applies (phases with different
+  // numbers of taps would need stages of their own each)
   if (nphase == 1 && found.size() == 1) {
     const PhaseTaps &pt = found[0];
     SplitLayout lay;
@@ -1815,7 +1830,8 @@ int build_dgrad_plan(const Geometry &g, Plan &pl) {
       const TileChoice tc = choose_tile(g.C, {npos}, stages, true, 4, 0, 16 * lay.sp.window, false, false, -1, lay.patch);
       pl.split = split_pays(lay, tc, stages, single, ktiles, bk) && split_tables(pl, t, lay, tc.bn, pt.ph, g.G, g.F, g.gvol);
       if (pl.split) {
-        pl.bm = tc.bm, pl.bn = tc.bn, pl.m_tiles = tc.m_tiles, pl.full_tiles = tc.full_tiles, pl.tail_split = tc.tail_split, pl.blocks_per_cu = tc.blocks_per_cu;
+        pl.bm = tc.bm, pl.bn = tc.bn, pl.m_tiles = tc.m_tiles, pl.full_tiles = tc.full_tiles;
+        pl.tail_split = tc.tail_split, pl.blocks_per_cu = tc.blocks_per_cu;
         Phase ph = pt.ph;
         ph.k_begin = 0, ph.blk_begin = 0;
         ph.k_count = (int)t.ktiles.size();
@@ -1912,7 +1928,8 @@ int build_dgrad_plan(const Geometry &g, Plan &pl) {
     set_divisors(coarse);
     const TileChoice tc = choose_tile((int)nphase * g.C, {(long long)coarse.npos}, coarse.k_count, true, g.dtype == MG_F64 ? 8 : 4, 1, bk, false, false);
     if (tc.bm != 0 && coarse.k_count > 0) {
-      pl.bm = tc.bm, pl.bn = tc.bn, pl.m_tiles = tc.m_tiles, pl.full_tiles = tc.full_tiles, pl.tail_split = tc.tail_split, pl.blocks_per_cu = tc.blocks_per_cu;
+      pl.bm = tc.bm, pl.bn = tc.bn, pl.m_tiles = tc.m_tiles, pl.full_tiles = tc.full_tiles;
+      pl.tail_split = tc.tail_split, pl.blocks_per_cu = tc.blocks_per_cu;
       pl.phase_rows = g.C;
       pl.phase_count = (int)nphase;
       pl.table_count = entries;
@@ -1997,7 +2014,8 @@ int build_dgrad_plan(const Geometry &g, Plan &pl) {
     set_divisors(coarse);
     const TileChoice tc = choose_tile(g.C, {(long long)coarse.npos}, (int)total_ktiles, true, 4, pl.nph, fbk, false, false);
     if (tc.bm != 0 && total_ktiles > 0) {
-      pl.bm = tc.bm, pl.bn = tc.bn, pl.m_tiles = tc.m_tiles, pl.full_tiles = tc.full_tiles, pl.tail_split = tc.tail_split, pl.blocks_per_cu = tc.blocks_per_cu;
+      pl.bm = tc.bm, pl.bn = tc.bn, pl.m_tiles = tc.m_tiles, pl.full_tiles = tc.full_tiles;
+      pl.tail_split = tc.tail_split, pl.blocks_per_cu = tc.blocks_per_cu;
       t.phases.push_back(coarse);
       pl.pos_blocks = (int)ceil_div(coarse.npos, pl.bn);
       return upload_plan(pl, t);
@@ -2031,7 +2049,8 @@ int build_dgrad_plan(const Geometry &g, Plan &pl) {
     }
     const TileChoice tc = choose_tile(g.C, npos, (int)std::max<long long>(min_ktiles, 0), pl.tap_major, g.dtype == MG_F64 ? 8 : 4, 1, bk, pl.table_rows,
                                       is_tiny(g), (int)(all_ktiles / std::max<long long>(all_pos, 1)));
-    pl.bm = tc.bm, pl.bn = tc.bn, pl.m_tiles = tc.m_tiles, pl.full_tiles = tc.full_tiles, pl.tail_split = tc.tail_split, pl.blocks_per_cu = tc.blocks_per_cu;
+    pl.bm = tc.bm, pl.bn = tc.bn, pl.m_tiles = tc.m_tiles, pl.full_tiles = tc.full_tiles;
+    pl.tail_split = tc.tail_split, pl.blocks_per_cu = tc.blocks_per_cu;
     deepen_if_tiny(g, pl);
   }
 
@@ -2689,8 +2708,9 @@ int pack_filters(const Geometry &g, const void *w, int mode, int depth, void **p
   return MG_OK;
 }
 
-// The filters of a plan on split operands (M rows of the product, `channels` channels contracted; row m's value under tap t of
-// channel c is w[m * m_stride + c * c_stride + t]) in the workspace; what the partial sums need follows.
+// The filters of a plan on split operands (M rows of the product, `channels` channels contracted; row m's value
+// under tap t of channel c is w[m * m_stride + c * c_stride + t]) in the workspace; what the partial sums need
+// follows.
 int pack_split(GemmParams &gp, const Plan &pl, const void *w, int M, int channels, long long m_stride, long long c_stride, void **partial) {
   gp.a_ld = (int)ceil_div(M, 16) * 16;
   gp.split_phases = pl.split_phases;
@@ -2712,8 +2732,8 @@ int pack_split(GemmParams &gp, const Plan &pl, const void *w, int M, int channel
   gp.split_w_bytes = (unsigned)((std::max(m_stride * M, c_stride * channels)) * sizeof(float));
   gp.split_w_mstride = (int)m_stride, gp.split_w_cstride = (int)c_stride;
   ScopedTiming timed(TAG_PACK_FILTERS);
-  launch_split_pack(static_cast<const float *>(w), scratch, pl.split_halves, pl.split_half_count, gp.redo, marks, M, channels, m_stride, c_stride, gp.a_ld,
-                    runtime().stream);
+  launch_split_pack(static_cast<const float *>(w), scratch, pl.split_halves, pl.split_half_count, gp.redo, marks, M, channels,
+                    m_stride, c_stride, gp.a_ld, runtime().stream);
   MG_HIP(hipGetLastError());
   return MG_OK;
 }

@@ -23,6 +23,25 @@ __device__ __forceinline__ TabEntry table_row(const int4v MG_CONSTANT *tab, int 
 // The wavefront-uniform value of x as a scalar register.
 __device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
 
+typedef int int8v __attribute__((ext_vector_type(8)));
+// A row of the phase table through the scalar data path (the index is wave-uniform).
+__device__ __forceinline__ Phase load_phase(const Phase *phases, int i) {
+  const int8v MG_CONSTANT *q = (const int8v MG_CONSTANT *)(phases + uniform(i));
+  const int8v a = q[0], b = q[1], c = q[2];
+  Phase ph;
+  ph.J[0] = a[0], ph.J[1] = a[1], ph.J[2] = a[2];
+  ph.o0[0] = a[3], ph.o0[1] = a[4], ph.o0[2] = a[5];
+  ph.k_begin = a[6], ph.k_count = a[7];
+  ph.blk_begin = b[0], ph.npos = b[1];
+  ph.by_jvol = FastDiv{(unsigned)b[2], (unsigned)b[3], (unsigned)b[4], 0u};
+  ph.by_j12 = FastDiv{(unsigned)b[6], (unsigned)b[7], (unsigned)c[0], 0u};
+  ph.by_j2 = FastDiv{(unsigned)c[2], (unsigned)c[3], (unsigned)c[4], 0u};
+  return ph;
+}
+__device__ __forceinline__ int phase_first_block(const Phase *phases, int i) {
+  return ((const int MG_CONSTANT *)(phases + uniform(i)))[8];
+}
+
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 

@@ -91,9 +91,10 @@ struct ShareFix {
   int tile, first_slot, slots, pad_;
 };
 
-// A phase of conv_split.hip.  Tap (a * count[1] + b) * count[2] + c reads at coordinate offsets d[0] + a * step[0],
-// d[1] + b * step[1], d[2] + c * step[2]; at most 31 of them.  A stage is 16 channels under `window` consecutive taps; tap t of the
-// window reads inner[t] rows (elements of a channel's plane) from the position's own, counted from the stage's row offset.
+// A phase of conv_split.hip.  Tap (a * count[1] + b) * count[2] + c reads at coordinate offsets d[0] + a *
+// step[0], d[1] + b * step[1], d[2] + c * step[2]; at most 31 of them.  A stage is 16 channels under `window`
+// consecutive taps; tap t of the window reads inner[t] rows (elements of a channel's plane) from the position's
+// own, counted from the stage's row offset.
 struct SplitPhase {
   int count[3], d[3], step[3];
   int window, inner_begin;  // inner_begin: into GemmParams::split_inner
@@ -173,8 +174,9 @@ struct GemmParams {
   int xcd_chunk;
   int phase_count;      // 0: off; else the number of stride phases (2 or 4)
   int phase_pairs;      // phases 2q, 2q + 1 are neighbours along the last axis of dst
-  // conv_split.hip: A is split into bf16 parts, a_ld a multiple of 16; ktiles holds stages, the names of KTile's fields aside:
-  // first half (tap of 16 channels) in A, channel offset, row offset, first tap, first channel, dead rows
+  // conv_split.hip: A is split into bf16 parts, a_ld a multiple of 16; ktiles holds stages, the names of
+  // KTile's fields aside:  first half (tap of 16 channels) in A, channel offset, row offset, first tap, first
+  // channel, dead rows
   const SplitPhase *split_phases;  // one per phase
   const int *split_inner;
   const int *split_tiles;  // per block of positions: the lowest row that any of its windows touches, a stage's row offset aside
@@ -184,13 +186,15 @@ struct GemmParams {
   const void *positions;  // row of src and taps of every position, 8 bytes each
   int npos;
   FastDiv by_sample;    // row -> sample
-  const void *split_w;  // the filter bank where it lies: row m's value under tap t of channel c at m * split_w_mstride + c * split_w_cstride + t
+  // the filter bank where it lies: row m's value under tap t of channel c at m * split_w_mstride + c * split_w_cstride + t
+  const void *split_w;
   unsigned split_w_bytes;
   unsigned *redo;  // whether there is a marked tile, then the marks, a bit each: see split_redo_kernel; cleared as the filters are packed
   int split_w_mstride, split_w_cstride;
 };
 
-// The table of positions of conv_split.hip (GemmParams::positions): positions (n, j) of J, sources at j + the taps' offsets in Q.
+// The table of positions of conv_split.hip (GemmParams::positions): positions (n, j) of J, sources at j + the
+// taps' offsets in Q.
 struct SplitPositions {
   int npos, J[3], Q[3];
   int sample_rows;
@@ -203,8 +207,8 @@ int split_patch_limit(int bm, int bn);
 int split_gemm_blocks_per_cu(int bm, int bn, int patch_rows);
 void launch_split_redo(const GemmParams &p, int bm, int bn, int tiles, hipStream_t s);
 bool launch_split_gemm(const GemmParams &p, int bm, int bn, bool odd, unsigned grid, hipStream_t s);
-void launch_split_pack(const float *w, void *packed, const void *halves, int count, unsigned *redo, int marks, int M, int channels, long long m_stride,
-                       long long c_stride, int ld, hipStream_t s);
+void launch_split_pack(const float *w, void *packed, const void *halves, int count, unsigned *redo, int marks, int M, int channels,
+                       long long m_stride, long long c_stride, int ld, hipStream_t s);
 void launch_split_positions(const SplitPositions &p, void *out, hipStream_t s);
 
 // Gather-GEMM with one position per lane, for few rows (the data gradient of a layer with a

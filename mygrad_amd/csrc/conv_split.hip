@@ -3,37 +3,44 @@
 //
 // v_mfma_f32_16x16x4_f32 does 157 TFLOP/s at best on this device and shares its issue with the vector
 // ALU (44 vector instructions next to 16 of them: 154 -> 110 TFLOP/s); v_mfma_f32_16x16x32_bf16 does
-// 1800 - 2000 and does not.  A float is the sum of three bf16 numbers exactly (8 + 8 + 8 bits of its
-// significand), x = x0 + x1 + x2, and
+// 1800 - 2000 and does not.  A float is the sum of three bf16 numbers (8 + 8 + 8 bits of its significand;
+// below 2^-110 see "what the split cannot represent"), x = x0 + x1 + x2, and
 //   x * w = x0 w0 + (x0 w1 + x1 w0) + (x0 w2 + x1 w1 + x2 w0) + at most 2^-24 |x w|,
 // six products, each exact in single precision: an effective peak of 300 - 330 TFLOP/s.
 //
-// Precision.  The large product and the five small ones have an accumulator each, added at the end.  An accumulator rounds once per
-// 32 terms of a product, whatever the terms are, and loses some bits of what it adds; in one accumulator for all six that
-// made sums of few terms less accurate than the single-precision instruction, which rounds only where a term is not zero.
-// Error against 64 bits (2-norm), one accumulator / two / single precision, (128,64,56,56) * (64,64,3,3):
-//   normal values 3.5e-7 / 1.4e-7 / 4.2e-7; behind a relu 3.4e-7 / 1.2e-7 / 3.0e-7; one element in 100 not zero 9.8e-8 / 3.7e-8 /
-//   4.9e-8; one product a sum 4.2e-8 / 2.6e-8 / 2.5e-8 (there what the six products leave out shows: no result is off by more than
-//   2^-23 of itself, where one rounding is 2^-24).
-// Two accumulators of 64 x 64 wave tiles do not fit 256 registers (70 - 85 of them spill: 186 us below become 246), those of 64 x 48 do but for
-// a dozen values that no step needs.
+// Precision.  The large product and the five small ones have an accumulator each, added at the end.  An
+// accumulator rounds once per 32 terms of a product, whatever the terms are, and loses some bits of what it
+// adds; in one accumulator for all six that made sums of few terms less accurate than the single-precision
+// instruction, which rounds only where a term is not zero.  Error against 64 bits (2-norm), (128,64,56,56) *
+// (64,64,3,3), one accumulator / two / single precision:
+//   normal values                    3.5e-7 / 1.4e-7 / 4.2e-7
+//   behind a relu                    3.4e-7 / 1.2e-7 / 3.0e-7
+//   one element in 100 not zero      9.8e-8 / 3.7e-8 / 4.9e-8
+//   one product a sum                4.2e-8 / 2.6e-8 / 2.5e-8
+// (In the last row what the six products leave out shows: no result is off by more than 2^-23 of itself, where
+// one rounding is 2^-24.)  Two accumulators of 64 x 64 wave tiles do not fit 256 registers (70 - 85 of them
+// spill: 186 us below become 246), those of 64 x 48 do but for a dozen values that no step needs.
 //
-// What bounds it: (128,64,56,56) * (64,64,3,3), 29.6 GFLOP, takes 178 - 194 us with its packing and the pass over marked tiles, from device to device
-// (single precision 232), some 165 - 180 by itself: 165 - 180 TFLOP/s of the 300.  Operands from LDS (64 x 48 and 48 x 64 waves: 21 reads of 16 bytes a lane for 72 matrix
-// instructions, 58 % of its bandwidth; 32 x 64 ones 18 for 48, 75 %: 201 us), and the turn between stages, where the waves of a block wait for
-// the patch to be split and parked; loads are hidden.  Smaller planes have smaller patches: (128,128,28,28) * (128,128,3,3), 29.6 GFLOP,
-// 230 -> 161 us; (16,96,16001) * (48,96,9), 21.2 GFLOP, 172 -> 130.
+// What bounds it: (128,64,56,56) * (64,64,3,3), 29.6 GFLOP, takes 178 - 194 us with its packing and the pass
+// over marked tiles on most devices (single precision 232), 164 - 166 by itself, 180 TFLOP/s of the 300; 194 by
+// itself on one where the filter gradient takes 280 us instead of 233.  Matrix pipes are busy 43 % of the
+// cycles, LDS 38 % (64 x 48 and 48 x 64 waves: 21 reads of 16 bytes a lane for 72 matrix instructions; 32 x 64
+// ones 18 for 48: 201 us for 186), the waves wait for 37 % of theirs: the turn between stages, where a block's
+// waves wait for the patch to be split and parked; loads are hidden.  Smaller planes have smaller patches:
+// (128,128,28,28) * (128,128,3,3), 29.6 GFLOP, 230 -> 161 us; (16,96,16001) * (48,96,9), 21.2 GFLOP, 172 -> 130.
 //
-// What the split cannot represent.  An infinite operand leaves Inf - Inf in
-// its second part and makes every sum that it takes part in a NaN, as an infinite or NaN operand or an overflow makes
-// it something not finite in any arithmetic.  And parts are multiples of 2^-133, the smallest number of bf16 (which the instruction takes as
-// it is, like every product and sum below 2^-126): of an operand below 2^-110 bits may be lost, below 2^-134 all of them.  K such losses
-// times the largest value of the other operand are less than the last bit of a sum of K * 2^-109 times that value.  So where a block has
-// a sum that is not finite, or has lost bits of an element or seen a filter value below 2^-109 and has a sum, zero included, below that bound,
-// it marks its tile, and split_redo_kernel computes marked tiles again on the single-precision instruction.  The bits of other
-// tiles do not depend on it, and few marked tiles cost little: the forward pass below 194 us as it is, 205 with one NaN, 252 with one sample in 20 of
-// values about 1e-38, 811 where every tile is marked (single precision 232).  (The whole pass on the single-precision kernels, three launches that
-// returned at once otherwise, took 381 for the first odd value and 9 more for none.)
+// What the split cannot represent.  An infinite operand leaves Inf - Inf in its second part and makes every sum
+// that it takes part in a NaN, as an infinite or NaN operand or an overflow makes it something not finite in
+// any arithmetic.  And parts are multiples of 2^-133, the smallest number of bf16 (which the instruction takes
+// as it is, like every product and sum below 2^-126): of an operand below 2^-110 bits may be lost, below 2^-134
+// all of them.  K such losses times the largest value of the other operand are less than the last bit of a sum
+// of K * 2^-109 times that value.  So where a block has a sum that is not finite, or has lost bits of an
+// element or seen a filter value below 2^-109 and has a sum, zero included, below that bound, it marks its
+// tile, and split_redo_kernel computes marked tiles again on the single-precision instruction.  The bits of
+// other tiles do not depend on it, and few marked tiles cost little: the forward pass below 194 us as it is,
+// 205 with one NaN, 252 with one sample in 20 of values about 1e-38, 811 where every tile is marked (single
+// precision 232).  (The whole pass on the single-precision kernels, three launches that returned at once
+// otherwise, took 381 for the first odd value and 9 more for none.)
 #include "conv_device.h"
 #include "conv_kernels.h"
 #include "internal.h"
@@ -53,7 +60,6 @@ typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-typedef int int8v __attribute__((ext_vector_type(8)));
 typedef int int16v __attribute__((ext_vector_type(16)));
 static_assert(sizeof(KTile) == sizeof(int8v) && sizeof(SplitPhase) == sizeof(int16v), "table rows");
 
@@ -66,11 +72,12 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void *base, un
 __device__ __forceinline__ unsigned bits_of(float v) { return __builtin_bit_cast(unsigned, v); }
 __device__ __forceinline__ float float_of(unsigned v) { return __builtin_bit_cast(float, v); }
 
-// a = h[0] + m[0] + l[0] and b likewise, exactly.  Every part is rounded to nearest (the last one, of at most eight bits, needs
-// none): x1 is at most 2^-8 of x and x2 2^-17, so what the six products leave out, x1 w2 + x2 w1 + x2 w2, is at most 2^-24 of x w and
-// has no sign of its own (with the first part cut off instead it was up to 2^-22).  A value that rounds to infinity leaves a
-// NaN in its second part.  Eleven vector instructions for two values.
-// The low sixteen bits of `lost` are set where the last part has lost some (see the head of the file).
+// a = h[0] + m[0] + l[0] and b likewise, exactly.  Every part is rounded to nearest (the last one, of at most
+// eight bits, needs none): x1 is at most 2^-8 of x and x2 2^-17, so what the six products leave out, x1 w2 + x2
+// w1 + x2 w2, is at most 2^-24 of x w and has no sign of its own (with the first part cut off instead it was up
+// to 2^-22).  A value that rounds to infinity leaves a NaN in its second part.  Eleven vector instructions for
+// two values.  The low sixteen bits of `lost` are set where the last part has lost some (see the head of the
+// file).
 __device__ __forceinline__ void split_pair(float a, float b, unsigned &h, unsigned &m, unsigned &l, unsigned &lost) {
   h = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{a, b}), bf16x2));
   const float ra = a - float_of(h << 16), rb = b - float_of(h & 0xffff0000u);
@@ -83,23 +90,6 @@ __device__ __forceinline__ void split_pair(float a, float b, unsigned &h, unsign
 // What a block finds out about an item's operands and sums, bit by bit.
 enum : unsigned { kNotFinite = 1, kLostElement = 2, kTinyFilter = 4, kLostSum = 8 };
 constexpr unsigned short kTinyBits = 18 << 7;  // 2^-109 in bf16
-
-__device__ __forceinline__ Phase load_phase(const Phase *phases, int i) {
-  const int8v MG_CONSTANT *q = (const int8v MG_CONSTANT *)(phases + uniform(i));
-  const int8v a = q[0], b = q[1], c = q[2];
-  Phase ph;
-  ph.J[0] = a[0], ph.J[1] = a[1], ph.J[2] = a[2];
-  ph.o0[0] = a[3], ph.o0[1] = a[4], ph.o0[2] = a[5];
-  ph.k_begin = a[6], ph.k_count = a[7];
-  ph.blk_begin = b[0], ph.npos = b[1];
-  ph.by_jvol = FastDiv{(unsigned)b[2], (unsigned)b[3], (unsigned)b[4], 0u};
-  ph.by_j12 = FastDiv{(unsigned)b[6], (unsigned)b[7], (unsigned)c[0], 0u};
-  ph.by_j2 = FastDiv{(unsigned)c[2], (unsigned)c[3], (unsigned)c[4], 0u};
-  return ph;
-}
-__device__ __forceinline__ int phase_first_block(const Phase *phases, int i) {
-  return ((const int MG_CONSTANT *)(phases + uniform(i)))[8];
-}
 
 // the element of dst at position ipos of the phase, row 0
 __device__ __forceinline__ float *dst_of(const GemmParams &p, const Phase &ph, int ipos) {
@@ -135,7 +125,8 @@ __global__ void __launch_bounds__(64 * MW * NW, WM == 16 ? 3 : 2) split_gemm_ker
   static_assert(WM % 16 == 0, "16 x 16 tiles");
   constexpr int PIECES = 12 * BM;  // of 16 bytes: a step's filters, [part][octet of K rows][row]
   constexpr int ALOADS = (PIECES + THREADS - 1) / THREADS;
-  // [2][PIECES] filters, then the patch: [octet of channels][row][part], p.patch_rows + 1 rows, the last one zeros; and three words (note)
+  // [2][PIECES] filters, then the patch: [octet of channels][row][part], p.patch_rows + 1 rows, the last one
+  // zeros; and three words (note)
   extern __shared__ __attribute__((aligned(16))) u32x4 lds[];
   u32x4 *const patch = lds + 2 * PIECES;
 
@@ -149,9 +140,12 @@ __global__ void __launch_bounds__(64 * MW * NW, WM == 16 ? 3 : 2) split_gemm_ker
     bool partial;
     Phase ph;
   };
-  // of the item, this lane's: bits lost of the elements that it has split, the smallest |filter value| that it has parked, less one (zeros aside)
+  // of the item, this lane's: bits lost of the elements that it has split, the smallest |filter value| that it
+  // has parked, less one (zeros aside)
   unsigned lost = 0;
   u16x2 tiniest = {0xffff, 0xffff};
+  // The walk over items is tap_gemm_kernel's.  (Shared by the two in a struct it changes that kernel's allocation of
+  // scalar registers: a 4096 x 4096 x 4096 product and its gradients 2931 -> 2943 us, where two runs differ by 0.3 %.)
   const bool shares = p.share_first != nullptr;
   const int share_begin = shares ? ((const int MG_CONSTANT *)p.share_first)[uniform((int)blockIdx.x)] : 0;
   const int share_end = shares ? ((const int MG_CONSTANT *)p.share_first)[uniform((int)blockIdx.x) + 1] : 0;
@@ -207,7 +201,8 @@ __global__ void __launch_bounds__(64 * MW * NW, WM == 16 ? 3 : 2) split_gemm_ker
   const unsigned piece_row = (unsigned)p.a_ld * 16u;  // bytes of one part of one octet of packed filters
   const unsigned c_step = (unsigned)p.src_cstride * 4u;
   const int octet_rows = p.patch_rows + 1;
-  unsigned *const note = reinterpret_cast<unsigned *>(patch + 2 * octet_rows * 3);  // what was found, the widest filter value, the widest element
+  // what was found, the widest filter value, the widest element
+  unsigned *const note = reinterpret_cast<unsigned *>(patch + 2 * octet_rows * 3);
   if (threadIdx.x < 6) patch[((int)threadIdx.x / 3 * octet_rows + p.patch_rows) * 3 + (int)threadIdx.x % 3] = u32x4{0, 0, 0, 0};
   int pi = 0;
   Item me;
@@ -218,9 +213,10 @@ __global__ void __launch_bounds__(64 * MW * NW, WM == 16 ? 3 : 2) split_gemm_ker
   int8v patch_e = {0, 0, 0, 0, 0, 0, 0, 0};  // first half, channel offset, row offset, first tap, first channel, dead rows
   bool patch_real = false;
   auto first_of = [&](const Item &it) -> int { return ((const int MG_CONSTANT *)p.split_tiles)[uniform(it.pos0 / BN)]; };
-  // A part of the patch's loads.  A thread takes four rows of four channels in each round; the rows begin on a multiple of four and therefore
-  // lie in one sample (a sample's rows are numbered up to a multiple of four; what is loaded for those beyond its last is of no use to
-  // anyone), and are loaded as one vector, whatever its alignment: 16 bytes a lane take the vector cache 16 cycles, 4 bytes 8 - 11.
+  // A part of the patch's loads.  A thread takes four rows of four channels in each round; the rows begin on a
+  // multiple of four and therefore lie in one sample (a sample's rows are numbered up to a multiple of four;
+  // what is loaded for those beyond its last is of no use to anyone), and are loaded as one vector, whatever
+  // its alignment: 16 bytes a lane take the vector cache 16 cycles, 4 bytes 8 - 11.
   const int quads = p.patch_rows / 4;
   auto quarter_of = [&](int idx) -> int { return (idx >= quads) + (idx >= 2 * quads) + (idx >= 3 * quads); };  // of the stage's channels
   auto request_part = [&](int k) {
@@ -236,7 +232,8 @@ __global__ void __launch_bounds__(64 * MW * NW, WM == 16 ? 3 : 2) split_gemm_ker
 #pragma unroll
     for (int u = 0; u < CHANNELS; ++u) {
       const int r = k * CHANNELS % 4 + u;
-      raw[round][r] = __builtin_amdgcn_raw_buffer_load_b128(src_buf, (int)(at | ((dead << (31 - r)) & kOutside)), (int)((unsigned)r * c_step), 0);
+      const unsigned lane_at = at | ((dead << (31 - r)) & kOutside);
+      raw[round][r] = __builtin_amdgcn_raw_buffer_load_b128(src_buf, (int)lane_at, (int)((unsigned)r * c_step), 0);
     }
   };
   auto park_patch = [&] {
@@ -272,7 +269,8 @@ __global__ void __launch_bounds__(64 * MW * NW, WM == 16 ? 3 : 2) split_gemm_ker
     const int window = sp[9];  // taps of the inner window
     const int inner = p.split_inner[sp[10] + min(lane, window - 1)];  // lane t: row offset of the window's tap t
 
-    // ---- this lane's positions: their row in the patch and the taps they have (bit by bit; none beyond the last position)
+    // ---- this lane's positions: their row in the patch and the taps they have (bit by bit; none beyond the
+    // last position)
     const int first_row = first_of(me);
     int row_at[TN];
     unsigned taps[TN];
@@ -348,7 +346,8 @@ __global__ void __launch_bounds__(64 * MW * NW, WM == 16 ? 3 : 2) split_gemm_ker
       }
     };
     int x_at[TN], x_next[TN];  // of the step under way and the one after it: 16-byte pieces from the start of the patch
-    // tap0: number of the window's first tap; q: first tap of the step within it; lead: rows of the patch ahead of the tile's first one
+    // tap0: number of the window's first tap; q: first tap of the step within it; lead: rows of the patch ahead
+    // of the tile's first one
     auto place = [&](int tap0, int q, bool single, int lead) {
       const int off0 = __builtin_amdgcn_readlane(inner, q), off1 = __builtin_amdgcn_readlane(inner, single ? q : q + 1);
       const int off = (second ? off1 : off0) + lead;
@@ -375,11 +374,13 @@ __global__ void __launch_bounds__(64 * MW * NW, WM == 16 ? 3 : 2) split_gemm_ker
       }
     };
 
-    // One K step (`step_no` of the item) whose operands' first position is in x[0] and whose filters are in w; the next step
-    // starts at tap `q_next` of its window, `single_next`: it is a window's odd last tap.  `turn`: the stage ends here.
+    // One K step (`step_no` of the item) whose operands' first position is in x[0] and whose filters are in w;
+    // the next step starts at tap `q_next` of its window, `single_next`: it is a window's odd last tap.
+    // `turn`: the stage ends here.
     bf16x8 x[2][3];
     int step_no = 0;
-    auto step = [&](auto single_c, auto turn_c, auto single_next_c, int half_after, int tap0_next, int q_next, int lead_next, int stage, int parts) {
+    auto step = [&](auto single_c, auto turn_c, auto single_next_c, int half_after, int tap0_next, int q_next, int lead_next,
+                    int stage, int parts) {
       constexpr bool SINGLE = decltype(single_c)::value, TURN = decltype(turn_c)::value, NEXT = decltype(single_next_c)::value;
       // smallest first; x0 w0 alone into the sum of large products, for a sum of a few of those is exact
       constexpr int PRODUCTS = SINGLE ? 4 : 6;
@@ -392,8 +393,9 @@ __global__ void __launch_bounds__(64 * MW * NW, WM == 16 ? 3 : 2) split_gemm_ker
         } else {
           park_filters((step_no + 1) & 1);
           __syncthreads();  // the next step's filters are there; nobody reads this one's patch any more
-          // the patch's loads are spread over the steps (all at once they fill the vector cache's queue, and every wave waits for
-          // memory there: 8000 cycles), ahead of the filters' so that parking those waits for nothing younger
+          // the patch's loads are spread over the steps (all at once they fill the vector cache's queue, and
+          // every wave waits for memory there: 8000 cycles), ahead of the filters' so that parking those waits
+          // for nothing younger
           if constexpr (!SINGLE) {
 #pragma unroll
             for (int k = 0; k < 4; ++k)
@@ -507,8 +509,9 @@ __global__ void __launch_bounds__(64 * MW * NW, WM == 16 ? 3 : 2) split_gemm_ker
         unsigned widest = 0;
         if ((found & kLostElement) != 0) {
           for (int at = (int)threadIdx.x; at < stages * window * 2 * BM; at += THREADS) {
-            const u32x4 firsts = __builtin_amdgcn_raw_buffer_load_b128(
-                a_buf, me.m0 + at % BM < p.a_ld ? (int)((unsigned)((table[0][0] * 2 + at / BM) * 3) * piece_row + (unsigned)(me.m0 + at % BM) * 16u) : (int)kOutside, 0, 0);
+            const int m = me.m0 + at % BM, octet = table[0][0] * 2 + at / BM;
+            const unsigned from = m < p.a_ld ? (unsigned)(octet * 3) * piece_row + (unsigned)m * 16u : kOutside;
+            const u32x4 firsts = __builtin_amdgcn_raw_buffer_load_b128(a_buf, (int)from, 0, 0);
 #pragma unroll
             for (int e = 0; e < 4; ++e) widest = max(widest, max((firsts[e] & 0x7fffu) << 16, firsts[e] & 0x7fff0000u));
           }
@@ -594,12 +597,14 @@ __global__ void __launch_bounds__(64 * MW * NW, WM == 16 ? 3 : 2) split_gemm_ker
   }
 }
 
-// The marked tiles (bm x bn, of one phase) of split_gemm_kernel again, on the single-precision instruction.  Where few are marked a block takes up
-// to 32 rows by 32 positions of one at a time, its waves a share of K each, which they add up in order: one marked tile is the work of
-// twelve blocks.  Where many are, a wave takes 16 TM rows by 64 positions over the whole of K.  Elements are gathered one by one (a tap that a
-// position does not have reads zero, as in the patch).  Filter values are the sums of their parts, which lie together as lanes want them,
-// but for lanes that find one among theirs which the parts do not hold.  Seldom anything to do: 4.5 us behind every pass.  Not built for the last
-// bit of speed: a step waits for its own loads (four parts of some 16 us a block is where the one way meets the other).
+// The marked tiles (bm x bn, of one phase) of split_gemm_kernel again, on the single-precision instruction.
+// Where few are marked a block takes up to 32 rows by 32 positions of one at a time, its waves a share of K
+// each, which they add up in order: one marked tile is the work of twelve blocks.  Where many are, a wave takes
+// 16 TM rows by 64 positions over the whole of K.  Elements are gathered one by one (a tap that a position does
+// not have reads zero, as in the patch).  Filter values are the sums of their parts, which lie together as
+// lanes want them, but for lanes that find one among theirs which the parts do not hold.  Seldom anything to
+// do: 4.5 us behind every pass.  Not built for the last bit of speed: a step waits for its own loads (four
+// parts of some 16 us a block is where the one way meets the other).
 constexpr int kRedoWaves = 8, kRedoBlocks = 512;  // a power of two
 
 template <int TM>
@@ -633,7 +638,8 @@ __global__ void __launch_bounds__(64 * kRedoWaves, 2) split_redo_kernel(const Ge
 #pragma unroll
     for (int j = 0; j < COLS; ++j) {
       typedef int int2v __attribute__((ext_vector_type(2)));
-      const int2v at = __builtin_bit_cast(int2v, __builtin_amdgcn_raw_buffer_load_b64(table_buf, (int)((unsigned)(pos0 + j * 16 + l16) * 8u), 0, 0));
+      const unsigned ipos = (unsigned)(pos0 + j * 16 + l16);
+      const int2v at = __builtin_bit_cast(int2v, __builtin_amdgcn_raw_buffer_load_b64(table_buf, (int)(ipos * 8u), 0, 0));
       row_at[j] = at[0];
       taps[j] = (unsigned)at[1];
     }
@@ -655,8 +661,10 @@ __global__ void __launch_bounds__(64 * kRedoWaves, 2) split_redo_kernel(const Ge
         const unsigned at = (n * (unsigned)p.src_nstride + (unsigned)(row - (int)n * p.sample_rows + here[1] + octet * 8 * p.src_cstride)) * 4u;
         const unsigned from = has_tap && ((taps[j] >> (here[3] + q)) & 1u) != 0 ? at : kOutside;
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-          xs[j][e] = float_of(__builtin_amdgcn_raw_buffer_load_b32(src_buf, (int)(from | ((dead << (31 - e)) & kOutside)), (int)((unsigned)(e * p.src_cstride) * 4u), 0));
+        for (int e = 0; e < 8; ++e) {
+          const unsigned lane_at = from | ((dead << (31 - e)) & kOutside), channel_at = (unsigned)(e * p.src_cstride) * 4u;
+          xs[j][e] = float_of(__builtin_amdgcn_raw_buffer_load_b32(src_buf, (int)lane_at, (int)channel_at, 0));
+        }
       }
       float ws[ROWS][8];
 #pragma unroll
@@ -677,9 +685,11 @@ __global__ void __launch_bounds__(64 * kRedoWaves, 2) split_redo_kernel(const Ge
         }
         if (!whole) {
 #pragma unroll
-          for (int e = 0; e < 8; ++e)
-            ws[i][e] = float_of(__builtin_amdgcn_raw_buffer_load_b32(
-                w_buf, (int)((unsigned)(m * p.split_w_mstride + (here[4] + octet * 8 + e) * p.split_w_cstride + here[3] + q) * 4u | ((dead << (31 - e)) & kOutside)), 0, 0));
+          for (int e = 0; e < 8; ++e) {
+            const int c = here[4] + octet * 8 + e;
+            const unsigned from = (unsigned)(m * p.split_w_mstride + c * p.split_w_cstride + here[3] + q) * 4u;
+            ws[i][e] = float_of(__builtin_amdgcn_raw_buffer_load_b32(w_buf, (int)(from | ((dead << (31 - e)) & kOutside)), 0, 0));
+          }
         }
       }
 #pragma unroll
@@ -752,14 +762,16 @@ __global__ void __launch_bounds__(64 * kRedoWaves, 2) split_redo_kernel(const Ge
 }
 
 // The filters of split_gemm_kernel, in three parts: piece [octet of K rows][part][m] holds the eight bf16
-// values of K rows 8 * octet .. + 7 of row m of the product, `ld` (a multiple of 16) pieces to a row.  Sixteen K rows
-// are 16 channels from c0 on under one tap, named by halves[K row / 16] = (c0, tap): row m's value is w[m * m_stride + c * c_stride + tap],
-// zero for c >= channels and m >= M.  A value that is not zero has a first part that is not, the smallest number of bf16 at least: that is how
-// split_gemm_kernel knows of those that have lost bits.  Also clears the marks of tiles, `marks` words of them.
+// values of K rows 8 * octet .. + 7 of row m of the product, `ld` (a multiple of 16) pieces to a row.  Sixteen
+// K rows are 16 channels from c0 on under one tap, named by halves[K row / 16] = (c0, tap): row m's value is
+// w[m * m_stride + c * c_stride + tap], zero for c >= channels and m >= M.  A value that is not zero has a
+// first part that is not, the smallest number of bf16 at least: that is how split_gemm_kernel knows of those
+// that have lost bits.  Also clears the marks of tiles, `marks` words of them.
 __global__ void __launch_bounds__(256) split_pack_kernel(const float *__restrict__ w, u32x4 *__restrict__ packed, const int2 *__restrict__ halves,
                                                          int count, unsigned *__restrict__ redo, int marks, int M, int channels, long long m_stride,
                                                          long long c_stride, int ld) {
-  for (unsigned i = (blockIdx.y * gridDim.x + blockIdx.x) * 256 + threadIdx.x; i < (unsigned)marks; i += gridDim.x * gridDim.y * 256) redo[i] = 0;
+  const unsigned block = blockIdx.y * gridDim.x + blockIdx.x, blocks = gridDim.x * gridDim.y;
+  for (unsigned i = block * 256 + threadIdx.x; i < (unsigned)marks; i += blocks * 256) redo[i] = 0;
   const int oct = blockIdx.x * 16 + (int)(threadIdx.x >> 4), m = blockIdx.y * 16 + (int)(threadIdx.x & 15);
   if (oct >= 2 * count) return;
   const int2 h = halves[oct / 2];
@@ -783,8 +795,8 @@ __global__ void __launch_bounds__(256) split_pack_kernel(const float *__restrict
   for (int part = 0; part < 3; ++part) packed[((long long)oct * 3 + part) * ld + m] = parts[part];
 }
 
-// (row, taps) of every position: the row of src (sample * sample_rows + element of a channel's plane) that its window starts
-// from, padding aside, and which taps have an element there, bit by bit.
+// (row, taps) of every position: the row of src (sample * sample_rows + element of a channel's plane) that its
+// window starts from, padding aside, and which taps have an element there, bit by bit.
 __global__ void __launch_bounds__(256) split_positions_kernel(const SplitPositions p, int2 *__restrict__ out) {
   const int idx = blockIdx.x * 256 + threadIdx.x;
   if (idx >= p.npos) return;
@@ -801,12 +813,14 @@ __global__ void __launch_bounds__(256) split_positions_kernel(const SplitPositio
   out[idx] = int2{n * p.sample_rows + (q0 * p.Q[1] + q1) * p.Q[2] + q2, (int)taps};
 }
 
-// rows of a wave; waves along the rows of a tile; 16 positions of a wave; waves along the positions; rounds of a patch (the fewest that hold it)
+// rows of a wave; waves along the rows of a tile; 16 positions of a wave; waves along the positions; rounds of
+// a patch (the fewest that hold it)
 #define MG_SPLIT_SHAPES(X) \
   X(32, 4, 4, 2, 1) X(64, 1, 3, 4, 2) X(32, 2, 4, 2, 1) X(32, 2, 4, 2, 2) X(48, 1, 4, 4, 2) X(32, 1, 4, 4, 2) X(16, 1, 4, 4, 2)
 
-// Rows of a patch that a tile has room for: those of its threads' rounds, and two blocks share a unit's LDS (alone on
-// it, a block's waves wait for their barriers: 256 filters, 3x3, stride 2, 27x27 161 us on patches of 540 rows, 134 on the other kernel).
+// Rows of a patch that a tile has room for: those of its threads' rounds, and two blocks share a unit's LDS
+// (alone on it, a block's waves wait for their barriers: 256 filters, 3x3, stride 2, 27x27 161 us on patches of
+// 540 rows, 134 on the other kernel).
 constexpr int patch_limit(int bm, int threads, int rounds) {
   const int held = threads * rounds, room = (80 * 1024 / 16 - 24 * bm - 1) / 6 - 1;
   return held < room ? held : room;
@@ -858,14 +872,18 @@ bool launch_split_gemm(const GemmParams &p, int bm, int bn, bool odd, unsigned g
 }
 
 void launch_split_redo(const GemmParams &p, int bm, int bn, int tiles, hipStream_t s) {
-  const auto kernel = bm % 64 == 0 ? split_redo_kernel<4> : bm == 48 ? split_redo_kernel<3> : bm == 32 ? split_redo_kernel<2> : split_redo_kernel<1>;
+  const auto kernel = bm % 64 == 0 ? split_redo_kernel<4>
+                      : bm == 48   ? split_redo_kernel<3>
+                      : bm == 32   ? split_redo_kernel<2>
+                                   : split_redo_kernel<1>;
   hipLaunchKernelGGL(kernel, dim3(kRedoBlocks), dim3(64 * kRedoWaves), 0, s, p, bm, bn, tiles);
 }
 
-void launch_split_pack(const float *w, void *packed, const void *halves, int count, unsigned *redo, int marks, int M, int channels, long long m_stride,
-                       long long c_stride, int ld, hipStream_t s) {
+void launch_split_pack(const float *w, void *packed, const void *halves, int count, unsigned *redo, int marks, int M, int channels,
+                       long long m_stride, long long c_stride, int ld, hipStream_t s) {
   hipLaunchKernelGGL(split_pack_kernel, dim3((unsigned)ceil_div(2 * count, 16), (unsigned)(ld / 16)), dim3(256), 0, s, w,
-                     static_cast<u32x4 *>(packed), static_cast<const int2 *>(halves), count, redo, marks, M, channels, m_stride, c_stride, ld);
+                     static_cast<u32x4 *>(packed), static_cast<const int2 *>(halves), count, redo, marks, M, channels, m_stride,
+                     c_stride, ld);
 }
 
 void launch_split_positions(const SplitPositions &p, void *out, hipStream_t s) {
