@@ -41,6 +41,9 @@ if ROOT not in sys.path:
     sys.path.insert(0, ROOT)
 
 PEAK_TFLOPS = {"f32": 157.3, "f64": 78.6}  # MI355X dense matrix peaks
+# A single-precision pass whose operands are in three bf16 parts issues six bf16 products for each of its own: a
+# sixth of the dense bf16 matrix peak.
+PEAK_SPLIT_TFLOPS = 2500.0 / 6
 PEAK_HBM_GBS = 8000.0
 
 # name -> definition.  "lit" shapes use the flooring placement of the window
@@ -241,6 +244,11 @@ def describe(name):
     lead, pooled, grid = pool_shapes(wl)
     how = "argmax recomputed from x in bwd" if wl.get("recompute") else "argmax kept from fwd, one byte per window"
     return f"{name}: max_pool {wl['dtype']} x{wl['x']} pool{wl['pool']} stride{wl['stride']} -> grid{grid} fwd+bwd ({how})"
+
+
+def peak_of(plan, peak):
+    """The peak that a pass with this plan note is priced against; `peak` unless it runs on another instruction."""
+    return PEAK_SPLIT_TFLOPS if plan.endswith("three bf16 parts") else peak
 
 
 class Step:
@@ -538,7 +546,7 @@ def run_gpu(name, steps, warmup, prewarm=None, time_every=None):
 
     step = Step(name)
     # The device clock climbs for a few hundred milliseconds after an idle period (measured:
-    # 2.15 - 2.3 GHz during the first tens of milliseconds of work, 2.38 - 2.40 GHz from then on,
+    # 2.15 - 2.3 GHz during the first tens of milliseconds of work, 2.37 - 2.46 GHz from then on,
     # see profiles/conv3a_sustained.txt): run the step untimed until it has settled, so that the
     # timed steps show the rate a job sustains rather than the ramp.
     prewarm = PREWARM_SECONDS if prewarm is None else prewarm
@@ -549,6 +557,11 @@ def run_gpu(name, steps, warmup, prewarm=None, time_every=None):
             step()
         _hip.synchronize()
         prewarmed += 10
+    pass_peak = {}
+    if step.wl["kind"] == "conv":
+        for _, fn, key in step.passes():
+            fn()
+            pass_peak[key] = peak_of(_hip.last_plan(), step.peak)
     for _ in range(warmup):
         step()
     _hip.synchronize()
@@ -589,7 +602,7 @@ def run_gpu(name, steps, warmup, prewarm=None, time_every=None):
         if k in roof["work"]:
             info["achieved"] = roof["work"][k] * roof["scale"] / (info["avg_ms"] * 1e-3)
             info["unit"] = roof["unit"]
-            info["frac"] = info["achieved"] / roof["peak"]
+            info["frac"] = info["achieved"] / pass_peak.get(k, roof["peak"])
             if moved:
                 info["on_definition_bytes"] = step.work[k] * roof["scale"] / (info["avg_ms"] * 1e-3)
     dominant = max((k for k in kernels if k in roof["work"]), key=lambda k: kernels[k]["avg_ms"] * kernels[k]["launches"])
@@ -618,7 +631,7 @@ def run_gpu(name, steps, warmup, prewarm=None, time_every=None):
             "bound": roof["bound"],
             "kernel": dominant,
             "achieved": dom["achieved"],
-            "peak": roof["peak"],
+            "peak": pass_peak.get(dominant, roof["peak"]),
             "unit": roof["unit"],
             "frac": dom["frac"],
             "traffic": traffic,
@@ -639,6 +652,8 @@ def short_plan(note):
         return note.split(": ", 1)[-1]
     family, tile, phases, fused, splits = m.group(2), m.group(3), int(m.group(4)), int(m.group(5)), int(m.group(6))
     extra = (f", {phases} phases" + (f" ({fused} fused)" if fused > 1 else "")) if phases > 1 else ""
+    if note.endswith("three bf16 parts"):
+        extra += ", three bf16 parts"
     return f"{family} {tile}{extra}" + (f", {splits} K splits" if m.group(1) == "wgrad" else "")
 
 
@@ -680,12 +695,12 @@ def run_sweep(names, steps=20, prewarm=0.25):
                     break
                 reps *= 4
             host_ms = elapsed / reps * 1e3
-            work = work_of[key]
+            work, peak = work_of[key], peak_of(plan, step.peak)
             rows.append({
                 "shape": name, "dtype": wl["dtype"], "kind": wl["kind"], "pass": label, "plan": plan, "launches": len(records) / steps,
                 "host_us": host_ms * 1e3, "kernel_us": kernel_ms * 1e3, "work": work, "unit": step.unit,
-                "achieved": work * step.scale / (host_ms * 1e-3), "frac": work * step.scale / (host_ms * 1e-3) / step.peak,
-                "kernel_frac": work * step.scale / (kernel_ms * 1e-3) / step.peak,
+                "achieved": work * step.scale / (host_ms * 1e-3), "frac": work * step.scale / (host_ms * 1e-3) / peak,
+                "kernel_frac": work * step.scale / (kernel_ms * 1e-3) / peak,
                 "small": wl["kind"] == "conv" and min(wl["x"][1], wl["w"][0]) < 32,
             })
         if wl["kind"] == "pool":

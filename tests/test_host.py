@@ -775,3 +775,14 @@ assert lib.mg_memcpy_d2h(back.ctypes.data, large.ptr + 16, 4096) == ok and np.ar
 print("refused")
 """
     assert "refused" in run_on_standins(tmp_path, program)
+
+
+def test_benchmark_prices_a_pass_against_the_instruction_that_runs_it():
+    import bench
+
+    plain = "fwd: tap-major tile 64x256x16, 1 phase(s) (1 fused per tile), 1568 position blocks x 1 row tiles, 1536 whole tiles + tail split 8, 2 block(s) per unit, K splits 1"
+    split = plain.replace("x16,", "x32,") + ", three bf16 parts"
+    assert bench.peak_of(plain, 157.3) == 157.3
+    # six bf16 products each: the conv3a layer's 29.6 GFLOP in 165 us are 179 TFLOP/s, less than the peak they have
+    assert 179 < bench.peak_of(split, 157.3) == 2500 / 6
+    assert bench.short_plan(split) == bench.short_plan(plain).replace("x16", "x32") + ", three bf16 parts"
