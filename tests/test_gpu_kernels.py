@@ -1621,7 +1621,7 @@ SPLIT_RULES = [
 
 
 @pytest.mark.parametrize("rule", range(len(SPLIT_RULES)))
-def test_which_passes_run_on_three_bf16_parts(abi, rule):
+def test_which_passes_run_on_three_bf16_parts(abi, monkeypatch, rule):
     from mygrad_amd import _hip
 
     x_shape, w_shape, p, split = SPLIT_RULES[rule]
@@ -1631,14 +1631,23 @@ def test_which_passes_run_on_three_bf16_parts(abi, rule):
     plan = _hip.last_plan()
     print(plan, flush=True)
     assert plan.endswith("three bf16 parts") == split
+    single = None
+    if split:
+        monkeypatch.setenv("MYGRAD_HIP_SPLIT", "0")
+        single = abi.conv_fwd(x, w, (1,) * len(p), p, (1,) * len(p))
+        assert not _hip.last_plan().endswith("three bf16 parts")
     # 200 of the results, each from its window; single precision rounds once a term, 2.5e-8 of the sum as it stands on average
     padded = np.pad(x, ((0, 0), (0, 0), *((q, q) for q in p)))
     flat = w.reshape(w_shape[0], -1).astype(np.float64)
     terms = flat.shape[1]
-    off = norm = 0.0
+    off = norm = off_single = 0.0
     for _ in range(200):
         n, *at = (rng.integers(size) for size in (x_shape[0], *out.shape[2:]))
         window = padded[(n, slice(None), *(slice(i, i + k) for i, k in zip(at, w_shape[2:])))]
         ref = flat @ window.reshape(-1).astype(np.float64)
         off, norm = off + np.sum((out[(n, slice(None), *at)] - ref) ** 2), norm + np.sum(ref**2)
+        if split:
+            off_single += np.sum((single[(n, slice(None), *at)] - ref) ** 2)
     assert np.sqrt(off / norm) <= 1.25 * 2.5e-8 * np.sqrt(terms / 2)
+    # no further off than the single-precision instruction, which rounds eight times as often
+    assert not split or off <= off_single
