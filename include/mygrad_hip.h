@@ -371,7 +371,7 @@ int mg_strided_copy(int elem_bytes, int nd, const int64_t *shape, const int64_t 
 
 /* out[b] = a @ x[b], a:(M, K) shared by the batch, x:(batch, K, N), out:(batch, M, N), all
  * C-contiguous.  Runs as the convolution of x with M one-tap filters (the same implicit-GEMM
- * kernels; the reduction has length K).  A stack of left operands times one right operand,
+ * kernels; the reduction has length K), a large float32 product on three bf16 parts instead.  A stack of left operands times one right operand,
  * (batch, M, K) @ (K, N), is the same call with batch = 1 and M := batch * M.
  * Replaces np.matmul in MatMul.__call__, src/mygrad/math/misc/ops.py:91-93. */
 int mg_matmul(int dtype, int64_t batch, int64_t M, int64_t K, int64_t N, const void *a, const void *x, void *out);

@@ -16,6 +16,7 @@
 #include "conv_device.h"
 #include "conv_kernels.h"
 #include "internal.h"
+#include "product_split.h"
 
 #include <algorithm>
 #include <array>
@@ -3138,23 +3139,44 @@ int matmul_desc(const char *who, int dtype, int64_t batch, int64_t M, int64_t K,
   d->X[MG_MAX_ND - 1] = d->G[MG_MAX_ND - 1] = N;
   return MG_OK;
 }
+
+// Whether the convolution's entry points would take the call (they say what is wrong with it if not), in float32.
+bool product_ready(const mg_conv_desc &d, const void *first, const void *second, const void *result) {
+  Geometry g;
+  return runtime().ready && d.dtype == MG_F32 && first && second && result && check_desc(&d, &g) == MG_OK;
+}
 }  // namespace
 
 int mg_matmul(int dtype, int64_t batch, int64_t M, int64_t K, int64_t N, const void *a, const void *x, void *out) {
   mg_conv_desc d;
   if (int rc = matmul_desc("mg_matmul", dtype, batch, M, K, N, &d)) return rc;
+  std::lock_guard<std::recursive_mutex> guard(api_mutex());
+  if (product_ready(d, a, x, out) && product_applies(M, batch * N, ceil_div(K, 8))) {
+    const int rc = product_forward(batch, M, K, N, a, x, out);
+    if (rc != MG_ERR_UNSUPPORTED) return rc;
+  }
   return mg_conv_fwd(&d, x, a, out);
 }
 
 int mg_matmul_da(int dtype, int64_t batch, int64_t M, int64_t K, int64_t N, const void *grad, const void *x, void *da) {
   mg_conv_desc d;
   if (int rc = matmul_desc("mg_matmul_da", dtype, batch, M, K, N, &d)) return rc;
+  std::lock_guard<std::recursive_mutex> guard(api_mutex());
+  if (product_ready(d, grad, x, da) && product_applies(M, K, batch * ceil_div(N, 8))) {
+    const int rc = product_da(batch, M, K, N, grad, x, da);
+    if (rc != MG_ERR_UNSUPPORTED) return rc;
+  }
   return mg_conv_wgrad(&d, grad, x, da);
 }
 
 int mg_matmul_dx(int dtype, int64_t batch, int64_t M, int64_t K, int64_t N, const void *grad, const void *a, void *dx) {
   mg_conv_desc d;
   if (int rc = matmul_desc("mg_matmul_dx", dtype, batch, M, K, N, &d)) return rc;
+  std::lock_guard<std::recursive_mutex> guard(api_mutex());
+  if (product_ready(d, grad, a, dx) && product_applies(K, batch * N, ceil_div(M, 8))) {
+    const int rc = product_dx(batch, M, K, N, grad, a, dx);
+    if (rc != MG_ERR_UNSUPPORTED) return rc;
+  }
   return mg_conv_dgrad(&d, grad, a, dx);
 }
 

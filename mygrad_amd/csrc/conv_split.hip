@@ -44,6 +44,7 @@
 #include "conv_device.h"
 #include "conv_kernels.h"
 #include "internal.h"
+#include "split_device.h"
 
 #include <algorithm>
 #include <array>
@@ -54,38 +55,8 @@ namespace mg {
 
 namespace {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 typedef int int16v __attribute__((ext_vector_type(16)));
 static_assert(sizeof(KTile) == sizeof(int8v) && sizeof(SplitPhase) == sizeof(int16v), "table rows");
-
-constexpr unsigned kOutside = 0x80000000u;  // a byte offset past the end of any tensor (each below 2 GiB): reads as zero
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void *base, unsigned bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)bytes, 0x00020000);
-}
-
-__device__ __forceinline__ unsigned bits_of(float v) { return __builtin_bit_cast(unsigned, v); }
-__device__ __forceinline__ float float_of(unsigned v) { return __builtin_bit_cast(float, v); }
-
-// a = h[0] + m[0] + l[0] and b likewise, exactly.  Every part is rounded to nearest (the last one, of at most
-// eight bits, needs none): x1 is at most 2^-8 of x and x2 2^-17, so what the six products leave out, x1 w2 + x2
-// w1 + x2 w2, is at most 2^-24 of x w and has no sign of its own (with the first part cut off instead it was up
-// to 2^-22).  A value that rounds to infinity leaves a NaN in its second part.  Eleven vector instructions for
-// two values.  The low sixteen bits of `lost` are set where the last part has lost some (see the head of the
-// file).
-__device__ __forceinline__ void split_pair(float a, float b, unsigned &h, unsigned &m, unsigned &l, unsigned &lost) {
-  h = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{a, b}), bf16x2));
-  const float ra = a - float_of(h << 16), rb = b - float_of(h & 0xffff0000u);
-  m = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{ra, rb}), bf16x2));
-  const float qa = ra - float_of(m << 16), qb = rb - float_of(m & 0xffff0000u);
-  l = __builtin_amdgcn_perm(bits_of(qb), bits_of(qa), 0x07060302u);
-  lost |= bits_of(qa) | bits_of(qb);
-}
 
 // What a block finds out about an item's operands and sums, bit by bit.
 enum : unsigned { kNotFinite = 1, kLostElement = 2, kTinyFilter = 4, kLostSum = 8 };

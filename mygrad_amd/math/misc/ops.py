@@ -3,7 +3,8 @@
 A matrix product is a convolution whose window has one element: ``a @ b`` with ``a:(M, K)``
 and ``b:(K, N)`` is the convolution of ``b`` -- K channels, N positions -- with M filters, and
 its two gradients are the convolution's.  The operation therefore runs on the convolution's
-implicit-GEMM kernels (``mg_matmul*`` in ``libmygrad_hip.so``) with no kernel of its own.
+implicit-GEMM kernels (``mg_matmul*`` in ``libmygrad_hip.so``); large float32 products on three
+bf16 parts have kernels of their own there.
 
 Operand patterns that run: both operands at most 2-D (vectors are promoted like
 ``np.matmul`` does); one operand a stack and the other at most 2-D (one launch: the stack is

@@ -80,6 +80,83 @@ def test_results_repeat_exactly(abi):
         assert np.array_equal(fn(*args), fn(*args))
 
 
+# (batch, M, K, N) of products on three bf16 parts: one value; one past, and short of, a panel of 128, a tile of 256 and a K step of 32, with
+# octets that end early; whole rounds of tiles and a rest that blocks share; batches along the columns and along the terms
+PARTS = [(1, 1, 1, 1), (1, 129, 31, 257), (1, 255, 33, 127), (2, 100, 65, 515), (3, 300, 129, 77), (1, 384, 1000, 640), (1, 4200, 40, 4100), (1, 96, 5000, 70)]
+
+
+@pytest.mark.parametrize("batch, M, K, N", PARTS)
+def test_large_products_on_three_bf16_parts(abi, monkeypatch, batch, M, K, N):
+    from mygrad_amd import _hip
+
+    rng = np.random.default_rng([7, batch, M, K, N])
+
+    def run(a, x, g, parts=True):
+        monkeypatch.setenv("MYGRAD_HIP_SPLIT", "1" if parts else "0")
+        monkeypatch.setenv("MYGRAD_HIP_SPLIT_MIN", "0")
+        results = []
+        for fn, args in ((abi.matmul, (a, x)), (abi.matmul_da, (g, x, M)), (abi.matmul_dx, (g, a))):
+            results.append(fn(*args))
+            assert ("three bf16 parts" in _hip.last_plan()) == parts
+        return results
+
+    def exact(a, x, g):
+        a, x, g = (v.astype(np.float64) for v in (a, x, g))
+        return a @ x, sum(g[b] @ x[b].T for b in range(batch)), a.T @ g
+
+    normal = lambda *shape: rng.standard_normal(shape).astype(np.float32)
+    a, x, g = normal(M, K), normal(batch, K, N), normal(batch, M, N)
+    # small integers: every sum is exact, and no value of a neighbour is in it
+    ints = [rng.integers(-2, 3, v.shape).astype(np.float32) for v in (a, x, g)]
+    whole = run(*ints)
+    for got, ref in zip(whole, exact(*ints)):
+        assert np.array_equal(got, ref)
+    # a sum of large products rounds off once in 32 terms, 5.06e-8 of itself as it stands then (cut off towards zero: 2^-23 * E[m^-2]^1/2 /
+    # 3^1/2, significands m spread evenly in their logarithm), what is left out of it and the last roundings 3.5e-8
+    plain, refs, terms = run(a, x, g, parts=False), exact(a, x, g), (K, batch * N, M)
+    for got, single, ref, count in zip(run(a, x, g), plain, refs, terms):
+        off = np.linalg.norm(got - ref)
+        assert off <= (1.25 * 5.06e-8 * np.sqrt(-(-count // 32) / 2) + 3.5e-8) * np.linalg.norm(ref)
+        # no further off than the single-precision instruction, which rounds once in a term
+        assert count < 30 or off <= np.linalg.norm(single - ref)
+    # one product a sum, the low bits of an operand below the smallest number of bf16 or not: what the six products leave out is 2^-24 of
+    # it, the five small ones round off 2^-29 each and the last sum 2^-24
+    few = np.zeros_like(a)
+    few[np.arange(min(M, K)), np.arange(min(M, K))] = rng.uniform(1, 2, min(M, K))
+    for tiny, other in ((1.0, 1.0), (1e-41, 3e4), (1e-38, 3e4), (1e-35, 3e36)):
+        for left, right in ((tiny, other), (other, tiny)):
+            args = few * np.float32(left), x * np.float32(right), g * np.float32(right)
+            for i in (0, 2):
+                got, ref = run(*args)[i], exact(*args)[i]
+                assert np.all(np.abs(got - ref) <= (2 + 5 / 32) * 2.0**-24 * np.abs(ref) + 2.0**-149)
+    # infinities, NaN and sums that overflow are those of single precision
+    for value in (np.inf, np.nan, 3e38):
+        odd = [v.copy() for v in (a * np.float32(4), x, g)]
+        for v in odd[1:]:
+            v[0, 0, 0] = value
+        odd[0][-1, -1] = value
+        with np.errstate(all="ignore"):
+            for got, single in zip(run(*odd), run(*odd, parts=False)):
+                finite = np.isfinite(single)
+                assert not finite.all() and np.array_equal(got[~finite], single[~finite], equal_nan=True)
+                assert np.all(np.isfinite(got[finite]))
+    for got, was in zip(run(*ints), whole):
+        assert np.array_equal(got, was)
+
+
+@pytest.mark.parametrize("sizes, parts", [((4096, 4096, 1024), (True, True, True)), ((1411, 3000, 3000), (True, True, True)),
+                                          ((72, 8611, 3924), (False, False, False)), ((1024, 1024, 1024), (False, False, False)),
+                                          ((4096, 24, 8192), (False, False, False))])
+def test_which_products_run_on_three_bf16_parts(abi, sizes, parts):
+    from mygrad_amd import _hip
+
+    M, K, N = sizes
+    a, x, g = (np.ones(shape, np.float32) for shape in ((M, K), (1, K, N), (1, M, N)))
+    for fn, args, terms, expected in zip((abi.matmul, abi.matmul_da, abi.matmul_dx), ((a, x), (g, x, M), (g, a)), (K, N, M), parts):
+        assert np.all(fn(*args) == terms)
+        assert ("three bf16 parts" in _hip.last_plan()) == expected
+
+
 BATCHED = [(1, 1, 1, 1), (3, 16, 16, 16), (5, 17, 3, 33), (2, 1, 70, 1), (300, 8, 8, 8), (7, 64, 40, 48), (4, 33, 6, 2), (2, 5, 0, 4),
            (3, 100, 129, 50),
            # 32 x 32 results or more per pair: 64 x 64 tiles staged in LDS -- whole tiles, ragged edges in M, N
