@@ -17,6 +17,7 @@
 #include "conv_kernels.h"
 #include "internal.h"
 #include "product_split.h"
+#include "wgrad_split.h"
 
 #include <algorithm>
 #include <array>
@@ -581,6 +582,8 @@ struct Plan {
   int split_half_count = 0, patch_rows = 0;
   bool split_odd = false;        // an odd number of taps per stage
   int split_npos = 0;            // positions (pos_tab: 8 bytes each)
+  WgradSplitPlan wsplit;         // filter gradient on three bf16 parts (wgrad_split.hip): fw != 0
+  unsigned *words = nullptr;     // kWgradSplitWords words of memory, zero between calls
   bool single_dense_phase = false;  // positions enumerate the destination tensor in order
   bool table_rows = false;          // tap-major kernel whose K tiles are rows of the gather table (channel count no multiple of the K tile)
   int table_count = 0;              // data gradient on table rows: rows of the (padded) table = rows of the packed filters
@@ -1151,7 +1154,7 @@ int upload_plan(Plan &pl, Tables &t) {
   const size_t off_si = off_sp + padded_bytes(t.split_phases);
   const size_t off_st = off_si + padded_bytes(t.split_inner);
   const size_t off_sh = off_st + padded_bytes(t.split_tiles);
-  const size_t total = off_sh + padded_bytes(t.split_halves) + 256;
+  const size_t off_words = off_sh + padded_bytes(t.split_halves), total = off_words + kWgradSplitWords * 4;
   std::vector<char> host(total, 0);
   auto put = [&](size_t off, const void *src, size_t n) {
     if (n) memcpy(host.data() + off, src, n);
@@ -1177,6 +1180,7 @@ int upload_plan(Plan &pl, Tables &t) {
   }
   char *base = static_cast<char *>(pl.blob);
   pl.zeros = base;  // the first 256 bytes stay zero: target of padding loads
+  pl.words = reinterpret_cast<unsigned *>(base + off_words);
   pl.tab = reinterpret_cast<TabEntry *>(base + off_tab);
   pl.arow = reinterpret_cast<int *>(base + off_arow);
   pl.phases = reinterpret_cast<Phase *>(base + off_ph);
@@ -2229,6 +2233,13 @@ int build_pos_table(const Geometry &g, Plan &pl) {
   return MG_OK;
 }
 
+// Whether a filter gradient may run on three bf16 parts.
+bool wgrad_split_applies(const Geometry &g, const Plan &pl) {
+  const char *least = getenv("MYGRAD_HIP_SPLIT_MIN");
+  return g.dtype == MG_F32 && pl.tap_major && split_on() && (!getenv("MYGRAD_HIP_WGRAD_TILE") || least) &&
+         conv_flops(g) >= (least ? atof(least) : 4e9);
+}
+
 int build_wgrad_plan(const Geometry &g, Plan &pl) {
   Tables t;
   const bool f64 = g.dtype == MG_F64;
@@ -2294,6 +2305,7 @@ int build_wgrad_plan(const Geometry &g, Plan &pl) {
   auto fits = [&](const Cand &c) { return c.bm - g.F < 16; };
   auto chunk_of = [&](const Cand &c, long long sp) { return ceil_div(ceil_div(kpos, c.bk), sp) * c.bk; };
   long long best_splits = 1;
+  double single_time = 0;  // modelled, us
   pl.bm = 0;
   // MYGRAD_HIP_WGRAD_TILE="rows,columns" (diagnostics and the tests of every tile shape; part of the
   // plan's key): that candidate or, where it does not apply, the usual choice
@@ -2345,6 +2357,7 @@ int build_wgrad_plan(const Geometry &g, Plan &pl) {
       if (c == usual) consider(usual_splits);
     }
     pl.run_tiles = (int)std::max<long long>(1, std::min<long long>(1024, chunk_of(*usual, usual_splits)) / pl.bk);
+    single_time = least;
   }
   pl.tap_major = pl.bm != 0;
   if (!pl.tap_major) {
@@ -2410,7 +2423,20 @@ int build_wgrad_plan(const Geometry &g, Plan &pl) {
     fwd_table(g, t.tab);
   }
   if (int rc = upload_plan(pl, t)) return rc;
-  return build_pos_table(g, pl);
+  if (int rc = build_pos_table(g, pl)) return rc;
+  if (wgrad_split_applies(g, pl)) {
+    pl.wsplit = plan_wgrad_split(g.N, g.C, g.F, g.X, g.G, g.W, g.S, g.D, g.P, cus);
+    // Table rows: 0.57 of the instruction's rate (0.40 - 0.66, 59 layers).  With a tenth in favour of the single-precision kernels
+    // 106 of 362 drawn layers of 4 - 30 GFLOP run on parts, 1.18 times as fast in the mean, 3 % slower or more in 8 of them: most
+    // of those with eight or nine taps to a tile, few with fewer, of which the tile's other products are of no use
+    // ((69,205,38,11) * (481,205,3,1) 755 us on parts, 168 without).
+    if (pl.table_rows) {
+      const double padded = 2.0 * (double)(ceil_div(g.F, pl.bm) * pl.bm) * (double)(col_tiles * pl.bn) * (double)kpos;
+      single_time = 8.0 + padded / (0.57 * 157.3e6);
+    }
+    if (!getenv("MYGRAD_HIP_SPLIT_MIN") && pl.wsplit.time > 0.9 * (pl.table_rows ? single_time : 1.05 * single_time)) pl.wsplit = WgradSplitPlan();
+  }
+  return MG_OK;
 }
 
 void free_tables(Plan &pl) {
@@ -2430,6 +2456,7 @@ int get_plan(ConvOp op, const mg_conv_desc *d, const Geometry &g, Plan **out) {
   if (const char *least = getenv("MYGRAD_HIP_SPLIT_MIN")) key.append("m").append(least);
   if (const char *tile = getenv("MYGRAD_HIP_TILE")) key.append(tile);
   if (const char *tile = getenv("MYGRAD_HIP_WGRAD_TILE")) key.append("w").append(tile);
+  if (const char *tile = getenv("MYGRAD_HIP_SPLIT_TILE")) key.append("v").append(tile);
   if (const char *row = getenv("MYGRAD_HIP_FUSE_MIN_ROW")) key.append("r").append(row);
   if (const char *limit = getenv("MYGRAD_HIP_BUFFER_LIMIT")) key.append("b").append(limit);
   auto it = plans().find(key);
@@ -2457,6 +2484,9 @@ int get_plan(ConvOp op, const mg_conv_desc *d, const Geometry &g, Plan **out) {
              pl.thin ? "one position per lane" : pl.tap_major ? "tap-major" : "table-driven", pl.table_rows ? ", table rows" : pl.phase_rows ? ", stride phases as rows" : "",
              pl.fold_row ? ", folded taps" : "", pl.bm, pl.bn, pl.split ? 32 : pl.bk, pl.nphases, pl.nph, pl.pos_blocks, pl.m_tiles, pl.full_tiles, tail,
              pl.blocks_per_cu, pl.splits, pl.split ? ", three bf16 parts" : "");
+    if (pl.wsplit.fw != 0)
+      snprintf(pl.note, sizeof pl.note, "wgrad: tile %dx%d of 16 channels by 9 taps, %d quads of %d rows, %d ahead, %d tasks, %d segments, %d tiles, K splits %d, %.0f us, three bf16 parts",
+               32 * pl.wsplit.fw, pl.wsplit.cw, pl.wsplit.p.quads, pl.wsplit.p.rows, pl.wsplit.p.depth, pl.wsplit.tasks, 1 << pl.wsplit.p.seg_shift, pl.wsplit.p.tiles, pl.wsplit.p.splits, pl.wsplit.time);
     // MYGRAD_HIP_TRACE=1 reports, once per new descriptor, what was planned
     static const bool trace = getenv("MYGRAD_HIP_TRACE") != nullptr;
     if (trace) fprintf(stderr, "[mygrad_hip] plan %s (K chunk %d)\n", pl.note, pl.kchunk);
@@ -2984,9 +3014,17 @@ int conv_wgrad_impl(const Geometry &g, const Plan &pl, const void *grad, const v
   const bool staged = pl.splits > 1 || (pl.tap_major && !pl.table_rows && g.wvol > 1);
   const int ct = (int)((staged ? pl.depth : g.C) * g.wvol);
   void *target = dw;
-  if (staged)
-    if (int rc = workspace((size_t)pl.splits * g.F * ct * sizeof(T), &target)) return rc;
   WgradParams wp{};
+  const size_t parts_bytes = pl.wsplit.fw != 0 ? wgrad_split_scratch(pl.wsplit) : 0;
+  void *scratch = nullptr;
+  if (staged || parts_bytes != 0) {
+    if (int rc = workspace(parts_bytes + (staged ? (size_t)pl.splits * g.F * ct * sizeof(T) : 0), &scratch)) return rc;
+    if (staged) target = static_cast<char *>(scratch) + parts_bytes;
+    if (parts_bytes != 0) {  // (the kernel below is then for a gradient that the parts cannot hold)
+      wp.gate = pl.words;
+      if (int rc = launch_wgrad_split(pl.wsplit, grad, x, scratch, pl.words, s)) return rc;
+    }
+  }
   wp.grad = grad;
   wp.x = x;
   wp.out = target;
@@ -3041,6 +3079,10 @@ int conv_wgrad_impl(const Geometry &g, const Plan &pl, const void *grad, const v
     if (!launched) return fail(MG_ERR_UNSUPPORTED, "no filter-gradient kernel for tile %d x %d", pl.bm, pl.bn);
   }
   MG_HIP(hipGetLastError());
+  if (parts_bytes != 0) {
+    const WgradSums single{staged ? static_cast<const float *>(target) : nullptr, pl.splits, ct, pl.tap_major && !pl.table_rows};
+    return launch_wgrad_split_reduce(pl.wsplit, single, dw, scratch, pl.words, s);
+  }
   if (staged) {
     const int count = g.F * ct;
     ScopedTiming timed(TAG_WGRAD_REDUCE);

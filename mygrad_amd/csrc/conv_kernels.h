@@ -287,6 +287,7 @@ struct WgradParams {
   // shift_from on are the last, shifted channel block; column col there is channel col - col_shift.
   int shift_from, col_shift;
   int run_tiles;  // K tiles that an accumulator sums up before they are added to the total (tap-major, single precision)
+  const unsigned *gate;  // tap-major kernels: not null: there is something to do only where it is not zero (see wgrad_split.h)
 };
 
 }  // namespace mg

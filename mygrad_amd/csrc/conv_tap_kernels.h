@@ -1009,6 +1009,7 @@ __global__ void __launch_bounds__(256) tail_fixup_kernel(const GemmParams p) {
 // the position table whenever the plan has one.
 template <typename T, int BM, int BN, int BK, int WM, int WN, bool WIDE, bool TABLE = false, bool POS = false>
 __global__ void __launch_bounds__(512) tap_wgrad_kernel(const WgradParams p) {
+  if (p.gate != nullptr && *p.gate == 0) return;
   static_assert(TABLE || !POS, "POS selects between the two forms of the TABLE kernel");
   static_assert((BM / WM) * (BN / WN) == 4, "four wavefronts per block");
   static_assert(256 % BK == 0 && BK % 16 == 0 && BN % 16 == 0, "K tile");

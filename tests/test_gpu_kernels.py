@@ -1651,3 +1651,89 @@ def test_which_passes_run_on_three_bf16_parts(abi, monkeypatch, rule):
     assert np.sqrt(off / norm) <= 1.25 * 2.5e-8 * np.sqrt(terms / 2)
     # no further off than the single-precision instruction, which rounds eight times as often
     assert not split or off <= off_single
+
+
+# (x, w, stride, padding, dilation, tile): filter gradients on three bf16 parts, a kernel each (waves along filters, column tiles, quads of a row)
+SPLIT_GRADIENTS = [
+    ((8, 64, 9, 17), (64, 64, 3, 3), (1, 1), (1, 1), (1, 1), "2,2,2"),        # whole tiles; rows that end among four columns
+    ((5, 17, 13, 30), (70, 17, 2, 7), (1, 1), (0, 3), (1, 1), "2,2,2"),       # 14 taps: two chunks; runs of columns; one channel past a group
+    ((16, 33, 14, 13), (65, 33, 3, 3), (1, 2), (1, 1), (1, 1), "2,2,2"),      # strided: two tasks a wave; three column tiles
+    ((9, 16, 5, 7, 12), (33, 16, 3, 3, 3), (2, 1, 1), (1, 1, 0), (1, 1, 2), "1,2,4"),  # planes of a volume that are outside
+    ((8, 32, 11, 20), (31, 32, 2, 3), (1, 1), (1, 1), (1, 1), "1,2,2"),       # two rows a stage
+    ((8, 16, 27, 27), (130, 16, 3, 3), (2, 2), (1, 1), (1, 1), "4,2,1"),      # every other row and column; one column tile for two
+    ((3, 48, 12, 67), (40, 48, 3, 3), (1, 1), (1, 1), (1, 1), "1,1,8"),
+    ((1, 40, 6, 45), (32, 40, 1, 3), (1, 1), (0, 1), (1, 1), "1,1,4"),        # one sample: eight runs of columns
+    ((8, 45, 501), (83, 45, 9), (1,), (4,), (1,), "1,1,8"),                   # along the only axis
+    ((3, 16, 1003), (64, 16, 4), (1,), (2,), (2,), "2,2,2"),
+    ((2, 30, 301), (20, 30, 5), (2,), (0,), (2,), "1,2,4"),
+    ((64, 16, 1, 5), (16, 16, 1, 3), (1, 1), (0, 1), (1, 1), "1,1,8"),        # fewer columns than a stage has
+]
+
+
+@pytest.mark.parametrize("problem", range(len(SPLIT_GRADIENTS)))
+def test_filter_gradients_on_three_bf16_parts(abi, monkeypatch, problem):
+    from mygrad_amd import _hip
+
+    x_shape, w_shape, s, p, d, tile = SPLIT_GRADIENTS[problem]
+    rng = np.random.default_rng(3600 + problem)
+
+    def gradient(g, x, split=True):
+        with monkeypatch.context() as m:
+            m.setenv("MYGRAD_HIP_SPLIT_MIN", "0")
+            m.setenv("MYGRAD_HIP_SPLIT", "1" if split else "0")
+            m.setenv("MYGRAD_HIP_SPLIT_TILE", tile)
+            dw = abi.conv_wgrad(g, x, w_shape, s, p, d)
+            plan = _hip.last_plan()
+            print(plan, flush=True)
+            assert plan.endswith("three bf16 parts") == split
+        return dw
+
+    xi = rng.integers(-3, 4, x_shape).astype(np.float32)
+    grid = direct.conv_forward(xi, np.zeros(w_shape, np.float32), s, p, d).shape
+    gi = rng.integers(-2, 3, grid).astype(np.float32)
+    # small integers: every sum is exact
+    want = direct.conv_backward_w(gi, xi, w_shape, s, p, d).astype(np.float32)
+    whole = gradient(gi, xi)
+    assert np.array_equal(whole, want)
+    # against 64 bits: a sum takes two roundings for every 32 terms (its large products, and the small ones), each 5.06e-8 of it as it stands
+    # then (see test_products_of_three_bf16_parts), the rest 3.5e-8; 32 terms are four positions of eight segments, of which some are dead
+    x, g = rng.standard_normal(x_shape).astype(np.float32), rng.standard_normal(grid).astype(np.float32)
+    exact = direct.conv_backward_w(g.astype(np.float64), x.astype(np.float64), w_shape, s, p, d)
+    got, single = gradient(g, x), gradient(g, x, split=False)
+    assert not np.array_equal(got, single)
+    off, norm = np.linalg.norm(got - exact), np.linalg.norm(exact)
+    terms = grid[0] * np.prod(grid[2:])
+    assert off <= (1.25 * 5.06e-8 * np.sqrt(2 * 2 * terms / 64) + 3.5e-8) * norm
+    assert off <= np.linalg.norm(single - exact)
+    # what the parts cannot hold: the single-precision kernel's gradient, bit for bit, and the one after it on the parts again
+    for value in (np.inf, np.nan, 1e-40):
+        for odd in range(2):
+            operands = [g.copy(), x.copy()]
+            operands[odd][tuple(n // 2 for n in operands[odd].shape)] = value
+            assert np.array_equal(bits(gradient(*operands)), bits(gradient(*operands, split=False)))
+    assert np.array_equal(bits(gradient(gi, xi)), bits(whole))
+    assert np.array_equal(bits(gradient(g, x)), bits(got))
+
+
+# (x, w, stride, padding, whether the filter gradient runs on parts)
+SPLIT_GRADIENT_RULES = [
+    ((128, 64, 56, 56), (64, 64, 3, 3), (1, 1), (1, 1), True),
+    ((16, 45, 16001), (83, 45, 9), (1,), (4,), True),
+    ((8, 16, 32, 64, 64), (32, 16, 3, 3, 3), (1, 1, 1), (1, 1, 1), True),
+    ((16, 64, 28, 28), (64, 64, 3, 3), (1, 1), (1, 1), False),         # 0.9 GFLOP
+    ((69, 205, 38, 11), (481, 205, 3, 1), (1, 1), (1, 0), False),      # three taps of a tile's nine
+]
+
+
+@pytest.mark.parametrize("rule", range(len(SPLIT_GRADIENT_RULES)))
+def test_which_filter_gradients_run_on_three_bf16_parts(abi, rule):
+    from mygrad_amd import _hip
+
+    x_shape, w_shape, s, p, split = SPLIT_GRADIENT_RULES[rule]
+    grid = tuple((n + 2 * q - t) // v + 1 for n, q, t, v in zip(x_shape[2:], p, w_shape[2:], s))
+    x, g = np.ones(x_shape, np.float32), np.ones((x_shape[0], w_shape[0], *grid), np.float32)
+    dw = abi.conv_wgrad(g, x, w_shape, s, p, (1,) * len(p))
+    print(_hip.last_plan(), flush=True)
+    assert _hip.last_plan().endswith("three bf16 parts") == split
+    centre = tuple(t // 2 for t in w_shape[2:])  # of the window: without padding there
+    assert np.all(dw[(slice(None), slice(None), *centre)] == x_shape[0] * np.prod(grid))
