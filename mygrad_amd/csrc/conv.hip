@@ -15,6 +15,7 @@
 //             order by a second kernel (no atomics, run-to-run identical)
 #include "conv_device.h"
 #include "conv_kernels.h"
+#include "few_split.h"
 #include "internal.h"
 #include "product_split.h"
 #include "wgrad_split.h"
@@ -582,6 +583,7 @@ struct Plan {
   int split_half_count = 0, patch_rows = 0;
   bool split_odd = false;        // an odd number of taps per stage
   int split_npos = 0;            // positions (pos_tab: 8 bytes each)
+  FewPlan few;                   // forward pass with few terms to a sum on three bf16 parts (few_split.hip): tm != 0
   WgradSplitPlan wsplit;         // filter gradient on three bf16 parts (wgrad_split.hip): fw != 0
   unsigned *words = nullptr;     // kWgradSplitWords words of memory, zero between calls
   bool single_dense_phase = false;  // positions enumerate the destination tensor in order
@@ -1570,7 +1572,24 @@ bool split_tables(Plan &pl, Tables &t, const SplitLayout &lay, int bn, const Pha
   return true;
 }
 
+// Whether a forward pass runs on few_split.hip's kernel: where its modelled time is the smaller one, with an eighth in favour of the
+// others, whose time (fitted to 80 layers of 0.2 - 30 GFLOP and up to 192 terms, 8 in 10 within 18 %) is the less certain one, and from 0.4
+// GFLOP on (below, 14 - 37 us, a few microseconds are in it either way).  Those of the 80 that it takes are 1.03 - 1.7 times as fast; most of
+// the rest are layers of few terms, bound by their stores: (111,1,211,211) * (11,1,3,3) 27.5 us and 44.4 there.
+// MYGRAD_HIP_FEW=0: none does; MYGRAD_HIP_FEW=10 tm + tn: every one that can, in that shape (tests; part of the plan's key).
+bool few_applies(const Geometry &g, Plan &pl) {
+  const char *shape = getenv("MYGRAD_HIP_FEW");
+  const int want = shape ? atoi(shape) : -1;
+  if (g.dtype != MG_F32 || !split_on() || want == 0 || !fits_buffer_loads(g)) return false;
+  if (want < 0 && (getenv("MYGRAD_HIP_TILE") || conv_flops(g) < 4e8 || g.C * g.wvol < 6)) return false;
+  pl.few = plan_few_split(g.N, g.C, g.F, g.X, g.G, g.W, g.S, g.D, g.P, runtime().props.multiProcessorCount);
+  const double others = 18.6 + 12.3e-9 * conv_flops(g) + 0.076e-6 * 4.0 * (double)g.N * g.F * (double)g.gvol + 0.052e-6 * 4.0 * (double)g.N * g.C * (double)g.xvol;
+  if (want < 0 && pl.few.time > 0.875 * others) pl.few = FewPlan();
+  return pl.few.tm != 0;
+}
+
 int build_fwd_plan(const Geometry &g, Plan &pl) {
+  if (few_applies(g, pl)) return MG_OK;
   Tables t;
   // (one tap and few channels: one position per lane takes 34.7 - 40.3 us for (64,C,112,112) * (64,C,1,1), C = 2 -
   // 11, whole K tiles of 16 with dead rows 41.9 - 44.3)
@@ -2457,6 +2476,7 @@ int get_plan(ConvOp op, const mg_conv_desc *d, const Geometry &g, Plan **out) {
   if (const char *tile = getenv("MYGRAD_HIP_TILE")) key.append(tile);
   if (const char *tile = getenv("MYGRAD_HIP_WGRAD_TILE")) key.append("w").append(tile);
   if (const char *tile = getenv("MYGRAD_HIP_SPLIT_TILE")) key.append("v").append(tile);
+  if (const char *shape = getenv("MYGRAD_HIP_FEW")) key.append("f").append(shape);
   if (const char *row = getenv("MYGRAD_HIP_FUSE_MIN_ROW")) key.append("r").append(row);
   if (const char *limit = getenv("MYGRAD_HIP_BUFFER_LIMIT")) key.append("b").append(limit);
   auto it = plans().find(key);
@@ -2487,6 +2507,9 @@ int get_plan(ConvOp op, const mg_conv_desc *d, const Geometry &g, Plan **out) {
     if (pl.wsplit.fw != 0)
       snprintf(pl.note, sizeof pl.note, "wgrad: tile %dx%d of 16 channels by 9 taps, %d quads of %d rows, %d ahead, %d tasks, %d segments, %d tiles, K splits %d, %.0f us, three bf16 parts",
                32 * pl.wsplit.fw, pl.wsplit.cw, pl.wsplit.p.quads, pl.wsplit.p.rows, pl.wsplit.p.depth, pl.wsplit.tasks, 1 << pl.wsplit.p.seg_shift, pl.wsplit.p.tiles, pl.wsplit.p.splits, pl.wsplit.time);
+    if (pl.few.tm != 0)
+      snprintf(pl.note, sizeof pl.note, "fwd: few terms, tile %dx%d, %d steps, patch of %d x %d, %d tiles%s by %d, %.0f us, three bf16 parts", 16 * pl.few.tm,
+               128 * pl.few.tn, pl.few.p.steps, pl.few.p.patch_rows, pl.few.p.pitch, pl.few.p.items, pl.few.p.along ? " of rows" : "", pl.few.p.m_tiles, pl.few.time);
     // MYGRAD_HIP_TRACE=1 reports, once per new descriptor, what was planned
     static const bool trace = getenv("MYGRAD_HIP_TRACE") != nullptr;
     if (trace) fprintf(stderr, "[mygrad_hip] plan %s (K chunk %d)\n", pl.note, pl.kchunk);
@@ -2815,6 +2838,7 @@ int run_thin(const Plan &pl, ThinParams &tp, const void *w, int tag) {
 
 template <typename T>
 int conv_fwd_impl(const Geometry &g, const Plan &pl, const void *x, const void *w, void *out) {
+  if (pl.few.tm != 0) return launch_few_split(pl.few, x, w, out, runtime().stream);
   if (pl.thin) {
     ThinParams tp{};
     tp.src = static_cast<const float *>(x);

@@ -1737,3 +1737,73 @@ def test_which_filter_gradients_run_on_three_bf16_parts(abi, rule):
     assert _hip.last_plan().endswith("three bf16 parts") == split
     centre = tuple(t // 2 for t in w_shape[2:])  # of the window: without padding there
     assert np.all(dw[(slice(None), slice(None), *centre)] == x_shape[0] * np.prod(grid))
+
+
+# (x, w, stride, padding, dilation, shape): forward passes with few terms on three bf16 parts (10 * (16 filters) + 16 positions of a wave)
+FEW_TERMS = [
+    ((3, 3, 33, 45), (64, 3, 7, 7), (2, 2), (3, 3), (1, 1), 43),    # a first layer; the last tile of a plane is short
+    ((2, 3, 40, 67), (70, 3, 3, 3), (1, 1), (1, 1), (1, 1), 42),    # two tiles of filters, most of the second one's beyond the last
+    ((5, 1, 9, 9), (8, 1, 5, 5), (1, 1), (0, 0), (1, 1), 22),       # fewer positions than a wave has
+    ((2, 5, 30, 21), (33, 5, 3, 4), (3, 1), (2, 0), (2, 3), 24),    # unequal axes
+    ((3, 21, 1501), (17, 21, 9), (1,), (4,), (1,), 24),             # 189 terms; runs of a row
+    ((2, 2, 4000), (40, 2, 15), (2,), (0,), (2,), 43),
+    ((1, 24, 6, 700), (48, 24, 1, 3), (1, 1), (0, 1), (1, 1), 42),  # rows longer than a tile: along them
+    ((4, 7, 5, 600), (65, 7, 2, 2), (1, 1), (0, 0), (1, 1), 43),
+    ((1, 1, 3), (1, 1, 1), (1,), (0,), (1,), 22),                   # one term
+]
+
+
+@pytest.mark.parametrize("problem", range(len(FEW_TERMS)))
+def test_forward_of_few_terms_on_three_bf16_parts(abi, monkeypatch, problem):
+    from mygrad_amd import _hip
+
+    x_shape, w_shape, s, p, d, shape = FEW_TERMS[problem]
+    rng = np.random.default_rng(3700 + problem)
+
+    def forward(x, w, few=True):
+        with monkeypatch.context() as m:
+            m.setenv("MYGRAD_HIP_FEW", str(shape if few else 0))
+            m.setenv("MYGRAD_HIP_SPLIT", "1" if few else "0")
+            out = abi.conv_fwd(x, w, s, p, d)
+            assert ("few terms" in _hip.last_plan()) == few
+        return out
+
+    xi, wi = rng.integers(-3, 4, x_shape).astype(np.float32), rng.integers(-2, 3, w_shape).astype(np.float32)
+    # small integers: every sum is exact
+    whole = forward(xi, wi)
+    assert np.array_equal(whole, direct.conv_forward(xi, wi, s, p, d))
+    # against 64 bits: as in test_filter_gradients_on_three_bf16_parts, a rounding for every 32 terms
+    x, w = rng.standard_normal(x_shape).astype(np.float32), rng.standard_normal(w_shape).astype(np.float32)
+    exact = direct.conv_forward(x.astype(np.float64), w.astype(np.float64), s, p, d)
+    got, single = forward(x, w), forward(x, w, few=False)
+    off, norm, terms = np.linalg.norm(got - exact), np.linalg.norm(exact), int(np.prod(w_shape[1:]))
+    assert off <= (1.25 * 5.06e-8 * np.sqrt(-(-terms // 32) / 2) + 3.5e-8) * norm
+    assert terms < 6 or off <= np.linalg.norm(single - exact)
+    # what the parts cannot hold: single precision's values, and the bits of far results as they were
+    for value in (np.inf, np.nan, 3e38, 1e-40):
+        for odd in range(2):
+            operands = [x * np.float32(4), w * np.float32(4)]
+            operands[odd][tuple(n // 2 for n in operands[odd].shape)] = value
+            with np.errstate(all="ignore"):
+                some, plain, far = forward(*operands), forward(*operands, few=False), forward(x * np.float32(4), w * np.float32(4))
+            finite = np.isfinite(plain)
+            assert np.array_equal(some[~finite], plain[~finite], equal_nan=True) and np.all(np.isfinite(some[finite]))
+            if odd == 0 and x_shape[0] > 1:
+                assert np.array_equal(bits(some[0]), bits(far[0]))
+    # one term a sum, of values below the smallest number of bf16: the single-precision instruction's results, to its rounding
+    tiny = np.zeros_like(w)
+    tiny.reshape(w_shape[0], -1)[:, 0] = 1e-41
+    assert np.array_equal(forward(x * np.float32(2.0**40), tiny), forward(x * np.float32(2.0**40), tiny, few=False))
+    assert np.array_equal(bits(forward(xi, wi)), bits(whole))
+
+
+@pytest.mark.parametrize("x_shape, w_shape, s, p, few", [((64, 3, 225, 225), (64, 3, 7, 7), 2, 3, True), ((25, 24, 6716), (178, 24, 5), 1, 2, True),
+                                                         ((111, 1, 211, 211), (11, 1, 3, 3), 2, 2, False), ((100, 16, 16, 16), (32, 16, 3, 3), 1, 1, False),
+                                                         ((4, 3, 16, 64, 64), (32, 3, 3, 3, 3), 1, 1, False), ((128, 64, 56, 56), (64, 64, 3, 3), 1, 1, False)])
+def test_which_forward_passes_run_as_few_terms(abi, x_shape, w_shape, s, p, few):
+    from mygrad_amd import _hip
+
+    out = abi.conv_fwd(np.ones(x_shape, np.float32), np.ones(w_shape, np.float32), s, p)
+    assert ("few terms" in _hip.last_plan()) == few
+    middle = tuple(n // 2 for n in out.shape[2:])
+    assert np.all(out[(slice(None), slice(None), *middle)] == np.prod(w_shape[1:]))
