@@ -3039,10 +3039,15 @@ int conv_wgrad_impl(const Geometry &g, const Plan &pl, const void *grad, const v
   const int ct = (int)((staged ? pl.depth : g.C) * g.wvol);
   void *target = dw;
   WgradParams wp{};
-  const size_t parts_bytes = pl.wsplit.fw != 0 ? wgrad_split_scratch(pl.wsplit) : 0;
+  size_t parts_bytes = pl.wsplit.fw != 0 ? wgrad_split_scratch(pl.wsplit) : 0;
+  const size_t staged_bytes = staged ? (size_t)pl.splits * g.F * ct * sizeof(T) : 0;
   void *scratch = nullptr;
+  if (parts_bytes != 0 && workspace(parts_bytes + staged_bytes, &scratch)) {
+    (void)hipGetLastError();
+    parts_bytes = 0;  // the kernels that need less stay
+  }
   if (staged || parts_bytes != 0) {
-    if (int rc = workspace(parts_bytes + (staged ? (size_t)pl.splits * g.F * ct * sizeof(T) : 0), &scratch)) return rc;
+    if (int rc = workspace(parts_bytes + staged_bytes, &scratch)) return rc;
     if (staged) target = static_cast<char *>(scratch) + parts_bytes;
     if (parts_bytes != 0) {  // (the kernel below is then for a gradient that the parts cannot hold)
       wp.gate = pl.words;

@@ -25,7 +25,13 @@ hipError_t hipGetLastError() { return hipSuccess; }
 hipError_t hipStreamCreateWithFlags(hipStream_t *stream, unsigned) { return *stream = reinterpret_cast<hipStream_t>(1), hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
-hipError_t hipMalloc(void **ptr, size_t size) { return *ptr = malloc(size), hipSuccess; }
+// STANDIN_LARGEST=bytes: larger blocks cannot be had
+hipError_t hipMalloc(void **ptr, size_t size) {
+  const char *largest = getenv("STANDIN_LARGEST");
+  if (largest && size > strtoull(largest, nullptr, 10)) return hipErrorOutOfMemory;
+  return *ptr = malloc(size), hipSuccess;
+}
+hipError_t hipFuncSetAttribute(const void *, hipFuncAttribute, int) { return hipSuccess; }
 hipError_t hipFree(void *ptr) { return free(ptr), hipSuccess; }
 hipError_t hipHostMalloc(void **ptr, size_t size, unsigned) { return *ptr = malloc(size), hipSuccess; }
 hipError_t hipHostFree(void *ptr) { return free(ptr), hipSuccess; }

@@ -777,6 +777,25 @@ print("refused")
     assert "refused" in run_on_standins(tmp_path, program)
 
 
+@pytest.mark.parametrize("largest", [1 << 30, 12 << 20])
+def test_filter_gradients_without_memory_for_their_parts_still_run(tmp_path, largest):
+    """Products on bf16 parts that cannot have their workspace leave the pass to the kernels that need less."""
+    program = f"""
+import os
+import numpy as np
+from mygrad_amd import _device, _hip
+lib = _hip.lib()
+desc = _hip.conv_desc(np.float32, (128, 64, 56, 56), (64, 64, 3, 3), (56, 56), (1, 1), (1, 1), (1, 1))
+buf = _device.DeviceBuffer(4 * 128 * 64 * 56 * 56)
+os.environ["STANDIN_LARGEST"] = "{largest}"
+for _ in range(2):
+    _hip.check(lib.mg_conv_wgrad(desc, buf.ptr, buf.ptr, buf.ptr))
+assert _hip.last_plan().endswith("three bf16 parts")
+print("ran")
+"""
+    assert "ran" in run_on_standins(tmp_path, program)
+
+
 def test_benchmark_prices_a_pass_against_the_instruction_that_runs_it():
     import bench
 
