@@ -462,6 +462,7 @@ bool product_applies(long long M, long long columns, long long octets) {
   if (flag && flag[0] == '0') return false;
   if ((getenv("MYGRAD_HIP_TILE") || getenv("MYGRAD_HIP_WGRAD_TILE")) && !least) return false;  // a tile of the convolution kernels was asked for
   if (M > (1 << 30) || columns > (1 << 30) || octets > (1 << 17)) return false;
+  if (ceil_div(M, kProductPanel) + ceil_div(columns, kProductPanel) > 65500) return false;  // (the packing's grid has a row for each)
   const double flops = 2.0 * (double)M * (double)columns * (double)octets * 8.0;
   if (least) return flops >= atof(least);
   if (flops < 4e9) return false;

@@ -805,3 +805,16 @@ def test_benchmark_prices_a_pass_against_the_instruction_that_runs_it():
     # six bf16 products each: the conv3a layer's 29.6 GFLOP in 165 us are 179 TFLOP/s, less than the peak they have
     assert 179 < bench.peak_of(split, 157.3) == 2500 / 6
     assert bench.short_plan(split) == bench.short_plan(plain).replace("x16", "x32") + ", three bf16 parts"
+
+
+def test_products_of_more_panels_than_a_grid_has_rows_stay_off_the_parts(tmp_path):
+    program = """
+import ctypes
+from mygrad_amd import _hip
+lib = _hip.lib()
+for rows, parts in ((8_380_000, True), (8_400_000, False)):
+    _hip.check(lib.mg_matmul(0, 1, rows, 16, 32, 1 << 40, 1 << 40, 1 << 40))
+    assert ("three bf16 parts" in _hip.last_plan()) == parts, (rows, _hip.last_plan())
+print("ran")
+"""
+    assert "ran" in run_on_standins(tmp_path, program, MYGRAD_HIP_SPLIT_MIN="0")
