@@ -328,6 +328,8 @@ __global__ void __launch_bounds__(512, 2) product_gemm_kernel(const ProductParam
     here.step = here.end - 1;
     forward(here);
   }
+  // (the zeros requested behind the last stage are on their way into LDS that the next block may have)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
 // Behind the products: the partial sums of the tiles whose K steps were shared, added in the order of K (the first
