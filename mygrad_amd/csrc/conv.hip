@@ -16,6 +16,7 @@
 #include "conv_device.h"
 #include "conv_kernels.h"
 #include "few_split.h"
+#include "few_wgrad.h"
 #include "internal.h"
 #include "product_split.h"
 #include "wgrad_split.h"
@@ -584,6 +585,7 @@ struct Plan {
   bool split_odd = false;        // an odd number of taps per stage
   int split_npos = 0;            // positions (pos_tab: 8 bytes each)
   FewPlan few;                   // forward pass with few terms to a sum on three bf16 parts (few_split.hip): tm != 0
+  FewGradPlan few_grad;          // filter gradient with few terms to a filter (few_wgrad.hip): tm != 0
   WgradSplitPlan wsplit;         // filter gradient on three bf16 parts (wgrad_split.hip): fw != 0
   unsigned *words = nullptr;     // kWgradSplitWords words of memory, zero between calls
   bool single_dense_phase = false;  // positions enumerate the destination tensor in order
@@ -2254,9 +2256,7 @@ int build_pos_table(const Geometry &g, Plan &pl) {
 
 // Whether a filter gradient may run on three bf16 parts.
 bool wgrad_split_applies(const Geometry &g, const Plan &pl) {
-  const char *least = getenv("MYGRAD_HIP_SPLIT_MIN");
-  return g.dtype == MG_F32 && pl.tap_major && split_on() && (!getenv("MYGRAD_HIP_WGRAD_TILE") || least) &&
-         conv_flops(g) >= (least ? atof(least) : 4e9);
+  return g.dtype == MG_F32 && pl.tap_major && split_on() && (!getenv("MYGRAD_HIP_WGRAD_TILE") || getenv("MYGRAD_HIP_SPLIT_MIN"));
 }
 
 int build_wgrad_plan(const Geometry &g, Plan &pl) {
@@ -2444,16 +2444,25 @@ int build_wgrad_plan(const Geometry &g, Plan &pl) {
   if (int rc = upload_plan(pl, t)) return rc;
   if (int rc = build_pos_table(g, pl)) return rc;
   if (wgrad_split_applies(g, pl)) {
-    pl.wsplit = plan_wgrad_split(g.N, g.C, g.F, g.X, g.G, g.W, g.S, g.D, g.P, cus);
-    // Table rows: 0.57 of the instruction's rate (0.40 - 0.66, 59 layers).  With a tenth in favour of the single-precision kernels
-    // 106 of 362 drawn layers of 4 - 30 GFLOP run on parts, 1.18 times as fast in the mean, 3 % slower or more in 8 of them: most
-    // of those with eight or nine taps to a tile, few with fewer, of which the tile's other products are of no use
-    // ((69,205,38,11) * (481,205,3,1) 755 us on parts, 168 without).
-    if (pl.table_rows) {
+    const char *least = getenv("MYGRAD_HIP_SPLIT_MIN"), *shape = getenv("MYGRAD_HIP_FEW");
+    if (pl.table_rows) {  // 0.57 of the instruction's rate (0.40 - 0.66, 59 layers)
       const double padded = 2.0 * (double)(ceil_div(g.F, pl.bm) * pl.bm) * (double)(col_tiles * pl.bn) * (double)kpos;
       single_time = 8.0 + padded / (0.57 * 157.3e6);
     }
-    if (!getenv("MYGRAD_HIP_SPLIT_MIN") && pl.wsplit.time > 0.9 * (pl.table_rows ? single_time : 1.05 * single_time)) pl.wsplit = WgradSplitPlan();
+    if (conv_flops(g) >= (least ? atof(least) : 4e9)) {
+      pl.wsplit = plan_wgrad_split(g.N, g.C, g.F, g.X, g.G, g.W, g.S, g.D, g.P, cus);
+      // With a tenth in favour of the single-precision kernels 106 of 362 drawn layers of 4 - 30 GFLOP run on parts, 1.18 times as fast in
+      // the mean, 3 % slower or more in 8 of them: most of those with eight or nine taps to a tile, few with fewer, of which the tile's
+      // other products are of no use ((69,205,38,11) * (481,205,3,1) 755 us on parts, 168 without).
+      if (!least && pl.wsplit.time > 0.9 * (pl.table_rows ? single_time : 1.05 * single_time)) pl.wsplit = WgradSplitPlan();
+    }
+    // Few terms to a filter: a ninth in favour of the others.  Most of 91 drawn layers stay ((32,3,224,224) * (64,3,3,3) 101 us and 140 there:
+    // 27 terms do not pay for their splitting); MYGRAD_HIP_FEW as in few_applies.
+    const int want = shape ? atoi(shape) : -1;
+    if (want > 0 || (want < 0 && !least && conv_flops(g) >= 4e8)) {
+      pl.few_grad = plan_few_wgrad(g.N, g.C, g.F, g.X, g.G, g.W, g.S, g.D, g.P, cus);
+      if (want < 0 && pl.few_grad.time > 0.9 * (pl.wsplit.fw != 0 ? std::min(pl.wsplit.time, single_time) : single_time)) pl.few_grad = FewGradPlan();
+    }
   }
   return MG_OK;
 }
@@ -2507,6 +2516,9 @@ int get_plan(ConvOp op, const mg_conv_desc *d, const Geometry &g, Plan **out) {
     if (pl.wsplit.fw != 0)
       snprintf(pl.note, sizeof pl.note, "wgrad: tile %dx%d of 16 channels by 9 taps, %d quads of %d rows, %d ahead, %d tasks, %d segments, %d tiles, K splits %d, %.0f us, three bf16 parts",
                32 * pl.wsplit.fw, pl.wsplit.cw, pl.wsplit.p.quads, pl.wsplit.p.rows, pl.wsplit.p.depth, pl.wsplit.tasks, 1 << pl.wsplit.p.seg_shift, pl.wsplit.p.tiles, pl.wsplit.p.splits, pl.wsplit.time);
+    if (pl.few_grad.tm != 0)
+      snprintf(pl.note, sizeof pl.note, "wgrad: few terms, tile %dx%d, patch of %d x %d, K splits %d, %.0f us, three bf16 parts", 16 * pl.few_grad.tm,
+               32 * pl.few_grad.tk, pl.few_grad.p.at.patch_rows, pl.few_grad.p.at.pitch, pl.few_grad.p.splits, pl.few_grad.time);
     if (pl.few.tm != 0)
       snprintf(pl.note, sizeof pl.note, "fwd: few terms, tile %dx%d, %d steps, patch of %d x %d, %d tiles%s by %d, %.0f us, three bf16 parts", 16 * pl.few.tm,
                128 * pl.few.tn, pl.few.p.steps, pl.few.p.patch_rows, pl.few.p.pitch, pl.few.p.items, pl.few.p.along ? " of rows" : "", pl.few.p.m_tiles, pl.few.time);
@@ -3039,7 +3051,7 @@ int conv_wgrad_impl(const Geometry &g, const Plan &pl, const void *grad, const v
   const int ct = (int)((staged ? pl.depth : g.C) * g.wvol);
   void *target = dw;
   WgradParams wp{};
-  size_t parts_bytes = pl.wsplit.fw != 0 ? wgrad_split_scratch(pl.wsplit) : 0;
+  size_t parts_bytes = pl.few_grad.tm != 0 ? few_wgrad_scratch(pl.few_grad) : pl.wsplit.fw != 0 ? wgrad_split_scratch(pl.wsplit) : 0;
   const size_t staged_bytes = staged ? (size_t)pl.splits * g.F * ct * sizeof(T) : 0;
   void *scratch = nullptr;
   if (parts_bytes != 0 && workspace(parts_bytes + staged_bytes, &scratch)) {
@@ -3051,7 +3063,7 @@ int conv_wgrad_impl(const Geometry &g, const Plan &pl, const void *grad, const v
     if (staged) target = static_cast<char *>(scratch) + parts_bytes;
     if (parts_bytes != 0) {  // (the kernel below is then for a gradient that the parts cannot hold)
       wp.gate = pl.words;
-      if (int rc = launch_wgrad_split(pl.wsplit, grad, x, scratch, pl.words, s)) return rc;
+      if (int rc = pl.few_grad.tm != 0 ? launch_few_wgrad(pl.few_grad, grad, x, scratch, pl.words, s) : launch_wgrad_split(pl.wsplit, grad, x, scratch, pl.words, s)) return rc;
     }
   }
   wp.grad = grad;
@@ -3110,6 +3122,7 @@ int conv_wgrad_impl(const Geometry &g, const Plan &pl, const void *grad, const v
   MG_HIP(hipGetLastError());
   if (parts_bytes != 0) {
     const WgradSums single{staged ? static_cast<const float *>(target) : nullptr, pl.splits, ct, pl.tap_major && !pl.table_rows};
+    if (pl.few_grad.tm != 0) return launch_few_wgrad_reduce(pl.few_grad, single, dw, scratch, pl.words, s);
     return launch_wgrad_split_reduce(pl.wsplit, single, dw, scratch, pl.words, s);
   }
   if (staged) {

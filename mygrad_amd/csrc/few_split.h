@@ -16,8 +16,9 @@ struct FewParams {
   // A tile's positions are consecutive in the plane of results: runs of the whole plane, or (along) of a row.
   int along, run_tiles; // tiles of a plane, or of a row
   int sample_tiles, items;  // tiles of a sample, of all samples
-  // A tile's patch of x, [channel][row][column], zeros outside: patch_rows rows of `pitch` columns
-  int patch_rows, pitch, patch;  // (patch: in all)
+  // A tile's patch of x, [channel][row][column], zeros outside: patch_rows rows of `pitch` columns, the windows' first one behind `lead`
+  // others, so that it begins on a multiple of four (-1: rows of up to 64 columns, as they come)
+  int patch_rows, pitch, lead, patch;  // (patch: in all)
   int m_tiles;
   FastDiv by_sample, by_run, by_row, by_patch_rows, by_window, by_w2;
 };

@@ -1,18 +1,17 @@
 // Forward pass of single-precision layers with few terms to a sum, such as a first layer's 3 x 7 x 7, on the bf16 matrix
 // instructions: see conv_split.hip for the arithmetic and its accuracy (two accumulators).
 //
-// What bounds it: (64,3,225,225) * (64,3,7,7), stride 2, 15.4 GFLOP, takes 141 us (187 with one position per lane on the
+// What bounds it: (64,3,225,225) * (64,3,7,7), stride 2, 15.4 GFLOP, takes 138 us (184 - 187 with one position per lane on the
 // single-precision instruction); 100 - 110 of them without its loads and stores (92 GFLOP of parts and 8 % of dead terms, 46 us at
 // the instruction's rate: eight waves to a unit, which all wait for a tile's patch, hide little of each other's latency), 69 with nothing
-// but loads and stores (209 MB).  (48,4,123,123) * (84,4,5,5) 186 -> 157, (25,24,6716) * (178,24,5) 118 -> 82.
+// but loads and stores (209 MB; loads of four bytes a lane, 141 us in all).  (48,4,123,123) * (84,4,5,5) 186 -> 157, (25,24,6716) * (178,24,5) 118 -> 82.
 // Error against 64 bits (2-norm), normal values: 6.9e-8 (single precision 2.2e-7); at 27 terms 3.7e-8 (9.5e-8).
 //
 // What the parts cannot represent (an infinity, a NaN, an overflow, low bits below the smallest number of bf16): the wave that
 // meets it computes its results again on the single-precision instruction, from the patch and the filters themselves; no other
 // result's bits depend on it.
-#include "few_split.h"
+#include "few_device.h"
 #include "internal.h"
-#include "split_device.h"
 
 #include <algorithm>
 #include <cstdlib>
@@ -22,15 +21,6 @@ namespace mg {
 namespace {
 
 constexpr int kWaves = 8;
-
-// Four bytes a lane from a buffer straight into LDS, the lanes' words one behind the other from byte `to` on.
-__device__ __forceinline__ void load_words_to_lds(__amdgpu_buffer_rsrc_t buffer, unsigned lane_at, unsigned at, unsigned to) {
-  typedef __attribute__((address_space(3))) void *LdsPointer;
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(buffer, (LdsPointer)(unsigned long long)to, 4, (int)lane_at, (int)at, 0, 0);
-}
-
-// This wave's loads have landed and its LDS reads are done; then all waves of the block are here.
-__device__ __forceinline__ void landed() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // A block keeps 16 TM filters, split, in LDS, and walks over tiles of 128 TN positions, 16 TN of them a wave.  The patch of x that a
 // tile's windows touch goes into LDS as it is (two of them: the next tile's is loaded meanwhile); a lane reads the eight
@@ -50,38 +40,15 @@ __global__ void __launch_bounds__(64 * kWaves, 2) few_split_kernel(const FewPara
   const int grid = (int)gridDim.x, place = grid % 8 == 0 ? (int)(blockIdx.x & 7) * (grid / 8) + (int)(blockIdx.x >> 3) : (int)blockIdx.x;
   const int m0 = place % p.m_tiles * BM, stride = grid / p.m_tiles;
 
-  struct Tile {
-    int n, q0, row, col;  // sample, first position, its row and (along) column
-  };
-  auto locate = [&](int item) -> Tile {
-    const int n = (int)p.by_sample.div((unsigned)item), rest = item - n * p.sample_tiles;
-    if (p.along) {
-      const int row = (int)p.by_run.div((unsigned)rest), col = (rest - row * p.run_tiles) * BN;
-      return Tile{n, row * p.G2 + col, row, col};
-    }
-    const int q0 = rest * BN;
-    return Tile{n, q0, (int)p.by_row.div((unsigned)q0), 0};
-  };
   const unsigned patches_at = (unsigned)reinterpret_cast<unsigned long long>((__attribute__((address_space(3))) char *)lds) + (unsigned)(pieces * 16 + (terms + 32) * 4);
   // the wave's share of a tile's patch: every eighth row of a channel, `count` of them from number `from` on
   const int lines = p.C * p.patch_rows, own_lines = (lines - wave + kWaves - 1) / kWaves;
-  auto request = [&](const Tile &t, int buf, int from, int count) {
-    const int x1 = t.row * p.S1 - p.P1, x2 = t.col * p.S2 - p.P2;
-    for (int own = from; own < min(from + count, own_lines); ++own) {
-      const int line = wave + own * kWaves;
-      const int c = (int)p.by_patch_rows.div((unsigned)line), r = x1 + line - c * p.patch_rows;
-      const bool there = (unsigned)r < (unsigned)p.X1;
-      const __amdgpu_buffer_rsrc_t x = buffer_of(p.x, there ? p.x_bytes : 0u);
-      const unsigned at = there ? (unsigned)(((t.n * p.C + c) * p.X1 + r) * p.X2) * 4u : 0u, to = patches_at + (unsigned)(buf * p.patch + line * p.pitch) * 4u;
-      for (int q = 0; q < p.pitch; q += 64) {
-        const int column = x2 + q + lane;
-        if (q + lane < p.pitch) load_words_to_lds(x, (unsigned)column < (unsigned)p.X2 ? (unsigned)column * 4u : kOutside, at, to + (unsigned)q * 4u);
-      }
-    }
+  auto request = [&](const FewTile &t, int buf, int from, int count) {
+    for (int own = from; own < min(from + count, own_lines); ++own) few_request_line(p, t, wave + own * kWaves, patches_at + (unsigned)(buf * p.patch) * 4u, lane);
   };
   int item = place / p.m_tiles;
   if (item >= p.items) return;
-  request(locate(item), 0, 0, own_lines);
+  request(few_tile<BN>(p, item), 0, 0, own_lines);
 
   // ---- the filters of the block, and where their terms lie
   if (threadIdx.x == 0) *tiny = 0;
@@ -110,24 +77,24 @@ __global__ void __launch_bounds__(64 * kWaves, 2) few_split_kernel(const FewPara
     for (int part = 0; part < 3; ++part) lds[((oct / 4 * 3 + part) * 4 + oct % 4) * BM + m] = parts[part];
   }
   if ((lost & 0xffffu) != 0) atomicOr(tiny, 1u);
-  landed();
+  few_landed();
   const bool lossy = uniform((int)*tiny) != 0;  // parts do not hold some filter value
 
   const u32x4 *const filters = lds + lk * BM + l16;
   const int4v *const mine_at = reinterpret_cast<const int4v *>(term_at) + lk * 2;
   for (int buf = 0; item < p.items; buf ^= 1) {
-    const Tile t = locate(item);
-    const int end = p.along ? min(t.q0 + BN, (t.row + 1) * p.G2) : min(t.q0 + BN, p.gvol), first = t.q0 + wave * 16 * TN;
+    const FewTile t = few_tile<BN>(p, item);
+    const int end = t.end, first = t.q0 + wave * 16 * TN;
     const char *const patch = reinterpret_cast<const char *>(patches + buf * p.patch);
     item += stride;
-    const Tile ahead = locate(min(item, p.items - 1));
+    const FewTile ahead = few_tile<BN>(p, min(item, p.items - 1));
     const int per_step = item < p.items ? (own_lines + p.steps - 1) / p.steps : 0;
 
     int base[TN];  // bytes: of the lane's positions, in the patch (beyond the last one: that one's)
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
       const int q = min(first + j * 16 + l16, end - 1), row = (int)p.by_row.div((unsigned)q);
-      base[j] = ((row - t.row) * p.S1 * p.pitch + (q - row * p.G2 - t.col) * p.S2) * 4;
+      base[j] = ((row - t.row) * p.S1 * p.pitch + (q - row * p.G2 - t.col) * p.S2 + max(p.lead, 0)) * 4;
     }
     f32x4 acc[TN][TM], low[TN][TM];  // sums of the large product and of the five small ones
 #pragma unroll
@@ -239,7 +206,7 @@ __global__ void __launch_bounds__(64 * kWaves, 2) few_split_kernel(const FewPara
         }
       }
     }
-    landed();  // the next patch is there, and nobody reads this one any more
+    few_landed();  // the next patch is there, and nobody reads this one any more
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
       const int m = m0 + i * 16 + l16;
@@ -269,7 +236,7 @@ size_t few_lds(const FewPlan &pl) { return (size_t)pl.p.steps * 12 * 16 * pl.tm 
 
 }  // namespace
 
-// The shape and the walk with the least modelled time, in us: fitted to 160 timed (layer, shape), 9 in 10 within 7 % of it.
+// The shape and the walk with the least modelled time, in us: fitted to 160 timed (layer, shape), 9 in 10 within 9 % of it.
 FewPlan plan_few_split(int N, int C, int F, const int *X, const int *G, const int *W, const int *S, const int *D, const int *P, int cus) {
   FewPlan best;
   const long long K = (long long)C * W[1] * W[2], gvol = (long long)G[1] * G[2];
@@ -291,9 +258,11 @@ FewPlan plan_few_split(int N, int C, int F, const int *X, const int *G, const in
     p.m_tiles = (int)ceil_div(F, bm);
     if (p.m_tiles > cus) continue;
     for (const int along : {0, 1}) {
-      p.along = along;
+      p.along = along, p.lead = -1;
       const long long rows = along ? 1 : std::min<long long>(G[1], ceil_div(bn - 1, G[2]) + 1), columns = along ? std::min(bn, G[2]) : G[2];
-      const long long patch_rows = (rows - 1) * S[1] + (long long)(W[1] - 1) * D[1] + 1, pitch = (columns - 1) * S[2] + (long long)(W[2] - 1) * D[2] + 1;
+      const long long patch_rows = (rows - 1) * S[1] + (long long)(W[1] - 1) * D[1] + 1, needed = (columns - 1) * S[2] + (long long)(W[2] - 1) * D[2] + 1;
+      long long pitch = needed;
+      if (needed > 64) p.lead = (4 - P[2] % 4) % 4, pitch = ceil_div(p.lead + needed, 4) * 4;
       if (patch_rows > kLds || pitch > kLds || C * patch_rows * pitch * 8 > kLds) continue;
       p.patch_rows = (int)patch_rows, p.pitch = (int)pitch, p.patch = (int)ceil_div(C * patch_rows * pitch, 4) * 4;
       if (few_lds(pl) > (size_t)kLds) continue;
@@ -306,8 +275,8 @@ FewPlan plan_few_split(int N, int C, int F, const int *X, const int *G, const in
       const int per = std::max(1, std::min(p.items, cus / p.m_tiles));
       pl.grid = per * p.m_tiles;
       const double rounds = (double)ceil_div(p.items, per);
-      const double requests = (double)(C * patch_rows * ceil_div(pitch, 64));
-      pl.time = 8.8 + 0.29 * p.steps + rounds * (0.82 + 0.159 * p.steps * pl.tn * pl.tm + 0.0104 * requests) + 0.132e-6 * 4.0 * (double)N * F * (double)gvol;
+      const double requests = (double)(C * patch_rows * (p.lead < 0 ? 1 : ceil_div(pitch, 256) + (X[2] % 4 != 0)));
+      pl.time = 8.2 + 0.208 * p.steps + rounds * (0.895 + 0.162 * p.steps * pl.tn * pl.tm + 0.0155 * requests) + 0.137e-6 * 4.0 * (double)N * F * (double)gvol;
       if (best.tm == 0 || pl.time < best.time) best = pl;
     }
   }

@@ -3,6 +3,7 @@
 #include "wgrad_split.h"
 #include "internal.h"
 #include "split_device.h"
+#include "wgrad_sums.h"
 
 #include <algorithm>
 #include <cstdlib>
@@ -378,24 +379,9 @@ __global__ void __launch_bounds__(256) wgrad_split_reduce_kernel(const WgradSpli
       if (f < p.F && c < p.C && frag < at.taps) p.dw[((long long)f * p.C + c) * p.wvol + at.t0 * p.W[1] * p.W[2] + at.tap + frag] = sum;
     }
   } else if (single.partial != nullptr) {
-    for (int i = (int)blockIdx.x * 256 + t; i < p.F * p.C * p.wvol; i += (int)gridDim.x * 256) {
-      const int tap = i % p.wvol, c = i / p.wvol % p.C, f = i / p.wvol / p.C;
-      // (the last group of 16 channels is moved back to end with the last channel, see WGroup; those of the one before it are that one's)
-      const int moved = single.groups && c / 16 * 16 + 16 > p.C ? 16 - p.C % 16 : 0;
-      const int column = single.groups ? (c / 16 * p.wvol + tap) * 16 + c % 16 + moved : c * p.wvol + tap;
-      p.dw[i] = sum_in_order(single.partial + (long long)f * single.ct + column, (long long)p.F * single.ct, single.splits);
-    }
+    reduce_single(single, p.dw, p.F, p.C, p.wvol);
   }
-  // The last block to have read it leaves the word as it was.  (Counted by 32 lines of memory first: one counter for all takes 10 ns a block.)
-  __syncthreads();
-  if (t == 0) {
-    const unsigned lines = min(gridDim.x, 32u), line = blockIdx.x % lines;
-    unsigned *const arrived = p.words + 32 * (1 + line);
-    if (atomicAdd(arrived, 1u) + 1 == (gridDim.x - line + lines - 1) / lines) {
-      *arrived = 0;
-      if (atomicAdd(&p.words[1], 1u) + 1 == lines) p.words[0] = p.words[1] = 0;
-    }
-  }
+  leave_words(p.words);
 }
 
 // waves along filters, column tiles and K; tasks of a wave

@@ -1807,3 +1807,52 @@ def test_which_forward_passes_run_as_few_terms(abi, x_shape, w_shape, s, p, few)
     assert ("few terms" in _hip.last_plan()) == few
     middle = tuple(n // 2 for n in out.shape[2:])
     assert np.all(out[(slice(None), slice(None), *middle)] == np.prod(w_shape[1:]))
+
+
+@pytest.mark.parametrize("problem", [n for n, case in enumerate(FEW_TERMS) if np.prod(case[1][1:]) <= 160])
+def test_filter_gradients_of_few_terms_on_three_bf16_parts(abi, monkeypatch, problem):
+    from mygrad_amd import _hip
+
+    x_shape, w_shape, s, p, d, _ = FEW_TERMS[problem]
+    rng = np.random.default_rng(3800 + problem)
+
+    def gradient(g, x, few=True):
+        with monkeypatch.context() as m:
+            m.setenv("MYGRAD_HIP_FEW", "1" if few else "0")
+            m.setenv("MYGRAD_HIP_SPLIT", "1" if few else "0")
+            dw = abi.conv_wgrad(g, x, w_shape, s, p, d)
+            assert ("few terms" in _hip.last_plan()) == few
+        return dw
+
+    xi = rng.integers(-3, 4, x_shape).astype(np.float32)
+    grid = direct.conv_forward(xi, np.zeros(w_shape, np.float32), s, p, d).shape
+    gi = rng.integers(-2, 3, grid).astype(np.float32)
+    # small integers: every sum is exact
+    whole = gradient(gi, xi)
+    assert np.array_equal(whole, direct.conv_backward_w(gi, xi, w_shape, s, p, d))
+    # against 64 bits: two roundings for every 32 terms, as in test_filter_gradients_on_three_bf16_parts
+    x, g = rng.standard_normal(x_shape).astype(np.float32), rng.standard_normal(grid).astype(np.float32)
+    exact = direct.conv_backward_w(g.astype(np.float64), x.astype(np.float64), w_shape, s, p, d)
+    got, single = gradient(g, x), gradient(g, x, few=False)
+    off, terms = np.linalg.norm(got - exact), grid[0] * np.prod(grid[2:])
+    assert off <= (1.25 * 5.06e-8 * np.sqrt(2 * 2 * terms / 64) + 3.5e-8) * np.linalg.norm(exact)
+    assert terms < 30 or off <= np.linalg.norm(single - exact)
+    # what the parts cannot hold: the single-precision kernel's gradient, bit for bit, and the one after it on the parts again
+    for value in (np.inf, np.nan, 1e-40):
+        for odd in range(2):
+            operands = [g.copy(), x.copy()]
+            operands[odd][tuple(n // 2 for n in operands[odd].shape)] = value
+            assert np.array_equal(bits(gradient(*operands)), bits(gradient(*operands, few=False)))
+    assert np.array_equal(bits(gradient(gi, xi)), bits(whole))
+
+
+@pytest.mark.parametrize("x_shape, w_shape, s, p, few", [((64, 3, 225, 225), (64, 3, 7, 7), 2, 3, True), ((91, 8, 14715), (26, 8, 15), 1, 7, False),
+                                                         ((32, 3, 224, 224), (64, 3, 3, 3), 1, 1, False), ((128, 64, 56, 56), (64, 64, 3, 3), 1, 1, False)])
+def test_which_filter_gradients_run_as_few_terms(abi, x_shape, w_shape, s, p, few):
+    from mygrad_amd import _hip
+
+    x = np.ones(x_shape, np.float32)
+    grid = tuple((n + 2 * p - t) // s + 1 for n, t in zip(x_shape[2:], w_shape[2:]))
+    dw = abi.conv_wgrad(np.ones((x_shape[0], w_shape[0], *grid), np.float32), x, w_shape, s, p)
+    assert ("few terms" in _hip.last_plan()) == few
+    assert np.all(dw[(slice(None), slice(None), *(t // 2 for t in w_shape[2:]))] == x_shape[0] * np.prod(grid))
