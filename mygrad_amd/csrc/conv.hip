@@ -29,6 +29,7 @@
 #include <cstring>
 #include <map>
 #include <string>
+#include <unistd.h>
 #include <vector>
 
 namespace mg {
@@ -2476,18 +2477,9 @@ void free_tables(Plan &pl) {
 int get_plan(ConvOp op, const mg_conv_desc *d, const Geometry &g, Plan **out) {
   std::string key(reinterpret_cast<const char *>(d), sizeof *d);
   key.push_back((char)op);
-  key.push_back(tiny_plans_enabled() ? 't' : 'T');
-  key.push_back(thin_on() ? 'n' : 'N');
-  key.push_back(phase_rows_enabled() ? 'p' : 'P');
-  key.push_back(pos_table_enabled() ? 'q' : 'Q');
-  key.push_back(split_on() ? 's' : 'S');
-  if (const char *least = getenv("MYGRAD_HIP_SPLIT_MIN")) key.append("m").append(least);
-  if (const char *tile = getenv("MYGRAD_HIP_TILE")) key.append(tile);
-  if (const char *tile = getenv("MYGRAD_HIP_WGRAD_TILE")) key.append("w").append(tile);
-  if (const char *tile = getenv("MYGRAD_HIP_SPLIT_TILE")) key.append("v").append(tile);
-  if (const char *shape = getenv("MYGRAD_HIP_FEW")) key.append("f").append(shape);
-  if (const char *row = getenv("MYGRAD_HIP_FUSE_MIN_ROW")) key.append("r").append(row);
-  if (const char *limit = getenv("MYGRAD_HIP_BUFFER_LIMIT")) key.append("b").append(limit);
+  // every switch that is set, whichever pass reads it: one walk over the environment (a look for each switch is one as well)
+  for (char **e = environ; *e; ++e)
+    if (strncmp(*e, "MYGRAD_HIP_", 11) == 0) key.append(*e).push_back('\0');
   auto it = plans().find(key);
   if (it == plans().end()) {
     if (plans().size() >= 256) {
@@ -3235,7 +3227,7 @@ int mg_matmul(int dtype, int64_t batch, int64_t M, int64_t K, int64_t N, const v
   mg_conv_desc d;
   if (int rc = matmul_desc("mg_matmul", dtype, batch, M, K, N, &d)) return rc;
   std::lock_guard<std::recursive_mutex> guard(api_mutex());
-  if (product_ready(d, a, x, out) && product_applies(M, batch * N, ceil_div(K, 8))) {
+  if (dtype == MG_F32 && product_applies(M, batch * N, ceil_div(K, 8)) && product_ready(d, a, x, out)) {
     const int rc = product_forward(batch, M, K, N, a, x, out);
     if (rc != MG_ERR_UNSUPPORTED) return rc;
   }
@@ -3246,7 +3238,7 @@ int mg_matmul_da(int dtype, int64_t batch, int64_t M, int64_t K, int64_t N, cons
   mg_conv_desc d;
   if (int rc = matmul_desc("mg_matmul_da", dtype, batch, M, K, N, &d)) return rc;
   std::lock_guard<std::recursive_mutex> guard(api_mutex());
-  if (product_ready(d, grad, x, da) && product_applies(M, K, batch * ceil_div(N, 8))) {
+  if (dtype == MG_F32 && product_applies(M, K, batch * ceil_div(N, 8)) && product_ready(d, grad, x, da)) {
     const int rc = product_da(batch, M, K, N, grad, x, da);
     if (rc != MG_ERR_UNSUPPORTED) return rc;
   }
@@ -3257,7 +3249,7 @@ int mg_matmul_dx(int dtype, int64_t batch, int64_t M, int64_t K, int64_t N, cons
   mg_conv_desc d;
   if (int rc = matmul_desc("mg_matmul_dx", dtype, batch, M, K, N, &d)) return rc;
   std::lock_guard<std::recursive_mutex> guard(api_mutex());
-  if (product_ready(d, grad, a, dx) && product_applies(K, batch * N, ceil_div(M, 8))) {
+  if (dtype == MG_F32 && product_applies(K, batch * N, ceil_div(M, 8)) && product_ready(d, grad, a, dx)) {
     const int rc = product_dx(batch, M, K, N, grad, a, dx);
     if (rc != MG_ERR_UNSUPPORTED) return rc;
   }

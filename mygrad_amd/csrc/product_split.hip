@@ -460,14 +460,15 @@ ProductPlan plan_product(long long M, long long columns, long long steps) {
 // 6 % at most; the others are faster by 1.37 in the mean.
 // MYGRAD_HIP_SPLIT_MIN=flops takes the place of the rule (tests).
 bool product_applies(long long M, long long columns, long long octets) {
-  const char *flag = getenv("MYGRAD_HIP_SPLIT"), *least = getenv("MYGRAD_HIP_SPLIT_MIN");
+  const char *least = getenv("MYGRAD_HIP_SPLIT_MIN");
+  const double flops = 2.0 * (double)M * (double)columns * (double)octets * 8.0;
+  if (flops < (least ? atof(least) : 4e9)) return false;
+  const char *flag = getenv("MYGRAD_HIP_SPLIT");
   if (flag && flag[0] == '0') return false;
   if ((getenv("MYGRAD_HIP_TILE") || getenv("MYGRAD_HIP_WGRAD_TILE")) && !least) return false;  // a tile of the convolution kernels was asked for
   if (M > (1 << 30) || columns > (1 << 30) || octets > (1 << 17)) return false;
   if (ceil_div(M, kProductPanel) + ceil_div(columns, kProductPanel) > 65500) return false;  // (the packing's grid has a row for each)
-  const double flops = 2.0 * (double)M * (double)columns * (double)octets * 8.0;
-  if (least) return flops >= atof(least);
-  if (flops < 4e9) return false;
+  if (least) return true;
   const long long steps = ceil_div(octets, 4);
   const ProductPlan pl = plan_product(M, columns, steps);
   const double read = (double)(M + columns) * (double)octets * 32.0;
