@@ -3033,6 +3033,13 @@ void launch_wgrad(WgradParams &wp, bool tap_major, bool table_rows, hipStream_t 
   }
 }
 
+// Runs of splits per element of a filter gradient's reduction: four or sixteen where one thread per element would leave units idle.
+int reduce_runs(bool groups, long long count, int splits) {
+  const long long blocks = ceil_div(count, 256), cus = runtime().props.multiProcessorCount;
+  if (blocks < cus / 8 && splits >= 64) return 16;
+  return groups && blocks < cus && splits >= 16 ? 4 : 1;
+}
+
 template <typename T>
 int conv_wgrad_impl(const Geometry &g, const Plan &pl, const void *grad, const void *x, void *dw) {
   hipStream_t s = runtime().stream;
@@ -3041,6 +3048,8 @@ int conv_wgrad_impl(const Geometry &g, const Plan &pl, const void *grad, const v
   // single tap (a matrix product), where the two orders are the same, and a single split.
   const bool staged = pl.splits > 1 || (pl.tap_major && !pl.table_rows && g.wvol > 1);
   const int ct = (int)((staged ? pl.depth : g.C) * g.wvol);
+  const bool groups = pl.tap_major && !pl.table_rows;  // columns by tap groups of 16 channels
+  const int runs = reduce_runs(groups, (long long)g.F * ct, pl.splits);
   void *target = dw;
   WgradParams wp{};
   size_t parts_bytes = pl.few_grad.tm != 0 ? few_wgrad_scratch(pl.few_grad) : pl.wsplit.fw != 0 ? wgrad_split_scratch(pl.wsplit) : 0;
@@ -3113,31 +3122,22 @@ int conv_wgrad_impl(const Geometry &g, const Plan &pl, const void *grad, const v
   }
   MG_HIP(hipGetLastError());
   if (parts_bytes != 0) {
-    const WgradSums single{staged ? static_cast<const float *>(target) : nullptr, pl.splits, ct, pl.tap_major && !pl.table_rows};
+    const WgradSums single{staged ? static_cast<const float *>(target) : nullptr, pl.splits, runs, ct, groups};
     if (pl.few_grad.tm != 0) return launch_few_wgrad_reduce(pl.few_grad, single, dw, scratch, pl.words, s);
     return launch_wgrad_split_reduce(pl.wsplit, single, dw, scratch, pl.words, s);
   }
   if (staged) {
     const int count = g.F * ct;
     ScopedTiming timed(TAG_WGRAD_REDUCE);
-    if (pl.tap_major && !pl.table_rows) {
-      // four or sixteen runs of splits per element when one thread per element would leave units idle
-      if (ceil_div(count, 256) < runtime().props.multiProcessorCount / 8 && pl.splits >= 64)
-        hipLaunchKernelGGL((tap_reduce_kernel<T, 16>), dim3((unsigned)ceil_div(count, 16)), dim3(256), 0, s,
-                           static_cast<const T *>(target), static_cast<T *>(dw), g.F, g.C, (int)g.wvol, pl.splits, ct);
-      else if (ceil_div(count, 256) < runtime().props.multiProcessorCount && pl.splits >= 16)
-        hipLaunchKernelGGL((tap_reduce_kernel<T, 4>), dim3((unsigned)ceil_div(count, 64)), dim3(256), 0, s,
-                           static_cast<const T *>(target), static_cast<T *>(dw), g.F, g.C, (int)g.wvol, pl.splits, ct);
-      else
-        hipLaunchKernelGGL((tap_reduce_kernel<T, 1>), dim3((unsigned)ceil_div(count, 256)), dim3(256), 0, s,
-                           static_cast<const T *>(target), static_cast<T *>(dw), g.F, g.C, (int)g.wvol, pl.splits, ct);
+    const dim3 grid((unsigned)ceil_div(count, 256 / runs));
+    const T *const part = static_cast<const T *>(target);
+    T *const out = static_cast<T *>(dw);
+    if (groups) {
+      const auto kernel = runs == 16 ? tap_reduce_kernel<T, 16> : runs == 4 ? tap_reduce_kernel<T, 4> : tap_reduce_kernel<T, 1>;
+      hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, part, out, g.F, g.C, (int)g.wvol, pl.splits, ct);
     } else {
-      if (ceil_div(count, 256) < runtime().props.multiProcessorCount / 8 && pl.splits >= 64)
-        hipLaunchKernelGGL((splitk_reduce_kernel<T, 16>), dim3((unsigned)ceil_div(count, 16)), dim3(256), 0, s,
-                           static_cast<const T *>(target), static_cast<T *>(dw), count, pl.splits);
-      else
-        hipLaunchKernelGGL((splitk_reduce_kernel<T, 1>), dim3((unsigned)ceil_div(count, 256)), dim3(256), 0, s,
-                           static_cast<const T *>(target), static_cast<T *>(dw), count, pl.splits);
+      const auto kernel = runs == 16 ? splitk_reduce_kernel<T, 16> : splitk_reduce_kernel<T, 1>;
+      hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, part, out, count, pl.splits);
     }
     MG_HIP(hipGetLastError());
   }

@@ -46,10 +46,11 @@ WgradSplitPlan plan_wgrad_split(int N, int C, int F, const int *X, const int *G,
 size_t wgrad_split_scratch(const WgradSplitPlan &pl);
 
 // The sums of the single-precision kernels, where the parts cannot hold a gradient: [split][F][ct], columns by tap groups of 16
-// channels (see WGroup) or in dw's own order; nullptr: they are in dw.
+// channels (see WGroup) or in dw's own order; nullptr: they are in dw.  They are added as that kernel's own reduction adds them: the
+// splits in `runs` runs, in order, then the runs.
 struct WgradSums {
   const float *partial;
-  int splits, ct;
+  int splits, runs, ct;
   bool groups;
 };
 

@@ -13,7 +13,12 @@ __device__ __forceinline__ void reduce_single(const WgradSums &single, float *dw
     // (the last group of 16 channels is moved back to end with the last channel, see WGroup; those of the one before it are that one's)
     const int moved = single.groups && c / 16 * 16 + 16 > C ? 16 - C % 16 : 0;
     const int column = single.groups ? (c / 16 * wvol + tap) * 16 + c % 16 + moved : c * wvol + tap;
-    dw[i] = sum_in_order(single.partial + (long long)f * single.ct + column, (long long)F * single.ct, single.splits);
+    const float *const from = single.partial + (long long)f * single.ct + column;
+    const long long stride = (long long)F * single.ct;
+    const int per = (single.splits + single.runs - 1) / single.runs;
+    float sum = sum_in_order(from, stride, min(per, single.splits));
+    for (int first = per; first < single.splits; first += per) sum += sum_in_order(from + first * stride, stride, min(per, single.splits - first));
+    dw[i] = sum;
   }
 }
 

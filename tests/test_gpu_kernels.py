@@ -1667,6 +1667,9 @@ SPLIT_GRADIENTS = [
     ((3, 16, 1003), (64, 16, 4), (1,), (2,), (2,), "2,2,2"),
     ((2, 30, 301), (20, 30, 5), (2,), (0,), (2,), "1,2,4"),
     ((64, 16, 1, 5), (16, 16, 1, 3), (1, 1), (0, 1), (1, 1), "1,1,8"),        # fewer columns than a stage has
+    # single-precision kernels behind them whose splits are added in sixteen and in four runs
+    ((8, 16, 4001), (16, 16, 9), (1,), (4,), (1,), "1,1,8"),
+    ((8, 32, 4001), (64, 32, 9), (1,), (4,), (1,), "2,2,2"),
 ]
 
 
@@ -1750,6 +1753,7 @@ FEW_TERMS = [
     ((1, 24, 6, 700), (48, 24, 1, 3), (1, 1), (0, 1), (1, 1), 42),  # rows longer than a tile: along them
     ((4, 7, 5, 600), (65, 7, 2, 2), (1, 1), (0, 0), (1, 1), 43),
     ((1, 1, 3), (1, 1, 1), (1,), (0,), (1,), 22),                   # one term
+    ((8, 3, 64, 64), (16, 3, 3, 3), (1, 1), (1, 1), (1, 1), 22),    # a single-precision filter gradient whose splits are added in sixteen runs
 ]
 
 
