@@ -175,7 +175,8 @@ __global__ void __launch_bounds__(512, 2) wgrad_split_kernel(const WgradSplitPar
       if constexpr (ALONG) {
         const int col = walk_col[s][e] + moved[s];
         outside = (unsigned)col < tick_limit[s] ? 0u : kOutside;
-        if (moved[s] == 0) at += (unsigned)max(3 - col, 0) * 4u;
+        // (in any tick of a walk that begins ahead of a row: with more padding than a tick has columns, a later one meets the row's first)
+        if (whole[s] == 0) at += (unsigned)max(3 - col, 0) * 4u;
       }
       raw[s][e] = __builtin_amdgcn_raw_buffer_load_b128(from, (int)(at | outside), 0, 0);
     }

@@ -1670,6 +1670,15 @@ SPLIT_GRADIENTS = [
     # single-precision kernels behind them whose splits are added in sixteen and in four runs
     ((8, 16, 4001), (16, 16, 9), (1,), (4,), (1,), "1,1,8"),
     ((8, 32, 4001), (64, 32, 9), (1,), (4,), (1,), "2,2,2"),
+    # Along the only axis, padded by more than a stage's columns: the second stage of a walk, or a later one, begins one to three columns
+    # ahead of its rows too.  (Filters enough that a block has several stages of a walk.)
+    *(((8, 32, 701), (300, 32, 9), (1,), (p,), (1,), "2,2,2") for p in (9, 10, 11)),
+    *(((8, 16, 1501), (256, 16, t), (1,), (p,), (1,), "1,2,4") for p, t in ((17, 18), (18, 18), (19, 20), (26, 27))),
+    *(((8, 16, 2001), (300, 16, 5), (1,), (p,), (1,), "1,1,8") for p in (33, 34, 35)),
+    *(((8, 32, 1401), (300, 32, 2), (2,), (p,), (1,), "2,2,2") for p in (17, 18, 19)),
+    ((8, 16, 1501), (256, 16, 9), (2,), (35,), (1,), "1,2,4"),
+    ((8, 16, 1501), (256, 16, 8), (1,), (21,), (3,), "1,2,4"),
+    ((8, 16, 3, 901), (250, 16, 3, 9), (1, 1), (0, 18), (1, 1), "1,2,4"),     # three rows to the only row of results
 ]
 
 
