@@ -818,3 +818,19 @@ for rows, parts in ((8_380_000, True), (8_400_000, False)):
 print("ran")
 """
     assert "ran" in run_on_standins(tmp_path, program, MYGRAD_HIP_SPLIT_MIN="0")
+
+
+def test_products_before_the_library_is_initialised_are_refused(tmp_path):
+    """Whatever their size: those that would run on three bf16 parts ask for the device's properties."""
+    program = """
+import ctypes
+from mygrad_amd import _hip
+lib = ctypes.CDLL(_hip.library_path())
+for name in ("mg_matmul", "mg_matmul_da", "mg_matmul_dx"):
+    entry = getattr(lib, name)
+    entry.argtypes = [ctypes.c_int, *(ctypes.c_int64,) * 4, *(ctypes.c_void_p,) * 3]
+    small, large = (entry(0, 1, n, n, n, 1 << 40, 1 << 40, 1 << 40) for n in (16, 4096))
+    assert small == large == _hip.MG_ERR_NOT_INIT, (name, small, large)
+print("refused")
+"""
+    assert "refused" in run_on_standins(tmp_path, program)
