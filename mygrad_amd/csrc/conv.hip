@@ -3227,7 +3227,7 @@ int mg_matmul(int dtype, int64_t batch, int64_t M, int64_t K, int64_t N, const v
   mg_conv_desc d;
   if (int rc = matmul_desc("mg_matmul", dtype, batch, M, K, N, &d)) return rc;
   std::lock_guard<std::recursive_mutex> guard(api_mutex());
-  if (dtype == MG_F32 && runtime().ready && product_applies(M, batch * N, ceil_div(K, 8)) && product_ready(d, a, x, out)) {
+  if (dtype == MG_F32 && runtime().ready && product_applies(M, batch * N, 1, K) && product_ready(d, a, x, out)) {
     const int rc = product_forward(batch, M, K, N, a, x, out);
     if (rc != MG_ERR_UNSUPPORTED) return rc;
   }
@@ -3238,7 +3238,7 @@ int mg_matmul_da(int dtype, int64_t batch, int64_t M, int64_t K, int64_t N, cons
   mg_conv_desc d;
   if (int rc = matmul_desc("mg_matmul_da", dtype, batch, M, K, N, &d)) return rc;
   std::lock_guard<std::recursive_mutex> guard(api_mutex());
-  if (dtype == MG_F32 && runtime().ready && product_applies(M, K, batch * ceil_div(N, 8)) && product_ready(d, grad, x, da)) {
+  if (dtype == MG_F32 && runtime().ready && product_applies(M, K, batch, N) && product_ready(d, grad, x, da)) {
     const int rc = product_da(batch, M, K, N, grad, x, da);
     if (rc != MG_ERR_UNSUPPORTED) return rc;
   }
@@ -3249,7 +3249,7 @@ int mg_matmul_dx(int dtype, int64_t batch, int64_t M, int64_t K, int64_t N, cons
   mg_conv_desc d;
   if (int rc = matmul_desc("mg_matmul_dx", dtype, batch, M, K, N, &d)) return rc;
   std::lock_guard<std::recursive_mutex> guard(api_mutex());
-  if (dtype == MG_F32 && runtime().ready && product_applies(K, batch * N, ceil_div(M, 8)) && product_ready(d, grad, a, dx)) {
+  if (dtype == MG_F32 && runtime().ready && product_applies(K, batch * N, 1, M) && product_ready(d, grad, a, dx)) {
     const int rc = product_dx(batch, M, K, N, grad, a, dx);
     if (rc != MG_ERR_UNSUPPORTED) return rc;
   }

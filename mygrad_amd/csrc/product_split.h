@@ -41,8 +41,8 @@ struct ProductParams {
 constexpr int kProductPanel = 128;                      // rows
 constexpr int kProductPanelBytes = kProductPanel * 32 * 6;  // of one K step
 
-// Whether a product of `octets` octets of K is large enough to run there.
-bool product_applies(long long M, long long columns, long long octets);
+// Whether a product with `runs` runs of `run` terms to a sum is large enough to run there.
+bool product_applies(long long M, long long columns, long long runs, long long run);
 
 // mg_matmul, mg_matmul_da and mg_matmul_dx in float32; MG_ERR_UNSUPPORTED, and nothing done, where there is no memory
 // for the parts.

@@ -146,13 +146,17 @@ def test_large_products_on_three_bf16_parts(abi, monkeypatch, batch, M, K, N):
 
 @pytest.mark.parametrize("sizes, parts", [((4096, 4096, 1024), (True, True, True)), ((1411, 3000, 3000), (True, True, True)),
                                           ((72, 8611, 3924), (False, False, False)), ((1024, 1024, 1024), (False, False, False)),
-                                          ((4096, 24, 8192), (False, False, False))])
+                                          ((4096, 24, 8192), (False, False, False)),
+                                          # stacks: a run of `a`'s gradient has no more terms than a matrix has columns, and is padded to eight on parts
+                                          ((1024, 1024, 1, 8192), (True, False, True)), ((4096, 4096, 1, 64), (False, False, False)),
+                                          ((1024, 1024, 2, 4096), (True, False, True)), ((1024, 1024, 9, 2048), (True, False, True)),
+                                          ((2000, 2000, 33, 64), (True, True, True))])
 def test_which_products_run_on_three_bf16_parts(abi, sizes, parts):
     from mygrad_amd import _hip
 
-    M, K, N = sizes
-    a, x, g = (np.ones(shape, np.float32) for shape in ((M, K), (1, K, N), (1, M, N)))
-    for fn, args, terms, expected in zip((abi.matmul, abi.matmul_da, abi.matmul_dx), ((a, x), (g, x, M), (g, a)), (K, N, M), parts):
+    M, K, N, batch = (*sizes, 1)[:4]
+    a, x, g = (np.ones(shape, np.float32) for shape in ((M, K), (batch, K, N), (batch, M, N)))
+    for fn, args, terms, expected in zip((abi.matmul, abi.matmul_da, abi.matmul_dx), ((a, x), (g, x, M), (g, a)), (K, batch * N, M), parts):
         assert np.all(fn(*args) == terms)
         assert ("three bf16 parts" in _hip.last_plan()) == expected
 
