@@ -436,7 +436,7 @@ WgradSplitPlan plan_wgrad_split(int N, int C, int F, const int *X, const int *G,
       p.chunks = (int)ceil_div(taps, kFrags);
       int tap_rows = 0;
       for (int c = 0; c < p.chunks; ++c) tap_rows = std::max(tap_rows, std::min(taps - 1, (c + 1) * kFrags - 1) / W[2] - c * kFrags / W[2] + 1);
-      const long long live = (p.rows - 1) * S[1] + (long long)(tap_rows - 1) * D[1] + 1, locs = (4 * quads - 1) * S[2] + (long long)(W[2] - 1) * D[2] + 1;
+      const long long live = (p.rows - 1ll) * S[1] + (tap_rows - 1ll) * D[1] + 1, locs = (4ll * quads - 1) * S[2] + (W[2] - 1ll) * D[2] + 1;
       if (live > 64 || locs > 64) continue;  // (far more than LDS holds)
       p.new_rows = pl.along ? (int)live : p.rows * S[1];
       p.depth = std::max(0, (int)ceil_div(live - p.new_rows, p.new_rows));

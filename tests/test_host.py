@@ -834,3 +834,18 @@ for name in ("mg_matmul", "mg_matmul_da", "mg_matmul_dx"):
 print("refused")
 """
     assert "refused" in run_on_standins(tmp_path, program)
+
+
+def test_filter_gradients_of_the_largest_strides_stay_off_the_parts(tmp_path):
+    """A window that is moved nowhere may have any stride: 7 * 613566757 is 3 modulo 2**32, a patch that would fit."""
+    program = """
+import numpy as np
+from mygrad_amd import _hip
+lib = _hip.lib()
+for stride, parts in ((1, True), (613566757, False), (2**31 - 1, False)):
+    desc = _hip.conv_desc(np.float32, (64, 16, 3), (64, 16, 3), (1,), (stride,), (0,), (1,))
+    _hip.check(lib.mg_conv_wgrad(desc, 1 << 40, 1 << 40, 1 << 40))
+    assert ("three bf16 parts" in _hip.last_plan()) == parts, (stride, _hip.last_plan())
+print("ran")
+"""
+    assert "ran" in run_on_standins(tmp_path, program, MYGRAD_HIP_SPLIT_MIN="0", MYGRAD_HIP_SPLIT_TILE="2,2,2")
