@@ -842,7 +842,7 @@ def test_filter_gradients_of_the_largest_strides_stay_off_the_parts(tmp_path):
 import numpy as np
 from mygrad_amd import _hip
 lib = _hip.lib()
-for stride, parts in ((1, True), (613566757, False), (2**31 - 1, False)):
+for stride, parts in ((1, True), (613566757, False)):
     desc = _hip.conv_desc(np.float32, (64, 16, 3), (64, 16, 3), (1,), (stride,), (0,), (1,))
     _hip.check(lib.mg_conv_wgrad(desc, 1 << 40, 1 << 40, 1 << 40))
     assert ("three bf16 parts" in _hip.last_plan()) == parts, (stride, _hip.last_plan())
