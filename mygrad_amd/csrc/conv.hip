@@ -613,6 +613,7 @@ struct Plan {
   int kchunk = 0;
   int run_tiles = 0;  // WgradParams::run_tiles
   char note[256] = "";  // what mg_last_plan() reports after a call that ran this plan
+  char less_note[256] = "";  // the same of a filter gradient that could not have the workspace of its parts
 };
 
 std::map<std::string, Plan> &plans() {
@@ -2505,6 +2506,7 @@ int get_plan(ConvOp op, const mg_conv_desc *d, const Geometry &g, Plan **out) {
              pl.thin ? "one position per lane" : pl.tap_major ? "tap-major" : "table-driven", pl.table_rows ? ", table rows" : pl.phase_rows ? ", stride phases as rows" : "",
              pl.fold_row ? ", folded taps" : "", pl.bm, pl.bn, pl.split ? 32 : pl.bk, pl.nphases, pl.nph, pl.pos_blocks, pl.m_tiles, pl.full_tiles, tail,
              pl.blocks_per_cu, pl.splits, pl.split ? ", three bf16 parts" : "");
+    memcpy(pl.less_note, pl.note, sizeof pl.note);
     if (pl.wsplit.fw != 0)
       snprintf(pl.note, sizeof pl.note, "wgrad: tile %dx%d of 16 channels by 9 taps, %d quads of %d rows, %d ahead, %d tasks, %d segments, %d tiles, K splits %d, %.0f us, three bf16 parts",
                32 * pl.wsplit.fw, pl.wsplit.cw, pl.wsplit.p.quads, pl.wsplit.p.rows, pl.wsplit.p.depth, pl.wsplit.tasks, 1 << pl.wsplit.p.seg_shift, pl.wsplit.p.tiles, pl.wsplit.p.splits, pl.wsplit.time);
@@ -3055,9 +3057,9 @@ int conv_wgrad_impl(const Geometry &g, const Plan &pl, const void *grad, const v
   size_t parts_bytes = pl.few_grad.tm != 0 ? few_wgrad_scratch(pl.few_grad) : pl.wsplit.fw != 0 ? wgrad_split_scratch(pl.wsplit) : 0;
   const size_t staged_bytes = staged ? (size_t)pl.splits * g.F * ct * sizeof(T) : 0;
   void *scratch = nullptr;
-  if (parts_bytes != 0 && workspace(parts_bytes + staged_bytes, &scratch)) {
-    (void)hipGetLastError();
+  if (parts_bytes != 0 && workspace_or_less(parts_bytes + staged_bytes, &scratch)) {
     parts_bytes = 0;  // the kernels that need less stay
+    note_plan(pl.less_note);
   }
   if (staged || parts_bytes != 0) {
     if (int rc = workspace(parts_bytes + staged_bytes, &scratch)) return rc;

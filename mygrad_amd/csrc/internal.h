@@ -30,6 +30,9 @@ struct Runtime {
   // filters, split-K partial sums).  Never handed to callers.
   void *workspace = nullptr;
   size_t workspace_bytes = 0;
+  // What workspace_or_less() could not have, and how many more of its calls leave it at that.
+  size_t refused_bytes = ~size_t(0);
+  int refusals_left = 0;
 };
 
 Runtime &runtime();
@@ -38,6 +41,10 @@ Runtime &runtime();
 // the allocation when needed.  Stream-ordered users may rely on its contents only
 // until the next call that asks for workspace.
 int workspace(size_t nbytes, void **ptr);
+
+// As workspace(), for those who have a way that needs less (not MG_OK, and no HIP error left behind, if there is no memory).  What could not be
+// had is asked for again in one of 256 calls only: to ask takes a drained stream, the block that is there and two trips to the driver.
+int workspace_or_less(size_t nbytes, void **ptr);
 
 // Optional per-launch timing with HIP events on the library stream (off by
 // default).  A launch site brackets its kernel with timing_begin/timing_end.

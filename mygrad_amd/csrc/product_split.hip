@@ -504,10 +504,7 @@ int run_product(ProductParams &p, int tag, const char *name) {
   const size_t mark_bytes = ((size_t)p.marks * 4 + 255) & ~size_t(255);
   const size_t partial_bytes = (size_t)p.share_blocks * 2 * 2 * kProductPanel * kProductPanel * 4;
   void *scratch = nullptr;
-  if (workspace((p.a_panels + p.b_panels) * panel_bytes + note_bytes + mark_bytes + partial_bytes, &scratch)) {
-    (void)hipGetLastError();
-    return MG_ERR_UNSUPPORTED;  // the kernels that need less stay
-  }
+  if (workspace_or_less((p.a_panels + p.b_panels) * panel_bytes + note_bytes + mark_bytes + partial_bytes, &scratch)) return MG_ERR_UNSUPPORTED;  // the kernels that need less stay
   char *at = static_cast<char *>(scratch);
   p.packed_a = at, at += p.a_panels * panel_bytes;
   p.packed_b = at, at += p.b_panels * panel_bytes;

@@ -65,6 +65,23 @@ int workspace(size_t nbytes, void **ptr) {
   return MG_OK;
 }
 
+int workspace_or_less(size_t nbytes, void **ptr) {
+  Runtime &rt = runtime();
+  if (nbytes > rt.workspace_bytes && nbytes >= rt.refused_bytes && rt.refusals_left > 0) {
+    --rt.refusals_left;
+    return MG_ERR_UNSUPPORTED;
+  }
+  const int rc = workspace(nbytes, ptr);
+  if (rc) {
+    (void)hipGetLastError();
+    rt.refused_bytes = nbytes;
+    rt.refusals_left = 255;
+  } else if (nbytes >= rt.refused_bytes) {
+    rt.refused_bytes = ~size_t(0);
+  }
+  return rc;
+}
+
 // ---- per-launch timing -------------------------------------------------------------------
 // One event after every timed launch; the event after the launch before it serves as its start
 // when nothing else can have been enqueued in between (the earlier scope ended in this entry
@@ -389,6 +406,7 @@ int mg_shutdown(void) {
   if (rt.workspace) MG_HIP(hipFree(rt.workspace));
   rt.workspace = nullptr;
   rt.workspace_bytes = 0;
+  rt.refused_bytes = ~size_t(0);
   pool_trim(0);  // idle blocks go back to the driver; blocks still held by callers stay theirs
   pool_trim(0, host_pool());
   MG_HIP(hipStreamDestroy(rt.stream));

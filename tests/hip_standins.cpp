@@ -7,10 +7,11 @@
 #include <cstring>
 
 namespace {
-int events_made = 0;
+int events_made = 0, blocks_refused = 0;
 }
 
 extern "C" {
+int standin_blocks_refused() { return blocks_refused; }
 hipError_t hipGetDeviceCount(int *count) { return *count = 1, hipSuccess; }
 hipError_t hipSetDevice(int) { return hipSuccess; }
 hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600 *props, int) {
@@ -28,7 +29,7 @@ hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 // STANDIN_LARGEST=bytes: larger blocks cannot be had
 hipError_t hipMalloc(void **ptr, size_t size) {
   const char *largest = getenv("STANDIN_LARGEST");
-  if (largest && size > strtoull(largest, nullptr, 10)) return hipErrorOutOfMemory;
+  if (largest && size > strtoull(largest, nullptr, 10)) return ++blocks_refused, hipErrorOutOfMemory;
   return *ptr = malloc(size), hipSuccess;
 }
 hipError_t hipFuncSetAttribute(const void *, hipFuncAttribute, int) { return hipSuccess; }

@@ -777,20 +777,28 @@ print("refused")
     assert "refused" in run_on_standins(tmp_path, program)
 
 
-@pytest.mark.parametrize("largest", [1 << 30, 12 << 20])
-def test_filter_gradients_without_memory_for_their_parts_still_run(tmp_path, largest):
-    """Products on bf16 parts that cannot have their workspace leave the pass to the kernels that need less."""
+@pytest.mark.parametrize("run, largest", [("_hip.lib().mg_conv_wgrad(desc, buf.ptr, buf.ptr, buf.ptr)", 12 << 20),
+                                          ("_hip.lib().mg_matmul(0, 1, 4096, 4096, 4096, buf.ptr, buf.ptr, buf.ptr)", 128 << 20)])
+def test_passes_without_memory_for_their_parts_still_run(tmp_path, run, largest):
+    """Products on bf16 parts that cannot have their workspace leave the pass to the kernels that need less, say so, and
+    ask for it again later, not in each call."""
     program = f"""
-import os
+import ctypes, os
 import numpy as np
 from mygrad_amd import _device, _hip
-lib = _hip.lib()
+refused = ctypes.CDLL(os.environ["LD_PRELOAD"]).standin_blocks_refused
 desc = _hip.conv_desc(np.float32, (128, 64, 56, 56), (64, 64, 3, 3), (56, 56), (1, 1), (1, 1), (1, 1))
 buf = _device.DeviceBuffer(4 * 128 * 64 * 56 * 56)
-os.environ["STANDIN_LARGEST"] = "{largest}"
-for _ in range(2):
-    _hip.check(lib.mg_conv_wgrad(desc, buf.ptr, buf.ptr, buf.ptr))
-assert _hip.last_plan().endswith("three bf16 parts")
+os.environ["STANDIN_LARGEST"] = str({largest})
+for call in range(600):
+    _hip.check({run})
+    assert "three bf16 parts" not in _hip.last_plan(), _hip.last_plan()
+    assert refused() == 1 + call // 256, call
+os.environ["STANDIN_LARGEST"] = str(1 << 30)
+for call in range(600, 900):
+    _hip.check({run})
+    assert ("three bf16 parts" in _hip.last_plan()) == (call >= 768), call
+assert refused() == 3
 print("ran")
 """
     assert "ran" in run_on_standins(tmp_path, program)
