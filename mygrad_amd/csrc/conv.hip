@@ -2479,7 +2479,7 @@ int get_plan(ConvOp op, const mg_conv_desc *d, const Geometry &g, Plan **out) {
   std::string key(reinterpret_cast<const char *>(d), sizeof *d);
   key.push_back((char)op);
   // every switch that is set, whichever pass reads it: one walk over the environment (a look for each switch is one as well)
-  for (char **e = environ; *e; ++e)
+  for (char **e = environ; e && *e; ++e)  // (clearenv() leaves none at all)
     if (strncmp(*e, "MYGRAD_HIP_", 11) == 0) key.append(*e).push_back('\0');
   auto it = plans().find(key);
   if (it == plans().end()) {

@@ -857,3 +857,18 @@ for stride, parts in ((1, True), (613566757, False)):
 print("ran")
 """
     assert "ran" in run_on_standins(tmp_path, program, MYGRAD_HIP_SPLIT_MIN="0", MYGRAD_HIP_SPLIT_TILE="2,2,2")
+
+
+def test_passes_run_without_an_environment(tmp_path):
+    program = """
+import ctypes
+import numpy as np
+from mygrad_amd import _hip
+lib = _hip.lib()
+desc = _hip.conv_desc(np.float32, (2, 3, 9, 9), (4, 3, 3, 3), (7, 7), (1, 1), (0, 0), (1, 1))
+_hip.check(lib.mg_conv_fwd(desc, 1 << 40, 1 << 40, 1 << 40))  # (the runtime's own first launch reads it)
+ctypes.CDLL(None).clearenv()
+_hip.check(lib.mg_conv_dgrad(desc, 1 << 40, 1 << 40, 1 << 40))
+print("ran", flush=True)
+"""
+    assert "ran" in run_on_standins(tmp_path, program)
