@@ -36,4 +36,15 @@ __device__ __forceinline__ void split_pair(float a, float b, unsigned &h, unsign
   lost |= bits_of(qa) | bits_of(qb);
 }
 
+// The largest |value| so far (a NaN stays): one instruction for two values.
+__device__ __forceinline__ void widen(float &widest, float a, float b) {
+  widest = __builtin_elementwise_maximum(widest, __builtin_elementwise_maximum(__builtin_fabsf(a), __builtin_fabsf(b)));
+}
+
+// What a product can have lost where an operand of `lost` has low bits below the smallest number of bf16, 2^-133, is 2^-133 of the other operand; a
+// sum of `terms` of them is as good as any where it is 2^24 times that.
+__device__ __forceinline__ float least_sum(bool lost_a, float widest_a, bool lost_b, float widest_b, int terms) {
+  return ((lost_a ? widest_b : 0.0f) + (lost_b ? widest_a : 0.0f)) * (float)terms * 0x1p-109f;
+}
+
 }  // namespace mg

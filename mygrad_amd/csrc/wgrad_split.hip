@@ -16,6 +16,7 @@ namespace {
 
 constexpr int kFrags = kWgradSplitFrags, kColumns = kFrags * 16;
 constexpr int kSumStride = kColumns + 4;  // floats between the filters of a tile's sums in LDS
+constexpr int kSums = 8 * 32 * kSumStride;  // floats of them: eight waves of 32 filters
 constexpr int kMiddle = 4;  // taps of a stage ahead of which the second half of the waves parks
 constexpr int kLoc = 48;                  // pieces of 16 bytes of 16 channels at one location: [part][channel]
 constexpr int kDump = 3 * kLoc + 2 * 16 + 16;  // pieces behind the rings for what nobody reads
@@ -185,7 +186,11 @@ __global__ void __launch_bounds__(512, 2) wgrad_split_kernel(const WgradSplitPar
 #pragma unroll
     for (int e = 0; e < 4; ++e) request(e);
   };
-  unsigned lost = 0;
+  // of a task's values: bits that the parts have lost, and the widest one
+  unsigned lost[TASKS];
+  float widest[TASKS];
+#pragma unroll
+  for (int s = 0; s < TASKS; ++s) lost[s] = 0, widest[s] = 0.0f;
   // splits and parks what was requested
   auto park = [&](int group) MG_INLINE {
 #pragma unroll
@@ -211,7 +216,9 @@ __global__ void __launch_bounds__(512, 2) wgrad_split_kernel(const WgradSplitPar
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
           unsigned h, m, l;
-          split_pair(float_of(raw[s][2 * e][u]), float_of(raw[s][2 * e + 1][u]), h, m, l, lost);
+          const float a = float_of(raw[s][2 * e][u]), b = float_of(raw[s][2 * e + 1][u]);
+          split_pair(a, b, h, m, l, lost[s]);
+          widen(widest[s], a, b);
           parts[0][e] = h, parts[1][e] = m, parts[2][e] = l;
         }
 #pragma unroll
@@ -343,17 +350,48 @@ __global__ void __launch_bounds__(512, 2) wgrad_split_kernel(const WgradSplitPar
       const f32x4 sum = j < kOwnLow ? acc[j][i] + low[j < kOwnLow ? j : 0][i] : acc[j][i];
       *reinterpret_cast<f32x4 *>(sums + (((kq * CW + cw) * FT + fw * 32 + i * 16 + l16) * kSumStride + j * 16 + lk * 4)) = sum;
     }
+  // Of every channel and filter of the tile, where any has lost bits: the widest value, and whether it has.
+  constexpr int ROWS = FT + CW * 16;  // filters, then channels
+  unsigned *const notes = reinterpret_cast<unsigned *>(sums + kSums), *const waves = notes + 2 * ROWS;
+  bool any = false;
+#pragma unroll
+  for (int s = 0; s < TASKS; ++s) any |= has[s] && (lost[s] & 0xffffu) != 0;
+  any = __any(any);
+  if (lane == 0) waves[wave] = any;
   __syncthreads();
+#pragma unroll
+  for (int w = 0; w < 8; ++w) any |= waves[w] != 0;
+  if (any) {  // seldom
+    for (int i = (int)threadIdx.x; i < 2 * ROWS; i += 512) notes[i] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < TASKS; ++s) {
+      if (!has[s]) continue;
+      const int number = wave + 8 * s, row = tasks[s].is_x ? FT + min((number - GTASKS) / xtasks, CW - 1) * 16 + l16 : (number * 2 + (lk >> 1)) / KW * 16 + l16;
+      atomicMax(&notes[row], bits_of(widest[s]));
+      if ((lost[s] & 0xffffu) != 0) atomicOr(&notes[ROWS + row], 1u);
+    }
+    __syncthreads();
+  }
   float *const out = p.partial + (long long)(split * p.tiles + tile) * (CW * FT * kColumns);
-  bool odd = (lost & 0xffffu) != 0;  // bits of an operand were lost, or a sum is not finite
+  bool odd = false;  // a sum is not finite, or bits that it would have were lost
+  const int terms = (last_stage - first_stage) * (KW * 4 * 8);
   for (int e = (int)threadIdx.x; e < CW * FT * kColumns / 4; e += 512) {
     const int f = e / (kColumns / 4), c = e % (kColumns / 4) * 4;  // (f: column tile, filter)
     f32x4 sum = *reinterpret_cast<const f32x4 *>(sums + f * kSumStride + c);
 #pragma unroll
     for (int k = 1; k < KW; ++k) sum += *reinterpret_cast<const f32x4 *>(sums + (k * CW * FT + f) * kSumStride + c);
     *reinterpret_cast<f32x4 *>(out + f * kColumns + c) = sum;
+    const bool live = c / 16 < columns_of(p, first_columns + f / FT).taps;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) odd |= !(__builtin_fabsf(sum[q]) < __builtin_inff()) && c / 16 < columns_of(p, first_columns + f / FT).taps;
+    for (int q = 0; q < 4; ++q) odd |= !(__builtin_fabsf(sum[q]) < __builtin_inff()) && live;
+    if (any && live) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int g = f % FT, x = FT + f / FT * 16 + c % 16 + q;
+        odd |= !(__builtin_fabsf(sum[q]) >= least_sum(notes[ROWS + g] != 0, float_of(notes[g]), notes[ROWS + x] != 0, float_of(notes[x]), terms));
+      }
+    }
   }
   if (__any(odd) && lane == 0) atomicOr(&p.words[0], 1u);
 }
@@ -400,7 +438,7 @@ constexpr int kLds = 160 * 1024;
 
 size_t lds_bytes(const WgradSplitPlan &pl) {
   const size_t rings = (size_t)pl.cw * (pl.p.depth + 2) * pl.p.new_rows * pl.p.row_locs * kLoc;
-  return std::max<size_t>((pl.kw * 4 * 2 * pl.fw * kLoc + rings + kDump) * 16, (size_t)8 * 32 * kSumStride * 4);
+  return std::max<size_t>((pl.kw * 4 * 2 * pl.fw * kLoc + rings + kDump) * 16, (size_t)(kSums + 2 * (32 * pl.fw + 16 * pl.cw) + 8) * 4);
 }
 
 }  // namespace

@@ -1653,6 +1653,25 @@ def test_which_passes_run_on_three_bf16_parts(abi, monkeypatch, rule):
     assert not split or off <= off_single
 
 
+def lost_bits_of_operands(gradient, g, x, distinct=True):
+    """Values below 2**-109 have bits that three bf16 parts lose.  One among others (and a filter or channel that is zero throughout): no sum can
+    tell, and the gradient stays on the parts.  A filter's or a channel's worth of them: the single-precision gradient, bit for bit."""
+    for odd in range(2):
+        operands = [g.copy(), x.copy()]
+        middle = tuple(n // 2 for n in operands[odd].shape)
+        if middle[1] + 1 < operands[odd].shape[1]:
+            operands[odd][:, -1] = 0
+        operands[odd][middle] = 0
+        without = gradient(*operands)
+        assert not distinct or not np.array_equal(without, gradient(*operands, False))
+        for value in (1e-36, 1e-40):
+            operands[odd][middle] = value
+            assert np.array_equal(bits(gradient(*operands)), bits(without))
+        operands[odd][:, 0] *= np.float32(1e-41)
+        operands[1 - odd] *= np.float32(2.0**40)
+        assert np.array_equal(bits(gradient(*operands)), bits(gradient(*operands, False)))
+
+
 # (x, w, stride, padding, dilation, tile): filter gradients on three bf16 parts, a kernel each (waves along filters, column tiles, quads of a row)
 SPLIT_GRADIENTS = [
     ((8, 64, 9, 17), (64, 64, 3, 3), (1, 1), (1, 1), (1, 1), "2,2,2"),        # whole tiles; rows that end among four columns
@@ -1718,11 +1737,12 @@ def test_filter_gradients_on_three_bf16_parts(abi, monkeypatch, problem):
     assert off <= (1.25 * 5.06e-8 * np.sqrt(2 * 2 * terms / 64) + 3.5e-8) * norm
     assert off <= np.linalg.norm(single - exact)
     # what the parts cannot hold: the single-precision kernel's gradient, bit for bit, and the one after it on the parts again
-    for value in (np.inf, np.nan, 1e-40):
+    for value in (np.inf, np.nan):
         for odd in range(2):
             operands = [g.copy(), x.copy()]
             operands[odd][tuple(n // 2 for n in operands[odd].shape)] = value
             assert np.array_equal(bits(gradient(*operands)), bits(gradient(*operands, split=False)))
+    lost_bits_of_operands(gradient, g, x)
     assert np.array_equal(bits(gradient(gi, xi)), bits(whole))
     assert np.array_equal(bits(gradient(g, x)), bits(got))
 
@@ -1851,11 +1871,12 @@ def test_filter_gradients_of_few_terms_on_three_bf16_parts(abi, monkeypatch, pro
     assert off <= (1.25 * 5.06e-8 * np.sqrt(2 * 2 * terms / 64) + 3.5e-8) * np.linalg.norm(exact)
     assert terms < 30 or off <= np.linalg.norm(single - exact)
     # what the parts cannot hold: the single-precision kernel's gradient, bit for bit, and the one after it on the parts again
-    for value in (np.inf, np.nan, 1e-40):
+    for value in (np.inf, np.nan):
         for odd in range(2):
             operands = [g.copy(), x.copy()]
             operands[odd][tuple(n // 2 for n in operands[odd].shape)] = value
             assert np.array_equal(bits(gradient(*operands)), bits(gradient(*operands, few=False)))
+    lost_bits_of_operands(gradient, g, x, terms >= 30)
     assert np.array_equal(bits(gradient(gi, xi)), bits(whole))
 
 
