@@ -5,8 +5,8 @@
 // returns at once (227 there, 68 TFLOP/s): 25 tiles a block of about 5.5 us each, of which the products are 1.8 at the
 // instruction's rate; the modelled time puts 1.5 of the rest on the requests of the next tile.  Four bytes a request and lane it took 217.  (112,44,3493) * (237,44,3) 402 -> 302.  Error against 64 bits (2-norm), normal values: 2.4e-7 (single precision 1.0e-6).
 //
-// What the parts cannot represent (lost bits of an element, a sum that is not finite) sets a word, and the single-precision kernel behind computes the
-// gradient (see wgrad_split.h).
+// What the parts cannot represent (a sum that is not finite, or smaller than what lost bits of its operands can have been worth) sets a word, and the
+// single-precision kernel behind computes the gradient (see wgrad_split.h).
 #include "few_wgrad.h"
 #include "few_device.h"
 #include "internal.h"
@@ -170,7 +170,11 @@ __global__ void __launch_bounds__(64 * kWaves, 2) few_wgrad_kernel(const FewGrad
 #pragma unroll
     for (int i = 0; i < TM; ++i)
       if (OWN) acc[j][i] += low[j % LOWS][i];
-  if (__any((lost & 0xffffu) != 0) && lane == 0) atomicOr(&params.words[0], 1u);
+  // (behind what the block loads, and behind its sums)
+  constexpr int ROWS = BM + BK;  // filters, then columns
+  unsigned *const notes = reinterpret_cast<unsigned *>(lds + max(2 * (GRAD + kPositions + p.patch), 2 * BM * SUMS)), *const waves = notes + 2 * ROWS;
+  const bool own_lost = __any((lost & 0xffffu) != 0);
+  if (lane == 0) waves[wave] = own_lost;
   float *const sums = lds + l16 * SUMS + cw * TK * 16 + lk * 4;
 #pragma unroll
   for (int round = 0; round < 2; ++round) {
@@ -190,8 +194,47 @@ __global__ void __launch_bounds__(64 * kWaves, 2) few_wgrad_kernel(const FewGrad
         for (int i = 0; i < TM; ++i) acc[j][i] += *reinterpret_cast<const f32x4 *>(sums + (kq >> (round + 1)) * BM * SUMS + i * 16 * SUMS + j * 16);
     }
   }
+  bool any = false;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) any |= waves[w] != 0;
+  if (any) {  // seldom: a second look at the block's values, for the widest of every filter and column, and whether it has lost bits
+    for (int r = (int)threadIdx.x; r < 2 * ROWS; r += 64 * kWaves) notes[r] = 0;
+    auto look = [&](int row) {
+      float widest = 0.0f;
+      unsigned h, m, l, low = 0;
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) split_pair(raw[e], raw[e + 1], h, m, l, low), widen(widest, raw[e], raw[e + 1]);
+      atomicMax(&notes[row], bits_of(widest));
+      if ((low & 0xffffu) != 0) atomicOr(&notes[ROWS + row], 1u);
+    };
+    item = first_item;
+    request(item, 0);
+    few_landed();
+    for (int buf = 0; item < p.items; buf ^= 1) {
+      const FewTile here = few_tile<kPositions>(p, item);
+      const int from = kq * 32 + lk * 8, live = here.end - here.q0 - from;
+      item += params.splits;
+      if (item < p.items) request(item, buf ^ 1);
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        const float *const row = lds + buf * GRAD + (i * 16 + l16) * kPositions;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) raw[e] = e < live ? row[(((from + e) / 4) ^ l16) * 4 + e % 4] : 0.0f;
+        look(i * 16 + l16);
+      }
+#pragma unroll
+      for (int j = 0; j < TK; ++j) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          raw[e] = *reinterpret_cast<const float *>(reinterpret_cast<const char *>(patches + buf * p.patch) + (position_at[buf * kPositions + from + e] + term_at[j]));
+        look(BM + (cw * TK + j) * 16 + l16);
+      }
+      few_landed();
+    }
+  }
   if (kq != 0) return;
-  bool odd = false;
+  const int terms = ((p.items - first_item - 1) / params.splits + 1) * kPositions;
+  bool odd = false;  // a sum is not finite, or smaller than what lost bits can have been worth
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
     const int m = m0 + i * 16 + l16;
@@ -205,6 +248,10 @@ __global__ void __launch_bounds__(64 * kWaves, 2) few_wgrad_kernel(const FewGrad
         if (k >= p.K) continue;
         out[k] = acc[j][i][q];
         odd |= !(__builtin_fabsf(acc[j][i][q]) < __builtin_inff());
+        if (any) {
+          const int f = i * 16 + l16, c = BM + k;
+          odd |= !(__builtin_fabsf(acc[j][i][q]) >= least_sum(notes[ROWS + f] != 0, float_of(notes[f]), notes[ROWS + c] != 0, float_of(notes[c]), terms));
+        }
       }
   }
   if (__any(odd) && lane == 0) atomicOr(&params.words[0], 1u);
@@ -237,7 +284,7 @@ constexpr int kLds = 160 * 1024;
 
 size_t few_lds(const FewGradPlan &pl) {
   const size_t bm = 16 * pl.tm;
-  return std::max<size_t>(2 * (bm * kPositions + kPositions + pl.p.at.patch), 2 * bm * (32 * pl.tk + 4)) * 4;
+  return (std::max<size_t>(2 * (bm * kPositions + kPositions + pl.p.at.patch), 2 * bm * (32 * pl.tk + 4)) + 2 * (bm + 32 * pl.tk) + kWaves) * 4;
 }
 
 }  // namespace
