@@ -199,13 +199,14 @@ __global__ void __launch_bounds__(64 * kWaves, 2) few_wgrad_kernel(const FewGrad
   for (int w = 0; w < kWaves; ++w) any |= waves[w] != 0;
   if (any) {  // seldom: a second look at the block's values, for the widest of every filter and column, and whether it has lost bits
     for (int r = (int)threadIdx.x; r < 2 * ROWS; r += 64 * kWaves) notes[r] = 0;
-    auto look = [&](int row) {
-      float widest = 0.0f;
-      unsigned h, m, l, low = 0;
+    float widest[TM + TK];
+    unsigned low[TM + TK];
 #pragma unroll
-      for (int e = 0; e < 8; e += 2) split_pair(raw[e], raw[e + 1], h, m, l, low), widen(widest, raw[e], raw[e + 1]);
-      atomicMax(&notes[row], bits_of(widest));
-      if ((low & 0xffffu) != 0) atomicOr(&notes[ROWS + row], 1u);
+    for (int r = 0; r < TM + TK; ++r) widest[r] = 0.0f, low[r] = 0;
+    auto look = [&](int r) {
+      unsigned h, m, l;
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) split_pair(raw[e], raw[e + 1], h, m, l, low[r]), widen(widest[r], raw[e], raw[e + 1]);
     };
     item = first_item;
     request(item, 0);
@@ -220,17 +221,24 @@ __global__ void __launch_bounds__(64 * kWaves, 2) few_wgrad_kernel(const FewGrad
         const float *const row = lds + buf * GRAD + (i * 16 + l16) * kPositions;
 #pragma unroll
         for (int e = 0; e < 8; ++e) raw[e] = e < live ? row[(((from + e) / 4) ^ l16) * 4 + e % 4] : 0.0f;
-        look(i * 16 + l16);
+        look(i);
       }
 #pragma unroll
       for (int j = 0; j < TK; ++j) {
 #pragma unroll
         for (int e = 0; e < 8; ++e)
           raw[e] = *reinterpret_cast<const float *>(reinterpret_cast<const char *>(patches + buf * p.patch) + (position_at[buf * kPositions + from + e] + term_at[j]));
-        look(BM + (cw * TK + j) * 16 + l16);
+        look(TM + j);
       }
       few_landed();
     }
+#pragma unroll
+    for (int r = 0; r < TM + TK; ++r) {
+      const int row = (r < TM ? r : TM + cw * TK + r - TM) * 16 + l16;
+      atomicMax(&notes[row], bits_of(widest[r]));
+      if ((low[r] & 0xffffu) != 0) atomicOr(&notes[ROWS + row], 1u);
+    }
+    __syncthreads();
   }
   if (kq != 0) return;
   const int terms = ((p.items - first_item - 1) / params.splits + 1) * kPositions;

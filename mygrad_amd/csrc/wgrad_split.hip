@@ -101,6 +101,7 @@ __global__ void __launch_bounds__(512, 2) wgrad_split_kernel(const WgradSplitPar
     const int in_walk = min(p.stages - stage % p.stages, last_stage - stage);
     ticks += in_walk + p.depth, stage += in_walk;
   }
+  const int all_ticks = ticks;
   int to_request = ticks, left = 0, filling = 0, next_stage = first_stage, octet = 0, strip = 0;
   // Of the walk, segment by segment of the thread: byte offset in its first tick, and the place (row; ALONG: column) whose
   // distance from the walk's beginning decides whether four columns are there at all.
@@ -186,29 +187,28 @@ __global__ void __launch_bounds__(512, 2) wgrad_split_kernel(const WgradSplitPar
 #pragma unroll
     for (int e = 0; e < 4; ++e) request(e);
   };
-  // of a task's values: bits that the parts have lost, and the widest one
-  unsigned lost[TASKS];
-  float widest[TASKS];
+  // what lies outside of a task's rows, among what was requested, is zero
+  auto clear_outside = [&](int s) MG_INLINE {
+    if ((ALONG ? moved[s] : 1) < whole[s]) return;
 #pragma unroll
-  for (int s = 0; s < TASKS; ++s) lost[s] = 0, widest[s] = 0.0f;
+    for (int e = 0; e < 4; ++e) {
+      int end;
+      const int col = columns_at(tasks[s], e, end) + (ALONG ? moved[s] : 0);
+      u32x4 v = raw[s][e];
+      v = col < 0 && (col & 1) != 0 ? u32x4{0, v[0], v[1], v[2]} : v;
+      v = col < 0 && ((-col) & 2) != 0 ? u32x4{0, 0, v[0], v[1]} : v;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) raw[s][e][u] = col + u < end ? v[u] : 0u;
+    }
+  };
+  unsigned lost = 0;
   // splits and parks what was requested
   auto park = [&](int group) MG_INLINE {
 #pragma unroll
     for (int s = 0; s < TASKS; ++s) {
       if (!has[s]) continue;
       const Task &t = tasks[s];
-      if ((ALONG ? moved[s] : 1) >= whole[s]) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          int end;
-          const int col = columns_at(t, e, end) + (ALONG ? moved[s] : 0);
-          u32x4 v = raw[s][e];
-          v = col < 0 && (col & 1) != 0 ? u32x4{0, v[0], v[1], v[2]} : v;
-          v = col < 0 && ((-col) & 2) != 0 ? u32x4{0, 0, v[0], v[1]} : v;
-#pragma unroll
-          for (int u = 0; u < 4; ++u) raw[s][e][u] = col + u < end ? v[u] : 0u;
-        }
-      }
+      clear_outside(s);
       u32x2 *const to = reinterpret_cast<u32x2 *>(lds + t.put + group * t.put_group) + half;
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
@@ -216,9 +216,7 @@ __global__ void __launch_bounds__(512, 2) wgrad_split_kernel(const WgradSplitPar
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
           unsigned h, m, l;
-          const float a = float_of(raw[s][2 * e][u]), b = float_of(raw[s][2 * e + 1][u]);
-          split_pair(a, b, h, m, l, lost[s]);
-          widen(widest[s], a, b);
+          split_pair(float_of(raw[s][2 * e][u]), float_of(raw[s][2 * e + 1][u]), h, m, l, lost);
           parts[0][e] = h, parts[1][e] = m, parts[2][e] = l;
         }
 #pragma unroll
@@ -350,31 +348,53 @@ __global__ void __launch_bounds__(512, 2) wgrad_split_kernel(const WgradSplitPar
       const f32x4 sum = j < kOwnLow ? acc[j][i] + low[j < kOwnLow ? j : 0][i] : acc[j][i];
       *reinterpret_cast<f32x4 *>(sums + (((kq * CW + cw) * FT + fw * 32 + i * 16 + l16) * kSumStride + j * 16 + lk * 4)) = sum;
     }
-  // Of every channel and filter of the tile, where any has lost bits: the widest value, and whether it has.
   constexpr int ROWS = FT + CW * 16;  // filters, then channels
   unsigned *const notes = reinterpret_cast<unsigned *>(sums + kSums), *const waves = notes + 2 * ROWS;
+  const bool own_lost = __any((lost & 0xffffu) != 0);
+  if (lane == 0) waves[wave] = own_lost;
+  __syncthreads();
   bool any = false;
 #pragma unroll
-  for (int s = 0; s < TASKS; ++s) any |= has[s] && (lost[s] & 0xffffu) != 0;
-  any = __any(any);
-  if (lane == 0) waves[wave] = any;
-  __syncthreads();
-#pragma unroll
   for (int w = 0; w < 8; ++w) any |= waves[w] != 0;
-  if (any) {  // seldom
+  // Seldom: a second look at the block's values, for the widest of every filter and channel, and whether it has lost bits.  (64 channels, 3 x 3, 56 x 56:
+  // 166 us without a lost bit, 219 - 225 with one, 305 with some in every block, 390 - 410 where any sent the gradient to the
+  // single-precision kernel.  With the widest values kept along the way all take 169, and the layers along one axis 3 % more.)
+  if (any) {
     for (int i = (int)threadIdx.x; i < 2 * ROWS; i += 512) notes[i] = 0;
+    float widest[TASKS];
+    unsigned low[TASKS];
+#pragma unroll
+    for (int s = 0; s < TASKS; ++s) widest[s] = 0.0f, low[s] = 0;
+    to_request = all_ticks, left = 0, next_stage = first_stage;
+    while (to_request > 0) {
+      advance();
+      request_all();
+#pragma unroll
+      for (int s = 0; s < TASKS; ++s) {
+        clear_outside(s);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int u = 0; u < 4; u += 2) {
+            const float a = float_of(raw[s][e][u]), b = float_of(raw[s][e][u + 1]);
+            unsigned h, m, l;
+            split_pair(a, b, h, m, l, low[s]);
+            widen(widest[s], a, b);
+          }
+      }
+    }
     __syncthreads();
 #pragma unroll
     for (int s = 0; s < TASKS; ++s) {
       if (!has[s]) continue;
       const int number = wave + 8 * s, row = tasks[s].is_x ? FT + min((number - GTASKS) / xtasks, CW - 1) * 16 + l16 : (number * 2 + (lk >> 1)) / KW * 16 + l16;
       atomicMax(&notes[row], bits_of(widest[s]));
-      if ((lost[s] & 0xffffu) != 0) atomicOr(&notes[ROWS + row], 1u);
+      if ((low[s] & 0xffffu) != 0) atomicOr(&notes[ROWS + row], 1u);
     }
     __syncthreads();
   }
   float *const out = p.partial + (long long)(split * p.tiles + tile) * (CW * FT * kColumns);
-  bool odd = false;  // a sum is not finite, or bits that it would have were lost
+  bool odd = false;  // a sum is not finite, or smaller than what lost bits can have been worth
   const int terms = (last_stage - first_stage) * (KW * 4 * 8);
   for (int e = (int)threadIdx.x; e < CW * FT * kColumns / 4; e += 512) {
     const int f = e / (kColumns / 4), c = e % (kColumns / 4) * 4;  // (f: column tile, filter)
