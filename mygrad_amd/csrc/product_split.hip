@@ -253,16 +253,13 @@ __global__ void __launch_bounds__(512, 2) product_gemm_kernel(const ProductParam
 #pragma unroll
       for (int i = 0; i < 4; ++i) acc[j][i] += low[j][i];
     const TilePlace at = tile_place(here.tile, p.m_tiles, n_tiles);
-    unsigned largest = 0, smallest = ~0u;
+    unsigned largest = 0;
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          largest = max(largest, bits_of(acc[j][i][q]) << 1);
-          smallest = min(smallest, bits_of(acc[j][i][q]) << 1);
-        }
+        for (int q = 0; q < 4; ++q) largest = max(largest, bits_of(acc[j][i][q]) << 1);
     // the widest values of either operand and which of them have lost bits: bit 0
     unsigned a_note = 0, b_note = 0;
     for (int i = (int)threadIdx.x; i < (PM + PN) * p.steps; i += 512) {
@@ -285,7 +282,15 @@ __global__ void __launch_bounds__(512, 2) product_gemm_kernel(const ProductParam
         atomicMax(&note[2], b_note);
         __syncthreads();
         const float bound = ((found & 2u ? float_of(note[1] >> 1) : 0.0f) + (found & 1u ? float_of(note[2] >> 1) : 0.0f)) * (float)(p.steps * 32) * 0x1p-109f;
-        if (!(float_of(smallest >> 1) >= bound)) atomicOr(&note[0], 4u);
+        bool below = false;  // (sums beyond the results' edges are zeros that nobody stores)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+              below |= at.m * BM + wm + i * 16 + l16 < p.M && at.n * BN + wn + j * 16 + lk * 4 + q < p.columns && !(__builtin_fabsf(acc[j][i][q]) >= bound);
+        if (below) atomicOr(&note[0], 4u);
         __syncthreads();
         found = (unsigned)uniform((int)note[0]);
       }

@@ -129,6 +129,15 @@ def test_large_products_on_three_bf16_parts(abi, monkeypatch, batch, M, K, N):
             for i in (0, 2):
                 got, ref = run(*args)[i], exact(*args)[i]
                 assert np.all(np.abs(got - ref) <= (2 + 5 / 32) * 2.0**-24 * np.abs(ref) + 2.0**-149)
+    # one value of low bits that parts lose, in the last row and column: no sum can tell, and all stay on the parts
+    for which in range(3):
+        args = [v.copy() for v in (a, x, g)]
+        where = tuple(n - 1 for n in args[which].shape)
+        args[which][where] = 0
+        without = run(*args)
+        args[which][where] = 1e-36
+        for got, was, count in zip(run(*args), without, terms):
+            assert count < 100 or np.array_equal(got.view(np.uint32), was.view(np.uint32))
     # infinities, NaN and sums that overflow are those of single precision
     for value in (np.inf, np.nan, 3e38):
         odd = [v.copy() for v in (a * np.float32(4), x, g)]
