@@ -377,9 +377,18 @@ __global__ void __launch_bounds__(256) product_finish_kernel(const ProductParams
   __shared__ float as[32 * LD], bs[32 * LD];
   const int lane = t & 63, l16 = lane & 15, lk = lane >> 4, wave = uniform(t >> 6);
   const int wm = wave / 2 * 32, wn = wave % 2 * 32, row = t & 63, oct = t >> 6;
-  for (int unit = (int)blockIdx.x - fix_blocks; unit < p.tiles * 8; unit += kProductRedoBlocks) {
-    const int tile = unit / 8, sub = unit % 8;
-    if (!marked(tile)) continue;
+  // the blocks take the marked tiles' eighths in turn (by the number of a tile, those of one column of tiles would meet in a few blocks)
+  int word = 0, before = 0;  // of the marks; tiles marked in the words before it
+  for (int turn = (int)blockIdx.x - fix_blocks;; turn += kProductRedoBlocks) {
+    int skip = turn / 8 - before;
+    while (word < p.marks - 1 && __popc(p.redo[1 + word]) <= skip) {
+      const int here = __popc(p.redo[1 + word++]);
+      before += here, skip -= here;
+    }
+    if (word >= p.marks - 1) break;
+    unsigned marks = p.redo[1 + word];
+    while (skip-- > 0) marks &= marks - 1;
+    const int tile = word * 32 + __ffs(marks) - 1, sub = turn % 8;
     const TilePlace at = tile_place(tile, p.m_tiles, n_tiles);
     const int m0 = at.m * PM * kProductPanel + sub / (2 * PN) * 64, n0 = at.n * PN * kProductPanel + sub % (2 * PN) * 64;
     f32x4 acc[2][2];
