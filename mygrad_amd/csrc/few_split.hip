@@ -29,12 +29,13 @@ constexpr int kWaves = 8;
 template <int TM, int TN>
 __global__ void __launch_bounds__(64 * kWaves, 2) few_split_kernel(const FewParams p) {
   constexpr int BM = 16 * TM, BN = 16 * TN * kWaves;
-  // filters [step][part][octet of terms][row]; where a term lies in the patch, for one step more; two patches; a word
+  // filters [step][part][octet of terms][row]; where a term lies in the patch, for one step more; two patches; of each filter the widest
+  // value, and whether it has lost bits
   extern __shared__ __attribute__((aligned(16))) u32x4 lds[];
   const int pieces = p.steps * 12 * BM, terms = p.steps * 32;
   int *const term_at = reinterpret_cast<int *>(lds + pieces);
   float *const patches = reinterpret_cast<float *>(term_at + terms + 32);
-  unsigned *const tiny = reinterpret_cast<unsigned *>(patches + 2 * p.patch);
+  unsigned *const notes = reinterpret_cast<unsigned *>(patches + 2 * p.patch);
   const int lane = (int)threadIdx.x & 63, l16 = lane & 15, lk = lane >> 4, wave = uniform((int)threadIdx.x >> 6);
   // blocks are dealt to the eight XCDs in turn: an XCD's blocks take neighbouring tiles
   const int grid = (int)gridDim.x, place = grid % 8 == 0 ? (int)(blockIdx.x & 7) * (grid / 8) + (int)(blockIdx.x >> 3) : (int)blockIdx.x;
@@ -51,16 +52,18 @@ __global__ void __launch_bounds__(64 * kWaves, 2) few_split_kernel(const FewPara
   request(few_tile<BN>(p, item), 0, 0, own_lines);
 
   // ---- the filters of the block, and where their terms lie
-  if (threadIdx.x == 0) *tiny = 0;
+  if (threadIdx.x < 2 * BM) notes[threadIdx.x] = 0;
   for (int k = (int)threadIdx.x; k < terms + 32; k += 64 * kWaves) {
     const int c = (int)p.by_window.div((unsigned)k), tap = k - c * (int)p.by_window.d, t1 = (int)p.by_w2.div((unsigned)tap), t2 = tap - t1 * p.W2;
     term_at[k] = k < p.K ? ((c * p.patch_rows + t1 * p.D1) * p.pitch + t2 * p.D2) * 4 : 0;
   }
   __syncthreads();
-  unsigned lost = 0;
+  unsigned lost;
   for (int at = (int)threadIdx.x; at < p.steps * 4 * BM; at += 64 * kWaves) {
     const int m = at % BM, oct = at / BM;
     u32x4 parts[3];
+    float widest = 0.0f;
+    lost = 0;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       float v[2];
@@ -71,14 +74,16 @@ __global__ void __launch_bounds__(64 * kWaves, 2) few_split_kernel(const FewPara
       }
       unsigned first, second, third;
       split_pair(v[0], v[1], first, second, third, lost);
+      widen(widest, v[0], v[1]);
       parts[0][e] = first, parts[1][e] = second, parts[2][e] = third;
     }
+    atomicMax(&notes[m], bits_of(widest));
+    if ((lost & 0xffffu) != 0) atomicOr(&notes[BM + m], 1u);
 #pragma unroll
     for (int part = 0; part < 3; ++part) lds[((oct / 4 * 3 + part) * 4 + oct % 4) * BM + m] = parts[part];
   }
-  if ((lost & 0xffffu) != 0) atomicOr(tiny, 1u);
   few_landed();
-  const bool lossy = uniform((int)*tiny) != 0;  // parts do not hold some filter value
+  const bool lossy = __any(notes[BM + lane % BM] != 0);  // some filter value has lost bits
 
   const u32x4 *const filters = lds + lk * BM + l16;
   const int4v *const mine_at = reinterpret_cast<const int4v *>(term_at) + lk * 2;
@@ -186,8 +191,44 @@ __global__ void __launch_bounds__(64 * kWaves, 2) few_split_kernel(const FewPara
 #pragma unroll
         for (int q = 0; q < 4; ++q) largest = max(largest, bits_of(acc[j][i][q]) << 1);
       }
-    // What the parts cannot hold: the wave's results again on the single-precision instruction.
-    if (lossy || __any((lost & 0xffffu) != 0 || largest >= 2u * (255u << 23))) {
+    // What the parts cannot hold: the wave's results again on the single-precision instruction.  Lost bits count where a result is not far above
+    // what they can have been worth; the widest values of the wave's positions are looked up then.
+    bool again = __any(largest >= 2u * (255u << 23));
+    if (!again && (lossy || __any((lost & 0xffffu) != 0))) {
+      bool below = false;
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        float widest = 0.0f;
+        unsigned low = 0;
+        for (int step = 0; step < p.steps; ++step) {
+          int terms[8];
+          read_terms_at(step, terms);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) raw[e] = *reinterpret_cast<const float *>(patch + (base[j] + terms[e]));
+#pragma unroll
+          for (int e = 0; e < 8; e += 2) {
+            unsigned h, m, l;
+            split_pair(raw[e], raw[e + 1], h, m, l, low);
+            widen(widest, raw[e], raw[e + 1]);
+          }
+        }
+#pragma unroll
+        for (int d = 16; d < 64; d *= 2) {
+          widest = fmaxf(widest, __shfl_xor(widest, d));
+          low |= (unsigned)__shfl_xor((int)low, d);
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const float widest_x = __shfl(widest, lk * 4 + q);
+          const bool lost_x = ((unsigned)__shfl((int)low, lk * 4 + q) & 0xffffu) != 0;
+#pragma unroll
+          for (int i = 0; i < TM; ++i)
+            below |= !(__builtin_fabsf(acc[j][i][q]) >= least_sum(notes[BM + i * 16 + l16] != 0, float_of(notes[i * 16 + l16]), lost_x, widest_x, p.K));
+        }
+      }
+      again = __any(below);
+    }
+    if (again) {
 #pragma unroll
       for (int j = 0; j < TN; ++j)
 #pragma unroll
@@ -232,7 +273,7 @@ __global__ void __launch_bounds__(64 * kWaves, 2) few_split_kernel(const FewPara
 
 constexpr int kLds = 160 * 1024;
 
-size_t few_lds(const FewPlan &pl) { return (size_t)pl.p.steps * 12 * 16 * pl.tm * 16 + (pl.p.steps + 1) * 32 * 4 + 2 * (size_t)pl.p.patch * 4 + 16; }
+size_t few_lds(const FewPlan &pl) { return (size_t)pl.p.steps * 12 * 16 * pl.tm * 16 + (pl.p.steps + 1) * 32 * 4 + 2 * (size_t)pl.p.patch * 4 + 2 * 16 * pl.tm * 4; }
 
 }  // namespace
 

@@ -1823,6 +1823,16 @@ def test_forward_of_few_terms_on_three_bf16_parts(abi, monkeypatch, problem):
             assert np.array_equal(some[~finite], plain[~finite], equal_nan=True) and np.all(np.isfinite(some[finite]))
             if odd == 0 and x_shape[0] > 1:
                 assert np.array_equal(bits(some[0]), bits(far[0]))
+    # one value of low bits that parts lose, beside a filter and a sample of zeros: no sum can tell, and all stay on the parts
+    for odd in range(2):
+        operands = [x.copy(), w.copy()]
+        for v in operands:
+            v[len(v) // 2 + 1 :][:1] = 0
+        middle = tuple(n // 2 for n in operands[odd].shape)
+        operands[odd][middle] = 0
+        without = forward(*operands)
+        operands[odd][middle] = 1e-36
+        assert terms < 6 or np.array_equal(bits(forward(*operands)), bits(without))
     # one term a sum, of values below the smallest number of bf16: the single-precision instruction's results, to its rounding
     tiny = np.zeros_like(w)
     tiny.reshape(w_shape[0], -1)[:, 0] = 1e-41
