@@ -21,20 +21,6 @@ __device__ __forceinline__ FewTile few_tile(const FewParams &p, int item) {
   return FewTile{n, q0, (int)p.by_row.div((unsigned)q0), 0, min(q0 + POSITIONS, p.gvol)};
 }
 
-// BYTES a lane from a buffer straight into LDS, the lanes' pieces one behind the other from byte `to` on.
-template <int BYTES>
-__device__ __forceinline__ void few_to_lds(__amdgpu_buffer_rsrc_t buffer, unsigned lane_at, unsigned at, unsigned to) {
-  typedef __attribute__((address_space(3))) void *LdsPointer;
-  static_assert(BYTES == 4 || BYTES == 16, "a word or four a lane");
-  if (BYTES == 16)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(buffer, (LdsPointer)(unsigned long long)to, 16, (int)lane_at, (int)at, 0, 0);
-  else
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(buffer, (LdsPointer)(unsigned long long)to, 4, (int)lane_at, (int)at, 0, 0);
-}
-
-// This wave's loads have landed and its LDS reads are done; then all waves of the block are here.
-__device__ __forceinline__ void few_landed() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
 // Row `line` (of channel line / patch_rows) of the tile's patch into LDS, from byte `patch` on: sixteen bytes a lane (requests are what the
 // kernels wait for: 4 bytes a lane, four times as many, took the filter gradient of a 3 x 7 x 7 layer 217 us, 158 so), the four columns that
 // the end of a row cuts by themselves.
@@ -46,17 +32,17 @@ __device__ __forceinline__ void few_request_line(const FewParams &p, const FewTi
   const unsigned at = there ? (unsigned)(((t.n * p.C + c) * p.X1 + r) * p.X2) * 4u : 0u, to = patch + (unsigned)(line * p.pitch) * 4u;
   if (p.lead < 0) {  // a row that one request a word takes
     const int column = first - 1 + lane;
-    if (lane < p.pitch) few_to_lds<4>(x, (unsigned)column < (unsigned)p.X2 ? (unsigned)column * 4u : kOutside, at, to);
+    if (lane < p.pitch) to_lds<4>(x, (unsigned)column < (unsigned)p.X2 ? (unsigned)column * 4u : kOutside, at, to);
     return;
   }
   const int cut = (p.X2 & ~3) - first;  // patch column of the cut four, if they are
   for (int q = 0; q < p.pitch; q += 256) {
     const int mine = q + lane * 4, column = first + mine;
     if (mine < p.pitch && (mine != cut || (p.X2 & 3) == 0))
-      few_to_lds<16>(x, column >= 0 && column < p.X2 ? (unsigned)column * 4u : kOutside, at, to + (unsigned)q * 4u);
+      to_lds<16>(x, column >= 0 && column < p.X2 ? (unsigned)column * 4u : kOutside, at, to + (unsigned)q * 4u);
   }
   if ((p.X2 & 3) != 0 && cut >= 0 && cut < p.pitch) {
-    if (lane < 4) few_to_lds<4>(x, lane < (p.X2 & 3) ? (unsigned)(first + cut + lane) * 4u : kOutside, at, to + (unsigned)cut * 4u);
+    if (lane < 4) to_lds<4>(x, lane < (p.X2 & 3) ? (unsigned)(first + cut + lane) * 4u : kOutside, at, to + (unsigned)cut * 4u);
   }
 }
 

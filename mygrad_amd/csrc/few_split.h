@@ -30,6 +30,14 @@ struct FewPlan {
   FewParams p{};
 };
 
+constexpr int kFewLds = 160 * 1024;
+
+// How tiles of `bm` filters by `positions` (along: of a row) lie; false: their patches are too large, or the layer is none that the kernels take.
+// (LDS that they need beside the patches is not looked at.)
+bool few_geometry(FewParams &p, int N, int C, int F, const int *X, const int *G, const int *W, const int *S, const int *D, const int *P, int bm, int positions, bool along);
+// Loads that a tile's patch takes.
+long long few_requests(const FewParams &p);
+
 FewPlan plan_few_split(int N, int C, int F, const int *X, const int *G, const int *W, const int *S, const int *D, const int *P, int cus);
 int launch_few_split(const FewPlan &pl, const void *x, const void *w, void *out, hipStream_t s);
 

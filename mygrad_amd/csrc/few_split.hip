@@ -82,7 +82,7 @@ __global__ void __launch_bounds__(64 * kWaves, 2) few_split_kernel(const FewPara
 #pragma unroll
     for (int part = 0; part < 3; ++part) lds[((oct / 4 * 3 + part) * 4 + oct % 4) * BM + m] = parts[part];
   }
-  few_landed();
+  landed();
   const bool lossy = __any(notes[BM + lane % BM] != 0);  // some filter value has lost bits
 
   const u32x4 *const filters = lds + lk * BM + l16;
@@ -247,7 +247,7 @@ __global__ void __launch_bounds__(64 * kWaves, 2) few_split_kernel(const FewPara
         }
       }
     }
-    few_landed();  // the next patch is there, and nobody reads this one any more
+    landed();  // the next patch is there, and nobody reads this one any more
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
       const int m = m0 + i * 16 + l16;
@@ -271,17 +271,38 @@ __global__ void __launch_bounds__(64 * kWaves, 2) few_split_kernel(const FewPara
 
 #define MG_FEW_SHAPES(X) X(4, 3) X(4, 2) X(2, 4) X(2, 2)
 
-constexpr int kLds = 160 * 1024;
-
 size_t few_lds(const FewPlan &pl) { return (size_t)pl.p.steps * 12 * 16 * pl.tm * 16 + (pl.p.steps + 1) * 32 * 4 + 2 * (size_t)pl.p.patch * 4 + 2 * 16 * pl.tm * 4; }
 
 }  // namespace
 
+// Tiles of BM filters by `positions`, and their patches of x.
+bool few_geometry(FewParams &p, int N, int C, int F, const int *X, const int *G, const int *W, const int *S, const int *D, const int *P, int bm, int positions, bool along) {
+  const long long K = (long long)C * W[1] * W[2], gvol = (long long)G[1] * G[2];
+  if (X[0] != 1 || G[0] != 1 || W[0] != 1 || P[0] != 0 || gvol > 1 << 29 || N > 1 << 24) return false;
+  p.C = C, p.F = F, p.K = (int)K, p.steps = (int)ceil_div(K, 32);
+  p.X1 = X[1], p.X2 = X[2], p.G2 = G[2], p.gvol = (int)gvol;
+  p.S1 = S[1], p.S2 = S[2], p.D1 = D[1], p.D2 = D[2], p.P1 = P[1], p.P2 = P[2], p.W1 = W[1], p.W2 = W[2];
+  p.m_tiles = (int)ceil_div(F, bm), p.along = along, p.lead = -1;
+  const long long rows = along ? 1 : std::min<long long>(G[1], ceil_div(positions - 1, G[2]) + 1), columns = along ? std::min(positions, G[2]) : G[2];
+  const long long patch_rows = (rows - 1) * S[1] + (W[1] - 1ll) * D[1] + 1, needed = (columns - 1) * S[2] + (W[2] - 1ll) * D[2] + 1;
+  long long pitch = needed;
+  if (needed > 64) p.lead = (4 - P[2] % 4) % 4, pitch = ceil_div(p.lead + needed, 4) * 4;
+  if (patch_rows > kFewLds || pitch > kFewLds || C * patch_rows * pitch * 8 > kFewLds) return false;
+  p.patch_rows = (int)patch_rows, p.pitch = (int)pitch, p.patch = (int)ceil_div(C * patch_rows * pitch, 4) * 4;
+  p.run_tiles = (int)ceil_div(along ? G[2] : gvol, positions), p.sample_tiles = p.run_tiles * (along ? G[1] : 1);
+  if ((long long)N * p.sample_tiles > 1 << 30) return false;
+  p.items = N * p.sample_tiles;
+  p.by_sample = make_fastdiv((unsigned)p.sample_tiles), p.by_run = make_fastdiv((unsigned)p.run_tiles), p.by_row = make_fastdiv((unsigned)G[2]);
+  p.by_patch_rows = make_fastdiv((unsigned)patch_rows), p.by_window = make_fastdiv((unsigned)(W[1] * W[2])), p.by_w2 = make_fastdiv((unsigned)W[2]);
+  return true;
+}
+
+long long few_requests(const FewParams &p) { return (long long)p.C * p.patch_rows * (p.lead < 0 ? 1 : ceil_div(p.pitch, 256) + (p.X2 % 4 != 0)); }
+
 // The shape and the walk with the least modelled time, in us: fitted to 160 timed (layer, shape), 9 in 10 within 9 % of it.
 FewPlan plan_few_split(int N, int C, int F, const int *X, const int *G, const int *W, const int *S, const int *D, const int *P, int cus) {
   FewPlan best;
-  const long long K = (long long)C * W[1] * W[2], gvol = (long long)G[1] * G[2];
-  if (X[0] != 1 || G[0] != 1 || W[0] != 1 || P[0] != 0 || K > 192 || gvol > 1 << 29 || N > 1 << 24) return best;
+  if ((long long)C * W[1] * W[2] > 192) return best;
   int want = 0;
   if (const char *v = getenv("MYGRAD_HIP_FEW")) want = atoi(v);  // 10 tm + tn (tests)
 #define MG_SHAPE(TM, TN) {TM, TN},
@@ -292,32 +313,14 @@ FewPlan plan_few_split(int N, int C, int F, const int *X, const int *G, const in
     pl.tm = shape[0], pl.tn = shape[1];
     if (want > 10 ? want != 10 * pl.tm + pl.tn : (F > 32) != (pl.tm == 4)) continue;
     FewParams &p = pl.p;
-    const int bn = 16 * pl.tn * kWaves, bm = 16 * pl.tm;
-    p.C = C, p.F = F, p.K = (int)K, p.steps = (int)ceil_div(K, 32);
-    p.X1 = X[1], p.X2 = X[2], p.G2 = G[2], p.gvol = (int)gvol;
-    p.S1 = S[1], p.S2 = S[2], p.D1 = D[1], p.D2 = D[2], p.P1 = P[1], p.P2 = P[2], p.W1 = W[1], p.W2 = W[2];
-    p.m_tiles = (int)ceil_div(F, bm);
-    if (p.m_tiles > cus) continue;
-    for (const int along : {0, 1}) {
-      p.along = along, p.lead = -1;
-      const long long rows = along ? 1 : std::min<long long>(G[1], ceil_div(bn - 1, G[2]) + 1), columns = along ? std::min(bn, G[2]) : G[2];
-      const long long patch_rows = (rows - 1) * S[1] + (long long)(W[1] - 1) * D[1] + 1, needed = (columns - 1) * S[2] + (long long)(W[2] - 1) * D[2] + 1;
-      long long pitch = needed;
-      if (needed > 64) p.lead = (4 - P[2] % 4) % 4, pitch = ceil_div(p.lead + needed, 4) * 4;
-      if (patch_rows > kLds || pitch > kLds || C * patch_rows * pitch * 8 > kLds) continue;
-      p.patch_rows = (int)patch_rows, p.pitch = (int)pitch, p.patch = (int)ceil_div(C * patch_rows * pitch, 4) * 4;
-      if (few_lds(pl) > (size_t)kLds) continue;
-      p.run_tiles = (int)ceil_div(along ? G[2] : gvol, bn), p.sample_tiles = p.run_tiles * (along ? G[1] : 1);
-      if ((long long)N * p.sample_tiles > 1 << 30) continue;
-      p.items = N * p.sample_tiles;
-      p.by_sample = make_fastdiv((unsigned)p.sample_tiles), p.by_run = make_fastdiv((unsigned)p.run_tiles), p.by_row = make_fastdiv((unsigned)G[2]);
-      p.by_patch_rows = make_fastdiv((unsigned)patch_rows);
-      p.by_window = make_fastdiv((unsigned)(W[1] * W[2])), p.by_w2 = make_fastdiv((unsigned)W[2]);
+    const int bn = 16 * pl.tn * kWaves;
+    for (const bool along : {false, true}) {
+      if (!few_geometry(p, N, C, F, X, G, W, S, D, P, 16 * pl.tm, bn, along) || p.m_tiles > cus || few_lds(pl) > (size_t)kFewLds) continue;
       const int per = std::max(1, std::min(p.items, cus / p.m_tiles));
       pl.grid = per * p.m_tiles;
       const double rounds = (double)ceil_div(p.items, per);
-      const double requests = (double)(C * patch_rows * (p.lead < 0 ? 1 : ceil_div(pitch, 256) + (X[2] % 4 != 0)));
-      pl.time = 8.2 + 0.208 * p.steps + rounds * (0.895 + 0.162 * p.steps * pl.tn * pl.tm + 0.0155 * requests) + 0.137e-6 * 4.0 * (double)N * F * (double)gvol;
+      const double requests = (double)few_requests(p);
+      pl.time = 8.2 + 0.208 * p.steps + rounds * (0.895 + 0.162 * p.steps * pl.tn * pl.tm + 0.0155 * requests) + 0.137e-6 * 4.0 * (double)N * F * (double)p.gvol;
       if (best.tm == 0 || pl.time < best.time) best = pl;
     }
   }
@@ -332,7 +335,7 @@ int launch_few_split(const FewPlan &pl, const void *x, const void *w, void *out,
   ScopedTiming timed(TAG_CONV_FWD);
 #define MG_FEW(TM, TN)                                                                                                              \
   if (pl.tm == TM && pl.tn == TN) {                                                                                                 \
-    static const hipError_t allowed = hipFuncSetAttribute((const void *)few_split_kernel<TM, TN>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds); \
+    static const hipError_t allowed = hipFuncSetAttribute((const void *)few_split_kernel<TM, TN>, hipFuncAttributeMaxDynamicSharedMemorySize, kFewLds); \
     MG_HIP(allowed);                                                                                                                \
     hipLaunchKernelGGL((few_split_kernel<TM, TN>), dim3((unsigned)pl.grid), dim3(64 * kWaves), few_lds(pl), s, p);                   \
   }

@@ -47,7 +47,7 @@ __global__ void __launch_bounds__(64 * kWaves, 2) few_wgrad_kernel(const FewGrad
     for (int pair = wave; pair < BM / 2; pair += kWaves) {
       const int r = pair * 2 + lane / 32, q = ((lane & 31) ^ (r & 15)) * 4;
       const bool there = m0 + r < p.F && t.q0 + q < t.end;
-      few_to_lds<16>(grad, there ? at + (unsigned)(r * p.gvol + q) * 4u : kOutside, 0, lds_at + (unsigned)(buf * GRAD + pair * 2 * kPositions) * 4u);
+      to_lds<16>(grad, there ? at + (unsigned)(r * p.gvol + q) * 4u : kOutside, 0, lds_at + (unsigned)(buf * GRAD + pair * 2 * kPositions) * 4u);
     }
     if ((int)threadIdx.x < kPositions) {
       const int q = min(t.q0 + (int)threadIdx.x, t.end - 1), row = (int)p.by_row.div((unsigned)q);
@@ -87,7 +87,7 @@ __global__ void __launch_bounds__(64 * kWaves, 2) few_wgrad_kernel(const FewGrad
   int item = first_item;
   if (item < p.items) {
     request(item, 0);
-    few_landed();
+    landed();
   }
   for (int buf = 0; item < p.items; buf ^= 1) {
     const FewTile here = few_tile<kPositions>(p, item);
@@ -160,7 +160,7 @@ __global__ void __launch_bounds__(64 * kWaves, 2) few_wgrad_kernel(const FewGrad
 #pragma unroll
       for (int i = 0; i < TM; ++i) acc[TK - 1][i] += low[(TK - 1) % 2][i];
     }
-    few_landed();  // the next tile is there, and nobody reads this one any more
+    landed();  // the next tile is there, and nobody reads this one any more
   }
 
   // ---- the sums of the waves along the positions, two and two; acc[j][i][q] is filter 16 i + l16, column 16 (cw TK + j) + 4 lk + q
@@ -210,7 +210,7 @@ __global__ void __launch_bounds__(64 * kWaves, 2) few_wgrad_kernel(const FewGrad
     };
     item = first_item;
     request(item, 0);
-    few_landed();
+    landed();
     for (int buf = 0; item < p.items; buf ^= 1) {
       const FewTile here = few_tile<kPositions>(p, item);
       const int from = kq * 32 + lk * 8, live = here.end - here.q0 - from;
@@ -230,7 +230,7 @@ __global__ void __launch_bounds__(64 * kWaves, 2) few_wgrad_kernel(const FewGrad
           raw[e] = *reinterpret_cast<const float *>(reinterpret_cast<const char *>(patches + buf * p.patch) + (position_at[buf * kPositions + from + e] + term_at[j]));
         look(TM + j);
       }
-      few_landed();
+      landed();
     }
 #pragma unroll
     for (int r = 0; r < TM + TK; ++r) {
@@ -288,8 +288,6 @@ __global__ void __launch_bounds__(256) few_wgrad_reduce_kernel(const FewGradPara
 
 #define MG_FEW_GRADS(X) X(4, 1) X(4, 2) X(4, 3) X(4, 4) X(4, 5) X(2, 1) X(2, 2) X(2, 3) X(2, 4) X(2, 5)
 
-constexpr int kLds = 160 * 1024;
-
 size_t few_lds(const FewGradPlan &pl) {
   const size_t bm = 16 * pl.tm;
   return (std::max<size_t>(2 * (bm * kPositions + kPositions + pl.p.at.patch), 2 * bm * (32 * pl.tk + 4)) + 2 * (bm + 32 * pl.tk) + kWaves) * 4;
@@ -300,31 +298,15 @@ size_t few_lds(const FewGradPlan &pl) {
 // Modelled time in us: fitted to 85 timed layers, 9 in 10 within 6 % of it.
 FewGradPlan plan_few_wgrad(int N, int C, int F, const int *X, const int *G, const int *W, const int *S, const int *D, const int *P, int cus) {
   FewGradPlan best;
-  const long long K = (long long)C * W[1] * W[2], gvol = (long long)G[1] * G[2];
-  if (X[0] != 1 || G[0] != 1 || W[0] != 1 || P[0] != 0 || K > 160 || gvol > 1 << 29 || N > 1 << 24 || F > 4096) return best;
-  for (const int along : {0, 1}) {
+  const long long K = (long long)C * W[1] * W[2];
+  if (K > 160 || F > 4096) return best;
+  for (const bool along : {false, true}) {
     FewGradPlan pl;
     pl.tm = F > 32 ? 4 : 2, pl.tk = (int)ceil_div(K, 32);
     FewParams &p = pl.p.at;
-    p.C = C, p.F = F, p.K = (int)K;
-    p.X1 = X[1], p.X2 = X[2], p.G2 = G[2], p.gvol = (int)gvol;
-    p.S1 = S[1], p.S2 = S[2], p.D1 = D[1], p.D2 = D[2], p.P1 = P[1], p.P2 = P[2], p.W1 = W[1], p.W2 = W[2];
-    p.m_tiles = (int)ceil_div(F, 16 * pl.tm), p.along = along, p.lead = -1;
-    if (p.m_tiles > cus) continue;
-    const long long rows = along ? 1 : std::min<long long>(G[1], ceil_div(kPositions - 1, G[2]) + 1), columns = along ? std::min(kPositions, G[2]) : G[2];
-    const long long patch_rows = (rows - 1) * S[1] + (long long)(W[1] - 1) * D[1] + 1, needed = (columns - 1) * S[2] + (long long)(W[2] - 1) * D[2] + 1;
-    long long pitch = needed;
-    if (needed > 64) p.lead = (4 - P[2] % 4) % 4, pitch = ceil_div(p.lead + needed, 4) * 4;
-    if (patch_rows > kLds || pitch > kLds || C * patch_rows * pitch * 8 > kLds) continue;
-    p.patch_rows = (int)patch_rows, p.pitch = (int)pitch, p.patch = (int)ceil_div(C * patch_rows * pitch, 4) * 4;
-    if (few_lds(pl) > (size_t)kLds) continue;
-    p.run_tiles = (int)ceil_div(along ? G[2] : gvol, kPositions), p.sample_tiles = p.run_tiles * (along ? G[1] : 1);
-    if ((long long)N * p.sample_tiles > 1 << 30) continue;
-    p.items = N * p.sample_tiles;
-    p.by_sample = make_fastdiv((unsigned)p.sample_tiles), p.by_run = make_fastdiv((unsigned)p.run_tiles), p.by_row = make_fastdiv((unsigned)G[2]);
-    p.by_patch_rows = make_fastdiv((unsigned)patch_rows), p.by_window = make_fastdiv((unsigned)(W[1] * W[2])), p.by_w2 = make_fastdiv((unsigned)W[2]);
+    if (!few_geometry(p, N, C, F, X, G, W, S, D, P, 16 * pl.tm, kPositions, along) || p.m_tiles > cus || few_lds(pl) > (size_t)kFewLds) continue;
     pl.p.splits = std::max(1, std::min(p.items, cus / p.m_tiles));
-    const double rounds = (double)ceil_div(p.items, pl.p.splits), requests = (double)(C * patch_rows * (p.lead < 0 ? 1 : ceil_div(pitch, 256) + (X[2] % 4 != 0)) + 8 * pl.tm);
+    const double rounds = (double)ceil_div(p.items, pl.p.splits), requests = (double)(few_requests(p) + 8 * pl.tm);
     pl.time = 19.1 + rounds * (0.785 + 0.161 * pl.tm * pl.tk + 0.0157 * requests) + 0.518e-6 * 8.0 * (double)pl.p.splits * F * (double)K;
     if (best.tm == 0 || pl.time < best.time) best = pl;
   }
@@ -342,7 +324,7 @@ int launch_few_wgrad(const FewGradPlan &pl, const void *grad, const void *x, voi
   ScopedTiming timed(TAG_CONV_WGRAD);
 #define MG_FEW_GRAD(TM, TK)                                                                                                              \
   if (pl.tm == TM && pl.tk == TK) {                                                                                                 \
-    static const hipError_t allowed = hipFuncSetAttribute((const void *)few_wgrad_kernel<TM, TK>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds); \
+    static const hipError_t allowed = hipFuncSetAttribute((const void *)few_wgrad_kernel<TM, TK>, hipFuncAttributeMaxDynamicSharedMemorySize, kFewLds); \
     MG_HIP(allowed);                                                                                                                \
     hipLaunchKernelGGL((few_wgrad_kernel<TM, TK>), dim3((unsigned)(p.splits * p.at.m_tiles)), dim3(64 * kWaves), few_lds(pl), s, p);      \
   }

@@ -88,17 +88,6 @@ __global__ void __launch_bounds__(256) product_pack_kernel(const ProductParams p
   }
 }
 
-// Sixteen bytes a lane from a buffer straight into LDS, the lanes' pieces one behind the other from byte `to` on.
-// Whoever reads it waits with landed() (__syncthreads() would do too; what must not come in between are waits for
-// these loads in front of other LDS reads, and the compiler puts none there).
-__device__ __forceinline__ void load_to_lds(__amdgpu_buffer_rsrc_t buffer, unsigned lane_at, unsigned at, unsigned to) {
-  typedef __attribute__((address_space(3))) void *LdsPointer;
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(buffer, (LdsPointer)(unsigned long long)to, 16, (int)lane_at, (int)at, 0, 0);
-}
-
-// Every load of this wave has landed, and its LDS reads are done; then all waves of the block are here.
-__device__ __forceinline__ void landed() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
 // The tile'th tile: groups of four row tiles run along all columns, so that the 32 tiles of one XCD's blocks touch
 // four row tiles and eight column tiles.
 struct TilePlace {
@@ -174,7 +163,7 @@ __global__ void __launch_bounds__(512, 2) product_gemm_kernel(const ProductParam
     const int panel = k / 3;
     const unsigned piece = (unsigned)(wave + k % 3 * 8) * 1024u;
     const unsigned at = (unsigned)(panel < PM ? panel : panel - PM) * (unsigned)panel_bytes + (unsigned)ahead.step * kProductPanelBytes + piece;
-    load_to_lds(panel < PM ? a_buf : b_buf, lane_at, at, lds_base + (unsigned)stage * STAGE + (unsigned)panel * kProductPanelBytes + piece);
+    to_lds<16>(panel < PM ? a_buf : b_buf, lane_at, at, lds_base + (unsigned)stage * STAGE + (unsigned)panel * kProductPanelBytes + piece);
   };
   auto step_ahead = [&] {
     if (!ahead.live) return;

@@ -315,7 +315,9 @@ __global__ void __launch_bounds__(512, 2) wgrad_split_kernel(const WgradSplitPar
                   into = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, x[px == 0 && j % 2 != 0 ? 3 : px]),
                                                                  __builtin_bit_cast(bf16x8, g[i][pg]), onto, 0, 0, 0);
                 }
-                if (j > kOwnLow && (t == 2 || t == 3)) acc[j - 1][t - 2] += small[(j - 1) % 2][t - 2];
+                if constexpr (j > kOwnLow) {
+                  if (t == 2 || t == 3) acc[j - 1][t - 2] += small[(j - 1) % 2][t - 2];
+                }
                 if (j != LAST) {
                   if (t == 0) next_tap();
                   if (t == 0) read_x(0, j + 1), read_x(2, j + 1);
