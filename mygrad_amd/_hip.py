@@ -292,6 +292,7 @@ KERNEL_TAGS = {
     18: "sum_over",
     19: "permute",
     20: "batched_product",
+    21: "gated",
 }
 
 

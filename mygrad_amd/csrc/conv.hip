@@ -3102,7 +3102,7 @@ int conv_wgrad_impl(const Geometry &g, const Plan &pl, const void *grad, const v
   wp.shift_from = staged || pl.depth == g.C ? 1 << 30 : pl.depth - 16;
   wp.col_shift = pl.depth - g.C;
   {
-    ScopedTiming timed(TAG_CONV_WGRAD);
+    ScopedTiming timed(wp.gate != nullptr ? TAG_GATED : TAG_CONV_WGRAD);
     bool launched = false;
     if (pl.table_rows) {
 #define MG_LAUNCH_TABLE(TT, BM, BN, BK, WM, WN)             \

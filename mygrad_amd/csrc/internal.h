@@ -69,6 +69,7 @@ enum KernelTag {
   TAG_SUM_OVER = 18,
   TAG_PERMUTE = 19,
   TAG_BATCHED_PRODUCT = 20,
+  TAG_GATED = 21,  // the single-precision filter gradient behind one on parts: seldom anything to do
 };
 void timing_begin(int tag);
 void timing_end();

@@ -1771,6 +1771,20 @@ def test_which_filter_gradients_run_on_three_bf16_parts(abi, rule):
     assert np.all(dw[(slice(None), slice(None), *centre)] == x_shape[0] * np.prod(grid))
 
 
+def test_launches_behind_filter_gradients_on_parts_are_timed_apart(abi):
+    from mygrad_amd import _hip
+
+    x, g = np.ones((64, 64, 56, 56), np.float32), np.ones((64, 64, 56, 56), np.float32)
+    _hip.timing_enable(True)
+    try:
+        abi.conv_wgrad(g, x, (64, 64, 3, 3), (1, 1), (1, 1), (1, 1))
+        assert _hip.last_plan().endswith("three bf16 parts")
+        kernels = [kernel for kernel, _ in _hip.timing_read() if kernel != "copy"]
+    finally:
+        _hip.timing_enable(False)
+    assert kernels == ["conv_wgrad", "gated", "wgrad_reduce"]
+
+
 # (x, w, stride, padding, dilation, shape): forward passes with few terms on three bf16 parts (10 * (16 filters) + 16 positions of a wave)
 FEW_TERMS = [
     ((3, 3, 33, 45), (64, 3, 7, 7), (2, 2), (3, 3), (1, 1), 43),    # a first layer; the last tile of a plane is short
