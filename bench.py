@@ -449,8 +449,13 @@ class Step:
             self.scale = 1e-9
 
     def passes(self):
-        """(label, callable, key of the pass in self.work) for each pass of a convolution or pooling step."""
-        lib, check, d = self.lib, self.check, self.desc
+        """(label, callable, key of the pass in self.work) for each pass of a convolution, product or pooling step."""
+        lib, check = self.lib, self.check
+        if self.wl["kind"] == "matmul":
+            return [("fwd", lambda: check(lib.mg_matmul(self.code, *self.dims, self.w.ptr, self.x.ptr, self.out.ptr)), "conv_fwd"),
+                    ("dx", lambda: check(lib.mg_matmul_dx(self.code, *self.dims, self.g.ptr, self.w.ptr, self.dx.ptr)), "conv_dgrad"),
+                    ("da", lambda: check(lib.mg_matmul_da(self.code, *self.dims, self.g.ptr, self.x.ptr, self.dw.ptr)), "conv_wgrad")]
+        d = self.desc
         if self.wl["kind"] == "conv":
             out = [("fwd", lambda: check(lib.mg_conv_fwd(d, self.x.ptr, self.w.ptr, self.out.ptr)), "conv_fwd")]
             if not self.wl.get("constant_input"):
@@ -483,9 +488,8 @@ class Step:
             check(lib.mg_matmul_batched(self.code, B, K, M, N, 1, 0, self.w.ptr, self.g.ptr, self.dx.ptr))  # a^T @ grad
             return
         if self.wl["kind"] == "matmul":
-            check(lib.mg_matmul(self.code, *self.dims, self.w.ptr, self.x.ptr, self.out.ptr))
-            check(lib.mg_matmul_dx(self.code, *self.dims, self.g.ptr, self.w.ptr, self.dx.ptr))
-            check(lib.mg_matmul_da(self.code, *self.dims, self.g.ptr, self.x.ptr, self.dw.ptr))
+            for _, fn, _ in self.passes():
+                fn()
             return
         if self.wl["kind"] == "permute":
             item = 4 if self.wl["dtype"] == "f32" else 8
@@ -558,7 +562,7 @@ def run_gpu(name, steps, warmup, prewarm=None, time_every=None):
         _hip.synchronize()
         prewarmed += 10
     pass_peak = {}
-    if step.wl["kind"] == "conv":
+    if step.wl["kind"] in ("conv", "matmul"):
         for _, fn, key in step.passes():
             fn()
             pass_peak[key] = peak_of(_hip.last_plan(), step.peak)

@@ -170,6 +170,13 @@ def test_which_products_run_on_three_bf16_parts(abi, sizes, parts):
         assert ("three bf16 parts" in _hip.last_plan()) == expected
 
 
+def test_benchmark_prices_products_on_parts_against_their_own_peak():
+    import bench
+
+    kernels = bench.run_gpu("mm4k", 2, 1, prewarm=0.0)["kernels"]
+    assert all(0 < kernels[key]["frac"] < 1 for key in ("conv_fwd", "conv_dgrad", "conv_wgrad")), kernels
+
+
 BATCHED = [(1, 1, 1, 1), (3, 16, 16, 16), (5, 17, 3, 33), (2, 1, 70, 1), (300, 8, 8, 8), (7, 64, 40, 48), (4, 33, 6, 2), (2, 5, 0, 4),
            (3, 100, 129, 50),
            # 32 x 32 results or more per pair: 64 x 64 tiles staged in LDS -- whole tiles, ragged edges in M, N
