@@ -209,6 +209,7 @@ __global__ void __launch_bounds__(64 * kWaves, 2) few_wgrad_kernel(const FewGrad
       for (int e = 0; e < 8; e += 2) split_pair(raw[e], raw[e + 1], h, m, l, low[r]), widen(widest[r], raw[e], raw[e + 1]);
     };
     item = first_item;
+    __syncthreads();  // the sums, which lie where the loads go, have been read
     request(item, 0);
     landed();
     for (int buf = 0; item < p.items; buf ^= 1) {
