@@ -16,8 +16,15 @@ __device__ __forceinline__ void reduce_single(const WgradSums &single, float *dw
     const float *const from = single.partial + (long long)f * single.ct + column;
     const long long stride = (long long)F * single.ct;
     const int per = (single.splits + single.runs - 1) / single.runs;
-    float sum = sum_in_order(from, stride, min(per, single.splits));
-    for (int first = per; first < single.splits; first += per) sum += sum_in_order(from + first * stride, stride, min(per, single.splits - first));
+    // (seldom: not with sum_in_order()'s sixteen loads at a time, whose registers would halve the waves of the usual reduction beside it)
+    float sum = 0.0f;
+    for (int first = 0; first < single.splits; first += per) {
+      const int last = min(first + per, single.splits);
+      float run = from[first * stride];
+#pragma unroll 8
+      for (int k = first + 1; k < last; ++k) run += from[k * stride];
+      sum = first == 0 ? run : sum + run;
+    }
     dw[i] = sum;
   }
 }
