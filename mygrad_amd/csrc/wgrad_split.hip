@@ -49,7 +49,7 @@ __global__ void __launch_bounds__(512, 2) wgrad_split_kernel(const WgradSplitPar
   constexpr int GRAD = KW * 4 * 2 * FW * kLoc;  // pieces of grad: [16 filters][position][part][filter]; then the column tiles' rings [row][location][part][channel]
   const int lane = (int)threadIdx.x & 63, l16 = lane & 15, lk = lane >> 4, wave = uniform((int)threadIdx.x >> 6);
   const int fw = wave / (CW * KW), cw = wave / KW % CW, kq = wave % KW;
-  const int grid = (int)gridDim.x, place = grid % 8 == 0 ? (int)(blockIdx.x & 7) * (grid / 8) + (int)(blockIdx.x >> 3) : (int)blockIdx.x;
+  const int grid = (int)gridDim.x, xcd = (int)(blockIdx.x & 7), place = xcd * (grid / 8) + min(xcd, grid % 8) + (int)(blockIdx.x >> 3);
   const int tile = place % p.tiles, split = place / p.tiles, f0 = tile % p.f_tiles * FT, first_columns = tile / p.f_tiles * CW;
   const int first_stage = (int)(p.total * split / p.splits), last_stage = (int)(p.total * (split + 1) / p.splits);
   const int row_pieces = p.row_locs * kLoc, group_pieces = p.new_rows * row_pieces, ring_pieces = (p.depth + 2) * group_pieces;
