@@ -2455,8 +2455,10 @@ int build_wgrad_plan(const Geometry &g, Plan &pl) {
       pl.wsplit = plan_wgrad_split(g.N, g.C, g.F, g.X, g.G, g.W, g.S, g.D, g.P, cus);
       // With a tenth in favour of the single-precision kernels 106 of 362 drawn layers of 4 - 30 GFLOP run on parts, 1.18 times as fast in
       // the mean, 3 % slower or more in 8 of them: most of those with eight or nine taps to a tile, few with fewer, of which the tile's
-      // other products are of no use ((69,205,38,11) * (481,205,3,1) 755 us on parts, 168 without).
-      if (!least && pl.wsplit.time > 0.9 * (pl.table_rows ? single_time : 1.05 * single_time)) pl.wsplit = WgradSplitPlan();
+      // other products are of no use ((69,205,38,11) * (481,205,3,1) 755 us on parts, 168 without).  Of 74 drawn ones with stages of one quad,
+      // whose modelled time is the less certain one, five run there, 1.12 times as fast in the mean, the worst of them even (of 80 others nine, two of them 3 - 4 % slower); of three
+      // 3 x 3 layers of stride 2 (128,128,27,27) * (256,128,3,3) does (120 us, 128 without), (128,256,13,13) * (512,256,3,3) not (140 and 134).
+      if (!least && pl.wsplit.time > 0.9 * (pl.table_rows || pl.wsplit.p.quads == 1 ? single_time : 1.05 * single_time)) pl.wsplit = WgradSplitPlan();
     }
     // Few terms to a filter: a ninth in favour of the others.  Most of 91 drawn layers stay ((32,3,224,224) * (64,3,3,3) 101 us and 140 there:
     // 27 terms do not pay for their splitting); MYGRAD_HIP_FEW as in few_applies.

@@ -468,7 +468,9 @@ size_t lds_bytes(const WgradSplitPlan &pl) {
 // Every shape of the kernel and split of K that the problem fits, by modelled time, in us: fitted to 1700 timed (filter gradient,
 // shape, quads) of 480 layers drawn over the range of sizes, 8 in 10 within 9 % of it; what it chooses is 0.5 % slower than the best
 // in the mean.  A tick takes 2.1 - 3.3 us; one quad a row, of several to a stage, is left out: lines of memory are then touched by
-// eight walks, up to twice the modelled time.
+// eight walks, up to twice the modelled time.  Where a stage is one quad (wide patches: strides), what it takes is the lines, 128 bytes each,
+// that its sixteen bytes a row lie in, at 8 TB/s, where that is more: 9 in 10 of 77 layers within 14 % of it, two thirds more than modelled without
+// ((128,64,55,55) * (128,64,3,3) stride 2: 104 us modelled, 152 measured, 139 on the single-precision kernel).
 WgradSplitPlan plan_wgrad_split(int N, int C, int F, const int *X, const int *G, const int *W, const int *S, const int *D, const int *P, int cus) {
   WgradSplitPlan best;
   // MYGRAD_HIP_SPLIT_TILE="waves along filters,column tiles,quads of a row" (tests; part of the plan's key)
@@ -508,13 +510,20 @@ WgradSplitPlan plan_wgrad_split(int N, int C, int F, const int *X, const int *G,
       p.tiles = (int)tiles;
       p.total = (long long)p.octets * p.strips * p.stages;
       if (p.total >= 1ll << 30 || tiles >= 1ll << 16) continue;
+      double lines_time = 0;
+      if (quads == 1) {
+        const int planes_of = 8 >> std::min(p.seg_shift, 3), runs = 8 / planes_of;  // of an octet; of a row
+        auto lines = [&](int run, int row) { return planes_of * std::min(runs * (1 + (run * 4 - 4) / 128.0), row * 4 / 128.0 + 1); };
+        lines_time = 0.12e-6 * 128 * (double)p.total *
+                     (F * lines(4, G[2]) + std::min(C, 16 * pl.cw) * (double)ceil_div(p.columns, pl.cw) * lines(4 * p.x_quads, X[2]) * p.new_rows * (1 + (double)p.depth / p.stages));
+      }
       const long long most = std::min<long long>(p.total, std::max<long long>(1, 6 * cus / tiles));
       for (long long splits = 1; splits <= most; ++splits) {
         const double rounds = (double)ceil_div(splits * tiles, cus), stages = (double)ceil_div(p.total, splits);
         const double walks = p.total % (splits * p.stages) == 0 ? stages / p.stages : stages / p.stages + 1.0;
         const double tick = 1.19 + 0.121 * tasks + 0.065 * pl.cw * p.new_rows;
         const double traffic = (double)(splits * tiles) * (32 * pl.fw * pl.cw * kColumns) * 8e-6;  // of the partial sums, MB
-        pl.time = 11.9 + rounds * (11.6 + 0.98 * walks + (stages + walks * p.depth) * tick) + 0.102 * traffic;
+        pl.time = 11.9 + rounds * (11.6 + 0.98 * walks) + std::max(lines_time, rounds * (stages + walks * p.depth) * tick) + 0.102 * traffic;
         p.splits = (int)splits;
         if (best.fw == 0 || pl.time < best.time) best = pl;
       }

@@ -1754,6 +1754,7 @@ SPLIT_GRADIENT_RULES = [
     ((8, 16, 32, 64, 64), (32, 16, 3, 3, 3), (1, 1, 1), (1, 1, 1), True),
     ((16, 64, 28, 28), (64, 64, 3, 3), (1, 1), (1, 1), False),         # 0.9 GFLOP
     ((69, 205, 38, 11), (481, 205, 3, 1), (1, 1), (1, 0), False),      # three taps of a tile's nine
+    ((128, 64, 55, 55), (128, 64, 3, 3), (2, 2), (1, 1), False),       # stages of one quad, seven of which share a row's lines of memory
 ]
 
 
