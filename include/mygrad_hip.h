@@ -141,7 +141,10 @@ int mg_event_destroy(void *event);
  * records in launch order, sets *count to the number recorded and starts over.
  * Tags: 1 conv forward, 2 conv dgrad, 3 conv wgrad, 4 wgrad split-K reduction,
  * 5 filter packing, 6 max-pool forward, 7 max-pool backward, 8 device copy,
- * 9 element-wise kernel, 10 whole-array sum. */
+ * 9 element-wise kernel, 10 whole-array sum, 11 - 14 batch norm (statistics, application, the
+ * gradients' sums, their application), 15 and 16 repeat and its gradient, 17 window copy, 18 sum over
+ * axes, 19 permutation, 20 batched product, 21 the single-precision filter gradient behind one on
+ * three bf16 parts (which returns at once as a rule). */
 int mg_timing_enable(int on);
 int mg_timing_read(int32_t *tags, float *ms, int capacity, int *count);
 /* Suspends (1) or resumes (0) the recording without waiting for the stream and without

@@ -1579,7 +1579,8 @@ bool split_tables(Plan &pl, Tables &t, const SplitLayout &lay, int bn, const Pha
 // Whether a forward pass runs on few_split.hip's kernel: where its modelled time is the smaller one, with an eighth in favour of the
 // others, whose time (fitted to 80 layers of 0.2 - 30 GFLOP and up to 192 terms, 8 in 10 within 18 %) is the less certain one, and from 0.4
 // GFLOP on (below, 14 - 37 us, a few microseconds are in it either way).  Those of the 80 that it takes are 1.03 - 1.7 times as fast; most of
-// the rest are layers of few terms, bound by their stores: (111,1,211,211) * (11,1,3,3) 27.5 us and 44.4 there.
+// the rest are layers of few terms, bound by their stores: (111,1,211,211) * (11,1,3,3) 27.5 us and 44.4 there.  (Of 80 that it took among
+// others drawn later, 1.2 times as fast in the mean, seven were 3 % slower or more, of 0.4 - 1.3 GFLOP, by 3.3 us at most.)
 // MYGRAD_HIP_FEW=0: none does; MYGRAD_HIP_FEW=10 tm + tn: every one that can, in that shape (tests; part of the plan's key).
 bool few_applies(const Geometry &g, Plan &pl) {
   const char *shape = getenv("MYGRAD_HIP_FEW");
@@ -2456,7 +2457,7 @@ int build_wgrad_plan(const Geometry &g, Plan &pl) {
       // With a tenth in favour of the single-precision kernels 106 of 362 drawn layers of 4 - 30 GFLOP run on parts, 1.18 times as fast in
       // the mean, 3 % slower or more in 8 of them: most of those with eight or nine taps to a tile, few with fewer, of which the tile's
       // other products are of no use ((69,205,38,11) * (481,205,3,1) 755 us on parts, 168 without).  Of 74 drawn ones with stages of one quad,
-      // whose modelled time is the less certain one, five run there, 1.12 times as fast in the mean, the worst of them even (of 80 others nine, two of them 3 - 4 % slower); of three
+      // whose modelled time is the less certain one, five run there, 1.12 times as fast in the mean, the worst of them even (of 80 others seven, two of them 3 - 4 % slower); of three
       // 3 x 3 layers of stride 2 (128,128,27,27) * (256,128,3,3) does (120 us, 128 without), (128,256,13,13) * (512,256,3,3) not (140 and 134).
       if (!least && pl.wsplit.time > 0.9 * (pl.table_rows || pl.wsplit.p.quads == 1 ? single_time : 1.05 * single_time)) pl.wsplit = WgradSplitPlan();
     }

@@ -22,7 +22,7 @@ __device__ __forceinline__ FewTile few_tile(const FewParams &p, int item) {
 }
 
 // Row `line` (of channel line / patch_rows) of the tile's patch into LDS, from byte `patch` on: sixteen bytes a lane (requests are what the
-// kernels wait for: 4 bytes a lane, four times as many, took the filter gradient of a 3 x 7 x 7 layer 217 us, 158 so), the four columns that
+// kernels wait for: 4 bytes a lane, four times as many, took the filter gradient of a 3 x 7 x 7 layer 217 us, 158 so on the same device), the four columns that
 // the end of a row cuts by themselves.
 __device__ __forceinline__ void few_request_line(const FewParams &p, const FewTile &t, int line, unsigned patch, int lane) {
   const int c = (int)p.by_patch_rows.div((unsigned)line), r = t.row * p.S1 - p.P1 + line - c * p.patch_rows;

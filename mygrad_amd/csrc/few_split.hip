@@ -1,7 +1,7 @@
 // Forward pass of single-precision layers with few terms to a sum, such as a first layer's 3 x 7 x 7, on the bf16 matrix
 // instructions: see conv_split.hip for the arithmetic and its accuracy (two accumulators).
 //
-// What bounds it: (64,3,225,225) * (64,3,7,7), stride 2, 15.4 GFLOP, takes 138 us (184 - 187 with one position per lane on the
+// What bounds it: (64,3,225,225) * (64,3,7,7), stride 2, 15.4 GFLOP, takes 136 - 147 us (184 - 187 with one position per lane on the
 // single-precision instruction); 100 - 110 of them without its loads and stores (92 GFLOP of parts and 8 % of dead terms, 46 us at
 // the instruction's rate: eight waves to a unit, which all wait for a tile's patch, hide little of each other's latency), 69 with nothing
 // but loads and stores (209 MB; loads of four bytes a lane, 141 us in all).  (48,4,123,123) * (84,4,5,5) 186 -> 157, (25,24,6716) * (178,24,5) 118 -> 82.

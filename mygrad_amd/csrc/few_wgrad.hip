@@ -1,9 +1,11 @@
 // Filter gradient of single-precision layers with few terms to a filter, such as a first layer's 3 x 7 x 7, on the bf16
 // matrix instructions: see conv_split.hip for the arithmetic and its accuracy (two accumulators), few_split.hip for the patch.
 //
-// What bounds it: (64,3,225,225) * (64,3,7,7), stride 2, 15.4 GFLOP, takes 158 - 165 us with its reduction and the single-precision kernel that
-// returns at once (227 there, 68 TFLOP/s): 25 tiles a block of about 5.5 us each, of which the products are 1.8 at the
-// instruction's rate; the modelled time puts 1.5 of the rest on the requests of the next tile.  Four bytes a request and lane it took 217.  (112,44,3493) * (237,44,3) 402 -> 302.  Error against 64 bits (2-norm), normal values: 2.4e-7 (single precision 1.0e-6).
+// What bounds it: (64,3,225,225) * (64,3,7,7), stride 2, 15.4 GFLOP, takes 149 - 166 us, its reduction and the single-precision kernel that
+// returns at once 10 (227 there, 68 TFLOP/s): 25 tiles a block of about 5.5 us each, of which the products are 1.8 at the
+// instruction's rate; the modelled time puts 1.5 of the rest on the requests of the next tile.  Four bytes a request and lane it took 217, where
+// this took 158.  The matrix pipes are 32 % busy, seven vector instructions to a product.
+// (112,44,3493) * (237,44,3) 402 -> 302.  Error against 64 bits (2-norm), normal values: 2.4e-7 (single precision 1.0e-6).
 //
 // What the parts cannot represent (a sum that is not finite, or smaller than what lost bits of its operands can have been worth) sets a word, and the
 // single-precision kernel behind computes the gradient (see wgrad_split.h).

@@ -7,10 +7,10 @@
 // go into LDS as they lie, without a register or an address in between, and a wave's operands are its rows' pieces
 // of 16 bytes side by side, free of bank conflicts in either orientation of the matrix.
 //
-// What bounds it: 4096 x 4096 x 4096, 137.4 GFLOP, takes 55 us for the packing (128 MB read, 192 MB written, 5.7
-// TB/s), 490 - 500 for the products (825 GFLOP of parts, 1.66 PFLOP/s) and 4 for the pass behind them: 555 - 570,
-// single precision 965 - 1000.  The matrix pipes are 72 % busy at 2.04 GHz, what the device's power allows beside them, LDS
-// 18 %, when a wave requests its nine loads at once (535 us); spread over two sections of a step 490.
+// What bounds it: 4096 x 4096 x 4096, 137.4 GFLOP, takes 56 us for the packing (134 MB read, 202 MB written, 6.0
+// TB/s), 495 - 513 by device for the products (825 GFLOP of parts, 1.61 - 1.67 PFLOP/s; 570 - 590 in the first passes from idle) and
+// 5 for the pass behind them: 560 - 590, single precision 965 - 1000.  The matrix pipes are 80 % busy at 1.9 GHz, what the device's
+// power allows beside them, LDS 20 %.
 // Error against 64 bits (2-norm), normal values: 4.0e-7, single precision 1.15e-6; at 1024 terms 8.6e-8 and 2.9e-7, at 64
 // 5.0e-8 and 1.05e-7.
 #include "product_split.h"
